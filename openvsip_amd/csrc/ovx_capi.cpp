@@ -203,7 +203,7 @@ static HierArgs hier_args(const LineFFT &f)
   return a;
 }
 
-static bool offsets_fit(long rows_per_block, long ld)
+bool offsets_fit(long rows_per_block, long ld)
 {
   return (unsigned long)rows_per_block * (unsigned long)std::max(ld, 0l) * 8ul < (1ul << 32);
 }
@@ -687,6 +687,13 @@ static int variant_of(unsigned flags, long n = 0, long rows = 0)
   return LineFFT::default_variant(n);
 }
 
+// Variant of a real transform's half-length line: the first register-Stockham
+// configuration, which the one-pass real kernels are built on.
+static int real_variant(long h)
+{
+  return hier_supported(h) ? 1 : 0;
+}
+
 extern "C" int ovx_supported_length(long n)
 {
   if (n >= 1 && n <= kMaxRowN) return row_variants((int)n) > 0 ? 1 : 0;
@@ -818,7 +825,11 @@ extern "C" int ovx_fftm_real_plan_create(ovx_plan *plan, long rows, long cols, i
   p->flags = flags;
   if (n > 0) {
     const long h = n / 2;
-    int st = p->line.init(h, variant_of(flags, h, axis == OVX_ROW ? rows : cols));
+    // the one-pass real kernels are built on the register-Stockham
+    // configurations, so lengths that have one use it unless the caller names
+    // another variant
+    const int pick = variant_of(flags);
+    int st = p->line.init(h, (flags >> 8) & 0xffu ? pick : real_variant(h));
     if (st) return st;
     if ((st = p->wtab.alloc((size_t)(h / 2 + 1) * 8))) return st;
     hipError_t e = launch_unit_roots(n, h / 2 + 1, (float2 *)p->wtab.p, nullptr);
@@ -877,11 +888,37 @@ static int real_lines(ovx_plan p, long in_s0, long in_s1, long out_s0, long out_
   return OVX_OK;
 }
 
+// One launch for the whole call where the half-length line has a
+// register-Stockham configuration: z is the real side (read or written as
+// pairs), c or cr / ci the complex side.
+static int real_fused(ovx_plan p, const RealLines &g, const void *z, const void *c, const float *cr, const float *ci,
+                      hipStream_t s)
+{
+  if (!offsets_fit(p->line.rc.rows_per_block, std::max(g.ldz, g.ldc)))
+    return fail(OVX_ERR_UNSUPPORTED, "row stride too large for 32-bit buffer offsets");
+  RealArgs a;
+  a.z = (float2 *)z;
+  a.ldz = g.ldz;
+  a.c = (float2 *)c;
+  a.cr = (float *)cr;
+  a.ci = (float *)ci;
+  a.ldc = g.lines > 1 ? g.ldc : 0;
+  a.lines = g.lines;
+  a.tw = (const float2 *)p->line.tw.p;
+  a.wt = (const float2 *)p->wtab.p;
+  a.scale = p->scale;
+  hipError_t e = launch_row_real(p->line.rc, g.fwd ? -1 : +1, a, s);
+  return e == hipSuccess ? OVX_OK : hip_fail(e, "real Fftm launch");
+}
+
 // The device body: forward = h-point complex transform of the real line read
 // as pairs, then the r2c post-pass; inverse = c2r pre-pass, then the inverse
-// h-point transform in place.  `ldc` is the complex side's line stride.
+// h-point transform in place (both in one launch where real_fused has one).
+// `ldc` is the complex side's line stride.
 static int real_run(ovx_plan p, const RealLines &g, const void *din, void *dout, long ldc, hipStream_t s)
 {
+  if (p->line.kind == LineFFT::LDS)
+    return g.fwd ? real_fused(p, g, din, dout, nullptr, nullptr, s) : real_fused(p, g, dout, din, nullptr, nullptr, s);
   if (g.fwd) {
     int r = p->line.transform(-1, (const float2 *)din, g.ldz, (float2 *)dout, ldc, g.lines, 1.0f, s);
     if (r) return r;
@@ -1242,6 +1279,7 @@ extern "C" int ovx_fftm_r2c_split(ovx_plan p, const void *in, long in_s0, long i
   hipStream_t s = (hipStream_t)stream;
   const long hc = g.h + 1;
   auto run = [&](const void *din, SplitOut o) -> int {
+    if (p->line.kind == LineFFT::LDS) return real_fused(p, g, din, nullptr, o.re, o.im, s);
     // the h-point transform into the workspace, then the post-pass writes
     // the split spectrum straight from it
     int r = p->split_ws.alloc((size_t)g.lines * hc * 8);
@@ -1280,6 +1318,7 @@ extern "C" int ovx_fftm_c2r_split(ovx_plan p, const void *in_re, const void *in_
   hipStream_t s = (hipStream_t)stream;
   const long hc = g.h + 1;
   auto run = [&](SplitIn i, void *dout) -> int {
+    if (p->line.kind == LineFFT::LDS) return real_fused(p, g, dout, nullptr, i.re, i.im, s);
     // the pre-pass reads the split spectrum, then the inverse h-point
     // transform in place on the output
     hipError_t e = launch_c2r_pre_split(i.re, i.im, g.ldc, (float2 *)dout, g.ldz, g.lines, g.h,

@@ -49,6 +49,23 @@ hipError_t launch_row_fastconv_split(const RowConfig &cfg, const float *xr, cons
                                      const float2 *w, long ldw, float *yr, float *yi, long ldy, long rows,
                                      const float2 *tw, float scale, hipStream_t s);
 
+// Real <-> complex rows in one pass: `lines` real lines of 2 * cfg.n values,
+// read or written as cfg.n complex pairs at z (line stride ldz pairs), and
+// their half spectra of cfg.n + 1 values at c or, split, at cr / ci (line
+// stride ldc values).  dir -1: z to spectrum; +1: spectrum to z.  tw: the
+// configuration's twiddles; wt[k] = exp(-2 pi i k / (2 cfg.n)), k <= cfg.n / 2.
+struct RealArgs {
+  float2 *z = nullptr;
+  long ldz = 0;
+  float2 *c = nullptr;
+  float *cr = nullptr, *ci = nullptr;
+  long ldc = 0;
+  long lines = 0;
+  const float2 *tw = nullptr, *wt = nullptr;
+  float scale = 1.0f;
+};
+hipError_t launch_row_real(const RowConfig &cfg, int dir, const RealArgs &a, hipStream_t s);
+
 // Forward twiddle table of a radix plan: tw[twoff_s + (r-1)*Ns + k] =
 // exp(-2 pi i r k / (Ns R_s)) evaluated in FP64 on the device, rounded to FP32.
 hipError_t launch_twiddles(const RadixPlan &plan, float2 *tw, hipStream_t s);

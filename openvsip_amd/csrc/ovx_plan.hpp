@@ -13,6 +13,8 @@ namespace ovx {
 int fail(int code, const char *fmt, ...);
 int hip_fail(hipError_t e, const char *what);
 int current_device();
+// whether rows_per_block lines at stride ld stay within 32-bit byte offsets
+bool offsets_fit(long rows_per_block, long ld);
 
 // Owning device allocation (hipMalloc / hipFree).
 struct DevBuf {

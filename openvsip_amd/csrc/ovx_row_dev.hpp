@@ -102,4 +102,152 @@ __device__ __forceinline__ void row_fft_body(const float2 *__restrict__ in, long
                         tw, scale, row0, lrow, t, lds);
 }
 
+// ---------------------------------------------------------------- real transforms
+// A real line of n = 2N values is read as N complex pairs z; with Z = FFT_N(z)
+// and W = e^{-2 pi i/n} its spectrum is, for k = 0 .. N/2,
+//   X[k] = E + W^k O,  X[N-k] = conj(E - W^k O),
+//   E = (Z[k] + conj Z[N-k]) / 2,  O = -i (Z[k] - conj Z[N-k]) / 2
+// (Z[N] standing for Z[0]).  r2c_pair gives both from Z[k] and Z[N-k], c2r_pair
+// the way back: Z[k] = A + i C, Z[N-k] = conj(A - i C) with
+// A = X[k] + conj X[N-k], C = W^-k (X[k] - conj X[N-k]).
+__device__ __forceinline__ void r2c_pair(float2 zk, float2 zm, float2 w, float scale, float2 &xk, float2 &xm)
+{
+  const float2 e = make_float2(0.5f * (zk.x + zm.x), 0.5f * (zk.y - zm.y));
+  const float2 o = make_float2(0.5f * (zk.y + zm.y), -0.5f * (zk.x - zm.x));
+  const float2 wo = cmul(w, o);
+  const float2 d = csub(e, wo);
+  xk = cscale(cadd(e, wo), scale);
+  xm = cscale(make_float2(d.x, -d.y), scale);
+}
+__device__ __forceinline__ void c2r_pair(float2 xk, float2 xm, float2 w, float2 &zk, float2 &zm)
+{
+  const float2 a = make_float2(xk.x + xm.x, xk.y - xm.y);
+  const float2 c = cmulc(make_float2(xk.x - xm.x, xk.y + xm.y), w);
+  zk = make_float2(a.x - c.y, a.y + c.x);
+  zm = make_float2(a.x + c.y, c.x - a.y);
+}
+
+// The pairs (k, N-k) of one thread: k = t + T q for q < NQ, so that the thread
+// holds Z[k] itself (slot form) and finds Z[N-k] in another thread's upper
+// slots, through one LDS exchange of half the line.  The mirrored positions
+// N - k of a thread are at base(t) + T (NQ - 1 - q).  The middle k = N/2 of an
+// even N (its own mirror) is slot P/2 of thread 0.
+template <int N, int P>
+struct RealPairs {
+  static constexpr int T = N / P;
+  static constexpr int NQ = (P + 1) / 2;
+  static constexpr bool MID = P % 2 == 0;
+  static_assert(P % 2 == 0 || T == 1, "an odd number of values per thread only for one-thread lines");
+  __device__ static constexpr int mirror_base(int t) { return N - t - T * (NQ - 1); }
+  __device__ static constexpr int mirror_off(int q) { return T * (NQ - 1 - q); }
+};
+
+// Forward: real lines ix (as N complex pairs per line) to half spectra of
+// N + 1 values, times scale: iy stores element t + e of the spectrum at
+// st(v, e), iym element mirror_base(t) + e.  wt[k] = W^k, k <= N/2.  Geometry
+// contract as row_fastconv_io.
+template <int N, int P, typename IX, typename IY, typename LP>
+__device__ __forceinline__ void row_r2c_io(const IX &ix, const IY &iy, const IY &iym, long rows,
+                                           const float2 *__restrict__ tw, const float2 *__restrict__ wt, float scale,
+                                           long row0, int lrow, int t, LP lds)
+{
+  using E = Engine<N, P, (N / P <= 64)>;
+  using L = typename E::Layout;
+  using R = RealPairs<N, P>;
+  constexpr int T = E::T;
+  const bool valid = row0 + lrow < rows;
+  const rsrc_t rtw = make_rsrc(tw, (uint32_t)(E::plan.twtotal + 1) * 8u);
+  const rsrc_t rwt = make_rsrc(wt, (uint32_t)(N / 2 + 1) * 8u);
+  float2 v[P];
+#pragma unroll
+  for (int q = 0; q < P; ++q) v[q] = valid ? ix.ld((uint32_t)(T * q)) : make_float2(0.f, 0.f);
+  E::template fft<-1>(v, lds, t, rtw);
+  float2 w[R::NQ];
+#pragma unroll
+  for (int q = 0; q < R::NQ; ++q) w[q] = bload(rwt, (uint32_t)t * 8u, (uint32_t)(T * q) * 8u);
+#pragma unroll
+  for (int q = P / 2; q < P; ++q) lds_st(lds, L::idx(t + T * q), v[q]);
+  exchange_sync<(N / P <= 64)>();
+  float2 z[R::NQ];
+#pragma unroll
+  for (int q = 0; q < R::NQ; ++q) {
+    const int m = R::mirror_base(t) + R::mirror_off(q); // N - k, N itself for k = 0
+    z[q] = lds_ld(lds, L::idx(q == 0 && t == 0 ? N - 1 : m));
+  }
+  if (t == 0) z[0] = v[0];
+  if (!valid) return;
+#pragma unroll
+  for (int q = 0; q < R::NQ; ++q) {
+    float2 xk, xm;
+    r2c_pair(v[q], z[q], w[q], scale, xk, xm);
+    iy.st(xk, (uint32_t)(T * q));
+    iym.st(xm, (uint32_t)R::mirror_off(q));
+  }
+  if (R::MID && t == 0) {
+    float2 xk, xm;
+    r2c_pair(v[P / 2], v[P / 2], bload(rwt, 0u, (uint32_t)(N / 2) * 8u), scale, xk, xm);
+    iy.st(xk, (uint32_t)(N / 2));
+  }
+}
+
+// Inverse (unnormalised, times scale): half spectra of N + 1 values (ix at
+// t + e, ixm at mirror_base(t) + e; the imaginary parts of X[0] and X[N] are
+// ignored) to real lines, stored by iy as N complex pairs per line.
+template <int N, int P, typename IX, typename IY, typename LP>
+__device__ __forceinline__ void row_c2r_io(const IX &ix, const IX &ixm, const IY &iy, long rows,
+                                           const float2 *__restrict__ tw, const float2 *__restrict__ wt, float scale,
+                                           long row0, int lrow, int t, LP lds)
+{
+  constexpr bool WAVE = N / P <= 64;
+  using E = Engine<N, P, WAVE>;
+  using L = typename E::Layout;
+  using R = RealPairs<N, P>;
+  constexpr int T = E::T;
+  const bool valid = row0 + lrow < rows;
+  const rsrc_t rtw = make_rsrc(tw, (uint32_t)(E::plan.twtotal + 1) * 8u);
+  const rsrc_t rwt = make_rsrc(wt, (uint32_t)(N / 2 + 1) * 8u);
+  float2 v[P], xm[R::NQ], w[R::NQ], mid = make_float2(0.f, 0.f);
+  if (valid) {
+#pragma unroll
+    for (int q = 0; q < R::NQ; ++q) {
+      v[q] = ix.ld((uint32_t)(T * q));
+      xm[q] = ixm.ld((uint32_t)R::mirror_off(q));
+    }
+    if (R::MID && t == 0) mid = ix.ld((uint32_t)(N / 2));
+  } else {
+#pragma unroll
+    for (int q = 0; q < R::NQ; ++q) v[q] = xm[q] = make_float2(0.f, 0.f);
+  }
+#pragma unroll
+  for (int q = 0; q < R::NQ; ++q) w[q] = bload(rwt, (uint32_t)t * 8u, (uint32_t)(T * q) * 8u);
+  if (t == 0) v[0].y = xm[0].y = 0.f; // DC and Nyquist carry no imaginary part in a real signal
+#pragma unroll
+  for (int q = 0; q < R::NQ; ++q) {
+    float2 zk, zm;
+    c2r_pair(v[q], xm[q], w[q], zk, zm);
+    v[q] = zk;
+    const int m = R::mirror_base(t) + R::mirror_off(q);
+    if (q > 0) lds_st(lds, L::idx(m), zm);
+    else if (t > 0) lds_st(lds, L::idx(m), zm); // Z[N] of k = 0 is Z[0] itself
+  }
+  if (R::MID && t == 0) {
+    float2 zk, zm;
+    c2r_pair(mid, mid, bload(rwt, 0u, (uint32_t)(N / 2) * 8u), zk, zm);
+    lds_st(lds, L::idx(N / 2), zk);
+  }
+  exchange_sync<WAVE>();
+#pragma unroll
+  for (int q = R::NQ; q < P; ++q) v[q] = lds_ld(lds, L::idx(t + T * q));
+  exchange_sync<WAVE>();
+  E::template fft<+1>(v, lds, t, rtw);
+  if (scale != 1.0f) {
+#pragma unroll
+    for (int q = 0; q < P; ++q) v[q] = cscale(v[q], scale);
+  }
+  if (valid) {
+#pragma unroll
+    for (int q = 0; q < P; ++q) iy.st(v[q], (uint32_t)(T * q));
+  }
+}
+
 } // namespace ovx
