@@ -27,23 +27,44 @@ ROW = _lib.ROW
 COL = _lib.COL
 
 
-def _torch():
+# Bound on first use (the package imports without torch): the module, its
+# complex64, and a function giving the current stream's handle.  A call's own
+# Python work is what bounds the small transforms (a 2048-point Fft takes
+# 3.4 us on the device), and torch.cuda.current_stream() alone, which builds a
+# Stream object, was 1.5 us of it.
+_bound = None
+
+
+def _bind():
+    global _bound
     import torch
-    return torch
+    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    if raw is None:
+        def stream():
+            return torch.cuda.current_stream().cuda_stream
+    else:
+        device = torch.cuda.current_device
+
+        def stream():
+            return raw(device())
+    _bound = (torch, torch.complex64, stream)
+    return _bound
+
+
+def _torch():
+    return (_bound or _bind())[0]
 
 
 def _stream():
-    torch = _torch()
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    return (_bound or _bind())[2]()
 
 
 def _ptr(t):
-    return ctypes.c_void_p(t.data_ptr())
+    return t.data_ptr()
 
 
 def _check_tensor(t, name):
-    torch = _torch()
-    if t.dtype != torch.complex64:
+    if t.dtype is not (_bound or _bind())[1]:
         raise TypeError(f"{name} must be complex64 (complex<float>)")
     if not t.is_cuda:
         raise TypeError(f"{name} must be a GPU tensor")
@@ -118,13 +139,15 @@ class Fftm(_Plan):
                                          _flags(variant)))
 
     def __call__(self, x, out=None):
-        torch = _torch()
         _check_tensor(x, "input")
         if out is None:
-            out = torch.empty_like(x)
+            out = _torch().empty_like(x)
         _check_tensor(out, "output")
-        check(lib().ovx_fftm_out_of_place(self._h, _ptr(x), x.stride(0), x.stride(1), _ptr(out),
-                                          out.stride(0), out.stride(1), self.rows, self.cols, _stream()))
+        s, o = x.stride(), out.stride()
+        st = lib().ovx_fftm_out_of_place(self._h, x.data_ptr(), s[0], s[1], out.data_ptr(), o[0], o[1], self.rows,
+                                         self.cols, _stream())
+        if st:
+            check(st)
         return out
 
     def in_place(self, x):
@@ -152,8 +175,8 @@ class FftmReal(_Plan):
         return (self.rows // 2 + 1, self.cols)
 
     def __call__(self, x, out=None):
-        torch = _torch()
         if out is None:
+            torch = _torch()
             if self.direction == FFT_FWD:
                 shape = self.complex_shape()
                 dtype = torch.complex64
@@ -166,8 +189,11 @@ class FftmReal(_Plan):
                 out = torch.empty(shape[::-1], dtype=dtype, device=x.device).t()
         if not (x.is_cuda and out.is_cuda):
             raise ValueError("real Fftm tensors must live on the device")
-        check(lib().ovx_fftm_real_out_of_place(self._h, _ptr(x), x.stride(0), x.stride(1), _ptr(out),
-                                               out.stride(0), out.stride(1), self.rows, self.cols, _stream()))
+        s, o = x.stride(), out.stride()
+        st = lib().ovx_fftm_real_out_of_place(self._h, x.data_ptr(), s[0], s[1], out.data_ptr(), o[0], o[1],
+                                              self.rows, self.cols, _stream())
+        if st:
+            check(st)
         return out
 
 
@@ -178,12 +204,13 @@ class Fft(_Plan):
         check(lib().ovx_fft_plan_create(ctypes.byref(self._h), n, direction, scale, 0))
 
     def __call__(self, x, out=None):
-        torch = _torch()
         _check_tensor(x, "input")
         if out is None:
-            out = torch.empty_like(x)
-        check(lib().ovx_fft_out_of_place(self._h, _ptr(x), x.stride(0), _ptr(out), out.stride(0), self.n,
-                                         _stream()))
+            out = _torch().empty_like(x)
+        st = lib().ovx_fft_out_of_place(self._h, x.data_ptr(), x.stride(0), out.data_ptr(), out.stride(0), self.n,
+                                        _stream())
+        if st:
+            check(st)
         return out
 
 
@@ -205,26 +232,28 @@ class Fastconv(_Plan):
         check(lib().ovx_fastconv_plan_create(ctypes.byref(self._h), rows, n, self.scale, flags))
 
     def __call__(self, x, w, out=None, rows=None):
-        torch = _torch()
         _check_tensor(x, "input")
         _check_tensor(w, "spectrum")
         if out is None:
-            out = torch.empty_like(x)
+            out = _torch().empty_like(x)
         rows = x.shape[0] if rows is None else rows
         ldw = 0 if w.dim() == 1 else w.stride(0)
-        check(lib().ovx_fastconv_exec(self._h, _ptr(x), x.stride(0), _ptr(w), ldw, _ptr(out), out.stride(0),
-                                      rows, _stream()))
+        st = lib().ovx_fastconv_exec(self._h, x.data_ptr(), x.stride(0), w.data_ptr(), ldw, out.data_ptr(),
+                                     out.stride(0), rows, _stream())
+        if st:
+            check(st)
         return out
 
     def with_replica(self, x, replica, out=None, rows=None):
         """Fastconv against a resident replica (spectrum prepared once)."""
-        torch = _torch()
         _check_tensor(x, "input")
         if out is None:
-            out = torch.empty_like(x)
+            out = _torch().empty_like(x)
         rows = x.shape[0] if rows is None else rows
-        check(lib().ovx_fastconv_exec_replica(self._h, _ptr(x), x.stride(0), replica.id, _ptr(out),
-                                              out.stride(0), rows, _stream()))
+        st = lib().ovx_fastconv_exec_replica(self._h, x.data_ptr(), x.stride(0), replica.id, out.data_ptr(),
+                                             out.stride(0), rows, _stream())
+        if st:
+            check(st)
         return out
 
 
@@ -234,23 +263,28 @@ def vmmul(dim, v, m, out=None, alpha=1.0):
     m are complex64 or float32 GPU tensors of any strides; out (complex64
     when either is complex, else float32) may be m."""
     torch = _torch()
-    ok = (torch.complex64, torch.float32)
-    for t, name in ((v, "v"), (m, "m")):
-        if t.dtype not in ok or not t.is_cuda:
+    c64, f32 = torch.complex64, torch.float32
+    vt, mt = v.dtype, m.dtype
+    for t, d, name in ((v, vt, "v"), (m, mt, "m")):
+        if (d is not c64 and d is not f32) or not t.is_cuda:
             raise TypeError(f"{name} must be a complex64 or float32 GPU tensor")
-    if v.dim() != 1 or m.dim() != 2:
+    vs, ms = v.shape, m.shape
+    if len(vs) != 1 or len(ms) != 2:
         raise ValueError("v must be 1-D and m 2-D")
-    rows, cols = m.shape
-    if v.shape[0] != (cols if dim == 0 else rows):
-        raise ValueError(f"vmmul<{dim}>: vector length {v.shape[0]} does not match the matrix {rows}x{cols}")
-    odt = torch.complex64 if torch.complex64 in (v.dtype, m.dtype) else torch.float32
+    rows, cols = ms
+    if vs[0] != (cols if dim == 0 else rows):
+        raise ValueError(f"vmmul<{dim}>: vector length {vs[0]} does not match the matrix {rows}x{cols}")
+    odt = c64 if vt is c64 or mt is c64 else f32
     if out is None:
         out = torch.empty((rows, cols), dtype=odt, device=m.device)
-    if out.dtype != odt or tuple(out.shape) != (rows, cols):
+    if out.dtype is not odt or out.shape != ms:
         raise TypeError("out has the wrong type or shape")
-    check(lib().ovx_vmmul(dim, int(v.dtype == torch.complex64), _ptr(v), v.stride(0),
-                          int(m.dtype == torch.complex64), _ptr(m), m.stride(0), m.stride(1), _ptr(out),
-                          out.stride(0), out.stride(1), rows, cols, alpha, _stream()))
+    m0, m1 = m.stride()
+    o0, o1 = out.stride()
+    st = lib().ovx_vmmul(dim, vt is c64, v.data_ptr(), v.stride(0), mt is c64, m.data_ptr(), m0, m1, out.data_ptr(),
+                         o0, o1, rows, cols, alpha, _stream())
+    if st:
+        check(st)
     return out
 
 
@@ -363,12 +397,14 @@ class Correlation(_Plan):
         self.output_size = lib().ovx_corr_output_size(_lib.SUPPORT[support], m, n)
 
     def __call__(self, bias, ref, x, out=None):
-        torch = _torch()
         _check_tensor(ref, "reference")
         _check_tensor(x, "input")
         if out is None:
+            torch = _torch()
             out = torch.empty(self.output_size, dtype=torch.complex64, device=x.device)
-        check(lib().ovx_corr_exec(self._h, _lib.BIAS[bias], _ptr(ref), _ptr(x), _ptr(out), _stream()))
+        st = lib().ovx_corr_exec(self._h, _lib.BIAS[bias], ref.data_ptr(), x.data_ptr(), out.data_ptr(), _stream())
+        if st:
+            check(st)
         return out
 
 
@@ -384,11 +420,13 @@ class Convolution(_Plan):
         self.output_size = lib().ovx_conv_output_size(_lib.SUPPORT[support], m, n, decimation)
 
     def __call__(self, x, out=None):
-        torch = _torch()
         _check_tensor(x, "input")
         if out is None:
+            torch = _torch()
             out = torch.empty(self.output_size, dtype=torch.complex64, device=x.device)
-        check(lib().ovx_conv_exec(self._h, _ptr(x), _ptr(out), _stream()))
+        st = lib().ovx_conv_exec(self._h, x.data_ptr(), out.data_ptr(), _stream())
+        if st:
+            check(st)
         return out
 
 
