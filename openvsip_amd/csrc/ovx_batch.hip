@@ -67,12 +67,9 @@ __device__ __noinline__ void tile_hier_fastconv(lds_job &j, int row0_arg, lds_pt
   a.y = uniform(j.y);
   a.ldy = uniform(j.ldy);
   a.w = uniform(j.w);
-  a.ldw = 0;
   a.rows = uniform(j.rows);
   a.tw_outer = uniform(j.tw0);
   a.tw_wave = uniform(j.tw1);
-  a.scale = 1.0f;
-  a.natural = 0;
   const int lrow = (int)threadIdx.x / H::TR;
   const int t = (int)threadIdx.x % H::TR;
   // a tile of one row is only made for a row that exists
@@ -103,7 +100,7 @@ template <int NT, int N, int P>
 __device__ __noinline__ void tile_row_fastconv(lds_job &j, int row0_arg, lds_ptr lds)
 {
   const int row0 = __builtin_amdgcn_readfirstlane(row0_arg); // uniform, see uniform()
-  using E = Engine<N, P, (N / P <= 64)>;
+  using E = Engine<N, P, line_in_wave(N / P)>;
   static_assert(NT % E::T == 0 && (NT / E::T) * E::LROW <= BatchLds<NT>::value, "tile LDS");
   const int lrow = (int)threadIdx.x / E::T;
   const int t = (int)threadIdx.x % E::T;
@@ -115,7 +112,7 @@ template <int NT, int N, int P>
 __device__ __noinline__ void tile_row_fwd(lds_job &j, int row0_arg, lds_ptr lds)
 {
   const int row0 = __builtin_amdgcn_readfirstlane(row0_arg); // uniform, see uniform()
-  using E = Engine<N, P, (N / P <= 64)>;
+  using E = Engine<N, P, line_in_wave(N / P)>;
   static_assert(NT % E::T == 0 && (NT / E::T) * E::LROW <= BatchLds<NT>::value, "tile LDS");
   const int lrow = (int)threadIdx.x / E::T;
   const int t = (int)threadIdx.x % E::T;

@@ -26,15 +26,16 @@ static std::mutex g_path_mu;
 static std::map<std::pair<long, int>, std::unique_ptr<LineFFT>> g_paths;
 
 // Variant the batch tiles of an (n, rows) job run: the autotuner's batch
-// entry for (n, rows) when it has one, else the default -- for the 3 * 2^k
-// lengths the 12-values-per-thread register-Stockham configuration (variant
-// 1), which fits the 1024-thread persistent kernel's register budget, for
-// the others the standalone default.
+// entry for (n, rows) when it names a tile body (an older cache file may hold
+// other variant numbers), else at 2048 and 4096 points the register-Stockham
+// body, else the first.  Lengths without a tile run the standalone default.
 int batch_variant(long n, long rows)
 {
-  int v = tuned_batch_variant(n, rows);
-  if (v >= 0) return v;
-  return (n == 3072 || n == 6144 || n == 12288) ? 1 : LineFFT::default_variant(n);
+  const std::vector<int> cands = batch_candidates(n);
+  if (cands.empty()) return LineFFT::default_variant(n, rows);
+  const int v = tuned_batch_variant(n, rows);
+  if (std::find(cands.begin(), cands.end(), v) != cands.end()) return v;
+  return n == 2048 || n == 4096 ? cands.back() : cands.front();
 }
 
 const LineFFT *shared_path(long n, int variant, int *status)

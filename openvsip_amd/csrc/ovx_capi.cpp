@@ -90,9 +90,17 @@ static int make_row_twiddles(const RowConfig &rc, DevBuf &tw)
 }
 
 // Variant used when neither the caller nor the tuner picks one: the
-// hierarchical kernel, except at 2048 and 4096, where the register-Stockham
-// kernel (16 values per thread) measured faster at every row count tried.
-int LineFFT::default_variant(long n) { return (n == 2048 || n == 4096) ? 1 : 0; }
+// hierarchical fastconv at 8192 and 16384 points (256 rows: 12.9 against 14.6
+// and 24.1 against 24.5 us), the register-Stockham kernel at the lengths below,
+// where it is faster at every row count (1024: 6.2 against 5.3, 2048: 8.7
+// against 6.9, 4096: 8.7 against 8.1 us).
+int LineFFT::default_variant(long n, long rows)
+{
+  if (n < 1 || n > kMaxRowN || n == 8192 || n == 16384) return 0;
+  return row_variant(n, row_pick((int)n, rows));
+}
+
+int LineFFT::row_variant(long n, int config) { return hier_supported(n) ? config + 1 : config; }
 
 int LineFFT::variants(long n)
 {
@@ -113,7 +121,8 @@ int LineFFT::init(long n_, int variant_)
     if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
     if (e != hipSuccess) return hip_fail(e, "twiddle kernels");
     kind = HIER;
-    return OVX_OK;
+    if (!row_config((int)n, 0, &rc)) return fail(OVX_ERR_UNSUPPORTED, "no LDS-resident configuration for n=%ld", n);
+    return make_row_twiddles(rc, tw);
   }
   if (n >= 1 && n <= kMaxRowN && row_variants((int)n) > 0) {
     int v = hier_supported(n) ? variant - 1 : variant;
@@ -129,7 +138,8 @@ int LineFFT::init(long n_, int variant_)
     n2 = n / n1;
     if (!fs_length_supported(n1) || !fs_length_supported(n2))
       return fail(OVX_ERR_UNSUPPORTED, "transform length %ld is not supported by the gfx950 backend", n);
-    if (!row_config((int)n1, 0, &rc1) || !row_config((int)n2, 0, &rc2))
+    if (!row_config((int)n1, row_config_with((int)n1, 16), &rc1) ||
+        !row_config((int)n2, row_config_with((int)n2, 16), &rc2))
       return fail(OVX_ERR_UNSUPPORTED, "no line configuration for %ld x %ld", n1, n2);
     int st;
     if ((st = make_row_twiddles(rc1, tw1)) || (st = make_row_twiddles(rc2, tw2))) return st;
@@ -188,7 +198,7 @@ bool LineFFT::tables_ready() const
 {
   switch (kind) {
   case LDS: return tw.p != nullptr;
-  case HIER: return tw_outer.p != nullptr && tw_wave.p != nullptr;
+  case HIER: return tw_outer.p != nullptr && tw_wave.p != nullptr && tw.p != nullptr;
   case FOURSTEP: return tw1.p && tw2.p && tlo.p && thi.p;
   default: return false;
   }
@@ -269,39 +279,33 @@ int LineFFT::transform_ws(int dir, const float2 *in, long ld_in, float2 *out, lo
 }
 
 // The hierarchical fastconv launch (interleaved or split X and Y, set in
-// `a`): a single spectrum is permuted once into the kernel's [k1][k2] order
-// with the scale folded in; a coefficient matrix is read in natural order.
-int LineFFT::hier_fastconv(HierArgs a, int launch_kind, long ldx, const float2 *w, long ldw, long ldy, long lines,
-                           float scale, hipStream_t s, const ExtScratch *ext) const
+// `a`) against one spectrum, which is permuted once into the kernel's [k1][k2]
+// order with the scale folded in.  A coefficient matrix goes to the
+// register-Stockham kernel instead, which reads its rows in natural order,
+// coalesced: gathered here at a stride of n/1024 values (one 8-byte value of
+// every 128-byte line at 16384) they took 15.4 us at 256 x 8192 and 35.8 us at
+// 256 x 16384 against 14.5 and 26.0 us there, 1000 x 16384 135.6 against 99.6.
+int LineFFT::hier_fastconv(HierArgs a, int launch_kind, long ldx, const float2 *w, long ldy, long lines, float scale,
+                           hipStream_t s, const ExtScratch *ext) const
 {
-  if (!offsets_fit(hier_rows_per_block(n), std::max(std::max(ldx, ldy), ldw)))
+  if (!offsets_fit(hier_rows_per_block(n), std::max(ldx, ldy)))
     return fail(OVX_ERR_UNSUPPORTED, "row stride too large for 32-bit buffer offsets");
   a.ldx = ldx;
   a.ldy = ldy;
   a.rows = lines;
-  if (ldw == 0) {
-    float2 *wpp;
-    if (ext) {
-      if (ext->wp_elems < (size_t)n) return fail(OVX_ERR_UNSUPPORTED, "lent scratch too small for the spectrum");
-      wpp = ext->wp;
-    } else {
-      int st = wp.alloc((size_t)n * 8);
-      if (st) return st;
-      wpp = (float2 *)wp.p;
-    }
-    hipError_t e = launch_hier_permute(w, 0, wpp, n, 1, scale, s);
-    if (e != hipSuccess) return hip_fail(e, "spectrum permutation");
-    a.w = wpp;
-    a.ldw = 0;
-    a.natural = 0;
-    a.scale = 1.0f;
+  float2 *wpp;
+  if (ext) {
+    if (ext->wp_elems < (size_t)n) return fail(OVX_ERR_UNSUPPORTED, "lent scratch too small for the spectrum");
+    wpp = ext->wp;
   } else {
-    a.w = w;
-    a.ldw = ldw;
-    a.natural = 1;
-    a.scale = scale;
+    int st = wp.alloc((size_t)n * 8);
+    if (st) return st;
+    wpp = (float2 *)wp.p;
   }
-  hipError_t e = launch_hier(launch_kind, n, a, s);
+  hipError_t e = launch_hier_permute(w, 0, wpp, n, 1, scale, s);
+  if (e != hipSuccess) return hip_fail(e, "spectrum permutation");
+  a.w = wpp;
+  e = launch_hier(launch_kind, n, a, s);
   return e == hipSuccess ? OVX_OK : hip_fail(e, "fastconv launch");
 }
 
@@ -403,9 +407,6 @@ int LineFFT::fastconv_split_vec(const float *xr, const float *xi, long ldx, cons
   a.ldy = ldy;
   a.rows = lines;
   a.w = (const float2 *)wp.p;
-  a.ldw = 0;
-  a.natural = 0;
-  a.scale = 1.0f;
   e = launch_hier(HIER_FASTCONV_SPLIT, n, a, s);
   return e == hipSuccess ? OVX_OK : hip_fail(e, "fastconv launch");
 }
@@ -447,7 +448,7 @@ int LineFFT::fastconv_split(const float *xr, const float *xi, long ldx, const fl
     if ((e = launch_fs_col(1, a, lines, s)) != hipSuccess) return hip_fail(e, "four-step column pass");
     return OVX_OK;
   }
-  if (kind == LDS) {
+  if (kind == LDS || (kind == HIER && ldw != 0)) {
     long ld = std::max(std::max(ldx, ldy), ldw);
     if ((unsigned long)rc.rows_per_block * (unsigned long)ld * 8ul >= (1ul << 32))
       return fail(OVX_ERR_UNSUPPORTED, "row stride too large for 32-bit buffer offsets");
@@ -460,7 +461,7 @@ int LineFFT::fastconv_split(const float *xr, const float *xi, long ldx, const fl
   a.xi = xi;
   a.yr = yr;
   a.yi = yi;
-  return hier_fastconv(a, HIER_FASTCONV_SPLIT, ldx, w, ldw, ldy, lines, scale, s);
+  return hier_fastconv(a, HIER_FASTCONV_SPLIT, ldx, w, ldy, lines, scale, s);
 }
 
 int LineFFT::fastconv(const float2 *x, long ldx, const float2 *w, long ldw, float2 *y, long ldy, long lines,
@@ -468,13 +469,13 @@ int LineFFT::fastconv(const float2 *x, long ldx, const float2 *w, long ldw, floa
 {
   if (lines <= 0) return OVX_OK;
   if (!tables_ready()) return fail(OVX_ERR_STATE, "fastconv plan has no twiddle tables");
-  if (kind == HIER) {
+  if (kind == HIER && ldw == 0) {
     HierArgs a = hier_args(*this);
     a.x = x;
     a.y = y;
-    return hier_fastconv(a, HIER_FASTCONV, ldx, w, ldw, ldy, lines, scale, s, ext);
+    return hier_fastconv(a, HIER_FASTCONV, ldx, w, ldy, lines, scale, s, ext);
   }
-  if (kind == LDS) {
+  if (kind == LDS || (kind == HIER && ldw != 0)) {
     long ld = std::max(std::max(ldx, ldy), ldw);
     if ((unsigned long)rc.rows_per_block * (unsigned long)ld * 8ul >= (1ul << 32))
       return fail(OVX_ERR_UNSUPPORTED, "row stride too large for 32-bit buffer offsets");
@@ -552,9 +553,6 @@ int LineFFT::fastconv_prepared(const float2 *x, long ldx, const float2 *wprep, f
     a.ldy = ldy;
     a.rows = lines;
     a.w = wprep;
-    a.ldw = 0;
-    a.natural = 0;
-    a.scale = 1.0f;
     hipError_t e = launch_hier(HIER_FASTCONV, n, a, s);
     if (e != hipSuccess) return hip_fail(e, "fastconv launch");
     return OVX_OK;
@@ -684,14 +682,21 @@ static int variant_of(unsigned flags, long n = 0, long rows = 0)
     int t = tuned_variant(n, rows);
     if (t >= 0 && t < LineFFT::variants(n)) return t;
   }
-  return LineFFT::default_variant(n);
+  return LineFFT::default_variant(n, rows);
 }
 
-// Variant of a real transform's half-length line: the first register-Stockham
-// configuration, which the one-pass real kernels are built on.
-static int real_variant(long h)
+// Variant of a transform plan of `rows` lines: the flags' or a
+// register-Stockham configuration, which stores its result in natural order
+// straight from registers where the hierarchical kernel stages it through LDS
+// (256 rows, hierarchical / register-Stockham, forward and inverse: 8192
+// 10.3 / 10.0 and 12.0 / 10.0, 16384 18.2 / 17.0 and 20.6 / 16.9 us; 1000 rows
+// of 16384 68.9 / 64.0 and 78.4 / 63.9 us).  The autotuner times fastconv, so
+// its choice is not asked here.
+static int fft_variant_of(unsigned flags, long n, long rows)
 {
-  return hier_supported(h) ? 1 : 0;
+  if ((flags >> 8) & 0xffu) return variant_of(flags);
+  if (n < 1 || n > kMaxRowN) return 0;
+  return LineFFT::row_variant(n, row_pick((int)n, rows));
 }
 
 extern "C" int ovx_supported_length(long n)
@@ -721,7 +726,7 @@ extern "C" int ovx_fftm_plan_create(ovx_plan *plan, long rows, long cols, int ax
   p->flags = flags;
   long n = axis == OVX_ROW ? cols : rows;
   if (n > 0) {
-    int st = p->line.init(n, variant_of(flags, n, axis == OVX_ROW ? rows : cols));
+    int st = p->line.init(n, fft_variant_of(flags, n, axis == OVX_ROW ? rows : cols));
     if (st) return st;
   }
   *plan = p.release();
@@ -826,10 +831,8 @@ extern "C" int ovx_fftm_real_plan_create(ovx_plan *plan, long rows, long cols, i
   if (n > 0) {
     const long h = n / 2;
     // the one-pass real kernels are built on the register-Stockham
-    // configurations, so lengths that have one use it unless the caller names
-    // another variant
-    const int pick = variant_of(flags);
-    int st = p->line.init(h, (flags >> 8) & 0xffu ? pick : real_variant(h));
+    // configurations
+    int st = p->line.init(h, fft_variant_of(flags, h, axis == OVX_ROW ? rows : cols));
     if (st) return st;
     if ((st = p->wtab.alloc((size_t)(h / 2 + 1) * 8))) return st;
     hipError_t e = launch_unit_roots(n, h / 2 + 1, (float2 *)p->wtab.p, nullptr);
@@ -970,7 +973,7 @@ extern "C" int ovx_fastconv_plan_create(ovx_plan *plan, long rows, long n, float
     p->bf16x3 = true;
     // its stage plan and twiddles are those of the register-Stockham
     // configuration with 16 values per thread
-    int st = p->line.init(n, hier_supported(n) ? 1 : 0);
+    int st = p->line.init(n, LineFFT::row_variant(n, row_config_with((int)n, 16)));
     if (st) return st;
     if (p->line.kind != LineFFT::LDS || p->line.rc.p != 16 || p->line.rc.plan.twtotal != bf16x3_twiddle_count())
       return fail(OVX_ERR_STATE, "BF16x3 variant: unexpected stage plan");

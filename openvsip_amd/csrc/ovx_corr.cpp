@@ -45,8 +45,8 @@ static int ols_init(CorrState &c)
   c.L = choose_L(c.M);
   if (c.M - 1 >= c.L) return fail(OVX_ERR_UNSUPPORTED, "kernel length %ld too long for overlap-save", c.M);
   // the overlap-save kernel is built on the register-Stockham engine: take
-  // that path's configuration (variant 0 of it) and its twiddle table
-  int st = c.fftL.init(c.L, hier_supported(c.L) ? 1 : 0);
+  // its 16-values-per-thread configuration and that one's twiddle table
+  int st = c.fftL.init(c.L, LineFFT::row_variant(c.L, row_config_with(c.L, 16)));
   if (st) return st;
   if (c.fftL.kind != LineFFT::LDS || !c.fftL.tw.p)
     return fail(OVX_ERR_UNSUPPORTED, "no register-Stockham configuration for segment length %d", c.L);

@@ -8,6 +8,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <utility>
+
 namespace ovx {
 
 // ---------------------------------------------------------------- complex
@@ -165,6 +167,85 @@ template <int DIR> struct Dft<16, DIR> {
     }
   }
 };
+
+// 9 = 3 x 3: y[k1 + 3 k2] = DFT3_n( W9^{n k1} * DFT3_{n2}(x[n + 3 n2])[k1] )[k2]
+template <int DIR> struct Dft<9, DIR> {
+  __device__ __forceinline__ static void run(float2 *v)
+  {
+    const float d = (float)DIR;
+    const float2 w1 = make_float2(0.76604444311897803520f, d * 0.64278760968653932632f);  // W9
+    const float2 w2 = make_float2(0.17364817766693034885f, d * 0.98480775301220805937f);  // W9^2
+    const float2 w4 = make_float2(-0.93969262078590838405f, d * 0.34202014332566873304f); // W9^4
+    float2 z[3][3];
+#pragma unroll
+    for (int n = 0; n < 3; ++n) {
+      float2 a[3] = { v[n], v[n + 3], v[n + 6] };
+      Dft<3, DIR>::run(a);
+#pragma unroll
+      for (int k = 0; k < 3; ++k) z[n][k] = a[k];
+    }
+    z[1][1] = cmul(z[1][1], w1);
+    z[1][2] = cmul(z[1][2], w2);
+    z[2][1] = cmul(z[2][1], w2);
+    z[2][2] = cmul(z[2][2], w4);
+#pragma unroll
+    for (int k1 = 0; k1 < 3; ++k1) {
+      float2 b[3] = { z[0][k1], z[1][k1], z[2][k1] };
+      Dft<3, DIR>::run(b);
+#pragma unroll
+      for (int k2 = 0; k2 < 3; ++k2) v[k1 + 3 * k2] = b[k2];
+    }
+  }
+};
+
+// R = A * B with A, B coprime (Good's prime-factor mapping, no twiddles):
+// input n = (B n1 + A n2) mod R, output k with k = k1 mod A, k = k2 mod B.
+// All indices are compile-time, so the maps cost nothing.
+template <int A, int B, int DIR> struct DftCoprime {
+  static constexpr int out(int k1, int k2)
+  {
+    for (int k = 0; k < A * B; ++k)
+      if (k % A == k1 && k % B == k2) return k;
+    return 0;
+  }
+  template <int K1, int... K2>
+  __device__ __forceinline__ static void put(float2 *v, const float2 *b, std::integer_sequence<int, K2...>)
+  {
+    ((v[std::integral_constant<int, out(K1, K2)>::value] = b[K2]), ...);
+  }
+  template <int... K1>
+  __device__ __forceinline__ static void second(float2 *v, const float2 (&z)[B][A], std::integer_sequence<int, K1...>)
+  {
+    (
+        [&] {
+          float2 b[B];
+#pragma unroll
+          for (int n2 = 0; n2 < B; ++n2) b[n2] = z[n2][K1];
+          Dft<B, DIR>::run(b);
+          put<K1>(v, b, std::make_integer_sequence<int, B>());
+        }(),
+        ...);
+  }
+  __device__ __forceinline__ static void run(float2 *v)
+  {
+    float2 z[B][A];
+#pragma unroll
+    for (int n2 = 0; n2 < B; ++n2) {
+#pragma unroll
+      for (int n1 = 0; n1 < A; ++n1) z[n2][n1] = v[(B * n1 + A * n2) % (A * B)];
+      Dft<A, DIR>::run(z[n2]);
+    }
+    second(v, z, std::make_integer_sequence<int, A>());
+  }
+};
+template <int DIR> struct Dft<6, DIR> : DftCoprime<2, 3, DIR> {};
+template <int DIR> struct Dft<10, DIR> : DftCoprime<2, 5, DIR> {};
+template <int DIR> struct Dft<12, DIR> : DftCoprime<4, 3, DIR> {};
+template <int DIR> struct Dft<18, DIR> : DftCoprime<2, 9, DIR> {};
+template <int DIR> struct Dft<20, DIR> : DftCoprime<4, 5, DIR> {};
+template <int DIR> struct Dft<24, DIR> : DftCoprime<8, 3, DIR> {};
+template <int DIR> struct Dft<36, DIR> : DftCoprime<4, 9, DIR> {};
+template <int DIR> struct Dft<40, DIR> : DftCoprime<8, 5, DIR> {};
 
 // ---------------------------------------------------------------- buffer IO
 // Raw buffer loads/stores: one 128-bit descriptor per base pointer, a

@@ -37,6 +37,38 @@ struct RadixPlan {
 };
 
 constexpr bool divides(int a, int b) { return b % a == 0; }
+constexpr bool pow2(int a) { return (a & (a - 1)) == 0; }
+
+// Radices of a length that is no power of two: the fewest stages (each but the
+// last costs an LDS exchange of the whole line and a set of twiddles), then the
+// smallest sum of radices, every radix a divisor of P and no larger than the
+// one before it.
+struct RadixChoice {
+  int nst = 99, sum = 0;
+  int radix[16] = {};
+};
+constexpr RadixChoice fewest_stages(int rem, int P, int largest, int depth)
+{
+  RadixChoice best{};
+  if (rem == 1) {
+    best.nst = 0;
+    return best;
+  }
+  if (depth == 0) return best;
+  const int cand[14] = { 40, 36, 24, 20, 18, 16, 12, 10, 9, 8, 6, 5, 4, 3 };
+  for (int i = 0; i <= 14; ++i) {
+    const int r = i < 14 ? cand[i] : 2;
+    if (r > largest || !divides(r, rem) || !divides(r, P)) continue;
+    const RadixChoice c = fewest_stages(rem / r, P, r, depth - 1);
+    if (c.nst + 1 < best.nst || (c.nst + 1 == best.nst && c.sum + r < best.sum)) {
+      best.nst = c.nst + 1;
+      best.sum = c.sum + r;
+      best.radix[0] = r;
+      for (int k = 0; k < c.nst; ++k) best.radix[k + 1] = c.radix[k];
+    }
+  }
+  return best;
+}
 
 // Radix sequence for length N with P values per thread: radices must divide
 // P; larger radices first (the first stage needs no twiddles, so the stage
@@ -45,17 +77,31 @@ constexpr RadixPlan make_plan(int N, int P)
 {
   RadixPlan p{};
   p.nst = 0;
-  int rem = N;
-  const int cand[6] = { 16, 8, 4, 5, 3, 2 };
-  while (rem > 1) {
-    int chosen = 0;
-    for (int i = 0; i < 6; ++i) {
-      int r = cand[i];
-      if (divides(r, rem) && divides(r, P)) { chosen = r; break; }
+  if (pow2(N)) {
+    int rem = N;
+    const int cand[4] = { 16, 8, 4, 2 };
+    while (rem > 1) {
+      int chosen = 0;
+      for (int i = 0; i < 4; ++i) {
+        int r = cand[i];
+        if (divides(r, rem) && divides(r, P)) { chosen = r; break; }
+      }
+      if (chosen == 0) { p.nst = -1; return p; }
+      p.radix[p.nst++] = chosen;
+      rem /= chosen;
     }
-    if (chosen == 0) { p.nst = -1; return p; }
-    p.radix[p.nst++] = chosen;
-    rem /= chosen;
+  } else {
+    RadixChoice c{};
+    for (int depth = 1; depth <= 8 && c.nst > 8; ++depth) c = fewest_stages(N, P, 40, depth);
+    if (c.nst > 8) { p.nst = -1; return p; }
+    // powers of two first: the Ns of a stage is then a power of two up to the
+    // first radix that is not (j / Ns and j % Ns cost a shift and a mask, and
+    // its writes keep constant distances)
+    p.nst = 0;
+    for (int s = 0; s < c.nst; ++s)
+      if (pow2(c.radix[s])) p.radix[p.nst++] = c.radix[s];
+    for (int s = c.nst - 1; s >= 0; --s)
+      if (!pow2(c.radix[s])) p.radix[p.nst++] = c.radix[s];
   }
   int ns = 1, off = 0;
   for (int s = 0; s < p.nst; ++s) {
@@ -112,6 +158,10 @@ __device__ __forceinline__ void exchange_sync()
     __syncthreads();
   }
 }
+
+// Whether lines of T threads, packed one after the other, each lie within one
+// wavefront.
+constexpr bool line_in_wave(int T) { return T <= 64 && 64 % T == 0; }
 
 // ---------------------------------------------------------------- engine
 // Each stage's twiddles are loaded during the previous stage's LDS exchange

@@ -12,13 +12,11 @@ struct HierArgs {
   long ldx;
   float2 *y;
   long ldy;
-  const float2 *w;        // fastconv spectrum ([k1][k2] order unless natural)
-  long ldw;               // 0: one spectrum for all rows
+  const float2 *w;        // fastconv: one spectrum in [k1][k2] order, scale folded in
   long rows;
   const float2 *tw_outer; // (R0-1)*1024 entries
   const float2 *tw_wave;  // 1024-point engine table
-  float scale;            // applied unless 1
-  int natural;            // spectrum in natural order (gathered)
+  float scale;            // transforms: applied unless 1
   // HIER_FASTCONV_SPLIT: X and Y as split real / imaginary arrays (line
   // strides ldx, ldy in floats); x and y are unused
   const float *xr = nullptr, *xi = nullptr;

@@ -99,9 +99,7 @@ __device__ __forceinline__ void outer_inverse_store(const IO &iy, bool valid, LP
 }
 
 // ---------------------------------------------------------------- fastconv
-// w_perm: spectrum in [k1][k2] order (w_perm[k1*1024 + k2] = W[k1 + R0 k2]),
-// one vector (ldw = 0) or one per row; when natural != 0 the spectrum is in
-// natural order and gathered with stride R0 instead.
+// a.w: one spectrum in [k1][k2] order (w[k1*1024 + k2] = W[k1 + R0 k2]).
 // Body shared by the standalone kernel and the persistent batch kernel:
 // rows row0 + lrow of the job, thread t of the row, LDS row region `lds`.
 // Every thread of the workgroup must call it (it contains workgroup
@@ -119,7 +117,7 @@ __device__ __forceinline__ void hier_fastconv_body(const HierArgs &a, long row0,
   const bool valid = ONE_ROW || row < a.rows;
   const auto ix = hier_in<SPLIT>(a, row0, lrow, t);
   const auto iy = hier_out<SPLIT>(a, row0, lrow, t);
-  const rsrc_t rw = make_rsrc(a.w + row0 * a.ldw, 0xffffffffu);
+  const rsrc_t rw = make_rsrc(a.w, (uint32_t)N * 8u);
   const rsrc_t rtw = make_rsrc(a.tw_wave, (uint32_t)(H::WE::plan.twtotal + 1) * 8u);
   const rsrc_t rto = make_rsrc(a.tw_outer, (uint32_t)((R0 - 1) * H::NW) * 8u); // outer twiddles
 
@@ -142,24 +140,11 @@ __device__ __forceinline__ void hier_fastconv_body(const HierArgs &a, long row0,
     for (int s = 0; s < 16; ++s) u[s] = valid ? ix.ld((uint32_t)(64 * s)) : make_float2(0.f, 0.f);
   }
   H::WE::template fft<-1>(u, sl, l, rtw);
-  if (a.natural) {
-    const uint32_t vw = (uint32_t)(lrow * a.ldw + k1 + R0 * l) * 8u;
+  const uint32_t vw = (uint32_t)(k1 * NW + l) * 8u;
 #pragma unroll
-    for (int s = 0; s < 16; ++s) {
-      float2 ww = bload(rw, vw, (uint32_t)(R0 * 64 * s) * 8u);
-      u[s] = cmul(u[s], ww);
-    }
-  } else {
-    const uint32_t vw = (uint32_t)(lrow * a.ldw + k1 * NW + l) * 8u;
-#pragma unroll
-    for (int s = 0; s < 16; ++s) {
-      float2 ww = bload(rw, vw, (uint32_t)(64 * s) * 8u);
-      u[s] = cmul(u[s], ww);
-    }
-  }
-  if (a.scale != 1.0f) {
-#pragma unroll
-    for (int s = 0; s < 16; ++s) u[s] = cscale(u[s], a.scale);
+  for (int s = 0; s < 16; ++s) {
+    float2 ww = bload(rw, vw, (uint32_t)(64 * s) * 8u);
+    u[s] = cmul(u[s], ww);
   }
   H::WE::template fft<+1>(u, sl, l, rtw);
   if constexpr (R0 > 1) {

@@ -24,6 +24,10 @@ struct RowConfig {
 // Number of compiled configurations for length n (0 = not LDS-resident).
 int row_variants(int n);
 bool row_config(int n, int variant, RowConfig *out);
+// The configuration with p values per thread: its index, or -1.
+int row_config_with(int n, int p);
+// The configuration a transform or fastconv of `rows` lines runs by default.
+int row_pick(int n, long rows);
 // Largest length with an LDS-resident configuration.
 constexpr int kMaxRowN = 16384;
 

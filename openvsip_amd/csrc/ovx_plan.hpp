@@ -44,7 +44,8 @@ struct LineFFT {
   int variant = 0;
   RowConfig rc;
   DevBuf tw;
-  // hierarchical (outer stage + per-wave 1024-point transforms)
+  // hierarchical (outer stage + per-wave 1024-point transforms); `rc` and
+  // `tw` are then the register-Stockham path that takes coefficient matrices
   DevBuf tw_outer, tw_wave;
   // two-pass four-step (n = n1 * n2)
   long n1 = 0, n2 = 0;
@@ -78,8 +79,8 @@ struct LineFFT {
                       long ld_out, long lines, float scale, hipStream_t s) const;
   int fastconv_split_vec(const float *xr, const float *xi, long ldx, const float *wr, const float *wi, float *yr,
                          float *yi, long ldy, long lines, float scale, hipStream_t s) const;
-  int hier_fastconv(HierArgs a, int launch_kind, long ldx, const float2 *w, long ldw, long ldy, long lines,
-                    float scale, hipStream_t s, const ExtScratch *ext = nullptr) const;
+  int hier_fastconv(HierArgs a, int launch_kind, long ldx, const float2 *w, long ldy, long lines, float scale,
+                    hipStream_t s, const ExtScratch *ext = nullptr) const;
   int fs_fastconv(const float2 *x, long ldx, const float2 *wprep, long ldwp, float2 *y, long ldy, long lines,
                   hipStream_t s) const;
   // Spectrum layout the fastconv kernels of this path read: wp = scale * w
@@ -89,7 +90,10 @@ struct LineFFT {
   int fastconv_prepared(const float2 *x, long ldx, const float2 *wp, float2 *y, long ldy, long lines,
                         hipStream_t s) const;
   static int variants(long n);
-  static int default_variant(long n);
+  // variant a fastconv of `rows` lines runs unless the caller or the tuner
+  // picks one; variant of the register-Stockham configuration `config`
+  static int default_variant(long n, long rows);
+  static int row_variant(long n, int config);
   // every table the kernels of this path read has been allocated
   bool tables_ready() const;
 };

@@ -16,7 +16,7 @@ __device__ __forceinline__ void row_fastconv_io(const IX &ix, const IY &iy, cons
                                                 long rows, const float2 *__restrict__ tw, float scale, long row0,
                                                 int lrow, int t, LP lds)
 {
-  using E = Engine<N, P, (N / P <= 64)>;
+  using E = Engine<N, P, line_in_wave(N / P)>;
   constexpr int T = E::T;
   const long row = row0 + lrow;
   const bool valid = row < rows;
@@ -68,7 +68,7 @@ template <int N, int P, int DIR, typename IX, typename IY, typename LP>
 __device__ __forceinline__ void row_fft_io(const IX &ix, const IY &iy, long rows, const float2 *__restrict__ tw,
                                            float scale, long row0, int lrow, int t, LP lds)
 {
-  using E = Engine<N, P, (N / P <= 64)>;
+  using E = Engine<N, P, line_in_wave(N / P)>;
   constexpr int T = E::T;
   const long row = row0 + lrow;
   const bool valid = row < rows;
@@ -151,7 +151,7 @@ __device__ __forceinline__ void row_r2c_io(const IX &ix, const IY &iy, const IY 
                                            const float2 *__restrict__ tw, const float2 *__restrict__ wt, float scale,
                                            long row0, int lrow, int t, LP lds)
 {
-  using E = Engine<N, P, (N / P <= 64)>;
+  using E = Engine<N, P, line_in_wave(N / P)>;
   using L = typename E::Layout;
   using R = RealPairs<N, P>;
   constexpr int T = E::T;
@@ -167,7 +167,7 @@ __device__ __forceinline__ void row_r2c_io(const IX &ix, const IY &iy, const IY 
   for (int q = 0; q < R::NQ; ++q) w[q] = bload(rwt, (uint32_t)t * 8u, (uint32_t)(T * q) * 8u);
 #pragma unroll
   for (int q = P / 2; q < P; ++q) lds_st(lds, L::idx(t + T * q), v[q]);
-  exchange_sync<(N / P <= 64)>();
+  exchange_sync<line_in_wave(N / P)>();
   float2 z[R::NQ];
 #pragma unroll
   for (int q = 0; q < R::NQ; ++q) {
@@ -198,7 +198,7 @@ __device__ __forceinline__ void row_c2r_io(const IX &ix, const IX &ixm, const IY
                                            const float2 *__restrict__ tw, const float2 *__restrict__ wt, float scale,
                                            long row0, int lrow, int t, LP lds)
 {
-  constexpr bool WAVE = N / P <= 64;
+  constexpr bool WAVE = line_in_wave(N / P);
   using E = Engine<N, P, WAVE>;
   using L = typename E::Layout;
   using R = RealPairs<N, P>;

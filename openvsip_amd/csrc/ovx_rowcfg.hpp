@@ -1,7 +1,12 @@
 // ovx_rowcfg.hpp -- the compiled register-Stockham row configurations.
 #pragma once
+#include <algorithm>
+
+#include "ovx_engine.hpp"
 
 namespace ovx {
+
+constexpr long kRowSpread = 256; // workgroups that fill the chip, one per CU
 
 // Compiled configurations: (N, P).  Rows per block B makes blocks of at
 // least 256 threads for short lines.
@@ -12,17 +17,75 @@ struct RowCfg {
   static constexpr int NT = T * B;
 };
 
-// X(N, P): every compiled configuration; the first listed for an N is
-// variant 0 (the default).
+// The launch of `rows` lines: as few lines per workgroup (RowCfg::B at most)
+// as leave no more than one workgroup per CU, so that a few short lines spread
+// over the chip instead of sharing a CU.
+template <int N, int P>
+struct RowLaunch {
+  dim3 grid, block;
+  unsigned lds;
+  explicit RowLaunch(long rows)
+  {
+    using C = RowCfg<N, P>;
+    const long b = std::min<long>(C::B, std::max<long>((rows + kRowSpread - 1) / kRowSpread, 1));
+    grid = dim3((unsigned)((rows + b - 1) / b));
+    block = dim3((unsigned)(b * C::T));
+    lds = C::B == 1 ? 0 : (unsigned)(b * Engine<N, P>::LROW * sizeof(float2));
+  }
+};
+
+// Which lines a block handles: blockDim.x / T lines of T threads each, lines
+// contiguous in memory at stride ld.  Out-of-range lines (the tail block)
+// compute on zeros and store nothing, but still take part in every barrier.
+// Several lines' LDS is sized at launch (one row region per line); a line that
+// has the workgroup to itself has its region as a static array, whose address
+// the compiler folds into the accesses (sized at launch, fastconv 256 x 16384
+// took 25.4 instead of 24.5 us).
+extern __shared__ float2 row_lds[];
+
+template <int N, int P>
+struct RowPlace {
+  using E = Engine<N, P, line_in_wave(N / P)>;
+  static constexpr bool ONE = RowCfg<N, P>::B == 1;
+  int lrow, t;
+  long row0;
+  float2 *lds;
+  __device__ __forceinline__ RowPlace()
+  {
+    lrow = ONE ? 0 : (int)threadIdx.x / E::T;
+    t = ONE ? (int)threadIdx.x : (int)threadIdx.x % E::T;
+    row0 = ONE ? (long)blockIdx.x : (long)blockIdx.x * (long)(blockDim.x / E::T);
+    if constexpr (ONE) {
+      __shared__ float2 line[E::LROW];
+      lds = line;
+    } else {
+      lds = row_lds + lrow * E::LROW;
+    }
+  }
+};
+
+// X(N, P): every compiled configuration, a length's in the order of its variant
+// numbers.  P is chosen per length by measurement (one launch, fastconv of 1,
+// 256 and 4000 lines of data that no cache holds, us):
+//   fewer values per thread put more threads on a line, which is what a few
+//   lines need (2304: P 36 9.7 / 10.8, P 12 5.6 / 6.7; 384: P 24 6.7 / 7.6,
+//   P 6 4.2 / 4.9; 2048: P 16 5.9 / 6.9, P 8 4.6 / 5.7), more values per thread
+//   save stages, which is what many lines need (1536 at 4000: P 12 30.1, P 24
+//   25.1; 1024 at 4000: P 8 21.5, P 16 17.2).
+// Where one P is best or within a few per cent everywhere it is the only one;
+// else row_pick() chooses by the number of lines.  16 values per thread at
+// powers of two from 64 and 12 at 3072, 6144 and 12288 are also what the
+// four-step, overlap-save and batch kernels run.
 #define OVX_ROW_CONFIGS(X)                                                      \
-  X(2, 2) X(4, 4) X(8, 8) X(16, 16) X(32, 16) X(64, 16) X(128, 16) X(256, 16)   \
-  X(512, 16) X(1024, 16) X(2048, 16) X(4096, 16) X(8192, 16) X(16384, 16)       \
-  X(3, 3) X(6, 6) X(12, 12) X(24, 24) X(48, 24) X(96, 24) X(192, 24)            \
-  X(384, 24) X(768, 24) X(1536, 24) X(3072, 24) X(6144, 24) X(12288, 24)       \
-  X(3072, 12) X(6144, 12) X(12288, 12)                                          \
-  X(5, 5) X(10, 10) X(20, 20) X(40, 40) X(80, 40) X(160, 40) X(320, 40)         \
-  X(640, 40) X(1280, 40) X(2560, 40) X(5120, 40) X(10240, 40)                 \
-  X(9, 9) X(18, 18) X(36, 36) X(72, 36) X(144, 36) X(288, 36) X(576, 36)       \
-  X(1152, 36) X(2304, 36) X(4608, 36) X(9216, 36)
+  X(2, 2) X(4, 4) X(8, 8) X(16, 4) X(32, 4) X(64, 4) X(64, 16) X(128, 4)        \
+  X(128, 16) X(256, 4) X(256, 16) X(512, 8) X(512, 16) X(1024, 16) X(1024, 8)   \
+  X(2048, 16) X(2048, 8) X(4096, 16) X(8192, 16) X(16384, 16)                   \
+  X(3, 3) X(6, 6) X(12, 12) X(24, 24) X(48, 6) X(96, 6) X(192, 6) X(384, 12)    \
+  X(384, 6) X(768, 12) X(1536, 24) X(1536, 12) X(3072, 12) X(6144, 24)          \
+  X(6144, 12) X(12288, 24) X(12288, 12)                                         \
+  X(5, 5) X(10, 10) X(20, 20) X(40, 40) X(80, 10) X(160, 10) X(320, 20)         \
+  X(640, 20) X(640, 10) X(1280, 20) X(2560, 20) X(5120, 20) X(10240, 40)        \
+  X(9, 9) X(18, 18) X(36, 36) X(72, 6) X(144, 12) X(288, 12) X(576, 24)         \
+  X(576, 12) X(1152, 12) X(2304, 12) X(4608, 12) X(9216, 24)
 
 } // namespace ovx

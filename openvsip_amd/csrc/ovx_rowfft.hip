@@ -13,82 +13,56 @@
 
 namespace ovx {
 
-// Which lines a block handles: B lines of T threads each, lines contiguous in
-// memory at stride ld.  Out-of-range lines (the tail block) compute on zeros
-// and store nothing, but still take part in every barrier.
-template <int N, int P, int B>
-struct RowGeom {
-  static constexpr int T = N / P;
-  static constexpr int NT = T * B;
-};
-
-template <int N, int P, int B, int DIR>
-__global__ __launch_bounds__(N / P * B) void k_row_fft(const float2 *__restrict__ in, long ld_in,
-                                                      float2 *__restrict__ out, long ld_out, long rows,
-                                                      const float2 *__restrict__ tw, float scale)
+template <int N, int P, int DIR>
+__global__ __launch_bounds__((RowCfg<N, P>::NT)) void k_row_fft(const float2 *__restrict__ in, long ld_in,
+                                                               float2 *__restrict__ out, long ld_out, long rows,
+                                                               const float2 *__restrict__ tw, float scale)
 {
-  using E = Engine<N, P, (N / P <= 64)>;
-  __shared__ float2 lds_all[B * E::LROW];
-  const int lrow = (B == 1) ? 0 : (int)threadIdx.x / E::T;
-  const int t = (B == 1) ? (int)threadIdx.x : (int)threadIdx.x % E::T;
-  row_fft_body<N, P, DIR>(in, ld_in, out, ld_out, rows, tw, scale, (long)blockIdx.x * B, lrow, t,
-                          lds_all + lrow * E::LROW);
+  const RowPlace<N, P> r;
+  row_fft_body<N, P, DIR>(in, ld_in, out, ld_out, rows, tw, scale, r.row0, r.lrow, r.t, r.lds);
 }
 
-template <int N, int P, int B>
-__global__ __launch_bounds__(N / P * B) void k_row_fastconv(const float2 *__restrict__ x, long ldx,
-                                                           const float2 *__restrict__ w, long ldw,
-                                                           float2 *__restrict__ y, long ldy, long rows,
-                                                           const float2 *__restrict__ tw, float scale)
+template <int N, int P>
+__global__ __launch_bounds__((RowCfg<N, P>::NT)) void k_row_fastconv(const float2 *__restrict__ x, long ldx,
+                                                                    const float2 *__restrict__ w, long ldw,
+                                                                    float2 *__restrict__ y, long ldy, long rows,
+                                                                    const float2 *__restrict__ tw, float scale)
 {
-  using E = Engine<N, P, (N / P <= 64)>;
-  constexpr int T = E::T;
-  __shared__ float2 lds_all[B * E::LROW];
-  const int lrow = (B == 1) ? 0 : (int)threadIdx.x / T;
-  const int t = (B == 1) ? (int)threadIdx.x : (int)threadIdx.x % T;
-  row_fastconv_body<N, P>(x, ldx, w, ldw, y, ldy, rows, tw, scale, (long)blockIdx.x * B, lrow, t,
-                          lds_all + lrow * E::LROW);
+  const RowPlace<N, P> r;
+  row_fastconv_body<N, P>(x, ldx, w, ldw, y, ldy, rows, tw, scale, r.row0, r.lrow, r.t, r.lds);
 }
 
 // Split-storage forms: real and imaginary parts of the lines in two float
 // arrays with the same strides (the spectrum stays interleaved).
-template <int N, int P, int B, int DIR>
-__global__ __launch_bounds__(N / P * B) void k_row_fft_split(const float *__restrict__ in_re,
-                                                            const float *__restrict__ in_im, long ld_in,
-                                                            float *__restrict__ out_re, float *__restrict__ out_im,
-                                                            long ld_out, long rows, const float2 *__restrict__ tw,
-                                                            float scale)
+template <int N, int P, int DIR>
+__global__ __launch_bounds__((RowCfg<N, P>::NT)) void k_row_fft_split(const float *__restrict__ in_re,
+                                                                     const float *__restrict__ in_im, long ld_in,
+                                                                     float *__restrict__ out_re,
+                                                                     float *__restrict__ out_im, long ld_out,
+                                                                     long rows, const float2 *__restrict__ tw,
+                                                                     float scale)
 {
-  using E = Engine<N, P, (N / P <= 64)>;
-  __shared__ float2 lds_all[B * E::LROW];
-  const int lrow = (B == 1) ? 0 : (int)threadIdx.x / E::T;
-  const int t = (B == 1) ? (int)threadIdx.x : (int)threadIdx.x % E::T;
-  const long row0 = (long)blockIdx.x * B;
-  row_fft_io<N, P, DIR>(IoS{make_rsrc(in_re + row0 * ld_in, 0xffffffffu), make_rsrc(in_im + row0 * ld_in, 0xffffffffu),
-                            (uint32_t)(lrow * ld_in + t) * 4u},
-                        IoS{make_rsrc(out_re + row0 * ld_out, 0xffffffffu),
-                            make_rsrc(out_im + row0 * ld_out, 0xffffffffu), (uint32_t)(lrow * ld_out + t) * 4u},
-                        rows, tw, scale, row0, lrow, t, lds_all + lrow * E::LROW);
+  const RowPlace<N, P> r;
+  row_fft_io<N, P, DIR>(
+      IoS{make_rsrc(in_re + r.row0 * ld_in, 0xffffffffu), make_rsrc(in_im + r.row0 * ld_in, 0xffffffffu),
+          (uint32_t)(r.lrow * ld_in + r.t) * 4u},
+      IoS{make_rsrc(out_re + r.row0 * ld_out, 0xffffffffu), make_rsrc(out_im + r.row0 * ld_out, 0xffffffffu),
+          (uint32_t)(r.lrow * ld_out + r.t) * 4u},
+      rows, tw, scale, r.row0, r.lrow, r.t, r.lds);
 }
 
-template <int N, int P, int B>
-__global__ __launch_bounds__(N / P * B) void k_row_fastconv_split(const float *__restrict__ xr,
-                                                                 const float *__restrict__ xi, long ldx,
-                                                                 const float2 *__restrict__ w, long ldw,
-                                                                 float *__restrict__ yr, float *__restrict__ yi,
-                                                                 long ldy, long rows, const float2 *__restrict__ tw,
-                                                                 float scale)
+template <int N, int P>
+__global__ __launch_bounds__((RowCfg<N, P>::NT)) void k_row_fastconv_split(
+    const float *__restrict__ xr, const float *__restrict__ xi, long ldx, const float2 *__restrict__ w, long ldw,
+    float *__restrict__ yr, float *__restrict__ yi, long ldy, long rows, const float2 *__restrict__ tw, float scale)
 {
-  using E = Engine<N, P, (N / P <= 64)>;
-  __shared__ float2 lds_all[B * E::LROW];
-  const int lrow = (B == 1) ? 0 : (int)threadIdx.x / E::T;
-  const int t = (B == 1) ? (int)threadIdx.x : (int)threadIdx.x % E::T;
-  const long row0 = (long)blockIdx.x * B;
-  row_fastconv_io<N, P>(IoS{make_rsrc(xr + row0 * ldx, 0xffffffffu), make_rsrc(xi + row0 * ldx, 0xffffffffu),
-                            (uint32_t)(lrow * ldx + t) * 4u},
-                        IoS{make_rsrc(yr + row0 * ldy, 0xffffffffu), make_rsrc(yi + row0 * ldy, 0xffffffffu),
-                            (uint32_t)(lrow * ldy + t) * 4u},
-                        w, ldw, rows, tw, scale, row0, lrow, t, lds_all + lrow * E::LROW);
+  const RowPlace<N, P> r;
+  row_fastconv_io<N, P>(
+      IoS{make_rsrc(xr + r.row0 * ldx, 0xffffffffu), make_rsrc(xi + r.row0 * ldx, 0xffffffffu),
+          (uint32_t)(r.lrow * ldx + r.t) * 4u},
+      IoS{make_rsrc(yr + r.row0 * ldy, 0xffffffffu), make_rsrc(yi + r.row0 * ldy, 0xffffffffu),
+          (uint32_t)(r.lrow * ldy + r.t) * 4u},
+      w, ldw, rows, tw, scale, r.row0, r.lrow, r.t, r.lds);
 }
 
 // ---------------------------------------------------------------- twiddles
@@ -178,12 +152,11 @@ template <int N, int P>
 static hipError_t do_fft(int dir, const float2 *in, long ld_in, float2 *out, long ld_out, long rows,
                          const float2 *tw, float scale, hipStream_t s)
 {
-  using C = RowCfg<N, P>;
-  dim3 grid((unsigned)((rows + C::B - 1) / C::B)), block(C::NT);
+  const RowLaunch<N, P> l(rows);
   if (dir < 0)
-    hipLaunchKernelGGL((k_row_fft<N, P, C::B, -1>), grid, block, 0, s, in, ld_in, out, ld_out, rows, tw, scale);
+    hipLaunchKernelGGL((k_row_fft<N, P, -1>), l.grid, l.block, l.lds, s, in, ld_in, out, ld_out, rows, tw, scale);
   else
-    hipLaunchKernelGGL((k_row_fft<N, P, C::B, +1>), grid, block, 0, s, in, ld_in, out, ld_out, rows, tw, scale);
+    hipLaunchKernelGGL((k_row_fft<N, P, +1>), l.grid, l.block, l.lds, s, in, ld_in, out, ld_out, rows, tw, scale);
   return hipGetLastError();
 }
 
@@ -191,9 +164,8 @@ template <int N, int P>
 static hipError_t do_fastconv(const float2 *x, long ldx, const float2 *w, long ldw, float2 *y, long ldy,
                               long rows, const float2 *tw, float scale, hipStream_t s)
 {
-  using C = RowCfg<N, P>;
-  dim3 grid((unsigned)((rows + C::B - 1) / C::B)), block(C::NT);
-  hipLaunchKernelGGL((k_row_fastconv<N, P, C::B>), grid, block, 0, s, x, ldx, w, ldw, y, ldy, rows, tw, scale);
+  const RowLaunch<N, P> l(rows);
+  hipLaunchKernelGGL((k_row_fastconv<N, P>), l.grid, l.block, l.lds, s, x, ldx, w, ldw, y, ldy, rows, tw, scale);
   return hipGetLastError();
 }
 
@@ -201,13 +173,12 @@ template <int N, int P>
 static hipError_t do_fft_split(int dir, const float *ir, const float *ii, long ld_in, float *orr, float *oi,
                                long ld_out, long rows, const float2 *tw, float scale, hipStream_t s)
 {
-  using C = RowCfg<N, P>;
-  dim3 grid((unsigned)((rows + C::B - 1) / C::B)), block(C::NT);
+  const RowLaunch<N, P> l(rows);
   if (dir < 0)
-    hipLaunchKernelGGL((k_row_fft_split<N, P, C::B, -1>), grid, block, 0, s, ir, ii, ld_in, orr, oi, ld_out, rows,
+    hipLaunchKernelGGL((k_row_fft_split<N, P, -1>), l.grid, l.block, l.lds, s, ir, ii, ld_in, orr, oi, ld_out, rows,
                        tw, scale);
   else
-    hipLaunchKernelGGL((k_row_fft_split<N, P, C::B, +1>), grid, block, 0, s, ir, ii, ld_in, orr, oi, ld_out, rows,
+    hipLaunchKernelGGL((k_row_fft_split<N, P, +1>), l.grid, l.block, l.lds, s, ir, ii, ld_in, orr, oi, ld_out, rows,
                        tw, scale);
   return hipGetLastError();
 }
@@ -216,9 +187,8 @@ template <int N, int P>
 static hipError_t do_fastconv_split(const float *xr, const float *xi, long ldx, const float2 *w, long ldw, float *yr,
                                     float *yi, long ldy, long rows, const float2 *tw, float scale, hipStream_t s)
 {
-  using C = RowCfg<N, P>;
-  dim3 grid((unsigned)((rows + C::B - 1) / C::B)), block(C::NT);
-  hipLaunchKernelGGL((k_row_fastconv_split<N, P, C::B>), grid, block, 0, s, xr, xi, ldx, w, ldw, yr, yi, ldy, rows,
+  const RowLaunch<N, P> l(rows);
+  hipLaunchKernelGGL((k_row_fastconv_split<N, P>), l.grid, l.block, l.lds, s, xr, xi, ldx, w, ldw, yr, yi, ldy, rows,
                      tw, scale);
   return hipGetLastError();
 }
@@ -265,6 +235,31 @@ bool row_config(int n, int variant, RowConfig *out)
   if (!e) return false;
   e->fill(out, variant);
   return true;
+}
+
+int row_config_with(int n, int p)
+{
+  for (int v = 0;; ++v) {
+    const Entry *e = find_entry(n, v);
+    if (!e) return -1;
+    if (e->p == p) return v;
+  }
+}
+
+// The first configuration of a length, or for few lines (up to two per CU) the
+// one with fewer values per thread, as long as its lines keep to 256 threads:
+// fastconv of 256 lines, first / few-line form, 384 5.8 / 4.9, 576 6.9 / 5.2,
+// 640 7.6 / 6.3, 1024 5.3 / 4.7, 1536 7.1 / 7.1 (7.3 / 6.7 at 64), 2048
+// 6.9 / 5.7 us; of 1000 lines 5.9 / 5.6, 7.0 / 6.2, 7.6 / 7.4, 6.4 / 7.0,
+// 8.9 / 10.5 and 10.5 / 11.2 us.  Above 256 threads (6144, 12288) the form
+// with fewer values is the slower one from one line on.
+int row_pick(int n, long rows)
+{
+  const Entry *first = find_entry(n, 0);
+  if (first && rows <= 2 * kRowSpread)
+    for (int v = 1; const Entry *e = find_entry(n, v); ++v)
+      if (e->p < first->p && n / e->p <= 256) return v;
+  return 0;
 }
 
 hipError_t launch_row_fft(const RowConfig &cfg, int dir, const float2 *in, long ld_in, float2 *out, long ld_out,

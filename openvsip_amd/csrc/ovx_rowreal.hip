@@ -34,44 +34,33 @@ __device__ __forceinline__ auto real_cside(const RealArgs &a, long row0, int lro
 template <int N, int P, bool SPLIT>
 __global__ __launch_bounds__((RowCfg<N, P>::NT)) void k_row_r2c(RealArgs a)
 {
-  using E = Engine<N, P, (N / P <= 64)>;
-  constexpr int B = RowCfg<N, P>::B;
-  __shared__ float2 lds_all[B * E::LROW];
-  const int lrow = (B == 1) ? 0 : (int)threadIdx.x / E::T;
-  const int t = (B == 1) ? (int)threadIdx.x : (int)threadIdx.x % E::T;
-  const long row0 = (long)blockIdx.x * B;
-  row_r2c_io<N, P>(IoC{make_rsrc(a.z + row0 * a.ldz, 0xffffffffu), (uint32_t)(lrow * a.ldz + t) * 8u},
-                   real_cside<SPLIT>(a, row0, lrow, t),
-                   real_cside<SPLIT>(a, row0, lrow, RealPairs<N, P>::mirror_base(t)), a.lines, a.tw, a.wt, a.scale,
-                   row0, lrow, t, lds_all + lrow * E::LROW);
+  const RowPlace<N, P> r;
+  row_r2c_io<N, P>(IoC{make_rsrc(a.z + r.row0 * a.ldz, 0xffffffffu), (uint32_t)(r.lrow * a.ldz + r.t) * 8u},
+                   real_cside<SPLIT>(a, r.row0, r.lrow, r.t),
+                   real_cside<SPLIT>(a, r.row0, r.lrow, RealPairs<N, P>::mirror_base(r.t)), a.lines, a.tw, a.wt,
+                   a.scale, r.row0, r.lrow, r.t, r.lds);
 }
 
 template <int N, int P, bool SPLIT>
 __global__ __launch_bounds__((RowCfg<N, P>::NT)) void k_row_c2r(RealArgs a)
 {
-  using E = Engine<N, P, (N / P <= 64)>;
-  constexpr int B = RowCfg<N, P>::B;
-  __shared__ float2 lds_all[B * E::LROW];
-  const int lrow = (B == 1) ? 0 : (int)threadIdx.x / E::T;
-  const int t = (B == 1) ? (int)threadIdx.x : (int)threadIdx.x % E::T;
-  const long row0 = (long)blockIdx.x * B;
-  row_c2r_io<N, P>(real_cside<SPLIT>(a, row0, lrow, t),
-                   real_cside<SPLIT>(a, row0, lrow, RealPairs<N, P>::mirror_base(t)),
-                   IoC{make_rsrc(a.z + row0 * a.ldz, 0xffffffffu), (uint32_t)(lrow * a.ldz + t) * 8u}, a.lines, a.tw,
-                   a.wt, a.scale, row0, lrow, t, lds_all + lrow * E::LROW);
+  const RowPlace<N, P> r;
+  row_c2r_io<N, P>(real_cside<SPLIT>(a, r.row0, r.lrow, r.t),
+                   real_cside<SPLIT>(a, r.row0, r.lrow, RealPairs<N, P>::mirror_base(r.t)),
+                   IoC{make_rsrc(a.z + r.row0 * a.ldz, 0xffffffffu), (uint32_t)(r.lrow * a.ldz + r.t) * 8u}, a.lines,
+                   a.tw, a.wt, a.scale, r.row0, r.lrow, r.t, r.lds);
 }
 
 template <int N, int P>
 static hipError_t do_real(int dir, const RealArgs &a, hipStream_t s)
 {
-  using C = RowCfg<N, P>;
-  dim3 grid((unsigned)((a.lines + C::B - 1) / C::B)), block(C::NT);
+  const RowLaunch<N, P> l(a.lines);
   if (dir < 0) {
-    if (a.cr) hipLaunchKernelGGL((k_row_r2c<N, P, true>), grid, block, 0, s, a);
-    else hipLaunchKernelGGL((k_row_r2c<N, P, false>), grid, block, 0, s, a);
+    if (a.cr) hipLaunchKernelGGL((k_row_r2c<N, P, true>), l.grid, l.block, l.lds, s, a);
+    else hipLaunchKernelGGL((k_row_r2c<N, P, false>), l.grid, l.block, l.lds, s, a);
   } else {
-    if (a.cr) hipLaunchKernelGGL((k_row_c2r<N, P, true>), grid, block, 0, s, a);
-    else hipLaunchKernelGGL((k_row_c2r<N, P, false>), grid, block, 0, s, a);
+    if (a.cr) hipLaunchKernelGGL((k_row_c2r<N, P, true>), l.grid, l.block, l.lds, s, a);
+    else hipLaunchKernelGGL((k_row_c2r<N, P, false>), l.grid, l.block, l.lds, s, a);
   }
   return hipGetLastError();
 }

@@ -592,7 +592,7 @@ extern "C" int ovx_corr_reference_create(int support, long m, long n, const void
   while (L < 4 * (m - 1) && L < kMaxRowN) L *= 2;
   if (m - 1 >= L) return fail(OVX_ERR_UNSUPPORTED, "reference length %ld too long", m);
   c->L = (int)L;
-  int st = c->f.init(L, hier_supported(L) ? 1 : 0);
+  int st = c->f.init(L, LineFFT::row_variant(L, row_config_with((int)L, 16)));
   if (st) return st;
   if (c->f.kind != LineFFT::LDS || !c->f.tw.p) return fail(OVX_ERR_UNSUPPORTED, "no segment path for L=%ld", L);
   DevBuf href, hpad;
