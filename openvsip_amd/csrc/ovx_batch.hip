@@ -120,9 +120,8 @@ __device__ __noinline__ void tile_row_fwd(lds_job &j, int row0_arg, lds_ptr lds)
                          uniform(j.tw0), uniform(j.scale), row0, lrow, t, lds + lrow * E::LROW);
 }
 
-// Overlap-save segments seg0, seg0 + 1, ... (NT / (L/16) of them per tile); a
-// copy past the last segment runs with P = 0, which stores nothing, because
-// ols_body's barriers need every thread.
+// Overlap-save segments seg0, seg0 + 1, ... (NT / (L/16) of them per tile);
+// those past the last store nothing.
 template <int NT, int L>
 __device__ __noinline__ void tile_ols(lds_job &j, int seg0_arg, lds_ptr lds)
 {
@@ -132,10 +131,7 @@ __device__ __noinline__ void tile_ols(lds_job &j, int seg0_arg, lds_ptr lds)
   static_assert(NT % T == 0 && (NT / T) * Engine<L, 16>::LROW <= BatchLds<NT>::value, "tile LDS");
   const int t = (int)threadIdx.x % T;
   const int copy = (int)threadIdx.x / T;
-  const long seg = (long)seg0 + copy;
-  const long nseg = ((a.P - 1) * a.decimation + a.c_step) / a.c_step; // segments of this job
-  if (seg >= nseg) a.P = 0;
-  ols_body<L, 16>(a, seg, t, lds + copy * Engine<L, 16>::LROW);
+  ols_body<L, 16>(a, seg0, copy, t, lds + copy * Engine<L, 16>::LROW);
 }
 
 int batch_ols_segments_per_tile(int L)

@@ -28,64 +28,83 @@ struct CorrState {
   long out_off = 0;
   int L = 0;
   LineFFT fftL;
-  DevBuf hpad, H, ref_stage, in_stage, out_stage;
+  int Lp = 0; // values per thread of a segment
+  DevBuf H, ref_stage, in_stage, out_stage;
 };
 
-// Segment length: a power of two with room for the kernel overlap.
-static int choose_L(long M)
+// Segments of length L over the plan's outputs.
+static long segment_count(const CorrState &c, int L)
 {
-  long L = 64;
-  while (L < 4 * (M - 1) && L < kMaxRowN) L *= 2;
-  while (L - (M - 1) < 1 && L < kMaxRowN) L *= 2;
+  const long span = (c.P - 1) * c.D + 1, step = L - (c.M - 1);
+  return (span + step - 1) / step;
+}
+
+// Segments up to which a segment is a matter of latency: four per CU.
+constexpr long kOlsFew = 1024;
+
+// Segment length: the shortest power of two from 512 of which the kernel
+// overlap takes no more than half (the chain of stages is what a call waits
+// for: 65536 x 1024 takes 7.6 us in segments of 2048 and 11.6 in segments of
+// 4096), and while there are more segments than the chip runs at once, twice
+// that until the overlap is under 30 % (2 * 10^6 x 513: 17.5 us in segments
+// of 1024, 13.9 in 2048, 14.0 in 4096).
+static int choose_L(const CorrState &c)
+{
+  long L = 512;
+  while (L < 2 * (c.M - 1) && L < kMaxRowN) L *= 2;
+  while (L < kMaxRowN && segment_count(c, (int)L) > kOlsFew && 10 * (c.M - 1) > 3 * L) L *= 2;
   return (int)L;
 }
 
+// The reference's spectrum in every segment or once in a launch of its own.
+static bool ols_fuse_ref(const CorrState &c) { return !c.is_conv && segment_count(c, c.L) <= kOlsFew; }
+
 static int ols_init(CorrState &c)
 {
-  c.L = choose_L(c.M);
-  if (c.M - 1 >= c.L) return fail(OVX_ERR_UNSUPPORTED, "kernel length %ld too long for overlap-save", c.M);
-  // the overlap-save kernel is built on the register-Stockham engine: take
-  // its 16-values-per-thread configuration and that one's twiddle table
-  int st = c.fftL.init(c.L, LineFFT::row_variant(c.L, row_config_with(c.L, 16)));
+  if (c.M - 1 >= kMaxRowN) return fail(OVX_ERR_UNSUPPORTED, "kernel length %ld too long for overlap-save", c.M);
+  c.L = choose_L(c);
+  c.Lp = c.L <= 2048 ? 8 : 16;
+  // the overlap-save kernels are built on the register-Stockham engine: take
+  // the configuration of that length and values per thread and its twiddles
+  int st = c.fftL.init(c.L, LineFFT::row_variant(c.L, row_config_with(c.L, c.Lp)));
   if (st) return st;
-  if (c.fftL.kind != LineFFT::LDS || !c.fftL.tw.p)
+  if (c.fftL.kind != LineFFT::LDS || c.fftL.rc.p != c.Lp || !c.fftL.tw.p)
     return fail(OVX_ERR_UNSUPPORTED, "no register-Stockham configuration for segment length %d", c.L);
-  if ((st = c.hpad.alloc((size_t)c.L * 8))) return st;
-  if ((st = c.H.alloc((size_t)c.L * 8))) return st;
-  return OVX_OK;
+  return ols_fuse_ref(c) ? OVX_OK : c.H.alloc((size_t)c.L * 8);
 }
 
 // H = FFT_L(h padded); h is a device pointer of M values
 static int ols_spectrum(CorrState &c, const float2 *h, int reverse, hipStream_t s)
 {
-  hipError_t e = launch_ols_prep(h, c.M, reverse, (float2 *)c.hpad.p, c.L, s);
-  if (e != hipSuccess) return hip_fail(e, "kernel padding");
-  return c.fftL.transform(-1, (const float2 *)c.hpad.p, c.L, (float2 *)c.H.p, c.L, 1, 1.0f, s);
+  hipError_t e = launch_ols_spectrum(c.L, c.Lp, h, c.M, reverse, (float2 *)c.H.p, (const float2 *)c.fftL.tw.p, s);
+  return e == hipSuccess ? OVX_OK : hip_fail(e, "kernel spectrum");
 }
 
-static int ols_run(CorrState &c, const float2 *in, float2 *out, int conj_input, int unbiased, hipStream_t s)
+// ref: the correlation's reference when its spectrum is not in c.H
+static int ols_run(CorrState &c, const float2 *ref, const float2 *in, float2 *out, int conj_input, int unbiased,
+                   hipStream_t s)
 {
-  if (c.fftL.kind != LineFFT::LDS || !c.fftL.tw.p || !c.H.p)
+  if (c.fftL.kind != LineFFT::LDS || !c.fftL.tw.p || !(ref || c.H.p))
     return fail(OVX_ERR_STATE, "overlap-save plan has no twiddle table");
-  OlsArgs a;
+  OlsArgs a{};
   a.in = in;
   a.N = c.N;
   a.M = c.M;
-  a.H = (const float2 *)c.H.p;
+  a.H = ref ? nullptr : (const float2 *)c.H.p;
+  a.h = ref;
   a.tw = (const float2 *)c.fftL.tw.p;
   a.scale = 1.0f / (float)c.L;
   a.conj_input = conj_input;
   a.unbiased = unbiased;
   a.support = c.support;
-  a.decimation = c.D;
+  a.decimation = c.P > 1 ? c.D : 1; // a single output is c[out_off] whatever the decimation
+  a.dmagic = ols_magic(a.decimation);
   a.out_off = c.out_off;
   a.c_first = c.out_off;
   a.c_step = c.L - (c.M - 1);
   a.P = c.P;
   a.out = out;
-  long span = (c.P - 1) * c.D + 1; // c indices needed
-  long segments = (span + a.c_step - 1) / a.c_step;
-  hipError_t e = launch_ols(c.L, a, segments, s);
+  hipError_t e = launch_ols(c.L, c.Lp, a, segment_count(c, c.L), s);
   if (e != hipSuccess) return hip_fail(e, "overlap-save launch");
   return OVX_OK;
 }
@@ -127,7 +146,7 @@ size_t ovx_plan_s::device_bytes() const
   size_t b = line.device_bytes() + stage_in.bytes + stage_out.bytes + stage_w.bytes + u256.bytes + wtab.bytes +
              split_ws.bytes;
   if (corr)
-    b += corr->fftL.device_bytes() + corr->hpad.bytes + corr->H.bytes + corr->ref_stage.bytes +
+    b += corr->fftL.device_bytes() + corr->H.bytes + corr->ref_stage.bytes +
          corr->in_stage.bytes + corr->out_stage.bytes;
   return b;
 }
@@ -189,8 +208,9 @@ extern "C" int ovx_corr_exec(ovx_plan p, int bias, const void *ref, const void *
     din = (const float2 *)c.in_stage.p;
     dout = (float2 *)c.out_stage.p;
   }
-  if ((st = ols_spectrum(c, dref, 1, s))) return st;
-  if ((st = ols_run(c, din, dout, 1, bias == OVX_UNBIASED, s))) return st;
+  const bool fuse = ols_fuse_ref(c);
+  if (!fuse && (st = ols_spectrum(c, dref, 1, s))) return st;
+  if ((st = ols_run(c, fuse ? dref : nullptr, din, dout, 1, bias == OVX_UNBIASED, s))) return st;
   if (host) {
     hipError_t e = hipMemcpyAsync(out, c.out_stage.p, (size_t)c.P * 8, hipMemcpyDeviceToHost, s);
     if (e == hipSuccess) e = hipStreamSynchronize(s);
@@ -276,7 +296,7 @@ extern "C" int ovx_conv_exec(ovx_plan p, const void *in, void *out, void *stream
     din = (const float2 *)c.in_stage.p;
     dout = (float2 *)c.out_stage.p;
   }
-  if ((st = ols_run(c, din, dout, 0, 0, s))) return st;
+  if ((st = ols_run(c, nullptr, din, dout, 0, 0, s))) return st;
   if (host) {
     hipError_t e = hipMemcpyAsync(out, c.out_stage.p, (size_t)c.P * 8, hipMemcpyDeviceToHost, s);
     if (e == hipSuccess) e = hipStreamSynchronize(s);

@@ -13,58 +13,78 @@
 // gathers g[i0 - (M-1) + u] (zero outside [0, N)), runs forward FFT,
 // multiplies by H = FFT_L(h) / L, inverse FFT, and scatters the valid outputs
 // u >= M-1, applying the unbiased divisors (correlation) or the decimation
-// (convolution).  One block per segment; every segment is one "row".
+// (convolution).  One workgroup per segment.
+//
+// A call is bound by the latency of one segment's chain of stages (a 65536 x
+// 1024 correlation has 65 segments for 256 CUs), so short segments run with 8
+// values per thread (2048 points: 4.9 us with 8, 5.8 with 16) and one segment
+// per workgroup (four of 512 points in one: 4.2 against 3.4 us).  A
+// correlation's reference comes with the call; its spectrum is computed by
+// every segment for itself while the segment's input is on its way, which
+// adds 1.6 us to a 2048-point segment where a launch of its own took 3.4 us
+// and more.  With thousands of segments the extra transform is work, not
+// latency (3900 of 1024 points: 16.2 to 19.8 us), and H is computed once
+// (ols_fuse_ref).  65536 x 1024: 18.1 us in three launches before, 7.6 us now;
+// 10^6 x 129 taps, every fourth output: 12.4 and 6.5 us.
 #include "ovx_ols_dev.hpp"
 
 namespace ovx {
 
-template <int L, int P>
+template <int L, int P, bool REF>
 __global__ __launch_bounds__(L / P) void k_ols(OlsArgs a)
 {
   __shared__ float2 lds[Engine<L, P>::LROW];
-  ols_body<L, P>(a, blockIdx.x, threadIdx.x, lds);
+  ols_body<L, P, REF>(a, blockIdx.x, 0, threadIdx.x, lds);
 }
 
-// h_pad[u] = reversed (corr) or plain (conv) kernel, zero-padded to L
-__global__ void k_ols_prep(const float2 *__restrict__ h, long M, int reverse, float2 *__restrict__ out, long L)
+// H = FFT_L of the reversed (correlation) or plain (convolution) kernel,
+// zero-padded to L.
+template <int L, int P>
+__global__ __launch_bounds__(L / P) void k_ols_spectrum(const float2 *__restrict__ h, long M, int reverse,
+                                                        float2 *__restrict__ H, const float2 *__restrict__ tw)
 {
-  long u = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (u >= L) return;
-  float2 v = make_float2(0.f, 0.f);
-  if (u < M) v = h[reverse ? (M - 1 - u) : u];
-  out[u] = v;
+  using E = Engine<L, P, line_in_wave(L / P)>;
+  __shared__ float2 lds[E::LROW];
+  const int t = threadIdx.x;
+  float2 v[P];
+  ols_load_kernel<L, P>(h, M, reverse != 0, t, v);
+  E::template fft<-1>(v, lds, t, make_rsrc(tw, (uint32_t)(E::plan.twtotal + 1) * 8u));
+#pragma unroll
+  for (int q = 0; q < P; ++q) H[t + E::T * q] = v[q];
 }
 
-template <int L>
-static hipError_t do_ols(const OlsArgs &a, long segments, hipStream_t s)
-{
-  constexpr int P = L >= 16 ? 16 : L;
-  hipLaunchKernelGGL((k_ols<L, P>), dim3((unsigned)segments), dim3(L / P), 0, s, a);
-  return hipGetLastError();
-}
+// X(L, P): the compiled segments.  8 values per thread for the plans' short
+// segments; 16 for the longer ones and for every length of the server's
+// references, whose batch tiles run the same body.
+#define OVX_OLS_CONFIGS(X) \
+  X(512, 8) X(1024, 8) X(2048, 8) X(1024, 16) X(2048, 16) X(4096, 16) X(8192, 16) X(16384, 16)
 
-hipError_t launch_ols(int L, const OlsArgs &a, long segments, hipStream_t s)
+hipError_t launch_ols(int L, int P, const OlsArgs &a, long segments, hipStream_t s)
 {
   if (segments <= 0) return hipSuccess;
-  switch (L) {
-  case 64: return do_ols<64>(a, segments, s);
-  case 128: return do_ols<128>(a, segments, s);
-  case 256: return do_ols<256>(a, segments, s);
-  case 512: return do_ols<512>(a, segments, s);
-  case 1024: return do_ols<1024>(a, segments, s);
-  case 2048: return do_ols<2048>(a, segments, s);
-  case 4096: return do_ols<4096>(a, segments, s);
-  case 8192: return do_ols<8192>(a, segments, s);
-  case 16384: return do_ols<16384>(a, segments, s);
-  default: return hipErrorInvalidValue;
+  const dim3 grid((unsigned)segments);
+#define X(L_, P_)                                                                                  \
+  if (L == L_ && P == P_) {                                                                        \
+    if (a.H) hipLaunchKernelGGL((k_ols<L_, P_, false>), grid, dim3(L_ / P_), 0, s, a);             \
+    else hipLaunchKernelGGL((k_ols<L_, P_, true>), grid, dim3(L_ / P_), 0, s, a);                  \
+    return hipGetLastError();                                                                      \
   }
+  OVX_OLS_CONFIGS(X)
+#undef X
+  return hipErrorInvalidValue;
 }
 
-hipError_t launch_ols_prep(const float2 *h, long M, int reverse, float2 *out, long L, hipStream_t s)
+hipError_t launch_ols_spectrum(int L, int P, const float2 *h, long M, int reverse, float2 *H, const float2 *tw,
+                               hipStream_t s)
 {
-  long blocks = (L + 255) / 256;
-  hipLaunchKernelGGL(k_ols_prep, dim3((unsigned)blocks), dim3(256), 0, s, h, M, reverse, out, L);
-  return hipGetLastError();
+#define X(L_, P_)                                                                                                \
+  if (L == L_ && P == P_) {                                                                                      \
+    hipLaunchKernelGGL((k_ols_spectrum<L_, P_>), dim3(1), dim3(L_ / P_), 0, s, h, M, reverse, H, tw);            \
+    return hipGetLastError();                                                                                    \
+  }
+  OVX_OLS_CONFIGS(X)
+#undef X
+  return hipErrorInvalidValue;
 }
 
 } // namespace ovx

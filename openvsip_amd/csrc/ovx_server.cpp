@@ -69,7 +69,7 @@ static int corr_ref_get(int id, const CorrRef **out)
 
 static OlsArgs corr_ols_args(const CorrRef &c, const float2 *in, float2 *out, int bias)
 {
-  OlsArgs a;
+  OlsArgs a{};
   a.in = in;
   a.N = c.n;
   a.M = c.m;
@@ -320,7 +320,7 @@ int Server::launch_plain(Slot &s, Req &q)
     const CorrRef *cr;
     if ((st = corr_ref_get(r.ref, &cr))) return st;
     OlsArgs a = corr_ols_args(*cr, (const float2 *)r.x, (float2 *)r.y, r.bias);
-    hipError_t e = launch_ols(cr->L, a, corr_segments(*cr), s.stream);
+    hipError_t e = launch_ols(cr->L, 16, a, corr_segments(*cr), s.stream);
     if (e != hipSuccess) return hip_fail(e, "correlation launch");
     return OVX_OK;
   }
@@ -595,13 +595,13 @@ extern "C" int ovx_corr_reference_create(int support, long m, long n, const void
   int st = c->f.init(L, LineFFT::row_variant(L, row_config_with((int)L, 16)));
   if (st) return st;
   if (c->f.kind != LineFFT::LDS || !c->f.tw.p) return fail(OVX_ERR_UNSUPPORTED, "no segment path for L=%ld", L);
-  DevBuf href, hpad;
-  if ((st = href.alloc((size_t)m * 8)) || (st = hpad.alloc((size_t)L * 8)) || (st = c->H.alloc((size_t)L * 8)))
-    return st;
+  DevBuf href;
+  if ((st = href.alloc((size_t)m * 8)) || (st = c->H.alloc((size_t)L * 8))) return st;
   hipError_t e = hipMemcpy(href.p, ref, (size_t)m * 8, hipMemcpyHostToDevice);
-  if (e == hipSuccess) e = launch_ols_prep((const float2 *)href.p, m, 1, (float2 *)hpad.p, L, nullptr);
+  if (e == hipSuccess)
+    e = launch_ols_spectrum((int)L, 16, (const float2 *)href.p, m, 1, (float2 *)c->H.p, (const float2 *)c->f.tw.p,
+                            nullptr);
   if (e != hipSuccess) return hip_fail(e, "reference upload");
-  if ((st = c->f.transform(-1, (const float2 *)hpad.p, L, (float2 *)c->H.p, L, 1, 1.0f, nullptr))) return st;
   e = hipStreamSynchronize(nullptr);
   if (e != hipSuccess) return hip_fail(e, "reference spectrum");
   std::lock_guard<std::mutex> g(g_cref_mu);
