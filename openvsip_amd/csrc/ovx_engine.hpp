@@ -148,6 +148,11 @@ __device__ __forceinline__ float2 lds_ld(lds_ptr p, int i)
 // Block scope: every wave of the workgroup takes part in the line.
 // Wave scope: the line lives in one wavefront, whose LDS operations complete
 // in order; waiting for them (lgkmcnt 0) is enough, no workgroup barrier.
+// The empty statements keep the exchange's LDS accesses on their side of the
+// barrier: where a branch follows the exchange, the compiler has sunk its reads
+// past the closing barrier to their uses behind the branch (nothing in the
+// barrier instruction itself counts as a write to it), and another wave's next
+// exchange then overwrote values not yet read.
 template <bool WAVE>
 __device__ __forceinline__ void exchange_sync()
 {
