@@ -148,6 +148,7 @@ __device__ __forceinline__ FsArgs fs_args_of(const J &j)
   a.nbig = j.n;
   a.tw1 = j.tw0;
   a.tw2 = j.tw1;
+  a.tw2c = j.tw2c;
   a.tlo = j.tlo;
   a.thi = j.thi;
   a.sbits = j.sbits;
@@ -300,6 +301,7 @@ __global__ __launch_bounds__(FsCfg<L>::NT, 4) void k_batch_fs(const BatchJob *__
                                                                const int *__restrict__ ntiles)
 {
   using F = FsCfg<L>;
+  static_assert(F::NT / FsConv<L>::T * FsConv<L>::LROW <= F::LDS, "middle pass LDS");
   __shared__ float2 lds[F::LDS];
   const int total = *ntiles;
   const int tid = (int)threadIdx.x;
@@ -307,35 +309,35 @@ __global__ __launch_bounds__(FsCfg<L>::NT, 4) void k_batch_fs(const BatchJob *__
     const BatchTile tile = tiles[ti];
     const BatchJob &j = jobs[tile.job];
     FsArgs a = fs_args_of(j);
-    if constexpr (PASS == 0) { // column FFT * twiddle: fastconv x -> y, Fftm x -> workspace
+    if constexpr (PASS == 0) { // column FFT: fastconv x -> y, Fftm x -> workspace
       const bool fft = tile.op == BT_FS_FFT_A;
-      if (fft) a.scale = j.scale;
       a.in = j.x;
       a.ld_in = j.ldx;
       a.out = fft ? j.ws : j.y;
       a.ld_out = fft ? (long)j.n : j.ldy;
-      fs_col_body<L, F::P, F::C, 0>(a, tile.a, tile.b, tid, lds);
+      fs_col_body<L, F::P, F::C, -1>(a, tile.a, tile.b, tid, lds);
     } else if constexpr (PASS == 1) {
-      if (tile.op == BT_FS_B) { // fastconv: row FFT * W * IFFT * twiddle in place on y
+      if (tile.op == BT_FS_B) { // fastconv: middle pass in place on y
         a.in = j.y;
         a.ld_in = j.ldy;
         a.out = j.y;
         a.ld_out = j.ldy;
-        fs_row_body<L, F::P, F::C, 0>(a, tile.a, tile.b, tid, lds);
+        fs_conv_body<L, F::NT / FsConv<L>::T>(a, tile.a, tile.b >> kTileRowsShift,
+                                              tile.b & ((1 << kTileRowsShift) - 1), tid, lds);
       } else { // Fftm: workspace -> y in natural order, scaled
         a.scale = j.scale;
         a.in = j.ws;
         a.ld_in = j.n;
         a.out = j.y;
         a.ld_out = j.ldy;
-        fs_row_body<L, F::P, F::C, 1>(a, tile.a, tile.b, tid, lds);
+        fs_row_body<L, F::P, F::C, -1>(a, tile.a, tile.b, tid, lds);
       }
     } else { // fastconv pass 3: column IFFT in place on y
       a.in = j.y;
       a.ld_in = j.ldy;
       a.out = j.y;
       a.ld_out = j.ldy;
-      fs_col_body<L, F::P, F::C, 1>(a, tile.a, tile.b, tid, lds);
+      fs_col_body<L, F::P, F::C, +1>(a, tile.a, tile.b, tid, lds);
     }
     __syncthreads(); // LDS reuse by the next tile
   }
@@ -387,6 +389,13 @@ int batch_fs_lines_per_group(int n_line)
 {
   if (n_line == 256) return FsCfg<256>::C;
   if (n_line == 512) return FsCfg<512>::C;
+  return 0;
+}
+
+int batch_fs_conv_lines_per_group(int n_line)
+{
+  if (n_line == 256) return FsCfg<256>::NT / FsConv<256>::T;
+  if (n_line == 512) return FsCfg<512>::NT / FsConv<512>::T;
   return 0;
 }
 

@@ -13,7 +13,7 @@ enum BatchOp {
   BT_HIER_FASTCONV = 1, // rows [a, a + rows_per_tile) of a hierarchical-path job
   BT_ROW_FASTCONV = 2,  // rows [a, ...) of a register-Stockham-path job
   BT_FS_A = 3,          // four-step fastconv pass 1: row a, column group b
-  BT_FS_B = 4,          // pass 2: row a, line group b
+  BT_FS_B = 4,          // pass 2: rows from a, line group b
   BT_FS_C = 5,          // pass 3: row a, column group b
   BT_HIER_FFT_FWD = 6,  // forward Fftm rows of a hierarchical-path job
   BT_ROW_FFT_FWD = 7,   // forward Fftm rows of a register-Stockham-path job
@@ -33,6 +33,7 @@ struct BatchJob {
   const float2 *w;   // prepared spectrum (path layout, 1/n folded in)
   const float2 *tw0; // HIER: outer table; ROW: engine table; FS: n1 line table
   const float2 *tw1; // HIER: 1024-point wave table; FS: n2 line table
+  const float2 *tw2c; // FS: n2 line table of a fastconv's middle pass
   const float2 *tlo, *thi;
   int sbits;
   const float2 *tfull; // FS: full twiddle table or null
@@ -47,8 +48,9 @@ struct BatchTile {
   int job;
   int op;
   int a; // first row
-  int b; // line group (four-step)
+  int b; // line group (four-step); BT_FS_B: rows << kTileRowsShift | line group
 };
+constexpr int kTileRowsShift = 16;
 
 // Tile queues of a batch: queue 0 holds the LDS-resident tiles (rows,
 // overlap-save segments) of the 1024-thread persistent launch, queue
@@ -85,6 +87,7 @@ inline int batch_ols_queue(int L) { return batch_ols_mid_routed(L) ? kMidQueue :
 int batch_rows_per_tile(int path, int n);
 int batch_ols_segments_per_tile(int L);
 int batch_fs_lines_per_group(int n_line); // C of a four-step group of lines of length n_line
+int batch_fs_conv_lines_per_group(int n_line); // of a fastconv's middle pass
 int batch_fs_blocks_per_cu(int n_line);   // co-resident workgroups of a four-step pass launch
 bool batch_supported(int path, int n);
 

@@ -15,6 +15,7 @@
 
 #include "ovx_batch.hpp"
 #include "ovx_batch_host.hpp"
+#include "ovx_fourstep.hpp"
 #include "ovx_plan.hpp"
 
 namespace ovx {
@@ -111,6 +112,7 @@ int make_batch_job(const LineFFT &f, long rows, const float2 *x, long ldx, float
   } else {
     j.tw0 = (const float2 *)f.tw1.p;
     j.tw1 = (const float2 *)f.tw2.p;
+    j.tw2c = f.tw2c;
     j.tlo = (const float2 *)f.tlo.p;
     j.thi = (const float2 *)f.thi.p;
     j.sbits = f.sbits;
@@ -122,10 +124,37 @@ int make_batch_job(const LineFFT &f, long rows, const float2 *x, long ldx, float
   return OVX_OK;
 }
 
+long batch_conv_workgroups(int n1, int n2, long rows) { return rows * (n1 / batch_fs_conv_lines_per_group(n2)); }
+
+// Column-pass tiles of rows [r0, r1): eight rows at a time, their tiles in
+// turn, so that the workgroups of a row land on one XCD (the standalone
+// passes' placement).
+static void push_col_tiles(std::vector<BatchTile> &q, const BatchJob &j, int ji, int op, long r0, long r1)
+{
+  const int groups = j.n2 / batch_fs_lines_per_group(j.n1);
+  for (long r = r0; r < r1; r += 8)
+    for (int g = 0; g < groups; ++g)
+      for (long k = r; k < std::min(r + 8, r1); ++k) q.push_back(BatchTile{ ji, op, (int)k, g });
+}
+
+// The three passes of rows [r0, r1) of a four-step fastconv, one line group
+// per tile and `conv_rows` rows per middle-pass tile.
+static void push_fs_tiles(const BatchJob &j, int ji, long r0, long r1, int conv_rows,
+                          std::vector<BatchTile> q[kBatchQueues])
+{
+  push_col_tiles(q[fs_queue(0, j.n1)], j, ji, BT_FS_A, r0, r1);
+  const int lines = j.n1 / batch_fs_conv_lines_per_group(j.n2);
+  std::vector<BatchTile> &b = q[fs_queue(1, j.n2)];
+  for (long r = r0; r < r1; r += conv_rows)
+    for (int g = 0; g < lines; ++g)
+      b.push_back(BatchTile{ ji, BT_FS_B, (int)r, (int)std::min<long>(conv_rows, r1 - r) << kTileRowsShift | g });
+  push_col_tiles(q[fs_queue(2, j.n1)], j, ji, BT_FS_C, r0, r1);
+}
+
 // Tiles of job `ji`: LDS-resident rows go to the queue of their persistent
 // launch (batch_queue), the three four-step passes to their (pass, line
-// length) queues, one line group per tile.
-void make_batch_tiles(const BatchJob &j, int ji, std::vector<BatchTile> q[kBatchQueues])
+// length) queues.
+void make_batch_tiles(const BatchJob &j, int ji, std::vector<BatchTile> q[kBatchQueues], int conv_rows)
 {
   if (j.path == BP_HIER || j.path == BP_ROW) {
     int rpt = batch_rows_per_tile(j.path, j.n);
@@ -134,55 +163,57 @@ void make_batch_tiles(const BatchJob &j, int ji, std::vector<BatchTile> q[kBatch
     for (long r = 0; r < j.rows; r += rpt) dst.push_back(BatchTile{ ji, op, (int)r, 0 });
     return;
   }
-  const int gcol = j.n2 / batch_fs_lines_per_group(j.n1), grow = j.n1 / batch_fs_lines_per_group(j.n2);
-  std::vector<BatchTile> &a = q[fs_queue(0, j.n1)], &b = q[fs_queue(1, j.n2)], &c = q[fs_queue(2, j.n1)];
-  for (long r = 0; r < j.rows; ++r) {
-    for (int g = 0; g < gcol; ++g) a.push_back(BatchTile{ ji, BT_FS_A, (int)r, g });
-    for (int g = 0; g < grow; ++g) b.push_back(BatchTile{ ji, BT_FS_B, (int)r, g });
-    for (int g = 0; g < gcol; ++g) c.push_back(BatchTile{ ji, BT_FS_C, (int)r, g });
-  }
+  push_fs_tiles(j, ji, 0, j.rows, conv_rows, q);
 }
 
 std::vector<TileQueue> chunked_fs_queues(const std::vector<BatchJob> &jobs, const std::vector<int> &order,
                                          size_t chunk_bytes)
 {
+  struct Part {
+    int ji;
+    long r0, r1;
+  };
   std::vector<TileQueue> out;
-  std::vector<BatchTile> cq[kBatchQueues];
+  std::vector<Part> chunk;
   size_t used = 0;
   auto flush = [&] {
+    long workgroups = 0;
+    for (const Part &p : chunk) workgroups += batch_conv_workgroups(jobs[p.ji].n1, jobs[p.ji].n2, p.r1 - p.r0);
+    std::vector<BatchTile> cq[kBatchQueues];
+    for (const Part &p : chunk) push_fs_tiles(jobs[p.ji], p.ji, p.r0, p.r1, fs_conv_rows(workgroups), cq);
     for (int k = 1; k < kFsQueueEnd; ++k)
-      if (!cq[k].empty()) {
-        out.push_back(TileQueue{ fs_queue_line(k), fs_queue_pass(k), std::move(cq[k]) });
-        cq[k].clear();
-      }
+      if (!cq[k].empty()) out.push_back(TileQueue{ fs_queue_line(k), fs_queue_pass(k), std::move(cq[k]) });
+    chunk.clear();
     used = 0;
   };
   for (int ji : order) {
     const BatchJob &j = jobs[(size_t)ji];
     if (j.path != BP_FS) continue;
     const size_t row_bytes = (size_t)j.n * 8;
-    const int gcol = j.n2 / batch_fs_lines_per_group(j.n1), grow = j.n1 / batch_fs_lines_per_group(j.n2);
-    const int qa = fs_queue(0, j.n1), qb = fs_queue(1, j.n2), qc = fs_queue(2, j.n1);
-    for (long r = 0; r < j.rows; ++r) {
-      if (used > 0 && used + row_bytes > chunk_bytes) flush();
-      for (int g = 0; g < gcol; ++g) cq[qa].push_back(BatchTile{ ji, BT_FS_A, (int)r, g });
-      for (int g = 0; g < grow; ++g) cq[qb].push_back(BatchTile{ ji, BT_FS_B, (int)r, g });
-      for (int g = 0; g < gcol; ++g) cq[qc].push_back(BatchTile{ ji, BT_FS_C, (int)r, g });
-      used += row_bytes;
+    for (long r = 0; r < j.rows;) {
+      // as many rows as the chunk takes, at least one into an empty chunk
+      long fit = used < chunk_bytes ? (long)((chunk_bytes - used) / row_bytes) : 0;
+      if (fit == 0 && used > 0) {
+        flush();
+        continue;
+      }
+      fit = std::min(std::max(fit, 1l), j.rows - r);
+      chunk.push_back(Part{ ji, r, r + fit });
+      used += (size_t)fit * row_bytes;
+      r += fit;
     }
   }
-  flush();
+  if (!chunk.empty()) flush();
   return out;
 }
 
 void make_batch_fft_tiles(const BatchJob &j, int ji, std::vector<BatchTile> q[kBatchQueues])
 {
-  const int gcol = j.n2 / batch_fs_lines_per_group(j.n1), grow = j.n1 / batch_fs_lines_per_group(j.n2);
-  std::vector<BatchTile> &a = q[fs_queue(0, j.n1)], &b = q[fs_queue(1, j.n2)];
-  for (long r = 0; r < j.rows; ++r) {
-    for (int g = 0; g < gcol; ++g) a.push_back(BatchTile{ ji, BT_FS_FFT_A, (int)r, g });
-    for (int g = 0; g < grow; ++g) b.push_back(BatchTile{ ji, BT_FS_FFT_B, (int)r, g });
-  }
+  push_col_tiles(q[fs_queue(0, j.n1)], j, ji, BT_FS_FFT_A, 0, j.rows);
+  const int lines = j.n1 / batch_fs_lines_per_group(j.n2);
+  std::vector<BatchTile> &b = q[fs_queue(1, j.n2)];
+  for (long r = 0; r < j.rows; ++r)
+    for (int g = 0; g < lines; ++g) b.push_back(BatchTile{ ji, BT_FS_FFT_B, (int)r, g });
 }
 
 hipError_t capture_batch_launches(const BatchJob *jobs, BatchTile *const tiles[kBatchQueues], int *meta,
@@ -373,7 +404,7 @@ extern "C" int ovx_batch_commit(ovx_batch b, void *stream)
   // length) queue of a chunk, in pass order.
   std::vector<BatchTile> q[kBatchQueues];
   for (int i : order)
-    if (b->djobs[i].path != BP_FS) make_batch_tiles(b->djobs[i], i, q);
+    if (b->djobs[i].path != BP_FS) make_batch_tiles(b->djobs[i], i, q, 1);
   std::vector<TileQueue> queues;
   if (!q[0].empty()) queues.push_back(TileQueue{ 0, 0, std::move(q[0]) });
   if (!q[kMidQueue].empty()) queues.push_back(TileQueue{ kMidLine, 0, std::move(q[kMidQueue]) });

@@ -26,8 +26,13 @@ int batch_path_of(const LineFFT &f);
 int device_cu_count();
 int make_batch_job(const LineFFT &f, long rows, const float2 *x, long ldx, float2 *y, long ldy, const float2 *wprep,
                    BatchJob *job);
-// Tiles of job `ji` appended to the batch's queues (kBatchQueues of them).
-void make_batch_tiles(const BatchJob &j, int ji, std::vector<BatchTile> q[kBatchQueues]);
+// Tiles of job `ji` appended to the batch's queues (kBatchQueues of them);
+// conv_rows: rows per tile of a four-step job's middle pass.
+void make_batch_tiles(const BatchJob &j, int ji, std::vector<BatchTile> q[kBatchQueues], int conv_rows);
+// Middle-pass workgroups of one row each that `rows` rows of a four-step job
+// of n = n1 * n2 points make (fs_conv_rows turns their sum over a launch into
+// rows per tile).
+long batch_conv_workgroups(int n1, int n2, long rows);
 // Four-step forward Fftm tiles (x -> workspace -> y) of job `ji`.
 void make_batch_fft_tiles(const BatchJob &j, int ji, std::vector<BatchTile> q[kBatchQueues]);
 // Capture the launches of a batch into `graph` on stream `cap`: the

@@ -76,15 +76,15 @@ int DevBuf::alloc(size_t n)
 }
 
 // ---------------------------------------------------------------- line transforms
-// Build the twiddle table for an LDS-resident configuration.
-static int make_row_twiddles(const RowConfig &rc, DevBuf &tw)
+// Build the twiddle table for an LDS-resident configuration, with room for
+// `room` more entries after it; without `wait` the caller synchronizes.
+static int make_row_twiddles(const RowConfig &rc, DevBuf &tw, size_t room = 0, bool wait = true)
 {
-  size_t n = (size_t)std::max(rc.plan.twtotal, 1);
+  size_t n = (size_t)std::max(rc.plan.twtotal, 1) + room;
   int st = tw.alloc(n * sizeof(float2));
   if (st) return st;
   hipError_t e = launch_twiddles(rc.plan, (float2 *)tw.p, nullptr);
-  if (e != hipSuccess) return hip_fail(e, "twiddle kernel");
-  e = hipStreamSynchronize(nullptr);
+  if (e == hipSuccess && wait) e = hipStreamSynchronize(nullptr);
   if (e != hipSuccess) return hip_fail(e, "twiddle kernel");
   return OVX_OK;
 }
@@ -142,11 +142,17 @@ int LineFFT::init(long n_, int variant_)
         !row_config((int)n2, row_config_with((int)n2, 16), &rc2))
       return fail(OVX_ERR_UNSUPPORTED, "no line configuration for %ld x %ld", n1, n2);
     int st;
-    if ((st = make_row_twiddles(rc1, tw1)) || (st = make_row_twiddles(rc2, tw2))) return st;
+    if ((st = make_row_twiddles(rc1, tw1, 0, false)) ||
+        (st = make_row_twiddles(rc2, tw2, (size_t)fs_conv_twiddle_count(n2), false)))
+      return st;
+    float2 *conv = (float2 *)tw2.p + rc2.plan.twtotal;
+    tw2c = conv;
+    hipError_t e = launch_fs_conv_twiddles(n2, conv, nullptr);
+    if (e != hipSuccess) return hip_fail(e, "four-step twiddles");
     sbits = (lg + 1) / 2;
     long lo = 1l << sbits, hi = (n + lo - 1) / lo;
     if ((st = tlo.alloc(lo * 8)) || (st = thi.alloc(hi * 8))) return st;
-    hipError_t e = launch_unit_roots(n, lo, (float2 *)tlo.p, nullptr);
+    e = launch_unit_roots(n, lo, (float2 *)tlo.p, nullptr);
     if (e == hipSuccess) e = launch_unit_roots(n / lo, hi, (float2 *)thi.p, nullptr);
     if (e == hipSuccess && n <= kFsFullTwiddleMax) {
       // one coalesced load per element instead of two gathered ones and a
@@ -170,6 +176,7 @@ static FsArgs fs_args(const LineFFT &f)
   a.nbig = f.n;
   a.tw1 = (const float2 *)f.tw1.p;
   a.tw2 = (const float2 *)f.tw2.p;
+  a.tw2c = f.tw2c;
   a.tlo = (const float2 *)f.tlo.p;
   a.thi = (const float2 *)f.thi.p;
   a.sbits = f.sbits;
@@ -199,7 +206,7 @@ bool LineFFT::tables_ready() const
   switch (kind) {
   case LDS: return tw.p != nullptr;
   case HIER: return tw_outer.p != nullptr && tw_wave.p != nullptr && tw.p != nullptr;
-  case FOURSTEP: return tw1.p && tw2.p && tlo.p && thi.p;
+  case FOURSTEP: return tw1.p && tw2.p && tw2c && tlo.p && thi.p;
   default: return false;
   }
 }
@@ -265,14 +272,14 @@ int LineFFT::transform_ws(int dir, const float2 *in, long ld_in, float2 *out, lo
     a.ld_in = ld_in;
     a.out = ws;
     a.ld_out = n;
-    hipError_t e = launch_fs_col(dir < 0 ? 0 : 2, a, lines, s);
+    hipError_t e = launch_fs_col(dir, a, lines, s);
     if (e != hipSuccess) return hip_fail(e, "four-step column pass");
     a.in = ws;
     a.ld_in = n;
     a.out = out;
     a.ld_out = ld_out;
     a.scale = scale;
-    e = launch_fs_row(dir < 0 ? 1 : 2, a, lines, s);
+    e = launch_fs_row(dir, a, lines, s);
     if (e != hipSuccess) return hip_fail(e, "four-step row pass");
     return OVX_OK;
   }
@@ -334,7 +341,7 @@ int LineFFT::transform_split(int dir, const float *in_re, const float *in_im, lo
     a.ld_in = ld_in;
     a.out = (float2 *)work.p;
     a.ld_out = n;
-    hipError_t e = launch_fs_col(dir < 0 ? 0 : 2, a, lines, s);
+    hipError_t e = launch_fs_col(dir, a, lines, s);
     if (e != hipSuccess) return hip_fail(e, "four-step column pass");
     FsArgs b = fs_args(*this);
     b.in = (const float2 *)work.p;
@@ -343,7 +350,7 @@ int LineFFT::transform_split(int dir, const float *in_re, const float *in_im, lo
     b.out_im = out_im;
     b.ld_out = ld_out;
     b.scale = scale;
-    e = launch_fs_row(dir < 0 ? 1 : 2, b, lines, s);
+    e = launch_fs_row(dir, b, lines, s);
     return e == hipSuccess ? OVX_OK : hip_fail(e, "four-step row pass");
   }
   if (kind == LDS) {
@@ -436,16 +443,16 @@ int LineFFT::fastconv_split(const float *xr, const float *xi, long ldx, const fl
     a.ld_in = ldx;
     a.out = ws;
     a.ld_out = n;
-    if ((e = launch_fs_col(0, a, lines, s)) != hipSuccess) return hip_fail(e, "four-step column pass");
+    if ((e = launch_fs_col(-1, a, lines, s)) != hipSuccess) return hip_fail(e, "four-step column pass");
     a.in_re = a.in_im = nullptr;
     a.in = ws;
     a.ld_in = n;
-    if ((e = launch_fs_row(0, a, lines, s)) != hipSuccess) return hip_fail(e, "four-step row pass");
+    if ((e = launch_fs_conv(a, lines, s)) != hipSuccess) return hip_fail(e, "four-step row pass");
     a.out = nullptr;
     a.out_re = yr;
     a.out_im = yi;
     a.ld_out = ldy;
-    if ((e = launch_fs_col(1, a, lines, s)) != hipSuccess) return hip_fail(e, "four-step column pass");
+    if ((e = launch_fs_col(+1, a, lines, s)) != hipSuccess) return hip_fail(e, "four-step column pass");
     return OVX_OK;
   }
   if (kind == LDS || (kind == HIER && ldw != 0)) {
@@ -520,11 +527,11 @@ int LineFFT::fs_fastconv(const float2 *x, long ldx, const float2 *wprep, long ld
   a.out = y;
   a.ld_out = ldy;
   hipError_t e;
-  if ((e = launch_fs_col(0, a, lines, s)) != hipSuccess) return hip_fail(e, "four-step column pass");
+  if ((e = launch_fs_col(-1, a, lines, s)) != hipSuccess) return hip_fail(e, "four-step column pass");
   a.in = y;
   a.ld_in = ldy;
-  if ((e = launch_fs_row(0, a, lines, s)) != hipSuccess) return hip_fail(e, "four-step row pass");
-  if ((e = launch_fs_col(1, a, lines, s)) != hipSuccess) return hip_fail(e, "four-step column pass");
+  if ((e = launch_fs_conv(a, lines, s)) != hipSuccess) return hip_fail(e, "four-step row pass");
+  if ((e = launch_fs_col(+1, a, lines, s)) != hipSuccess) return hip_fail(e, "four-step column pass");
   return OVX_OK;
 }
 

@@ -160,7 +160,9 @@ __device__ __forceinline__ void exchange_sync()
     __builtin_amdgcn_s_waitcnt(0xc07f); // lgkmcnt(0), vmcnt/expcnt untouched
     __builtin_amdgcn_wave_barrier();
   } else {
+    asm volatile("" ::: "memory");
     __syncthreads();
+    asm volatile("" ::: "memory");
   }
 }
 
@@ -232,11 +234,53 @@ struct Engine {
     }
   }
 
+  // All twiddles of a thread in registers, loaded once for several transforms
+  // (a forward and an inverse transform use the same ones): stage S's
+  // M (R - 1) values from held_off(S).
+  static constexpr int held_off(int S)
+  {
+    int o = 0;
+    for (int s = 0; s < S; ++s)
+      if (plan.ns[s] > 1) o += (P / plan.radix[s]) * (plan.radix[s] - 1);
+    return o;
+  }
+  static constexpr int HELD = held_off(NST) > 0 ? held_off(NST) : 1;
+  template <int S = 0>
+  __device__ __forceinline__ static void load_held(int t, rsrc_t tw, float2 (&w)[HELD])
+  {
+    if constexpr (S < NST) {
+      constexpr int R = plan.radix[S], Ns = plan.ns[S], M = P / R;
+      if constexpr (Ns > 1) {
+#pragma unroll
+        for (int m = 0; m < M; ++m) {
+          const int k = (t + m * T) % Ns;
+#pragma unroll
+          for (int r = 1; r < R; ++r)
+            w[held_off(S) + m * (R - 1) + r - 1] =
+                bload(tw, (uint32_t)k * 8u, (uint32_t)(plan.twoff[S] + (r - 1) * Ns) * 8u);
+        }
+      }
+      load_held<S + 1>(t, tw, w);
+    }
+  }
+
   // One stage.  tw: concatenated forward twiddle table (FP32 values of FP64
   // W_{Ns R}^{r k}, layout tw[twoff_s + (r-1)*Ns + k]); w: this stage's
   // twiddles (loaded by the previous stage, or by the caller for stage 0).
   template <int S, int DIR, typename LP>
   __device__ __forceinline__ static void stage(float2 (&v)[P], LP lds, int t, rsrc_t tw, float2 (&w)[P])
+  {
+    butterflies<S, DIR>(v, lds, t, w, 0);
+    if constexpr (S != NST - 1) {
+      load_tw<S + 1>(t, tw, w);
+      read_back(v, lds, t);
+    }
+  }
+
+  // The arithmetic of stage S (its twiddles in w from `off`) and, unless it is
+  // the last, the write half of its exchange.
+  template <int S, int DIR, typename LP, int NW>
+  __device__ __forceinline__ static void butterflies(float2 (&v)[P], LP lds, int t, const float2 (&w)[NW], int off)
   {
     constexpr int R = plan.radix[S];
     constexpr int Ns = plan.ns[S];
@@ -250,7 +294,7 @@ struct Engine {
       const int j = t + m * T;
       if constexpr (Ns > 1) {
 #pragma unroll
-        for (int r = 1; r < R; ++r) a[r] = twmul<DIR>(a[r], w[m * (R - 1) + r - 1]);
+        for (int r = 1; r < R; ++r) a[r] = twmul<DIR>(a[r], w[off + m * (R - 1) + r - 1]);
       }
       Dft<R, DIR>::run(a);
       if constexpr (last) {
@@ -268,19 +312,21 @@ struct Engine {
         }
       }
     }
-    if constexpr (!last) {
-      load_tw<S + 1>(t, tw, w);
-      exchange_sync<WAVE>();
-      if constexpr (read_split()) {
-        const int b = Layout::idx(t);
+  }
+  // The read half of an exchange.
+  template <typename LP>
+  __device__ __forceinline__ static void read_back(float2 (&v)[P], LP lds, int t)
+  {
+    exchange_sync<WAVE>();
+    if constexpr (read_split()) {
+      const int b = Layout::idx(t);
 #pragma unroll
-        for (int q = 0; q < P; ++q) v[q] = lds_ld(lds, b + Layout::step(T * q));
-      } else {
+      for (int q = 0; q < P; ++q) v[q] = lds_ld(lds, b + Layout::step(T * q));
+    } else {
 #pragma unroll
-        for (int q = 0; q < P; ++q) v[q] = lds_ld(lds, Layout::idx(t + T * q));
-      }
-      exchange_sync<WAVE>();
+      for (int q = 0; q < P; ++q) v[q] = lds_ld(lds, Layout::idx(t + T * q));
     }
+    exchange_sync<WAVE>();
   }
 
   // One stage on its own (a caller that runs a single stage).
@@ -310,6 +356,17 @@ struct Engine {
     float2 w[P];
     load_tw<0>(t, tw, w); // stage 0 has Ns = 1: nothing
     stages_from<0, DIR>(v, lds, t, tw, w);
+  }
+
+  // The same with the twiddles held in registers (load_held).
+  template <int DIR, int S = 0, typename LP>
+  __device__ __forceinline__ static void fft_held(float2 (&v)[P], LP lds, int t, const float2 (&w)[HELD])
+  {
+    if constexpr (S < NST) {
+      butterflies<S, DIR>(v, lds, t, w, held_off(S));
+      if constexpr (S != NST - 1) read_back(v, lds, t);
+      fft_held<DIR, S + 1>(v, lds, t, w);
+    }
   }
 };
 

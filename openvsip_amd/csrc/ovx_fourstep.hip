@@ -3,9 +3,10 @@
 //
 // A line of N = N1*N2 is viewed as an N1 x N2 row-major matrix,
 // n = N2*n1 + n2.  Forward:
-//   column pass:  B[k1][n2] = W_N^{n2 k1} * sum_n1 A[n1][n2] W_N1^{n1 k1}
-//   row pass:     X[k1 + N1 k2] = sum_n2 B[k1][n2] W_N2^{n2 k2}
-// Inverse (k = k1 + N1 k2, n = N2 n1 + n2):
+//   column pass:  B[k1][n2] = sum_n1 A[n1][n2] W_N1^{n1 k1}
+//   row pass:     X[k1 + N1 k2] = sum_n2 W_N^{n2 k1} B[k1][n2] W_N2^{n2 k2}
+// The inverse is the same with conjugate factors; the way back of a fastconv
+// runs the passes in the other order:
 //   row pass:     U[k1][n2] = W_N^{-n2 k1} * sum_k2 X[k1 + N1 k2] W_N2^{-n2 k2}
 //   column pass:  x[N2 n1 + n2] = sum_k1 U[k1][n2] W_N1^{-n1 k1}
 // Fftm uses column pass + row pass with an LDS-staged transposed store
@@ -22,18 +23,52 @@
 
 namespace ovx {
 
-template <int L, int P, int C, int MODE, bool SIN, bool SOUT>
-__global__ __launch_bounds__(C *(L / P)) void k_fs_col(FsArgs a)
+// Row and column group of workgroup w: the groups of a row on one XCD
+// (workgroups go to the eight XCDs in turn), so that its accesses cover whole
+// matrix rows, not every eighth 128-byte run of each, which at a row of
+// 256 columns left an XCD two of its L2's sixteen channels.  256 x 256 lines,
+// 256 rows: 58 to 52 us; 512 x 512: 62 to 58.
+__device__ __forceinline__ void fs_place(unsigned w, unsigned groups, unsigned rows, long &row, long &group)
 {
-  __shared__ float2 lds_all[C * FsLds<L>::LROW];
-  fs_col_body<L, P, C, MODE, SIN, SOUT>(a, blockIdx.y, blockIdx.x, threadIdx.x, lds_all);
+  const unsigned whole = rows & ~7u;
+  if (w < whole * groups) {
+    row = (w / 8 / groups) * 8 + w % 8;
+    group = (w / 8) % groups;
+  } else {
+    const unsigned r = w - whole * groups;
+    row = whole + r / groups;
+    group = r % groups;
+  }
 }
 
-template <int L, int P, int C, int MODE, bool SOUT>
+template <int L, int P, int C, int DIR, bool SIN, bool SOUT>
+__global__ __launch_bounds__(C *(L / P)) void k_fs_col(FsArgs a, unsigned groups, unsigned rows)
+{
+  __shared__ float2 lds_all[C * FsLds<L>::LROW];
+  long row, group;
+  fs_place(blockIdx.x, groups, rows, row, group);
+  fs_col_body<L, P, C, DIR, SIN, SOUT>(a, row, group, threadIdx.x, lds_all);
+}
+
+template <int L, int P, int C, int DIR, bool SOUT>
 __global__ __launch_bounds__(C *(L / P)) void k_fs_row(FsArgs a)
 {
   __shared__ float2 lds_all[C * FsLds<L>::LROW];
-  fs_row_body<L, P, C, MODE, SOUT>(a, blockIdx.y, blockIdx.x, threadIdx.x, lds_all);
+  fs_row_body<L, P, C, DIR, SOUT>(a, blockIdx.y, blockIdx.x, threadIdx.x, lds_all);
+}
+
+// 256 threads: fewer lines per workgroup leave it sooner (C = 16 / 4 at 512:
+// 56 / 53 us)
+template <int L>
+struct FsConvCfg {
+  static constexpr int C = 256 / FsConv<L>::T;
+};
+template <int L>
+__global__ __launch_bounds__(256, 4) void k_fs_conv(FsArgs a, int rows, int per)
+{
+  __shared__ float2 lds_all[FsConvCfg<L>::C * FsConv<L>::LROW];
+  const int row0 = (int)blockIdx.y * per;
+  fs_conv_body<L, FsConvCfg<L>::C>(a, row0, min(per, rows - row0), blockIdx.x, threadIdx.x, lds_all);
 }
 
 // Wp[k1][k2] = scale * W[k1 + N1 k2] for `rows` coefficient rows (ldw = 0:
@@ -62,66 +97,96 @@ struct FsSplitCfg {
   static constexpr int NT = C * (L / P);
 };
 
-template <int L, int MODE>
+template <int L, int DIR>
 static hipError_t col_launch(const FsArgs &a, long rows, hipStream_t s)
 {
   using F = FsCfg<L>;
   using G = FsSplitCfg<L>;
   // split storage is read by a call's first pass or written by its last
+  const bool split = a.in_re || a.out_re;
+  const unsigned groups = (unsigned)(a.n2 / (split ? G::C : F::C));
+  const dim3 grid(groups * (unsigned)rows);
   if (a.in_re)
-    hipLaunchKernelGGL((k_fs_col<L, G::P, G::C, MODE, true, false>), dim3((unsigned)(a.n2 / G::C), (unsigned)rows),
-                       dim3(G::NT), 0, s, a);
+    hipLaunchKernelGGL((k_fs_col<L, G::P, G::C, DIR, true, false>), grid, dim3(G::NT), 0, s, a, groups, (unsigned)rows);
   else if (a.out_re)
-    hipLaunchKernelGGL((k_fs_col<L, G::P, G::C, MODE, false, true>), dim3((unsigned)(a.n2 / G::C), (unsigned)rows),
-                       dim3(G::NT), 0, s, a);
+    hipLaunchKernelGGL((k_fs_col<L, G::P, G::C, DIR, false, true>), grid, dim3(G::NT), 0, s, a, groups, (unsigned)rows);
   else
-    hipLaunchKernelGGL((k_fs_col<L, F::P, F::C, MODE, false, false>), dim3((unsigned)(a.n2 / F::C), (unsigned)rows),
-                       dim3(F::NT), 0, s, a);
+    hipLaunchKernelGGL((k_fs_col<L, F::P, F::C, DIR, false, false>), grid, dim3(F::NT), 0, s, a, groups,
+                       (unsigned)rows);
   return hipGetLastError();
 }
 
-template <int L, int MODE>
+template <int L, int DIR>
 static hipError_t row_launch(const FsArgs &a, long rows, hipStream_t s)
 {
   using F = FsCfg<L>;
   using G = FsSplitCfg<L>;
   if (a.out_re)
-    hipLaunchKernelGGL((k_fs_row<L, G::P, G::C, MODE, true>), dim3((unsigned)(a.n1 / G::C), (unsigned)rows),
+    hipLaunchKernelGGL((k_fs_row<L, G::P, G::C, DIR, true>), dim3((unsigned)(a.n1 / G::C), (unsigned)rows),
                        dim3(G::NT), 0, s, a);
   else
-    hipLaunchKernelGGL((k_fs_row<L, F::P, F::C, MODE, false>), dim3((unsigned)(a.n1 / F::C), (unsigned)rows),
+    hipLaunchKernelGGL((k_fs_row<L, F::P, F::C, DIR, false>), dim3((unsigned)(a.n1 / F::C), (unsigned)rows),
                        dim3(F::NT), 0, s, a);
+  return hipGetLastError();
+}
+
+// Rows per workgroup of the middle pass: as many as leave 8 workgroups a CU
+// (four rows) or 4 (two): 512 x 512 lines, 64 rows, 1 / 2 / 4 / 8 rows 56 / 46
+// / 44 / 51 us; 256 x 256, 64 rows, 18.4 / 17.8 / 19.5 / 24.0.
+int fs_conv_rows(long workgroups)
+{
+  return workgroups >= 4 * 2048 ? 4 : workgroups >= 2 * 1024 ? 2 : 1;
+}
+
+template <int L>
+static hipError_t conv_launch(const FsArgs &a, long rows, hipStream_t s)
+{
+  const long groups = a.n1 / FsConvCfg<L>::C;
+  const int per = fs_conv_rows(groups * rows);
+  hipLaunchKernelGGL((k_fs_conv<L>), dim3((unsigned)groups, (unsigned)((rows + per - 1) / per)), dim3(256), 0, s, a,
+                     (int)rows, per);
   return hipGetLastError();
 }
 
 #define OVX_FS_LENGTHS(X) X(128) X(256) X(512) X(1024) X(2048)
 
-hipError_t launch_fs_col(int mode, const FsArgs &a, long rows, hipStream_t s)
+hipError_t launch_fs_col(int dir, const FsArgs &a, long rows, hipStream_t s)
 {
   switch (a.n1) {
-#define X(L)                                                  \
-  case L:                                                     \
-    if (mode == 0) return col_launch<L, 0>(a, rows, s);       \
-    if (mode == 1) return col_launch<L, 1>(a, rows, s);       \
-    return col_launch<L, 2>(a, rows, s);
+#define X(L) \
+  case L: return dir < 0 ? col_launch<L, -1>(a, rows, s) : col_launch<L, +1>(a, rows, s);
     OVX_FS_LENGTHS(X)
 #undef X
   default: return hipErrorInvalidValue;
   }
 }
 
-hipError_t launch_fs_row(int mode, const FsArgs &a, long rows, hipStream_t s)
+hipError_t launch_fs_row(int dir, const FsArgs &a, long rows, hipStream_t s)
 {
   switch (a.n2) {
-#define X(L)                                                  \
-  case L:                                                     \
-    if (mode == 0) return row_launch<L, 0>(a, rows, s);       \
-    if (mode == 1) return row_launch<L, 1>(a, rows, s);       \
-    return row_launch<L, 2>(a, rows, s);
+#define X(L) \
+  case L: return dir < 0 ? row_launch<L, -1>(a, rows, s) : row_launch<L, +1>(a, rows, s);
     OVX_FS_LENGTHS(X)
 #undef X
   default: return hipErrorInvalidValue;
   }
+}
+
+hipError_t launch_fs_conv(const FsArgs &a, long rows, hipStream_t s)
+{
+  switch (a.n2) {
+#define X(L) \
+  case L: return conv_launch<L>(a, rows, s);
+    OVX_FS_LENGTHS(X)
+#undef X
+  default: return hipErrorInvalidValue;
+  }
+}
+
+int fs_conv_twiddle_count(long l) { return make_plan((int)l, FsConv<128>::P).twtotal; }
+hipError_t launch_fs_conv_twiddles(long l, float2 *tw, hipStream_t s)
+{
+  return launch_twiddles(make_plan((int)l, FsConv<128>::P), tw, s);
 }
 
 // tfull[k1 * n2 + c] = W_N^{k1 c}, N = n1 n2, from FP64 values rounded once.

@@ -11,6 +11,7 @@ struct FsArgs {
   long ld_out;
   long n1, n2, nbig;       // N = n1 * n2
   const float2 *tw1, *tw2; // line twiddles of the n1 and n2 plans
+  const float2 *tw2c;      // of the n2 plan of a fastconv's middle pass
   const float2 *tlo, *thi; // W_N^m = thi[m >> sbits] * tlo[m & (2^sbits - 1)]
   int sbits;
   const float2 *tfull;     // W_N^{k1 n2} at [k1 * n2count + n2], or null (two-level)
@@ -23,8 +24,16 @@ struct FsArgs {
   float *out_re = nullptr, *out_im = nullptr;
 };
 
-hipError_t launch_fs_col(int mode, const FsArgs &a, long rows, hipStream_t s);
-hipError_t launch_fs_row(int mode, const FsArgs &a, long rows, hipStream_t s);
+// Column pass of `rows` rows in direction dir; row pass of a transform; middle
+// pass of a fastconv.
+hipError_t launch_fs_col(int dir, const FsArgs &a, long rows, hipStream_t s);
+hipError_t launch_fs_row(int dir, const FsArgs &a, long rows, hipStream_t s);
+hipError_t launch_fs_conv(const FsArgs &a, long rows, hipStream_t s);
+// rows per workgroup of a middle pass of that many workgroups of one row
+int fs_conv_rows(long workgroups);
+// twiddle entries of a middle pass over lines of length l, and the table
+int fs_conv_twiddle_count(long l);
+hipError_t launch_fs_conv_twiddles(long l, float2 *tw, hipStream_t s);
 hipError_t launch_fs_permute(const float2 *w, long ldw, float2 *wp, long n1, long n2, long rows, float scale,
                              hipStream_t s);
 bool fs_length_supported(long l);

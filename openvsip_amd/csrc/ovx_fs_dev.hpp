@@ -23,9 +23,10 @@ __device__ __forceinline__ float2 big_twiddle(const float2 *__restrict__ tlo, co
 }
 
 // ---------------------------------------------------------------- column pass
-// MODE 0: forward column FFT, then * W_N^{n2 k1}      (fastconv / Fftm pass 1)
-// MODE 1: inverse column FFT, then * scale             (fastconv pass 3)
-// MODE 2: inverse column FFT, then * W_N^{-n2 k1}      (inverse Fftm pass 1)
+// Column FFT in direction DIR, times a.scale unless 1.  The twiddle
+// W_N^{n2 k1} between the two passes is applied by the row pass, where a line's
+// table entries are contiguous and serve both sides of a fastconv: read here,
+// at the columns' stride, they cost 15 us of a 67 us pass over 134 MB.
 // One group of C columns of one row: `group` selects columns
 // [group*C, group*C + C), `tid` is the thread within the group's C*(L/P)
 // threads, `lds_all` the group's C*LROW LDS elements.
@@ -49,7 +50,7 @@ __device__ __forceinline__ void fs_store(const FsArgs &a, long o, float2 v)
   }
 }
 
-template <int L, int P, int C, int MODE, bool SIN = false, bool SOUT = false, typename LP>
+template <int L, int P, int C, int DIR, bool SIN = false, bool SOUT = false, typename LP>
 __device__ __forceinline__ void fs_col_body(const FsArgs &a, long row, long group, int tid, LP lds_all)
 {
   using E = Engine<L, P>;
@@ -66,26 +67,8 @@ __device__ __forceinline__ void fs_col_body(const FsArgs &a, long row, long grou
   float2 v[P];
 #pragma unroll
   for (int q = 0; q < P; ++q) v[q] = fs_load<SIN>(a, ib + (long)(t + T * q) * N2);
-  if constexpr (MODE == 0) E::template fft<-1>(v, lds, t, rtw);
-  else E::template fft<+1>(v, lds, t, rtw);
-  if constexpr (MODE == 0 || MODE == 2) {
-    if (a.tfull) { // lanes of consecutive columns read consecutive entries
-      const float2 *tf = a.tfull + n2;
-#pragma unroll
-      for (int q = 0; q < P; ++q) {
-        float2 w = tf[(long)(t + T * q) * N2];
-        v[q] = (MODE == 0) ? cmul(v[q], w) : cmulc(v[q], w);
-      }
-    } else {
-#pragma unroll
-      for (int q = 0; q < P; ++q) {
-        const uint32_t k1 = (uint32_t)(t + T * q);
-        const uint32_t m = (uint32_t)n2 * k1; // < N1*N2: no reduction needed
-        float2 w = big_twiddle(a.tlo, a.thi, a.sbits, m);
-        v[q] = (MODE == 0) ? cmul(v[q], w) : cmulc(v[q], w);
-      }
-    }
-  } else {
+  E::template fft<DIR>(v, lds, t, rtw);
+  if (a.scale != 1.0f) {
 #pragma unroll
     for (int q = 0; q < P; ++q) v[q] = cscale(v[q], a.scale);
   }
@@ -94,17 +77,31 @@ __device__ __forceinline__ void fs_col_body(const FsArgs &a, long row, long grou
 }
 
 // ---------------------------------------------------------------- row pass
-// MODE 0: fastconv middle pass (in place allowed):
-//         forward row FFT, * Wp[k1][k2], inverse row FFT, * W_N^{-n2 k1}
-// MODE 1: forward row FFT, transposed store X[k1 + N1 k2], * scale
-// MODE 2: inverse row FFT, transposed store,               * scale
-// One group of C lines k1 in [group*C, group*C + C) of one row.
-template <int L, int P, int C, int MODE, bool SOUT = false, typename LP>
+// The twiddles W_N^{k1 n2} of line k1 at the thread's positions n2 = t + T q.
+template <int L, int P>
+__device__ __forceinline__ void fs_line_twiddles(const FsArgs &a, long k1, int t, float2 (&w)[P])
+{
+  constexpr int T = L / P;
+  if (a.tfull) {
+    const float2 *tf = a.tfull + k1 * L;
+#pragma unroll
+    for (int q = 0; q < P; ++q) w[q] = tf[t + T * q];
+  } else {
+#pragma unroll
+    for (int q = 0; q < P; ++q)
+      w[q] = big_twiddle(a.tlo, a.thi, a.sbits, (uint32_t)(t + T * q) * (uint32_t)k1); // < N1 N2
+  }
+}
+
+// Row pass of a transform in direction DIR: * W_N^{-+ k1 n2}, row FFT,
+// transposed store X[k1 + N1 k2], * scale.  One group of C lines k1 in
+// [group*C, group*C + C) of one row.
+template <int L, int P, int C, int DIR, bool SOUT = false, typename LP>
 __device__ __forceinline__ void fs_row_body(const FsArgs &a, long row, long group, int tid, LP lds_all)
 {
   // a line's L/P threads are consecutive; when they fit one wavefront its
   // exchanges need no workgroup barrier
-  using E = Engine<L, P, (L / P <= 64)>;
+  using E = Engine<L, P, line_in_wave(L / P)>;
   constexpr int T = E::T;
   constexpr int LROW = FsLds<L>::LROW;
   const int c = tid / T; // consecutive threads walk along a line
@@ -115,47 +112,86 @@ __device__ __forceinline__ void fs_row_body(const FsArgs &a, long row, long grou
   LP lds = lds_all + c * LROW;
   const float2 *src = a.in + row * a.ld_in + k1 * L;
 
-  float2 v[P];
+  float2 v[P], w[P];
 #pragma unroll
   for (int q = 0; q < P; ++q) v[q] = src[t + T * q];
-  if constexpr (MODE == 0) {
-    E::template fft<-1>(v, lds, t, rtw);
-    const float2 *wp = a.wp + row * a.ldwp + k1 * L;
+  fs_line_twiddles<L, P>(a, k1, t, w);
 #pragma unroll
-    for (int q = 0; q < P; ++q) v[q] = cmul(v[q], wp[t + T * q]);
-    E::template fft<+1>(v, lds, t, rtw);
-    if (a.tfull) {
-      const float2 *tf = a.tfull + k1 * L;
+  for (int q = 0; q < P; ++q) v[q] = twmul<DIR>(v[q], w[q]);
+  E::template fft<DIR>(v, lds, t, rtw);
+  if (a.scale != 1.0f) {
 #pragma unroll
-      for (int q = 0; q < P; ++q) v[q] = cmulc(v[q], tf[t + T * q]);
-    } else {
+    for (int q = 0; q < P; ++q) v[q] = cscale(v[q], a.scale);
+  }
+  // transpose through LDS: element k2 of line c -> out[k1_0 + c + N1 k2]
 #pragma unroll
-      for (int q = 0; q < P; ++q) {
-        const uint32_t n2 = (uint32_t)(t + T * q);
-        const uint32_t m = n2 * (uint32_t)k1;
-        v[q] = cmulc(v[q], big_twiddle(a.tlo, a.thi, a.sbits, m));
-      }
+  for (int q = 0; q < P; ++q) lds_st(lds, t + T * q, v[q]);
+  __syncthreads();
+  const int c2 = tid % C;
+  const int t2 = tid / C;
+  LP lsrc = lds_all + c2 * LROW;
+  const long ob = row * a.ld_out + group * C + c2;
+#pragma unroll
+  for (int q = 0; q < P; ++q) fs_store<SOUT>(a, ob + (long)(t2 + T * q) * N1, lds_ld(lsrc, t2 + T * q));
+}
+
+// Middle pass of a fastconv (in place allowed): * W_N^{k1 n2}, forward row
+// FFT, * Wp[k1][k2], inverse row FFT, * W_N^{-k1 n2}; C lines of rows row0 ..
+// row0 + nrows - 1.  A line's stage twiddles, its W_N entries (the same on both
+// sides) and, with one spectrum for all rows, its spectrum stay in registers
+// over the rows: what bounded this pass was neither HBM nor latency but the
+// loads through L1, 110 of which for 16 values of a line were tables and stage
+// twiddles against 16 of data.  8 values per thread leave the registers for
+// them (100 of 128 VGPRs; with 16 the 512-point lines spill).  512 x 512
+// lines, 64 rows: 63 us with every table read where it is used, 53 with the
+// stage twiddles held, 56 with 8 values and W_N held as well (and none of it
+// left to the column pass), 46 over 2 rows and 44 over 4; the same loads and
+// stores alone take 40.
+template <int L>
+struct FsConv {
+  static constexpr int P = 8;
+  static constexpr int T = L / P;
+  static constexpr int LROW = LdsLayout<L, P>::elems | 1;
+};
+template <int L, int C, typename LP>
+__device__ __forceinline__ void fs_conv_body(const FsArgs &a, long row0, int nrows, long group, int tid, LP lds_all)
+{
+  constexpr int P = FsConv<L>::P, T = FsConv<L>::T;
+  using E = Engine<L, P, line_in_wave(T)>;
+  const int c = tid / T;
+  const int t = tid % T;
+  const long k1 = group * C + c;
+  const rsrc_t rtw = make_rsrc(a.tw2c, (uint32_t)(E::plan.twtotal + 1) * 8u);
+  LP lds = lds_all + c * FsConv<L>::LROW;
+  const float2 *src = a.in + row0 * a.ld_in + k1 * L + t;
+  float2 *dst = a.out + row0 * a.ld_out + k1 * L + t;
+  const float2 *wp = a.wp + row0 * a.ldwp + k1 * L + t;
+
+  float2 w[P], ws[P], st[E::HELD];
+  fs_line_twiddles<L, P>(a, k1, t, w);
+#pragma unroll
+  for (int q = 0; q < P; ++q) ws[q] = wp[T * q];
+  E::load_held(t, rtw, st);
+#pragma unroll 1
+  for (int r = 0; r < nrows; ++r) {
+    float2 v[P];
+#pragma unroll
+    for (int q = 0; q < P; ++q) v[q] = src[T * q];
+#pragma unroll
+    for (int q = 0; q < P; ++q) v[q] = cmul(v[q], w[q]);
+    E::template fft_held<-1>(v, lds, t, st);
+#pragma unroll
+    for (int q = 0; q < P; ++q) v[q] = cmul(v[q], ws[q]);
+    if (a.ldwp && r + 1 < nrows) { // one spectrum per row: the next one
+      wp += a.ldwp;
+#pragma unroll
+      for (int q = 0; q < P; ++q) ws[q] = wp[T * q];
     }
-    const long ob = row * a.ld_out + k1 * L;
+    E::template fft_held<+1>(v, lds, t, st);
 #pragma unroll
-    for (int q = 0; q < P; ++q) fs_store<SOUT>(a, ob + t + T * q, v[q]);
-  } else {
-    if constexpr (MODE == 1) E::template fft<-1>(v, lds, t, rtw);
-    else E::template fft<+1>(v, lds, t, rtw);
-    if (a.scale != 1.0f) {
-#pragma unroll
-      for (int q = 0; q < P; ++q) v[q] = cscale(v[q], a.scale);
-    }
-    // transpose through LDS: element k2 of line c -> out[k1_0 + c + N1 k2]
-#pragma unroll
-    for (int q = 0; q < P; ++q) lds_st(lds, t + T * q, v[q]);
-    __syncthreads();
-    const int c2 = tid % C;
-    const int t2 = tid / C;
-    LP lsrc = lds_all + c2 * LROW;
-    const long ob = row * a.ld_out + group * C + c2;
-#pragma unroll
-    for (int q = 0; q < P; ++q) fs_store<SOUT>(a, ob + (long)(t2 + T * q) * N1, lds_ld(lsrc, t2 + T * q));
+    for (int q = 0; q < P; ++q) dst[T * q] = cmulc(v[q], w[q]);
+    src += a.ld_in;
+    dst += a.ld_out;
   }
 }
 

@@ -52,6 +52,7 @@ struct LineFFT {
   int sbits = 0;
   RowConfig rc1, rc2;
   DevBuf tw1, tw2, tlo, thi, tfull;
+  const float2 *tw2c = nullptr; // lines of a fastconv's middle pass, in tw2 after its own
   mutable DevBuf work, wp; // Fftm workspace, permuted spectrum
 
   int init(long n, int variant);

@@ -29,6 +29,7 @@
 
 #include "ovx_batch.hpp"
 #include "ovx_batch_host.hpp"
+#include "ovx_fourstep.hpp"
 #include "ovx_hier.hpp"
 #include "ovx_ols.hpp"
 #include "ovx_plan.hpp"
@@ -249,6 +250,14 @@ int Server::admit_and_launch(Slot &s, std::vector<Req *> &batch)
   std::vector<BatchJob> jobs;
   std::vector<BatchTile> q[kBatchQueues];
   size_t ws_off = 0;
+  long conv_wgs = 0; // middle-pass workgroups of the batch's four-step fastconvs
+  for (const Req *q0 : batch) {
+    int st;
+    const LineFFT *f = q0->r.kind == OVX_REQ_FASTCONV ? shared_path(q0->r.n, q0->r.rows, &st) : nullptr;
+    if (f && f->kind == LineFFT::FOURSTEP && batch_supported(BP_FS, (int)f->n))
+      conv_wgs += batch_conv_workgroups((int)f->n1, (int)f->n2, q0->r.rows);
+  }
+  const int conv_rows = fs_conv_rows(conv_wgs);
   for (size_t i = 0; i < batch.size(); ++i) {
     const ovx_request &r = batch[i]->r;
     int st;
@@ -274,7 +283,7 @@ int Server::admit_and_launch(Slot &s, std::vector<Req *> &batch)
       if ((st = replica_prepared(r.ref, &prep, &rn, f))) return st;
       if ((st = make_batch_job(*f, r.rows, (const float2 *)r.x, r.ldx, (float2 *)r.y, r.ldy, prep, &j))) return st;
       jobs.push_back(j);
-      make_batch_tiles(j, (int)i, q);
+      make_batch_tiles(j, (int)i, q, conv_rows);
     } else { // forward Fftm
       if ((st = make_batch_job(*f, r.rows, (const float2 *)r.x, r.ldx, (float2 *)r.y, r.ldy, nullptr, &j))) return st;
       j.scale = 1.0f;

@@ -283,7 +283,7 @@ int autotune_batch(long n, long rows, int *best_variant, double *best_us)
     if ((st = make_batch_job(f, rows, (const float2 *)x.p, n, (float2 *)y.p, n, (const float2 *)wp.p, &j))) break;
     std::vector<BatchJob> jobs(1, j);
     std::vector<BatchTile> q[kBatchQueues];
-    make_batch_tiles(j, 0, q);
+    make_batch_tiles(j, 0, q, 1);
     std::vector<TileQueue> queues;
     if (!q[0].empty()) queues.push_back(TileQueue{ 0, 0, std::move(q[0]) });
     if (!q[kMidQueue].empty()) queues.push_back(TileQueue{ kMidLine, 0, std::move(q[kMidQueue]) });
