@@ -32,105 +32,98 @@ struct BatchLds {
   static constexpr int value = NT == kBatchThreads ? kBatchLds : kBatchMidLds;
 };
 
-// The job descriptor of the current tile lives in LDS (copied once per tile
-// by the persistent loop); the tile functions read it from there.
-typedef __attribute__((address_space(3))) const BatchJob lds_job;
-
-// The tile functions are called (not inlined), so the compiler cannot see
-// that the descriptor is the same for every lane: pointers read from LDS
-// would sit in vector registers and every buffer access built on them would
-// need a loop over the distinct values.  Each field a tile function uses is
-// read into scalar registers through uniform().
-template <typename T>
-__device__ __forceinline__ T uniform(const __attribute__((address_space(3))) T &f)
+// A tile function's thread number, taken anew for each tile: what it computes
+// from it (LDS and memory offsets, table entries) cannot be moved out of the
+// loop over tiles, where the offsets of every size at once would not fit the
+// registers.  (Inlined without this the two kernels keep 268 and 1048 bytes a
+// thread in scratch memory; as functions that are called, the tile functions
+// each save and restore up to 49 registers a tile: 24 uneven instances,
+// 694 MB, 356 us called and 352 inlined.)
+__device__ __forceinline__ int tile_thread()
 {
-  static_assert(sizeof(T) % 4 == 0, "dword copy");
-  T u;
-  const __attribute__((address_space(3))) int *src = (const __attribute__((address_space(3))) int *)&f;
-  int *dst = (int *)&u;
-#pragma unroll
-  for (int i = 0; i < (int)(sizeof(T) / 4); ++i) dst[i] = __builtin_amdgcn_readfirstlane(src[i]);
-  return u;
+  int t = (int)threadIdx.x;
+  asm volatile("" : "+v"(t));
+  return t;
 }
 
 // Tile functions of a workgroup of NT threads: NT / (threads of a row) rows
 // (or overlap-save segments) per tile.
 template <int NT, int N>
-__device__ __noinline__ void tile_hier_fastconv(lds_job &j, int row0_arg, lds_ptr lds)
+__device__ __forceinline__ void tile_hier_fastconv(const BatchJob &j, int row0, lds_ptr lds)
 {
-  const int row0 = __builtin_amdgcn_readfirstlane(row0_arg); // uniform, see uniform()
   using H = Hier<N>;
   static_assert(NT % H::TR == 0 && (NT / H::TR) * H::LROW <= BatchLds<NT>::value, "tile LDS");
   HierArgs a{};
-  a.x = uniform(j.x);
-  a.ldx = uniform(j.ldx);
-  a.y = uniform(j.y);
-  a.ldy = uniform(j.ldy);
-  a.w = uniform(j.w);
-  a.rows = uniform(j.rows);
-  a.tw_outer = uniform(j.tw0);
-  a.tw_wave = uniform(j.tw1);
-  const int lrow = (int)threadIdx.x / H::TR;
-  const int t = (int)threadIdx.x % H::TR;
+  a.x = j.x;
+  a.ldx = j.ldx;
+  a.y = j.y;
+  a.ldy = j.ldy;
+  a.w = j.w;
+  a.rows = j.rows;
+  a.tw_outer = j.tw0;
+  a.tw_wave = j.tw1;
+  const int tid = tile_thread();
+  const int lrow = tid / H::TR;
+  const int t = tid % H::TR;
   // a tile of one row is only made for a row that exists
-  hier_fastconv_body<N, NT / H::TR == 1>(a, row0, lrow, t, lds + lrow * H::LROW);
+  hier_fastconv_body<N, NT / H::TR == 1, false>(a, row0, lrow, t, lds + lrow * H::LROW);
 }
 
 template <int NT, int N>
-__device__ __noinline__ void tile_hier_fwd(lds_job &j, int row0_arg, lds_ptr lds)
+__device__ __forceinline__ void tile_hier_fwd(const BatchJob &j, int row0, lds_ptr lds)
 {
-  const int row0 = __builtin_amdgcn_readfirstlane(row0_arg); // uniform, see uniform()
   using H = Hier<N>;
   static_assert(NT % H::TR == 0 && (NT / H::TR) * H::LROW <= BatchLds<NT>::value, "tile LDS");
   HierArgs a{};
-  a.x = uniform(j.x);
-  a.ldx = uniform(j.ldx);
-  a.y = uniform(j.y);
-  a.ldy = uniform(j.ldy);
-  a.rows = uniform(j.rows);
-  a.tw_outer = uniform(j.tw0);
-  a.tw_wave = uniform(j.tw1);
-  a.scale = uniform(j.scale);
-  const int lrow = (int)threadIdx.x / H::TR;
-  const int t = (int)threadIdx.x % H::TR;
+  a.x = j.x;
+  a.ldx = j.ldx;
+  a.y = j.y;
+  a.ldy = j.ldy;
+  a.rows = j.rows;
+  a.tw_outer = j.tw0;
+  a.tw_wave = j.tw1;
+  a.scale = j.scale;
+  const int tid = tile_thread();
+  const int lrow = tid / H::TR;
+  const int t = tid % H::TR;
   hier_fwd_body<N>(a, row0, lrow, t, lds + lrow * H::LROW);
 }
 
 template <int NT, int N, int P>
-__device__ __noinline__ void tile_row_fastconv(lds_job &j, int row0_arg, lds_ptr lds)
+__device__ __forceinline__ void tile_row_fastconv(const BatchJob &j, int row0, lds_ptr lds)
 {
-  const int row0 = __builtin_amdgcn_readfirstlane(row0_arg); // uniform, see uniform()
   using E = Engine<N, P, line_in_wave(N / P)>;
   static_assert(NT % E::T == 0 && (NT / E::T) * E::LROW <= BatchLds<NT>::value, "tile LDS");
-  const int lrow = (int)threadIdx.x / E::T;
-  const int t = (int)threadIdx.x % E::T;
-  row_fastconv_body<N, P>(uniform(j.x), uniform(j.ldx), uniform(j.w), 0, uniform(j.y), uniform(j.ldy),
-                          uniform(j.rows), uniform(j.tw0), 1.0f, row0, lrow, t, lds + lrow * E::LROW);
+  const int tid = tile_thread();
+  const int lrow = tid / E::T;
+  const int t = tid % E::T;
+  row_fastconv_body<N, P>(j.x, j.ldx, j.w, 0, j.y, j.ldy,
+                          j.rows, j.tw0, 1.0f, row0, lrow, t, lds + lrow * E::LROW);
 }
 
 template <int NT, int N, int P>
-__device__ __noinline__ void tile_row_fwd(lds_job &j, int row0_arg, lds_ptr lds)
+__device__ __forceinline__ void tile_row_fwd(const BatchJob &j, int row0, lds_ptr lds)
 {
-  const int row0 = __builtin_amdgcn_readfirstlane(row0_arg); // uniform, see uniform()
   using E = Engine<N, P, line_in_wave(N / P)>;
   static_assert(NT % E::T == 0 && (NT / E::T) * E::LROW <= BatchLds<NT>::value, "tile LDS");
-  const int lrow = (int)threadIdx.x / E::T;
-  const int t = (int)threadIdx.x % E::T;
-  row_fft_body<N, P, -1>(uniform(j.x), uniform(j.ldx), uniform(j.y), uniform(j.ldy), uniform(j.rows),
-                         uniform(j.tw0), uniform(j.scale), row0, lrow, t, lds + lrow * E::LROW);
+  const int tid = tile_thread();
+  const int lrow = tid / E::T;
+  const int t = tid % E::T;
+  row_fft_body<N, P, -1>(j.x, j.ldx, j.y, j.ldy, j.rows,
+                         j.tw0, j.scale, row0, lrow, t, lds + lrow * E::LROW);
 }
 
 // Overlap-save segments seg0, seg0 + 1, ... (NT / (L/16) of them per tile);
 // those past the last store nothing.
 template <int NT, int L>
-__device__ __noinline__ void tile_ols(lds_job &j, int seg0_arg, lds_ptr lds)
+__device__ __forceinline__ void tile_ols(const BatchJob &j, int seg0, lds_ptr lds)
 {
-  const int seg0 = __builtin_amdgcn_readfirstlane(seg0_arg); // uniform, see uniform()
-  OlsArgs a = uniform(j.ols);
+  const OlsArgs a = j.ols;
   constexpr int T = L / 16;
   static_assert(NT % T == 0 && (NT / T) * Engine<L, 16>::LROW <= BatchLds<NT>::value, "tile LDS");
-  const int t = (int)threadIdx.x % T;
-  const int copy = (int)threadIdx.x / T;
+  const int tid = tile_thread();
+  const int t = tid % T;
+  const int copy = tid / T;
   ols_body<L, 16>(a, seg0, copy, t, lds + copy * Engine<L, 16>::LROW);
 }
 
@@ -174,7 +167,7 @@ static_assert(batch_mid_routed(BP_HIER, 8192) && !batch_mid_routed(BP_HIER, 1638
               "run in the 512-thread one");
 
 template <int NT, int N>
-__device__ __forceinline__ void run_hier(bool fwd_only, lds_job &j, int a, lds_ptr lds)
+__device__ __forceinline__ void run_hier(bool fwd_only, const BatchJob &j, int a, lds_ptr lds)
 {
   if constexpr (runs_in<NT, BP_HIER, N>()) {
     if (fwd_only) tile_hier_fwd<NT, N>(j, a, lds);
@@ -182,7 +175,7 @@ __device__ __forceinline__ void run_hier(bool fwd_only, lds_job &j, int a, lds_p
   }
 }
 template <int NT, int N, int P>
-__device__ __forceinline__ void run_row(bool fwd_only, lds_job &j, int a, lds_ptr lds)
+__device__ __forceinline__ void run_row(bool fwd_only, const BatchJob &j, int a, lds_ptr lds)
 {
   if constexpr (runs_in<NT, BP_ROW, N>()) {
     if (fwd_only) tile_row_fwd<NT, N, P>(j, a, lds);
@@ -190,7 +183,7 @@ __device__ __forceinline__ void run_row(bool fwd_only, lds_job &j, int a, lds_pt
   }
 }
 template <int NT, int L>
-__device__ __forceinline__ void run_ols(lds_job &j, int a, lds_ptr lds)
+__device__ __forceinline__ void run_ols(const BatchJob &j, int a, lds_ptr lds)
 {
   if constexpr (ols_runs_in<NT, L>()) tile_ols<NT, L>(j, a, lds);
 }
@@ -202,16 +195,13 @@ __device__ __forceinline__ void run_ols(lds_job &j, int a, lds_ptr lds)
 // per tile).
 template <int NT>
 __device__ __forceinline__ void batch_loop(const BatchJob *__restrict__ jobs, const BatchTile *__restrict__ tiles,
-                                           const int *__restrict__ ntiles, float2 *lds_mem, BatchJob *s_job)
+                                           const int *__restrict__ ntiles, float2 *lds_mem)
 {
   const lds_ptr lds = as_lds(lds_mem);
-  lds_job &j = *(lds_job *)s_job;
-  static_assert(sizeof(BatchJob) % 4 == 0 && sizeof(BatchJob) / 4 <= NT, "job copy");
   const int total = *ntiles;
   for (int ti = blockIdx.x; ti < total; ti += gridDim.x) {
     const BatchTile tile = tiles[ti];
-    if (threadIdx.x < sizeof(BatchJob) / 4) ((int *)s_job)[threadIdx.x] = ((const int *)&jobs[tile.job])[threadIdx.x];
-    __syncthreads();
+    const BatchJob &j = jobs[tile.job]; // the same for every lane: scalar loads
     switch (tile.op) {
     case BT_HIER_FASTCONV:
     case BT_HIER_FFT_FWD: {
@@ -262,19 +252,17 @@ __global__ __launch_bounds__(kBatchThreads) void k_batch(const BatchJob *__restr
                                                           const int *__restrict__ ntiles)
 {
   __shared__ float2 lds_mem[kBatchLds];
-  __shared__ BatchJob s_job;
-  batch_loop<kBatchThreads>(jobs, tiles, ntiles, lds_mem, &s_job);
+  batch_loop<kBatchThreads>(jobs, tiles, ntiles, lds_mem);
 }
 
 // Two workgroups per CU: four waves per SIMD (the second launch bound is
-// waves per SIMD; the tile functions inherit it, so they fit 128 VGPRs) and
-// 2 x (67.6 KB + the descriptor) of LDS.
+// waves per SIMD: 128 VGPRs) and
+// 2 x 67.6 KB of LDS.
 __global__ __launch_bounds__(kBatchMidThreads, kBatchMidBlocksPerCu * kBatchMidThreads / 256) void k_batch_mid(
     const BatchJob *__restrict__ jobs, const BatchTile *__restrict__ tiles, const int *__restrict__ ntiles)
 {
   __shared__ float2 lds_mem[kBatchMidLds];
-  __shared__ BatchJob s_job;
-  batch_loop<kBatchMidThreads>(jobs, tiles, ntiles, lds_mem, &s_job);
+  batch_loop<kBatchMidThreads>(jobs, tiles, ntiles, lds_mem);
 }
 
 hipError_t launch_batch(const BatchJob *jobs, const BatchTile *tiles, const int *ntiles, int grid, hipStream_t s)
