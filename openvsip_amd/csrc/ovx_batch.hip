@@ -66,7 +66,7 @@ __device__ __forceinline__ void tile_hier_fastconv(const BatchJob &j, int row0, 
   const int lrow = tid / H::TR;
   const int t = tid % H::TR;
   // a tile of one row is only made for a row that exists
-  hier_fastconv_body<N, NT / H::TR == 1, false>(a, row0, lrow, t, lds + lrow * H::LROW);
+  hier_fastconv_body<N, NT / H::TR == 1, false, N == 16384>(a, row0, lrow, t, lds + lrow * H::LROW);
 }
 
 template <int NT, int N>

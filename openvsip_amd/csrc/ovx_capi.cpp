@@ -526,11 +526,14 @@ int LineFFT::fs_fastconv(const float2 *x, long ldx, const float2 *wprep, long ld
   a.ld_in = ldx;
   a.out = y;
   a.ld_out = ldy;
+  const size_t bytes = (size_t)lines * (size_t)n * sizeof(float2);
   hipError_t e;
+  a.stream = fs_streams_in(bytes);
   if ((e = launch_fs_col(-1, a, lines, s)) != hipSuccess) return hip_fail(e, "four-step column pass");
   a.in = y;
   a.ld_in = ldy;
   if ((e = launch_fs_conv(a, lines, s)) != hipSuccess) return hip_fail(e, "four-step row pass");
+  a.stream = fs_streams_out(bytes);
   if ((e = launch_fs_col(+1, a, lines, s)) != hipSuccess) return hip_fail(e, "four-step column pass");
   return OVX_OK;
 }

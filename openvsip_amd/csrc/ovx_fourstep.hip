@@ -41,13 +41,13 @@ __device__ __forceinline__ void fs_place(unsigned w, unsigned groups, unsigned r
   }
 }
 
-template <int L, int P, int C, int DIR, bool SIN, bool SOUT>
+template <int L, int P, int C, int DIR, bool SIN, bool SOUT, bool STREAM>
 __global__ __launch_bounds__(C *(L / P)) void k_fs_col(FsArgs a, unsigned groups, unsigned rows)
 {
   __shared__ float2 lds_all[C * FsLds<L>::LROW];
   long row, group;
   fs_place(blockIdx.x, groups, rows, row, group);
-  fs_col_body<L, P, C, DIR, SIN, SOUT>(a, row, group, threadIdx.x, lds_all);
+  fs_col_body<L, P, C, DIR, SIN, SOUT, STREAM, STREAM && (DIR > 0)>(a, row, group, threadIdx.x, lds_all);
 }
 
 template <int L, int P, int C, int DIR, bool SOUT>
@@ -107,11 +107,14 @@ static hipError_t col_launch(const FsArgs &a, long rows, hipStream_t s)
   const unsigned groups = (unsigned)(a.n2 / (split ? G::C : F::C));
   const dim3 grid(groups * (unsigned)rows);
   if (a.in_re)
-    hipLaunchKernelGGL((k_fs_col<L, G::P, G::C, DIR, true, false>), grid, dim3(G::NT), 0, s, a, groups, (unsigned)rows);
+    hipLaunchKernelGGL((k_fs_col<L, G::P, G::C, DIR, true, false, false>), grid, dim3(G::NT), 0, s, a, groups, (unsigned)rows);
   else if (a.out_re)
-    hipLaunchKernelGGL((k_fs_col<L, G::P, G::C, DIR, false, true>), grid, dim3(G::NT), 0, s, a, groups, (unsigned)rows);
+    hipLaunchKernelGGL((k_fs_col<L, G::P, G::C, DIR, false, true, false>), grid, dim3(G::NT), 0, s, a, groups, (unsigned)rows);
+  else if (a.stream)
+    hipLaunchKernelGGL((k_fs_col<L, F::P, F::C, DIR, false, false, true>), grid, dim3(F::NT), 0, s, a, groups,
+                       (unsigned)rows);
   else
-    hipLaunchKernelGGL((k_fs_col<L, F::P, F::C, DIR, false, false>), grid, dim3(F::NT), 0, s, a, groups,
+    hipLaunchKernelGGL((k_fs_col<L, F::P, F::C, DIR, false, false, false>), grid, dim3(F::NT), 0, s, a, groups,
                        (unsigned)rows);
   return hipGetLastError();
 }

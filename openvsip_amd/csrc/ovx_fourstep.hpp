@@ -1,6 +1,7 @@
 // ovx_fourstep.hpp -- launch interface of the two-pass four-step kernels.
 #pragma once
 #include <hip/hip_runtime.h>
+#include <stddef.h>
 
 namespace ovx {
 
@@ -22,7 +23,19 @@ struct FsArgs {
   // imaginary arrays at the strides ld_in / ld_out); null: in / out are used
   const float *in_re = nullptr, *in_im = nullptr;
   float *out_re = nullptr, *out_im = nullptr;
+  // interleaved column pass: non-temporal loads (forward) or loads and stores
+  // (inverse), see fs_streams_in / fs_streams_out
+  bool stream = false;
 };
+
+// Whether the first / last pass of a fastconv over `bytes` of rows goes past
+// the caches: X, which is read once, should not push Y out of the 256 MB
+// Infinity Cache, nor the result the rows of Y still to be read.  All ordinary
+// / first / last / both, us: 64 MB (32 x 262144) 75 / 72 / 77 / 77, 96 MB 106 /
+// 106 / 104 / 104, 128 MB 139 / 139 / 133 / 131, 256 MB 285 / 266 / 273 / 257;
+// 256 x 65536 127 / 124 / 120 / 120; at 32 MB 41 / 43 / 48 / 49.
+inline bool fs_streams_in(size_t bytes) { return bytes >= ((size_t)64 << 20); }
+inline bool fs_streams_out(size_t bytes) { return bytes >= ((size_t)96 << 20); }
 
 // Column pass of `rows` rows in direction dir; row pass of a transform; middle
 // pass of a fastconv.

@@ -30,27 +30,31 @@ __device__ __forceinline__ float2 big_twiddle(const float2 *__restrict__ tlo, co
 // One group of C columns of one row: `group` selects columns
 // [group*C, group*C + C), `tid` is the thread within the group's C*(L/P)
 // threads, `lds_all` the group's C*LROW LDS elements.
-// The passes' global reads and writes at element offset o from a call's
-// base: interleaved lines (a.in, a.out) or, when SPLIT, separate real and
-// imaginary arrays (a.in_re / a.in_im, a.out_re / a.out_im).
-template <bool SPLIT>
-__device__ __forceinline__ float2 fs_load(const FsArgs &a, long o)
+// The passes' global reads and writes: one row's buffer, element offsets of at
+// most N values.  Interleaved lines (a.in, a.out) or, when SPLIT, separate real
+// and imaginary arrays (a.in_re / a.in_im, a.out_re / a.out_im).  NT:
+// non-temporal (fs_streams_in(), fs_streams_out()).
+template <bool SPLIT, bool NT>
+__device__ __forceinline__ auto fs_in(const FsArgs &a, long row, uint32_t lane)
 {
-  if constexpr (SPLIT) return make_float2(a.in_re[o], a.in_im[o]);
-  else return a.in[o];
+  if constexpr (SPLIT)
+    return IoSx<NT, false>{ make_rsrc(a.in_re + row * a.ld_in, 0xffffffffu),
+                            make_rsrc(a.in_im + row * a.ld_in, 0xffffffffu), lane * 4u };
+  else
+    return IoCx<NT, false>{ make_rsrc(a.in + row * a.ld_in, 0xffffffffu), lane * 8u };
 }
-template <bool SPLIT>
-__device__ __forceinline__ void fs_store(const FsArgs &a, long o, float2 v)
+template <bool SPLIT, bool NT>
+__device__ __forceinline__ auto fs_out(const FsArgs &a, long row, uint32_t lane)
 {
-  if constexpr (SPLIT) {
-    a.out_re[o] = v.x;
-    a.out_im[o] = v.y;
-  } else {
-    a.out[o] = v;
-  }
+  if constexpr (SPLIT)
+    return IoSx<false, NT>{ make_rsrc(a.out_re + row * a.ld_out, 0xffffffffu),
+                            make_rsrc(a.out_im + row * a.ld_out, 0xffffffffu), lane * 4u };
+  else
+    return IoCx<false, NT>{ make_rsrc(a.out + row * a.ld_out, 0xffffffffu), lane * 8u };
 }
 
-template <int L, int P, int C, int DIR, bool SIN = false, bool SOUT = false, typename LP>
+template <int L, int P, int C, int DIR, bool SIN = false, bool SOUT = false, bool NTL = false, bool NTS = false,
+          typename LP>
 __device__ __forceinline__ void fs_col_body(const FsArgs &a, long row, long group, int tid, LP lds_all)
 {
   using E = Engine<L, P>;
@@ -58,22 +62,23 @@ __device__ __forceinline__ void fs_col_body(const FsArgs &a, long row, long grou
   constexpr int LROW = FsLds<L>::LROW;
   const int c = tid % C;
   const int t = tid / C;
-  const long n2 = group * C + c;
-  const long N2 = a.n2;
-  const long ib = row * a.ld_in + n2, ob = row * a.ld_out + n2;
+  const uint32_t N2 = (uint32_t)a.n2;
+  const uint32_t lane = (uint32_t)t * N2 + (uint32_t)(group * C + c);
+  const auto in = fs_in<SIN, NTL>(a, row, lane);
+  const auto out = fs_out<SOUT, NTS>(a, row, lane);
   const rsrc_t rtw = make_rsrc(a.tw1, (uint32_t)(E::plan.twtotal + 1) * 8u);
   LP lds = lds_all + c * LROW;
 
   float2 v[P];
 #pragma unroll
-  for (int q = 0; q < P; ++q) v[q] = fs_load<SIN>(a, ib + (long)(t + T * q) * N2);
+  for (int q = 0; q < P; ++q) v[q] = in.ld((uint32_t)(T * q) * N2);
   E::template fft<DIR>(v, lds, t, rtw);
   if (a.scale != 1.0f) {
 #pragma unroll
     for (int q = 0; q < P; ++q) v[q] = cscale(v[q], a.scale);
   }
 #pragma unroll
-  for (int q = 0; q < P; ++q) fs_store<SOUT>(a, ob + (long)(t + T * q) * N2, v[q]);
+  for (int q = 0; q < P; ++q) out.st(v[q], (uint32_t)(T * q) * N2);
 }
 
 // ---------------------------------------------------------------- row pass
@@ -107,14 +112,14 @@ __device__ __forceinline__ void fs_row_body(const FsArgs &a, long row, long grou
   const int c = tid / T; // consecutive threads walk along a line
   const int t = tid % T;
   const long k1 = group * C + c;
-  const long N1 = a.n1;
+  const uint32_t N1 = (uint32_t)a.n1;
   const rsrc_t rtw = make_rsrc(a.tw2, (uint32_t)(E::plan.twtotal + 1) * 8u);
   LP lds = lds_all + c * LROW;
-  const float2 *src = a.in + row * a.ld_in + k1 * L;
+  const auto in = fs_in<false, false>(a, row, (uint32_t)k1 * L + t);
 
   float2 v[P], w[P];
 #pragma unroll
-  for (int q = 0; q < P; ++q) v[q] = src[t + T * q];
+  for (int q = 0; q < P; ++q) v[q] = in.ld((uint32_t)(T * q));
   fs_line_twiddles<L, P>(a, k1, t, w);
 #pragma unroll
   for (int q = 0; q < P; ++q) v[q] = twmul<DIR>(v[q], w[q]);
@@ -130,9 +135,9 @@ __device__ __forceinline__ void fs_row_body(const FsArgs &a, long row, long grou
   const int c2 = tid % C;
   const int t2 = tid / C;
   LP lsrc = lds_all + c2 * LROW;
-  const long ob = row * a.ld_out + group * C + c2;
+  const auto out = fs_out<SOUT, false>(a, row, (uint32_t)t2 * N1 + (uint32_t)(group * C + c2));
 #pragma unroll
-  for (int q = 0; q < P; ++q) fs_store<SOUT>(a, ob + (long)(t2 + T * q) * N1, lds_ld(lsrc, t2 + T * q));
+  for (int q = 0; q < P; ++q) out.st(lds_ld(lsrc, t2 + T * q), (uint32_t)(T * q) * N1);
 }
 
 // Middle pass of a fastconv (in place allowed): * W_N^{k1 n2}, forward row
@@ -163,8 +168,7 @@ __device__ __forceinline__ void fs_conv_body(const FsArgs &a, long row0, int nro
   const long k1 = group * C + c;
   const rsrc_t rtw = make_rsrc(a.tw2c, (uint32_t)(E::plan.twtotal + 1) * 8u);
   LP lds = lds_all + c * FsConv<L>::LROW;
-  const float2 *src = a.in + row0 * a.ld_in + k1 * L + t;
-  float2 *dst = a.out + row0 * a.ld_out + k1 * L + t;
+  const uint32_t lane = (uint32_t)k1 * L + t;
   const float2 *wp = a.wp + row0 * a.ldwp + k1 * L + t;
 
   float2 w[P], ws[P], st[E::HELD];
@@ -174,9 +178,11 @@ __device__ __forceinline__ void fs_conv_body(const FsArgs &a, long row0, int nro
   E::load_held(t, rtw, st);
 #pragma unroll 1
   for (int r = 0; r < nrows; ++r) {
+    const auto in = fs_in<false, false>(a, row0 + r, lane);
+    const auto out = fs_out<false, false>(a, row0 + r, lane);
     float2 v[P];
 #pragma unroll
-    for (int q = 0; q < P; ++q) v[q] = src[T * q];
+    for (int q = 0; q < P; ++q) v[q] = in.ld((uint32_t)(T * q));
 #pragma unroll
     for (int q = 0; q < P; ++q) v[q] = cmul(v[q], w[q]);
     E::template fft_held<-1>(v, lds, t, st);
@@ -189,9 +195,7 @@ __device__ __forceinline__ void fs_conv_body(const FsArgs &a, long row0, int nro
     }
     E::template fft_held<+1>(v, lds, t, st);
 #pragma unroll
-    for (int q = 0; q < P; ++q) dst[T * q] = cmulc(v[q], w[q]);
-    src += a.ld_in;
-    dst += a.ld_out;
+    for (int q = 0; q < P; ++q) out.st(cmulc(v[q], w[q]), (uint32_t)(T * q));
   }
 }
 

@@ -21,7 +21,7 @@
 namespace ovx {
 
 // ---------------------------------------------------------------- kernels
-template <int N, bool SPLIT>
+template <int N, bool SPLIT, bool NTL>
 __global__ __launch_bounds__(Hier<N>::NT) void k_hier_fastconv(HierArgs a)
 {
   using H = Hier<N>;
@@ -29,7 +29,7 @@ __global__ __launch_bounds__(Hier<N>::NT) void k_hier_fastconv(HierArgs a)
   const int lrow = (H::B == 1) ? 0 : (int)threadIdx.x / H::TR;
   const int t = (H::B == 1) ? (int)threadIdx.x : (int)threadIdx.x % H::TR;
   // one row per block and a grid of exactly `rows` blocks: every row exists
-  hier_fastconv_body<N, H::B == 1, SPLIT>(a, (long)blockIdx.x * H::B, lrow, t, lds_all + lrow * H::LROW);
+  hier_fastconv_body<N, H::B == 1, SPLIT, NTL>(a, (long)blockIdx.x * H::B, lrow, t, lds_all + lrow * H::LROW);
 }
 
 template <int N, bool SPLIT>
@@ -88,13 +88,35 @@ __global__ void k_hier_outer_twiddles(float2 *two, int n, int count)
 }
 
 // ---------------------------------------------------------------- dispatch
+// Whether a 16384-point fastconv loads X non-temporally: a row has a CU to
+// itself, and with (nearly) all of them loading at once that is the faster way,
+// with part of them idle the slower one.  Ordinary / non-temporal, us: 64 rows
+// 17.4 / 18.7, 192 20.3 / 20.6, 224 21.4 / 21.3, 256 23.8 / 22.5, 300 37.8 /
+// 39.4, 512 44.4 / 44.0, 700 59.3 / 62.3, 1000 88.4 / 84.4.  Shorter rows share
+// a CU and load faster the ordinary way at any count.
+static bool hier_streams_in(long rows)
+{
+  const long last = rows % 256;
+  return rows >= 224 && (last == 0 || last >= 224);
+}
+
 template <int N>
 static hipError_t launch_kind(int kind, const HierArgs &a, hipStream_t s)
 {
   using H = Hier<N>;
   dim3 grid((unsigned)((a.rows + H::B - 1) / H::B)), block(H::NT);
-  if (kind == HIER_FASTCONV) hipLaunchKernelGGL((k_hier_fastconv<N, false>), grid, block, 0, s, a);
-  else if (kind == HIER_FASTCONV_SPLIT) hipLaunchKernelGGL((k_hier_fastconv<N, true>), grid, block, 0, s, a);
+  if (kind == HIER_FASTCONV || kind == HIER_FASTCONV_SPLIT) {
+    const bool split = kind == HIER_FASTCONV_SPLIT;
+    if constexpr (N == 16384) {
+      if (hier_streams_in(a.rows)) {
+        if (split) hipLaunchKernelGGL((k_hier_fastconv<N, true, true>), grid, block, 0, s, a);
+        else hipLaunchKernelGGL((k_hier_fastconv<N, false, true>), grid, block, 0, s, a);
+        return hipGetLastError();
+      }
+    }
+    if (split) hipLaunchKernelGGL((k_hier_fastconv<N, true, false>), grid, block, 0, s, a);
+    else hipLaunchKernelGGL((k_hier_fastconv<N, false, false>), grid, block, 0, s, a);
+  }
   else if (kind == HIER_FWD) hipLaunchKernelGGL((k_hier_fft_fwd<N, false>), grid, block, 0, s, a);
   else if (kind == HIER_INV) hipLaunchKernelGGL((k_hier_fft_inv<N, false>), grid, block, 0, s, a);
   else if (kind == HIER_FWD_SPLIT) hipLaunchKernelGGL((k_hier_fft_fwd<N, true>), grid, block, 0, s, a);

@@ -24,14 +24,14 @@ struct Hier {
 
 // Row accessors of the input and output lines of rows row0 + lrow, thread t:
 // interleaved (a.x, a.y) or split storage (a.xr/a.xi, a.yr/a.yi).
-template <bool SPLIT>
+template <bool SPLIT, bool NTL = false>
 __device__ __forceinline__ auto hier_in(const HierArgs &a, long row0, int lrow, int t)
 {
   if constexpr (SPLIT)
-    return IoS{make_rsrc(a.xr + row0 * a.ldx, 0xffffffffu), make_rsrc(a.xi + row0 * a.ldx, 0xffffffffu),
+    return IoSx<NTL>{make_rsrc(a.xr + row0 * a.ldx, 0xffffffffu), make_rsrc(a.xi + row0 * a.ldx, 0xffffffffu),
                (uint32_t)(lrow * a.ldx + t) * 4u};
   else
-    return IoC{make_rsrc(a.x + row0 * a.ldx, 0xffffffffu), (uint32_t)(lrow * a.ldx + t) * 8u};
+    return IoCx<NTL>{make_rsrc(a.x + row0 * a.ldx, 0xffffffffu), (uint32_t)(lrow * a.ldx + t) * 8u};
 }
 template <bool SPLIT>
 __device__ __forceinline__ auto hier_out(const HierArgs &a, long row0, int lrow, int t)
@@ -108,14 +108,17 @@ __device__ __forceinline__ void outer_inverse_store(const IO &iy, bool valid, LP
 // per block, one block per row), so no row needs the check.
 // SPLIT: X and Y in split storage (a.xr/a.xi, a.yr/a.yi); the spectrum is
 // interleaved either way.
-template <int N, bool ONE_ROW = false, bool SPLIT = false, typename LP>
+// NTL: non-temporal loads of X.  The wave transform's twiddles stay in
+// registers from the forward to the inverse transform, 27 loads of the 116
+// that a wave issued: 256 x 16384 24.0 to 22.5 us, 1000 x 8192 41.7 to 36.8.
+template <int N, bool ONE_ROW = false, bool SPLIT = false, bool NTL = false, typename LP>
 __device__ __forceinline__ void hier_fastconv_body(const HierArgs &a, long row0, int lrow, int t, LP lds)
 {
   using H = Hier<N>;
   constexpr int R0 = H::R0, NW = H::NW;
   const long row = row0 + lrow;
   const bool valid = ONE_ROW || row < a.rows;
-  const auto ix = hier_in<SPLIT>(a, row0, lrow, t);
+  const auto ix = hier_in<SPLIT, NTL>(a, row0, lrow, t);
   const auto iy = hier_out<SPLIT>(a, row0, lrow, t);
   const rsrc_t rw = make_rsrc(a.w, (uint32_t)N * 8u);
   const rsrc_t rtw = make_rsrc(a.tw_wave, (uint32_t)(H::WE::plan.twtotal + 1) * 8u);
@@ -139,14 +142,16 @@ __device__ __forceinline__ void hier_fastconv_body(const HierArgs &a, long row0,
 #pragma unroll
     for (int s = 0; s < 16; ++s) u[s] = valid ? ix.ld((uint32_t)(64 * s)) : make_float2(0.f, 0.f);
   }
-  H::WE::template fft<-1>(u, sl, l, rtw);
+  float2 st[H::WE::HELD];
+  H::WE::load_held(l, rtw, st);
+  H::WE::template fft_held<-1>(u, sl, l, st);
   const uint32_t vw = (uint32_t)(k1 * NW + l) * 8u;
 #pragma unroll
   for (int s = 0; s < 16; ++s) {
     float2 ww = bload(rw, vw, (uint32_t)(64 * s) * 8u);
     u[s] = cmul(u[s], ww);
   }
-  H::WE::template fft<+1>(u, sl, l, rtw);
+  H::WE::template fft_held<+1>(u, sl, l, st);
   if constexpr (R0 > 1) {
     if (k1 > 0) {
 #pragma unroll

@@ -6,6 +6,13 @@
 
 namespace ovx {
 
+// Whether the stage twiddles stay in registers from the forward to the inverse
+// transform (30 values at most here) instead of being loaded for each: 4096
+// points, 64 / 1000 rows 7.5 / 20.4 to 7.2 / 19.5 us, 2048 6.5 / 10.3 to 5.6 /
+// 9.9.  With 8 values a thread the early loads cost the few-line forms 0.5 us,
+// and longer lines have no registers left (16384: 25 to 36 us).
+constexpr bool row_holds_twiddles(int N, int P) { return P == 16 && N >= 1024 && N <= 4096; }
+
 // Rows row0 + lrow of the job, thread t of the row's T = N/P threads, LDS row
 // region `lds` (Engine LROW elements).  Every thread of the workgroup calls
 // it; rows at or beyond `rows` compute on zeros and store nothing.  ix / iy
@@ -32,7 +39,14 @@ __device__ __forceinline__ void row_fastconv_io(const IX &ix, const IY &iy, cons
 #pragma unroll
     for (int q = 0; q < P; ++q) v[q] = make_float2(0.f, 0.f);
   }
-  E::template fft<-1>(v, lds, t, rtw);
+  constexpr bool HOLD = row_holds_twiddles(N, P);
+  float2 st[E::HELD];
+  if constexpr (HOLD) {
+    E::load_held(t, rtw, st);
+    E::template fft_held<-1>(v, lds, t, st);
+  } else {
+    E::template fft<-1>(v, lds, t, rtw);
+  }
   // multiply by the replica spectrum; slot q holds frequency t + T q
 #pragma unroll
   for (int q = 0; q < P; ++q) {
@@ -43,7 +57,8 @@ __device__ __forceinline__ void row_fastconv_io(const IX &ix, const IY &iy, cons
 #pragma unroll
     for (int q = 0; q < P; ++q) v[q] = cscale(v[q], scale);
   }
-  E::template fft<+1>(v, lds, t, rtw);
+  if constexpr (HOLD) E::template fft_held<+1>(v, lds, t, st);
+  else E::template fft<+1>(v, lds, t, rtw);
   if (valid) {
 #pragma unroll
     for (int q = 0; q < P; ++q) iy.st(v[q], (uint32_t)(T * q));
