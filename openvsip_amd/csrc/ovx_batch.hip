@@ -310,7 +310,7 @@ __global__ __launch_bounds__(FsCfg<L>::NT, 4) void k_batch_fs(const BatchJob *__
         a.ld_in = j.ldy;
         a.out = j.y;
         a.ld_out = j.ldy;
-        fs_conv_body<L, F::NT / FsConv<L>::T>(a, tile.a, tile.b >> kTileRowsShift,
+        fs_conv_body<L, F::NT / FsConv<L>::T>(a, tile.a, tile.b >> kTileRowsShift, 1,
                                               tile.b & ((1 << kTileRowsShift) - 1), tid, lds);
       } else { // Fftm: workspace -> y in natural order, scaled
         a.scale = j.scale;

@@ -180,7 +180,7 @@ std::vector<TileQueue> chunked_fs_queues(const std::vector<BatchJob> &jobs, cons
     long workgroups = 0;
     for (const Part &p : chunk) workgroups += batch_conv_workgroups(jobs[p.ji].n1, jobs[p.ji].n2, p.r1 - p.r0);
     std::vector<BatchTile> cq[kBatchQueues];
-    for (const Part &p : chunk) push_fs_tiles(jobs[p.ji], p.ji, p.r0, p.r1, fs_conv_rows(workgroups), cq);
+    for (const Part &p : chunk) push_fs_tiles(jobs[p.ji], p.ji, p.r0, p.r1, fs_conv_rows(workgroups, false), cq);
     for (int k = 1; k < kFsQueueEnd; ++k)
       if (!cq[k].empty()) out.push_back(TileQueue{ fs_queue_line(k), fs_queue_pass(k), std::move(cq[k]) });
     chunk.clear();

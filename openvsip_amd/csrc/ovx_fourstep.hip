@@ -51,10 +51,12 @@ __global__ __launch_bounds__(C *(L / P)) void k_fs_col(FsArgs a, unsigned groups
 }
 
 template <int L, int P, int C, int DIR, bool SOUT>
-__global__ __launch_bounds__(C *(L / P)) void k_fs_row(FsArgs a)
+__global__ __launch_bounds__(C *(L / P)) void k_fs_row(FsArgs a, unsigned groups, unsigned rows)
 {
   __shared__ float2 lds_all[C * FsLds<L>::LROW];
-  fs_row_body<L, P, C, DIR, SOUT>(a, blockIdx.y, blockIdx.x, threadIdx.x, lds_all);
+  long row = blockIdx.x / groups, group = blockIdx.x % groups;
+  if (a.placed) fs_place(blockIdx.x, groups, rows, row, group);
+  fs_row_body<L, P, C, DIR, SOUT>(a, row, group, threadIdx.x, lds_all);
 }
 
 // 256 threads: fewer lines per workgroup leave it sooner (C = 16 / 4 at 512:
@@ -63,12 +65,29 @@ template <int L>
 struct FsConvCfg {
   static constexpr int C = 256 / FsConv<L>::T;
 };
+// Sets of `per` rows that the rows of one XCD (an eighth of `whole`) make.
+__host__ __device__ static inline int fs_conv_sets(int whole, int per) { return (whole / 8 + per - 1) / per; }
+
 template <int L>
-__global__ __launch_bounds__(256, 4) void k_fs_conv(FsArgs a, int rows, int per)
+__global__ __launch_bounds__(256, 4) void k_fs_conv(FsArgs a, int groups, int rows, int per)
 {
   __shared__ float2 lds_all[FsConvCfg<L>::C * FsConv<L>::LROW];
-  const int row0 = (int)blockIdx.y * per;
-  fs_conv_body<L, FsConvCfg<L>::C>(a, row0, min(per, rows - row0), blockIdx.x, threadIdx.x, lds_all);
+  const int w = (int)blockIdx.x;
+  int row0 = w / groups * per, nrows = min(per, rows - row0), step = 1, group = w % groups;
+  if (a.placed) { // fs_place()'s rows of one XCD: `per` of the rows x, x + 8, ...
+    const int whole = rows & ~7, split = fs_conv_sets(whole, per) * 8 * groups;
+    if (w < split) {
+      row0 = w / 8 / groups * 8 * per + w % 8;
+      nrows = min(per, (whole - row0 + 7) / 8);
+      step = 8;
+      group = w / 8 % groups;
+    } else {
+      row0 = whole + (w - split) / groups;
+      nrows = 1;
+      group = (w - split) % groups;
+    }
+  }
+  fs_conv_body<L, FsConvCfg<L>::C>(a, row0, nrows, step, group, threadIdx.x, lds_all);
 }
 
 // Wp[k1][k2] = scale * W[k1 + N1 k2] for `rows` coefficient rows (ldw = 0:
@@ -97,57 +116,85 @@ struct FsSplitCfg {
   static constexpr int NT = C * (L / P);
 };
 
+template <int L, int DIR, int C, bool SIN, bool SOUT, bool STREAM>
+static hipError_t col_launch_c(const FsArgs &a, long rows, hipStream_t s)
+{
+  constexpr int P = FsCfg<L>::P;
+  const unsigned groups = (unsigned)(a.n2 / C);
+  hipLaunchKernelGGL((k_fs_col<L, P, C, DIR, SIN, SOUT, STREAM>), dim3(groups * (unsigned)rows), dim3(C * (L / P)), 0,
+                     s, a, groups, (unsigned)rows);
+  return hipGetLastError();
+}
+
+// Columns per workgroup of the column pass: 16, or 8 where 16 make few
+// workgroups or few threads, so that each is done sooner.  16 / 8 columns, us: 256
+// x 256, 1 row 3.85 / 3.25, 8 rows 4.25 / 3.68, 256 x 512, 4 rows 4.36 / 3.74, 8
+// rows 4.78 / 4.64, 512 x 512, 2 rows 6.65 / 5.20, 4 rows 7.11 / 7.36, 1024 x
+// 1024, 1 row 11.6 / 9.5, 4 rows 15.9 / 18.8.  Split storage, read by a call's
+// first pass or written by its last, has 32 (FsSplitCfg); 64-byte runs of
+// 2048-point columns are not streamed (4 rows 229 us ordinary, 240 streamed).
 template <int L, int DIR>
 static hipError_t col_launch(const FsArgs &a, long rows, hipStream_t s)
 {
-  using F = FsCfg<L>;
-  using G = FsSplitCfg<L>;
-  // split storage is read by a call's first pass or written by its last
-  const bool split = a.in_re || a.out_re;
-  const unsigned groups = (unsigned)(a.n2 / (split ? G::C : F::C));
-  const dim3 grid(groups * (unsigned)rows);
-  if (a.in_re)
-    hipLaunchKernelGGL((k_fs_col<L, G::P, G::C, DIR, true, false, false>), grid, dim3(G::NT), 0, s, a, groups, (unsigned)rows);
-  else if (a.out_re)
-    hipLaunchKernelGGL((k_fs_col<L, G::P, G::C, DIR, false, true, false>), grid, dim3(G::NT), 0, s, a, groups, (unsigned)rows);
-  else if (a.stream)
-    hipLaunchKernelGGL((k_fs_col<L, F::P, F::C, DIR, false, false, true>), grid, dim3(F::NT), 0, s, a, groups,
-                       (unsigned)rows);
-  else
-    hipLaunchKernelGGL((k_fs_col<L, F::P, F::C, DIR, false, false, false>), grid, dim3(F::NT), 0, s, a, groups,
-                       (unsigned)rows);
+  constexpr int C = FsCfg<L>::C;
+  if (a.in_re) return col_launch_c<L, DIR, FsSplitCfg<L>::C, true, false, false>(a, rows, s);
+  if (a.out_re) return col_launch_c<L, DIR, FsSplitCfg<L>::C, false, true, false>(a, rows, s);
+  if constexpr (C == 16) {
+    const long groups = a.n2 / C * rows;
+    if (groups <= 64 || groups * FsCfg<L>::NT <= 32768) return col_launch_c<L, DIR, 8, false, false, false>(a, rows, s);
+    if (a.stream) return col_launch_c<L, DIR, C, false, false, true>(a, rows, s);
+  }
+  return col_launch_c<L, DIR, C, false, false, false>(a, rows, s);
+}
+
+template <int L, int DIR, int C, bool SPLIT>
+static hipError_t row_launch_c(FsArgs a, long rows, hipStream_t s)
+{
+  constexpr int P = FsCfg<L>::P, CL = C < FsSplitCfg<L>::C ? C : FsSplitCfg<L>::C;
+  const unsigned groups = (unsigned)(a.n1 / CL);
+  a.placed = fs_stays_in_l2(a.nbig, rows);
+  hipLaunchKernelGGL((k_fs_row<L, P, CL, DIR, SPLIT>), dim3(groups * (unsigned)rows), dim3(CL * (L / P)), 0, s, a,
+                     groups, (unsigned)rows);
   return hipGetLastError();
 }
 
+// Lines per workgroup of the row pass.  8 up to 64 MB of rows: twice the
+// workgroups where they are few, each sooner at its store, and the 64-byte runs
+// of neighbouring groups meet in L2; 16 beyond.  16 / 8 lines, us, both
+// passes: 256 x 512 lines, 24 rows 23.4 / 22.3, 256 x 256, 1 row 8.4 / 7.6, 512
+// x 512, 1 row 14.0 / 12.1, 128 x 256, 100 rows 22.6 / 21.0, 1000 rows 199 / 221;
+// 1024 x 1024, 8 rows 66.3 / 60.7.  Split storage, whose runs are half as long:
+// 32 lines, 8 where those would leave half the CUs without one (32 / 8, 256 x
+// 256, 1 row 10.9 / 8.5, 9 rows 11.8 / 10.3, 24 rows 14.5 / 15.2).
 template <int L, int DIR>
 static hipError_t row_launch(const FsArgs &a, long rows, hipStream_t s)
 {
-  using F = FsCfg<L>;
-  using G = FsSplitCfg<L>;
   if (a.out_re)
-    hipLaunchKernelGGL((k_fs_row<L, G::P, G::C, DIR, true>), dim3((unsigned)(a.n1 / G::C), (unsigned)rows),
-                       dim3(G::NT), 0, s, a);
-  else
-    hipLaunchKernelGGL((k_fs_row<L, F::P, F::C, DIR, false>), dim3((unsigned)(a.n1 / F::C), (unsigned)rows),
-                       dim3(F::NT), 0, s, a);
-  return hipGetLastError();
+    return rows * a.n1 < 128 * 32 ? row_launch_c<L, DIR, 8, true>(a, rows, s)
+                                  : row_launch_c<L, DIR, 32, true>(a, rows, s);
+  return rows * a.nbig * 8 <= (64l << 20) ? row_launch_c<L, DIR, 8, false>(a, rows, s)
+                                         : row_launch_c<L, DIR, FsCfg<L>::C, false>(a, rows, s);
 }
 
 // Rows per workgroup of the middle pass: as many as leave 8 workgroups a CU
-// (four rows) or 4 (two): 512 x 512 lines, 64 rows, 1 / 2 / 4 / 8 rows 56 / 46
-// / 44 / 51 us; 256 x 256, 64 rows, 18.4 / 17.8 / 19.5 / 24.0.
-int fs_conv_rows(long workgroups)
+// (four rows), or 3 (two; 2 where the rows are in L2): 512 x 512 lines, 64 rows,
+// 1 / 2 / 4 / 8 rows 56 / 46 / 44 / 51 us; the whole fastconv, 1 / 2 rows: 512
+// x 512, 12 rows 41.3 / 39.3, 9 rows 41.1 / 41.4, 1024 x 1024, 2 rows 41.0 /
+// 42.8; in L2, 256 x 512, 24 rows 33.0 / 31.2, 256 x 256, 40 rows 28.8 / 27.8, 32
+// rows 24.8 / 24.7, 16 rows 16.5 / 17.2.
+int fs_conv_rows(long workgroups, bool placed)
 {
-  return workgroups >= 4 * 2048 ? 4 : workgroups >= 2 * 1024 ? 2 : 1;
+  return workgroups >= 4 * 2048 ? 4 : workgroups >= 2 * (placed ? 512 : 768) ? 2 : 1;
 }
 
 template <int L>
-static hipError_t conv_launch(const FsArgs &a, long rows, hipStream_t s)
+static hipError_t conv_launch(FsArgs a, long rows, hipStream_t s)
 {
-  const long groups = a.n1 / FsConvCfg<L>::C;
-  const int per = fs_conv_rows(groups * rows);
-  hipLaunchKernelGGL((k_fs_conv<L>), dim3((unsigned)groups, (unsigned)((rows + per - 1) / per)), dim3(256), 0, s, a,
-                     (int)rows, per);
+  const int groups = (int)(a.n1 / FsConvCfg<L>::C), whole = (int)rows & ~7;
+  a.placed = fs_stays_in_l2(a.nbig, rows);
+  const int per = fs_conv_rows(groups * rows, a.placed);
+  const long sets = a.placed ? 8l * fs_conv_sets(whole, per) + (rows - whole) : (rows + per - 1) / per;
+  hipLaunchKernelGGL((k_fs_conv<L>), dim3((unsigned)(groups * sets)), dim3(256), 0, s, a, groups, (int)rows, per);
   return hipGetLastError();
 }
 

@@ -26,7 +26,23 @@ struct FsArgs {
   // interleaved column pass: non-temporal loads (forward) or loads and stores
   // (inverse), see fs_streams_in / fs_streams_out
   bool stream = false;
+  // row and middle passes: each row on the XCD of its column pass
+  // (fs_stays_in_l2)
+  bool placed = false;
 };
+
+// Whether a call's rows stay in the eight XCDs' L2s (4 MB each) from pass to
+// pass: the column pass works each row on one XCD, the next pass then does the
+// same.  Otherwise its groups go to the XCDs in turn, which suits rows that are
+// not in L2 better.  In turn / on the row's XCD, us: fastconv 256 x 256 lines,
+// 9 rows 16.8 / 14.7, 24 25.9 / 21.7, 40 33.0 / 27.8, 64 38.6 / 36.7, 96 54.0 /
+// 54.2; 256 x 512, 24 rows 35.9 / 31.2; rows of 2 MB and more, of which an L2
+// holds two: 512 x 512, 12 rows 41.3 / 42.5, 24 59 / 64.  Fftm 256 x 256, 24
+// rows 16.5 / 13.3, 256 x 512, 24 rows 22.3 / 21.7.
+inline bool fs_stays_in_l2(long n, long rows)
+{
+  return n * 8 <= (1l << 20) && rows * n * 8 <= 8 * (4l << 20);
+}
 
 // Whether the first / last pass of a fastconv over `bytes` of rows goes past
 // the caches: X, which is read once, should not push Y out of the 256 MB
@@ -43,7 +59,7 @@ hipError_t launch_fs_col(int dir, const FsArgs &a, long rows, hipStream_t s);
 hipError_t launch_fs_row(int dir, const FsArgs &a, long rows, hipStream_t s);
 hipError_t launch_fs_conv(const FsArgs &a, long rows, hipStream_t s);
 // rows per workgroup of a middle pass of that many workgroups of one row
-int fs_conv_rows(long workgroups);
+int fs_conv_rows(long workgroups, bool placed);
 // twiddle entries of a middle pass over lines of length l, and the table
 int fs_conv_twiddle_count(long l);
 hipError_t launch_fs_conv_twiddles(long l, float2 *tw, hipStream_t s);

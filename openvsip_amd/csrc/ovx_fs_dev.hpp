@@ -22,14 +22,6 @@ __device__ __forceinline__ float2 big_twiddle(const float2 *__restrict__ tlo, co
   return cmul(hi, lo);
 }
 
-// ---------------------------------------------------------------- column pass
-// Column FFT in direction DIR, times a.scale unless 1.  The twiddle
-// W_N^{n2 k1} between the two passes is applied by the row pass, where a line's
-// table entries are contiguous and serve both sides of a fastconv: read here,
-// at the columns' stride, they cost 15 us of a 67 us pass over 134 MB.
-// One group of C columns of one row: `group` selects columns
-// [group*C, group*C + C), `tid` is the thread within the group's C*(L/P)
-// threads, `lds_all` the group's C*LROW LDS elements.
 // The passes' global reads and writes: one row's buffer, element offsets of at
 // most N values.  Interleaved lines (a.in, a.out) or, when SPLIT, separate real
 // and imaginary arrays (a.in_re / a.in_im, a.out_re / a.out_im).  NT:
@@ -53,6 +45,14 @@ __device__ __forceinline__ auto fs_out(const FsArgs &a, long row, uint32_t lane)
     return IoCx<false, NT>{ make_rsrc(a.out + row * a.ld_out, 0xffffffffu), lane * 8u };
 }
 
+// ---------------------------------------------------------------- column pass
+// Column FFT in direction DIR, times a.scale unless 1.  The twiddle
+// W_N^{n2 k1} between the two passes is applied by the row pass, where a line's
+// table entries are contiguous and serve both sides of a fastconv: read here,
+// at the columns' stride, they cost 15 us of a 67 us pass over 134 MB.
+// One group of C columns of one row: `group` selects columns
+// [group*C, group*C + C), `tid` is the thread within the group's C*(L/P)
+// threads, `lds_all` the group's C*LROW LDS elements.
 template <int L, int P, int C, int DIR, bool SIN = false, bool SOUT = false, bool NTL = false, bool NTS = false,
           typename LP>
 __device__ __forceinline__ void fs_col_body(const FsArgs &a, long row, long group, int tid, LP lds_all)
@@ -101,6 +101,9 @@ __device__ __forceinline__ void fs_line_twiddles(const FsArgs &a, long k1, int t
 // Row pass of a transform in direction DIR: * W_N^{-+ k1 n2}, row FFT,
 // transposed store X[k1 + N1 k2], * scale.  One group of C lines k1 in
 // [group*C, group*C + C) of one row.
+// The result is written once, non-temporally where a run is 64 bytes or more:
+// 512 x 512 lines, 24 rows, both passes 42 to 36 us, 64 rows 95 to 88; 256 x
+// 256, 256 rows, 84 to 80; runs of 32 bytes (split, 2048 lines) 57 to 75.
 template <int L, int P, int C, int DIR, bool SOUT = false, typename LP>
 __device__ __forceinline__ void fs_row_body(const FsArgs &a, long row, long group, int tid, LP lds_all)
 {
@@ -135,14 +138,14 @@ __device__ __forceinline__ void fs_row_body(const FsArgs &a, long row, long grou
   const int c2 = tid % C;
   const int t2 = tid / C;
   LP lsrc = lds_all + c2 * LROW;
-  const auto out = fs_out<SOUT, false>(a, row, (uint32_t)t2 * N1 + (uint32_t)(group * C + c2));
+  const auto out = fs_out<SOUT, (C * (SOUT ? 4 : 8) >= 64)>(a, row, (uint32_t)t2 * N1 + (uint32_t)(group * C + c2));
 #pragma unroll
   for (int q = 0; q < P; ++q) out.st(lds_ld(lsrc, t2 + T * q), (uint32_t)(T * q) * N1);
 }
 
 // Middle pass of a fastconv (in place allowed): * W_N^{k1 n2}, forward row
-// FFT, * Wp[k1][k2], inverse row FFT, * W_N^{-k1 n2}; C lines of rows row0 ..
-// row0 + nrows - 1.  A line's stage twiddles, its W_N entries (the same on both
+// FFT, * Wp[k1][k2], inverse row FFT, * W_N^{-k1 n2}; C lines of the nrows rows
+// row0, row0 + step, ...  A line's stage twiddles, its W_N entries (the same on both
 // sides) and, with one spectrum for all rows, its spectrum stay in registers
 // over the rows: what bounded this pass was neither HBM nor latency but the
 // loads through L1, 110 of which for 16 values of a line were tables and stage
@@ -159,7 +162,7 @@ struct FsConv {
   static constexpr int LROW = LdsLayout<L, P>::elems | 1;
 };
 template <int L, int C, typename LP>
-__device__ __forceinline__ void fs_conv_body(const FsArgs &a, long row0, int nrows, long group, int tid, LP lds_all)
+__device__ __forceinline__ void fs_conv_body(const FsArgs &a, long row0, int nrows, int step, long group, int tid, LP lds_all)
 {
   constexpr int P = FsConv<L>::P, T = FsConv<L>::T;
   using E = Engine<L, P, line_in_wave(T)>;
@@ -178,8 +181,8 @@ __device__ __forceinline__ void fs_conv_body(const FsArgs &a, long row0, int nro
   E::load_held(t, rtw, st);
 #pragma unroll 1
   for (int r = 0; r < nrows; ++r) {
-    const auto in = fs_in<false, false>(a, row0 + r, lane);
-    const auto out = fs_out<false, false>(a, row0 + r, lane);
+    const auto in = fs_in<false, false>(a, row0 + r * step, lane);
+    const auto out = fs_out<false, false>(a, row0 + r * step, lane);
     float2 v[P];
 #pragma unroll
     for (int q = 0; q < P; ++q) v[q] = in.ld((uint32_t)(T * q));
@@ -189,7 +192,7 @@ __device__ __forceinline__ void fs_conv_body(const FsArgs &a, long row0, int nro
 #pragma unroll
     for (int q = 0; q < P; ++q) v[q] = cmul(v[q], ws[q]);
     if (a.ldwp && r + 1 < nrows) { // one spectrum per row: the next one
-      wp += a.ldwp;
+      wp += a.ldwp * step;
 #pragma unroll
       for (int q = 0; q < P; ++q) ws[q] = wp[T * q];
     }

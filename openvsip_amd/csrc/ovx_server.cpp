@@ -257,7 +257,7 @@ int Server::admit_and_launch(Slot &s, std::vector<Req *> &batch)
     if (f && f->kind == LineFFT::FOURSTEP && batch_supported(BP_FS, (int)f->n))
       conv_wgs += batch_conv_workgroups((int)f->n1, (int)f->n2, q0->r.rows);
   }
-  const int conv_rows = fs_conv_rows(conv_wgs);
+  const int conv_rows = fs_conv_rows(conv_wgs, false);
   for (size_t i = 0; i < batch.size(); ++i) {
     const ovx_request &r = batch[i]->r;
     int st;

@@ -19,6 +19,11 @@ REL_L2 = 1e-6
 # rows for two rows per workgroup, four times that for four
 CASES = [(32768, 1), (32768, 131), (32768, 517), (65536, 9), (65536, 67), (65536, 259), (131072, 35), (262144, 17),
          (524288, 9), (1 << 20, 5), (1 << 20, 17), (1 << 21, 3), (1 << 22, 2), (1 << 22, 9)]
+# up to 32 MB of rows of at most 1 MB: worked on one XCD from pass to pass, one
+# and two rows per workgroup, the last pair incomplete, fewer than eight rows,
+# rows left over from eights
+CASES += [(32768, 5), (32768, 96), (32768, 121), (65536, 41), (65536, 56), (65536, 64), (65536, 65), (131072, 7),
+          (131072, 31)]
 
 
 def rel(a, b):
