@@ -9,8 +9,8 @@
 // stride over their queues, workgroup w taking tiles w, w + grid, ...  Every
 // tile runs the same device body as the standalone kernels, so a job's
 // result is bitwise the same alone and in a batch.  Four-step jobs need their
-// three passes in order; each pass is a launch of its own over its queue, and
-// the host captures all of a batch's launches in one hipGraph.
+// three passes in order; each pass is a launch of its own over its queue.  A
+// batch's launches are captured in one hipGraph; the server issues its own.
 #include "ovx_batch.hpp"
 #include "ovx_fs_dev.hpp"
 #include "ovx_hier_dev.hpp"
@@ -46,12 +46,38 @@ __device__ __forceinline__ int tile_thread()
   return t;
 }
 
+// Tile `ti` of a queue: its span and its number in the span.  (Jobs and spans
+// are kernel arguments of their own, __restrict__: only so are the descriptor's
+// fields read by scalar loads, and the kernels free of scratch memory.)  The lanes of each
+// wave read 64 spans at once.
+struct Tile {
+  int job, op, row0, row1, conv_rows, k;
+};
+__device__ __forceinline__ Tile find_tile(const BatchSpan *__restrict__ spans, int nspans, int ti)
+{
+  const int lane = tile_thread() & 63;
+  for (int base = 0;; base += 64) {
+    int4 a = make_int4(0x7fffffff, 0, 0, 0);
+    int2 b = make_int2(0, 0);
+    if (base + lane < nspans) {
+      const BatchSpan *sp = spans + base + lane;
+      a = *(const int4 *)sp;
+      b = *(const int2 *)&sp->row1;
+    }
+    const int n = __popcll(__ballot(a.x <= ti)); // the spans that begin here or before
+    if (n == 64 && base + 64 < nspans && spans[base + 64].tile0 <= ti) continue;
+    auto of = [&](int v) { return __builtin_amdgcn_readlane(v, n - 1); };
+    return Tile{ of(a.y), of(a.z), of(a.w), of(b.x), of(b.y), ti - of(a.x) };
+  }
+}
+
 // Tile functions of a workgroup of NT threads: NT / (threads of a row) rows
 // (or overlap-save segments) per tile.
 template <int NT, int N>
-__device__ __forceinline__ void tile_hier_fastconv(const BatchJob &j, int row0, lds_ptr lds)
+__device__ __forceinline__ void tile_hier_fastconv(const BatchJob &j, const Tile &tile, lds_ptr lds)
 {
   using H = Hier<N>;
+  const int row0 = tile.row0 + tile.k * (NT / H::TR);
   static_assert(NT % H::TR == 0 && (NT / H::TR) * H::LROW <= BatchLds<NT>::value, "tile LDS");
   HierArgs a{};
   a.x = j.x;
@@ -70,9 +96,10 @@ __device__ __forceinline__ void tile_hier_fastconv(const BatchJob &j, int row0, 
 }
 
 template <int NT, int N>
-__device__ __forceinline__ void tile_hier_fwd(const BatchJob &j, int row0, lds_ptr lds)
+__device__ __forceinline__ void tile_hier_fwd(const BatchJob &j, const Tile &tile, lds_ptr lds)
 {
   using H = Hier<N>;
+  const int row0 = tile.row0 + tile.k * (NT / H::TR);
   static_assert(NT % H::TR == 0 && (NT / H::TR) * H::LROW <= BatchLds<NT>::value, "tile LDS");
   HierArgs a{};
   a.x = j.x;
@@ -90,9 +117,10 @@ __device__ __forceinline__ void tile_hier_fwd(const BatchJob &j, int row0, lds_p
 }
 
 template <int NT, int N, int P>
-__device__ __forceinline__ void tile_row_fastconv(const BatchJob &j, int row0, lds_ptr lds)
+__device__ __forceinline__ void tile_row_fastconv(const BatchJob &j, const Tile &tile, lds_ptr lds)
 {
   using E = Engine<N, P, line_in_wave(N / P)>;
+  const int row0 = tile.row0 + tile.k * (NT / E::T);
   static_assert(NT % E::T == 0 && (NT / E::T) * E::LROW <= BatchLds<NT>::value, "tile LDS");
   const int tid = tile_thread();
   const int lrow = tid / E::T;
@@ -102,9 +130,10 @@ __device__ __forceinline__ void tile_row_fastconv(const BatchJob &j, int row0, l
 }
 
 template <int NT, int N, int P>
-__device__ __forceinline__ void tile_row_fwd(const BatchJob &j, int row0, lds_ptr lds)
+__device__ __forceinline__ void tile_row_fwd(const BatchJob &j, const Tile &tile, lds_ptr lds)
 {
   using E = Engine<N, P, line_in_wave(N / P)>;
+  const int row0 = tile.row0 + tile.k * (NT / E::T);
   static_assert(NT % E::T == 0 && (NT / E::T) * E::LROW <= BatchLds<NT>::value, "tile LDS");
   const int tid = tile_thread();
   const int lrow = tid / E::T;
@@ -116,7 +145,7 @@ __device__ __forceinline__ void tile_row_fwd(const BatchJob &j, int row0, lds_pt
 // Overlap-save segments seg0, seg0 + 1, ... (NT / (L/16) of them per tile);
 // those past the last store nothing.
 template <int NT, int L>
-__device__ __forceinline__ void tile_ols(const BatchJob &j, int seg0, lds_ptr lds)
+__device__ __forceinline__ void tile_ols(const BatchJob &j, const Tile &tile, lds_ptr lds)
 {
   const OlsArgs a = j.ols;
   constexpr int T = L / 16;
@@ -124,7 +153,7 @@ __device__ __forceinline__ void tile_ols(const BatchJob &j, int seg0, lds_ptr ld
   const int tid = tile_thread();
   const int t = tid % T;
   const int copy = tid / T;
-  ols_body<L, 16>(a, seg0, copy, t, lds + copy * Engine<L, 16>::LROW);
+  ols_body<L, 16>(a, tile.row0 + tile.k * (NT / T), copy, t, lds + copy * Engine<L, 16>::LROW);
 }
 
 int batch_ols_segments_per_tile(int L)
@@ -167,25 +196,25 @@ static_assert(batch_mid_routed(BP_HIER, 8192) && !batch_mid_routed(BP_HIER, 1638
               "run in the 512-thread one");
 
 template <int NT, int N>
-__device__ __forceinline__ void run_hier(bool fwd_only, const BatchJob &j, int a, lds_ptr lds)
+__device__ __forceinline__ void run_hier(bool fwd_only, const BatchJob &j, const Tile &tile, lds_ptr lds)
 {
   if constexpr (runs_in<NT, BP_HIER, N>()) {
-    if (fwd_only) tile_hier_fwd<NT, N>(j, a, lds);
-    else tile_hier_fastconv<NT, N>(j, a, lds);
+    if (fwd_only) tile_hier_fwd<NT, N>(j, tile, lds);
+    else tile_hier_fastconv<NT, N>(j, tile, lds);
   }
 }
 template <int NT, int N, int P>
-__device__ __forceinline__ void run_row(bool fwd_only, const BatchJob &j, int a, lds_ptr lds)
+__device__ __forceinline__ void run_row(bool fwd_only, const BatchJob &j, const Tile &tile, lds_ptr lds)
 {
   if constexpr (runs_in<NT, BP_ROW, N>()) {
-    if (fwd_only) tile_row_fwd<NT, N, P>(j, a, lds);
-    else tile_row_fastconv<NT, N, P>(j, a, lds);
+    if (fwd_only) tile_row_fwd<NT, N, P>(j, tile, lds);
+    else tile_row_fastconv<NT, N, P>(j, tile, lds);
   }
 }
 template <int NT, int L>
-__device__ __forceinline__ void run_ols(const BatchJob &j, int a, lds_ptr lds)
+__device__ __forceinline__ void run_ols(const BatchJob &j, const Tile &tile, lds_ptr lds)
 {
-  if constexpr (ols_runs_in<NT, L>()) tile_ols<NT, L>(j, a, lds);
+  if constexpr (ols_runs_in<NT, L>()) tile_ols<NT, L>(j, tile, lds);
 }
 
 // The persistent loop of a launch of NT threads: workgroup w takes tiles w,
@@ -194,24 +223,23 @@ __device__ __forceinline__ void run_ols(const BatchJob &j, int a, lds_ptr lds)
 // queue (a shared atomic counter cost each workgroup a cross-XCD round trip
 // per tile).
 template <int NT>
-__device__ __forceinline__ void batch_loop(const BatchJob *__restrict__ jobs, const BatchTile *__restrict__ tiles,
-                                           const int *__restrict__ ntiles, float2 *lds_mem)
+__device__ __forceinline__ void batch_loop(const BatchJob *__restrict__ jobs, const BatchSpan *__restrict__ spans,
+                                           int nspans, int tiles, float2 *lds_mem)
 {
   const lds_ptr lds = as_lds(lds_mem);
-  const int total = *ntiles;
-  for (int ti = blockIdx.x; ti < total; ti += gridDim.x) {
-    const BatchTile tile = tiles[ti];
+  for (int ti = blockIdx.x; ti < tiles; ti += gridDim.x) {
+    const Tile tile = find_tile(spans, nspans, ti);
     const BatchJob &j = jobs[tile.job]; // the same for every lane: scalar loads
     switch (tile.op) {
     case BT_HIER_FASTCONV:
     case BT_HIER_FFT_FWD: {
       const bool fwd = tile.op == BT_HIER_FFT_FWD;
       switch (j.n) {
-      case 1024: run_hier<NT, 1024>(fwd, j, tile.a, lds); break;
-      case 2048: run_hier<NT, 2048>(fwd, j, tile.a, lds); break;
-      case 4096: run_hier<NT, 4096>(fwd, j, tile.a, lds); break;
-      case 8192: run_hier<NT, 8192>(fwd, j, tile.a, lds); break;
-      case 16384: run_hier<NT, 16384>(fwd, j, tile.a, lds); break;
+      case 1024: run_hier<NT, 1024>(fwd, j, tile, lds); break;
+      case 2048: run_hier<NT, 2048>(fwd, j, tile, lds); break;
+      case 4096: run_hier<NT, 4096>(fwd, j, tile, lds); break;
+      case 8192: run_hier<NT, 8192>(fwd, j, tile, lds); break;
+      case 16384: run_hier<NT, 16384>(fwd, j, tile, lds); break;
       default: break;
       }
       break;
@@ -220,24 +248,24 @@ __device__ __forceinline__ void batch_loop(const BatchJob *__restrict__ jobs, co
     case BT_ROW_FFT_FWD: {
       const bool fwd = tile.op == BT_ROW_FFT_FWD;
       switch (j.n) {
-      case 256: run_row<NT, 256, 16>(fwd, j, tile.a, lds); break;
-      case 512: run_row<NT, 512, 16>(fwd, j, tile.a, lds); break;
-      case 2048: run_row<NT, 2048, 16>(fwd, j, tile.a, lds); break;
-      case 4096: run_row<NT, 4096, 16>(fwd, j, tile.a, lds); break;
-      case 3072: run_row<NT, 3072, 12>(fwd, j, tile.a, lds); break;
-      case 6144: run_row<NT, 6144, 12>(fwd, j, tile.a, lds); break;
-      case 12288: run_row<NT, 12288, 12>(fwd, j, tile.a, lds); break;
+      case 256: run_row<NT, 256, 16>(fwd, j, tile, lds); break;
+      case 512: run_row<NT, 512, 16>(fwd, j, tile, lds); break;
+      case 2048: run_row<NT, 2048, 16>(fwd, j, tile, lds); break;
+      case 4096: run_row<NT, 4096, 16>(fwd, j, tile, lds); break;
+      case 3072: run_row<NT, 3072, 12>(fwd, j, tile, lds); break;
+      case 6144: run_row<NT, 6144, 12>(fwd, j, tile, lds); break;
+      case 12288: run_row<NT, 12288, 12>(fwd, j, tile, lds); break;
       default: break;
       }
       break;
     }
     case BT_OLS:
       switch (j.ols_len) {
-      case 1024: run_ols<NT, 1024>(j, tile.a, lds); break;
-      case 2048: run_ols<NT, 2048>(j, tile.a, lds); break;
-      case 4096: run_ols<NT, 4096>(j, tile.a, lds); break;
-      case 8192: run_ols<NT, 8192>(j, tile.a, lds); break;
-      case 16384: run_ols<NT, 16384>(j, tile.a, lds); break;
+      case 1024: run_ols<NT, 1024>(j, tile, lds); break;
+      case 2048: run_ols<NT, 2048>(j, tile, lds); break;
+      case 4096: run_ols<NT, 4096>(j, tile, lds); break;
+      case 8192: run_ols<NT, 8192>(j, tile, lds); break;
+      case 16384: run_ols<NT, 16384>(j, tile, lds); break;
       default: break;
       }
       break;
@@ -247,116 +275,123 @@ __device__ __forceinline__ void batch_loop(const BatchJob *__restrict__ jobs, co
   }
 }
 
-__global__ __launch_bounds__(kBatchThreads) void k_batch(const BatchJob *__restrict__ jobs,
-                                                          const BatchTile *__restrict__ tiles,
-                                                          const int *__restrict__ ntiles)
+__global__ __launch_bounds__(kBatchThreads) void k_batch(
+    const BatchJob *__restrict__ jobs, const BatchSpan *__restrict__ spans, int nspans, int tiles)
 {
   __shared__ float2 lds_mem[kBatchLds];
-  batch_loop<kBatchThreads>(jobs, tiles, ntiles, lds_mem);
+  batch_loop<kBatchThreads>(jobs, spans, nspans, tiles, lds_mem);
 }
 
 // Two workgroups per CU: four waves per SIMD (the second launch bound is
 // waves per SIMD: 128 VGPRs) and
 // 2 x 67.6 KB of LDS.
 __global__ __launch_bounds__(kBatchMidThreads, kBatchMidBlocksPerCu * kBatchMidThreads / 256) void k_batch_mid(
-    const BatchJob *__restrict__ jobs, const BatchTile *__restrict__ tiles, const int *__restrict__ ntiles)
+    const BatchJob *__restrict__ jobs, const BatchSpan *__restrict__ spans, int nspans, int tiles)
 {
   __shared__ float2 lds_mem[kBatchMidLds];
-  batch_loop<kBatchMidThreads>(jobs, tiles, ntiles, lds_mem);
+  batch_loop<kBatchMidThreads>(jobs, spans, nspans, tiles, lds_mem);
 }
 
-hipError_t launch_batch(const BatchJob *jobs, const BatchTile *tiles, const int *ntiles, int grid, hipStream_t s)
+hipError_t launch_batch(const BatchQueue &q, int grid, hipStream_t s)
 {
-  hipLaunchKernelGGL(k_batch, dim3(grid), dim3(kBatchThreads), 0, s, jobs, tiles, ntiles);
+  hipLaunchKernelGGL(k_batch, dim3(grid), dim3(kBatchThreads), 0, s, q.jobs, q.spans, q.nspans, q.tiles);
   return hipGetLastError();
 }
 
-hipError_t launch_batch_mid(const BatchJob *jobs, const BatchTile *tiles, const int *ntiles, int grid, hipStream_t s)
+hipError_t launch_batch_mid(const BatchQueue &q, int grid, hipStream_t s)
 {
-  hipLaunchKernelGGL(k_batch_mid, dim3(grid), dim3(kBatchMidThreads), 0, s, jobs, tiles, ntiles);
+  hipLaunchKernelGGL(k_batch_mid, dim3(grid), dim3(kBatchMidThreads), 0, s, q.jobs, q.spans, q.nspans, q.tiles);
   return hipGetLastError();
 }
 
 // ---------------------------------------------------------------- four-step passes
-// One line group of one row per workgroup (the standalone kernels' shape;
-// four waves per SIMD, the occupancy the LDS of L = 256 groups allows), so
-// co-resident workgroups run independently and overlap their loads with
-// other groups' arithmetic; workgroup w takes tiles w, w + grid, ...  The job
-// descriptor is read from global memory (uniform per tile, scalar loads).
+// Row and line group of tile k of a column pass over rows [row0, row1): eight
+// rows at a time, their tiles in turn, so that the workgroups of a row land on
+// one XCD (the standalone passes' placement).
+__device__ __forceinline__ void fs_col_tile(const Tile &t, int groups, int &row, int &group)
+{
+  const int rows = t.row1 - t.row0, whole = rows & ~7;
+  if (t.k < whole * groups) {
+    const int e = t.k / 8;
+    row = t.row0 + e / groups * 8 + t.k % 8;
+    group = e % groups;
+  } else {
+    const int e = t.k - whole * groups, left = rows - whole;
+    row = t.row0 + whole + e % left;
+    group = e / left;
+  }
+}
+
+// One line group per workgroup (the standalone kernels' shape; four waves per
+// SIMD, the occupancy the LDS of L = 256 groups allows), so co-resident
+// workgroups run independently and overlap their loads with other groups'
+// arithmetic.  The job descriptor is read from global memory (uniform per tile,
+// scalar loads).
 template <int L, int PASS>
-__global__ __launch_bounds__(FsCfg<L>::NT, 4) void k_batch_fs(const BatchJob *__restrict__ jobs,
-                                                               const BatchTile *__restrict__ tiles,
-                                                               const int *__restrict__ ntiles)
+__global__ __launch_bounds__(FsCfg<L>::NT, 4) void k_batch_fs(
+    const BatchJob *__restrict__ jobs, const BatchSpan *__restrict__ spans, int nspans)
 {
   using F = FsCfg<L>;
-  static_assert(F::NT / FsConv<L>::T * FsConv<L>::LROW <= F::LDS, "middle pass LDS");
+  constexpr int CC = F::NT / FsConv<L>::T; // lines of a middle-pass tile
+  static_assert(CC * FsConv<L>::LROW <= F::LDS, "middle pass LDS");
   __shared__ float2 lds[F::LDS];
-  const int total = *ntiles;
   const int tid = (int)threadIdx.x;
-  for (int ti = blockIdx.x; ti < total; ti += gridDim.x) {
-    const BatchTile tile = tiles[ti];
-    const BatchJob &j = jobs[tile.job];
-    FsArgs a = fs_args_of(j);
-    if constexpr (PASS == 0) { // column FFT: fastconv x -> y, Fftm x -> workspace
-      const bool fft = tile.op == BT_FS_FFT_A;
-      a.in = j.x;
-      a.ld_in = j.ldx;
-      a.out = fft ? j.ws : j.y;
-      a.ld_out = fft ? (long)j.n : j.ldy;
-      fs_col_body<L, F::P, F::C, -1>(a, tile.a, tile.b, tid, lds);
-    } else if constexpr (PASS == 1) {
-      if (tile.op == BT_FS_B) { // fastconv: middle pass in place on y
-        a.in = j.y;
-        a.ld_in = j.ldy;
-        a.out = j.y;
-        a.ld_out = j.ldy;
-        fs_conv_body<L, F::NT / FsConv<L>::T>(a, tile.a, tile.b >> kTileRowsShift, 1,
-                                              tile.b & ((1 << kTileRowsShift) - 1), tid, lds);
-      } else { // Fftm: workspace -> y in natural order, scaled
-        a.scale = j.scale;
-        a.in = j.ws;
-        a.ld_in = j.n;
-        a.out = j.y;
-        a.ld_out = j.ldy;
-        fs_row_body<L, F::P, F::C, -1>(a, tile.a, tile.b, tid, lds);
-      }
-    } else { // fastconv pass 3: column IFFT in place on y
+  const Tile tile = find_tile(spans, nspans, blockIdx.x);
+  const BatchJob &j = jobs[tile.job];
+  FsArgs a = fs_args_of(j);
+  int row, group;
+  if constexpr (PASS == 0) { // column FFT: fastconv x -> y, Fftm x -> workspace
+    const bool fft = tile.op == BT_FS_FFT_A;
+    a.in = j.x;
+    a.ld_in = j.ldx;
+    a.out = fft ? j.ws : j.y;
+    a.ld_out = fft ? (long)j.n : j.ldy;
+    fs_col_tile(tile, j.n2 / F::C, row, group);
+    fs_col_body<L, F::P, F::C, -1>(a, row, group, tid, lds);
+  } else if constexpr (PASS == 1) {
+    if (tile.op == BT_FS_B) { // fastconv: middle pass in place on y
       a.in = j.y;
       a.ld_in = j.ldy;
       a.out = j.y;
       a.ld_out = j.ldy;
-      fs_col_body<L, F::P, F::C, +1>(a, tile.a, tile.b, tid, lds);
+      const int groups = j.n1 / CC;
+      row = tile.row0 + tile.k / groups * tile.conv_rows;
+      fs_conv_body<L, CC>(a, row, min(tile.conv_rows, tile.row1 - row), 1, tile.k % groups, tid, lds);
+    } else { // Fftm: workspace -> y in natural order, scaled
+      a.scale = j.scale;
+      a.in = j.ws;
+      a.ld_in = j.n;
+      a.out = j.y;
+      a.ld_out = j.ldy;
+      const int groups = j.n1 / F::C;
+      fs_row_body<L, F::P, F::C, -1>(a, tile.row0 + tile.k / groups, tile.k % groups, tid, lds);
     }
-    __syncthreads(); // LDS reuse by the next tile
+  } else { // fastconv pass 3: column IFFT in place on y
+    a.in = j.y;
+    a.ld_in = j.ldy;
+    a.out = j.y;
+    a.ld_out = j.ldy;
+    fs_col_tile(tile, j.n2 / F::C, row, group);
+    fs_col_body<L, F::P, F::C, +1>(a, row, group, tid, lds);
   }
 }
 
 template <int L>
-static hipError_t launch_fs_pass(int pass, const BatchJob *jobs, const BatchTile *tiles, const int *ntiles, int grid,
-                                 hipStream_t s)
+static hipError_t launch_fs_pass(int pass, const BatchQueue &q, hipStream_t s)
 {
   constexpr int NT = FsCfg<L>::NT;
-  if (pass == 0) hipLaunchKernelGGL((k_batch_fs<L, 0>), dim3(grid), dim3(NT), 0, s, jobs, tiles, ntiles);
-  else if (pass == 1) hipLaunchKernelGGL((k_batch_fs<L, 1>), dim3(grid), dim3(NT), 0, s, jobs, tiles, ntiles);
-  else hipLaunchKernelGGL((k_batch_fs<L, 2>), dim3(grid), dim3(NT), 0, s, jobs, tiles, ntiles);
+  if (pass == 0) hipLaunchKernelGGL((k_batch_fs<L, 0>), dim3(q.tiles), dim3(NT), 0, s, q.jobs, q.spans, q.nspans);
+  else if (pass == 1) hipLaunchKernelGGL((k_batch_fs<L, 1>), dim3(q.tiles), dim3(NT), 0, s, q.jobs, q.spans, q.nspans);
+  else hipLaunchKernelGGL((k_batch_fs<L, 2>), dim3(q.tiles), dim3(NT), 0, s, q.jobs, q.spans, q.nspans);
   return hipGetLastError();
 }
 
-hipError_t launch_batch_fs(int n_line, int pass, const BatchJob *jobs, const BatchTile *tiles, const int *ntiles,
-                           int grid, hipStream_t s)
+hipError_t launch_batch_fs(int n_line, int pass, const BatchQueue &q, hipStream_t s)
 {
-  if (grid <= 0) return hipSuccess;
-  if (n_line == 256) return launch_fs_pass<256>(pass, jobs, tiles, ntiles, grid, s);
-  if (n_line == 512) return launch_fs_pass<512>(pass, jobs, tiles, ntiles, grid, s);
+  if (q.tiles <= 0) return hipSuccess;
+  if (n_line == 256) return launch_fs_pass<256>(pass, q, s);
+  if (n_line == 512) return launch_fs_pass<512>(pass, q, s);
   return hipErrorInvalidValue;
-}
-
-// Workgroups of a four-step pass that fit one CU together (LDS-bound).
-int batch_fs_blocks_per_cu(int n_line)
-{
-  if (n_line == 256) return (160 * 1024) / (FsCfg<256>::LDS * 8);
-  if (n_line == 512) return (160 * 1024) / (FsCfg<512>::LDS * 8);
-  return 1;
 }
 
 bool batch_supported(int path, int n)

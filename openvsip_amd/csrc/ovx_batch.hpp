@@ -10,19 +10,19 @@ namespace ovx {
 enum BatchPath { BP_HIER = 1, BP_ROW = 2, BP_FS = 3 };
 // Tile operations.
 enum BatchOp {
-  BT_HIER_FASTCONV = 1, // rows [a, a + rows_per_tile) of a hierarchical-path job
-  BT_ROW_FASTCONV = 2,  // rows [a, ...) of a register-Stockham-path job
-  BT_FS_A = 3,          // four-step fastconv pass 1: row a, column group b
-  BT_FS_B = 4,          // pass 2: rows from a, line group b
-  BT_FS_C = 5,          // pass 3: row a, column group b
+  BT_HIER_FASTCONV = 1, // a tile's worth of rows of a hierarchical-path job
+  BT_ROW_FASTCONV = 2,  // the same of a register-Stockham-path job
+  BT_FS_A = 3,          // four-step fastconv pass 1: a column group of a row
+  BT_FS_B = 4,          // pass 2: a line group of conv_rows rows
+  BT_FS_C = 5,          // pass 3: a column group of a row
   BT_HIER_FFT_FWD = 6,  // forward Fftm rows of a hierarchical-path job
   BT_ROW_FFT_FWD = 7,   // forward Fftm rows of a register-Stockham-path job
   BT_FS_FFT_A = 8,      // four-step forward Fftm pass 1: x -> workspace
   BT_FS_FFT_B = 9,      // pass 2: workspace -> y (natural order)
-  BT_OLS = 10           // one overlap-save segment (a = segment index)
+  BT_OLS = 10           // a tile's worth of overlap-save segments
 };
 
-struct BatchJob {
+struct alignas(16) BatchJob { // spans may follow a table of jobs
   int path;
   int n;
   long rows;
@@ -44,13 +44,18 @@ struct BatchJob {
   int ols_len;       // segment length L
 };
 
-struct BatchTile {
+// Consecutive tiles of a queue: one operation over rows (or segments) [row0,
+// row1) of one job.  A workgroup finds the span of its tile and works out rows
+// and line group itself.  The host wrote and copied a table of the tiles, 160 KB
+// for 32 mixed requests: with that, a copy per queue and a graph that launched
+// empty queues too the server took 340 us for them, now 262.
+struct alignas(16) BatchSpan {
+  int tile0; // first tile in the queue
   int job;
   int op;
-  int a; // first row
-  int b; // line group (four-step); BT_FS_B: rows << kTileRowsShift | line group
+  int row0, row1;
+  int conv_rows; // BT_FS_B: rows per tile
 };
-constexpr int kTileRowsShift = 16;
 
 // Tile queues of a batch: queue 0 holds the LDS-resident tiles (rows,
 // overlap-save segments) of the 1024-thread persistent launch, queue
@@ -88,20 +93,23 @@ int batch_rows_per_tile(int path, int n);
 int batch_ols_segments_per_tile(int L);
 int batch_fs_lines_per_group(int n_line); // C of a four-step group of lines of length n_line
 int batch_fs_conv_lines_per_group(int n_line); // of a fastconv's middle pass
-int batch_fs_blocks_per_cu(int n_line);   // co-resident workgroups of a four-step pass launch
 bool batch_supported(int path, int n);
 
-// One persistent launch over tiles[0 .. *ntiles): `grid` workgroups, workgroup
-// w taking tiles w, w + grid, ...
-hipError_t launch_batch(const BatchJob *jobs, const BatchTile *tiles, const int *ntiles, int grid, hipStream_t s);
+// A queue in device memory: spans by first tile, `tiles` tiles in all.
+struct BatchQueue {
+  const BatchJob *jobs;
+  const BatchSpan *spans;
+  int nspans, tiles;
+};
+// One persistent launch over a queue of LDS-resident tiles: `grid` workgroups,
+// workgroup w taking tiles w, w + grid, ...
+hipError_t launch_batch(const BatchQueue &q, int grid, hipStream_t s);
 // The same over the 512-thread queue (two workgroups per CU).
-hipError_t launch_batch_mid(const BatchJob *jobs, const BatchTile *tiles, const int *ntiles, int grid, hipStream_t s);
+hipError_t launch_batch_mid(const BatchQueue &q, int grid, hipStream_t s);
 constexpr int kBatchMidBlocksPerCu = 2;
-// Four-step pass `pass` (0, 1, 2) over tiles[0 .. *ntiles) of line length
-// n_line (256 or 512): `grid` workgroups of one line group each take tiles
-// blockIdx.x, blockIdx.x + grid, ... (no shared counter).
-hipError_t launch_batch_fs(int n_line, int pass, const BatchJob *jobs, const BatchTile *tiles, const int *ntiles,
-                           int grid, hipStream_t s);
+// Four-step pass `pass` (0, 1, 2) over a queue of line length n_line (256 or
+// 512), one tile per workgroup.
+hipError_t launch_batch_fs(int n_line, int pass, const BatchQueue &q, hipStream_t s);
 inline int fs_queue_pass(int q) { return (q - 1) / 2; }
 
 } // namespace ovx

@@ -126,44 +126,44 @@ int make_batch_job(const LineFFT &f, long rows, const float2 *x, long ldx, float
 
 long batch_conv_workgroups(int n1, int n2, long rows) { return rows * (n1 / batch_fs_conv_lines_per_group(n2)); }
 
-// Column-pass tiles of rows [r0, r1): eight rows at a time, their tiles in
-// turn, so that the workgroups of a row land on one XCD (the standalone
-// passes' placement).
-static void push_col_tiles(std::vector<BatchTile> &q, const BatchJob &j, int ji, int op, long r0, long r1)
+void TileQueue::push(int job, int op, long row0, long row1, long count, int conv_rows)
 {
-  const int groups = j.n2 / batch_fs_lines_per_group(j.n1);
-  for (long r = r0; r < r1; r += 8)
-    for (int g = 0; g < groups; ++g)
-      for (long k = r; k < std::min(r + 8, r1); ++k) q.push_back(BatchTile{ ji, op, (int)k, g });
+  if (count <= 0) return;
+  spans.push_back(BatchSpan{ tiles, job, op, (int)row0, (int)row1, conv_rows });
+  tiles += (int)count;
 }
 
-// The three passes of rows [r0, r1) of a four-step fastconv, one line group
-// per tile and `conv_rows` rows per middle-pass tile.
-static void push_fs_tiles(const BatchJob &j, int ji, long r0, long r1, int conv_rows,
-                          std::vector<BatchTile> q[kBatchQueues])
+hipError_t launch_queue(const TileQueue &q, const BatchJob *jobs, const BatchSpan *spans, hipStream_t s)
 {
-  push_col_tiles(q[fs_queue(0, j.n1)], j, ji, BT_FS_A, r0, r1);
-  const int lines = j.n1 / batch_fs_conv_lines_per_group(j.n2);
-  std::vector<BatchTile> &b = q[fs_queue(1, j.n2)];
-  for (long r = r0; r < r1; r += conv_rows)
-    for (int g = 0; g < lines; ++g)
-      b.push_back(BatchTile{ ji, BT_FS_B, (int)r, (int)std::min<long>(conv_rows, r1 - r) << kTileRowsShift | g });
-  push_col_tiles(q[fs_queue(2, j.n1)], j, ji, BT_FS_C, r0, r1);
+  if (q.tiles <= 0) return hipSuccess;
+  const BatchQueue bq{ jobs, spans, (int)q.spans.size(), q.tiles };
+  if (q.line == 0) return launch_batch(bq, std::min(q.tiles, device_cu_count()), s);
+  if (q.line == kMidLine) return launch_batch_mid(bq, std::min(q.tiles, kBatchMidBlocksPerCu * device_cu_count()), s);
+  return launch_batch_fs(q.line, q.pass, bq, s);
 }
 
-// Tiles of job `ji`: LDS-resident rows go to the queue of their persistent
-// launch (batch_queue), the three four-step passes to their (pass, line
-// length) queues.
-void make_batch_tiles(const BatchJob &j, int ji, std::vector<BatchTile> q[kBatchQueues], int conv_rows)
+void push_row_tiles(const BatchJob &j, int ji, bool fft, TileQueue &big, TileQueue &mid)
 {
-  if (j.path == BP_HIER || j.path == BP_ROW) {
-    int rpt = batch_rows_per_tile(j.path, j.n);
-    int op = j.path == BP_HIER ? BT_HIER_FASTCONV : BT_ROW_FASTCONV;
-    std::vector<BatchTile> &dst = q[batch_queue(j.path, j.n)];
-    for (long r = 0; r < j.rows; r += rpt) dst.push_back(BatchTile{ ji, op, (int)r, 0 });
+  const int rpt = batch_rows_per_tile(j.path, j.n);
+  const int op = j.path == BP_HIER ? (fft ? BT_HIER_FFT_FWD : BT_HIER_FASTCONV) : (fft ? BT_ROW_FFT_FWD : BT_ROW_FASTCONV);
+  TileQueue &q = batch_queue(j.path, j.n) == kMidQueue ? mid : big;
+  q.push(ji, op, 0, j.rows, (j.rows + rpt - 1) / rpt);
+}
+
+// The passes of rows [r0, r1) of a four-step job: a fastconv's three, with
+// `conv_rows` rows per middle-pass tile, or an Fftm's two.
+static void push_fs_tiles(const BatchJob &j, int ji, long r0, long r1, int conv_rows, TileQueue q[kBatchQueues])
+{
+  const bool fft = j.ws != nullptr;
+  const long rows = r1 - r0, cols = j.n2 / batch_fs_lines_per_group(j.n1);
+  q[fs_queue(0, j.n1)].push(ji, fft ? BT_FS_FFT_A : BT_FS_A, r0, r1, rows * cols);
+  if (fft) {
+    q[fs_queue(1, j.n2)].push(ji, BT_FS_FFT_B, r0, r1, rows * (j.n1 / batch_fs_lines_per_group(j.n2)));
     return;
   }
-  push_fs_tiles(j, ji, 0, j.rows, conv_rows, q);
+  const long sets = (rows + conv_rows - 1) / conv_rows;
+  q[fs_queue(1, j.n2)].push(ji, BT_FS_B, r0, r1, sets * (j.n1 / batch_fs_conv_lines_per_group(j.n2)), conv_rows);
+  q[fs_queue(2, j.n1)].push(ji, BT_FS_C, r0, r1, rows * cols);
 }
 
 std::vector<TileQueue> chunked_fs_queues(const std::vector<BatchJob> &jobs, const std::vector<int> &order,
@@ -177,12 +177,17 @@ std::vector<TileQueue> chunked_fs_queues(const std::vector<BatchJob> &jobs, cons
   std::vector<Part> chunk;
   size_t used = 0;
   auto flush = [&] {
-    long workgroups = 0;
-    for (const Part &p : chunk) workgroups += batch_conv_workgroups(jobs[p.ji].n1, jobs[p.ji].n2, p.r1 - p.r0);
-    std::vector<BatchTile> cq[kBatchQueues];
+    long workgroups = 0; // of the fastconvs' middle pass
+    for (const Part &p : chunk)
+      if (!jobs[p.ji].ws) workgroups += batch_conv_workgroups(jobs[p.ji].n1, jobs[p.ji].n2, p.r1 - p.r0);
+    TileQueue cq[kBatchQueues];
     for (const Part &p : chunk) push_fs_tiles(jobs[p.ji], p.ji, p.r0, p.r1, fs_conv_rows(workgroups, false), cq);
-    for (int k = 1; k < kFsQueueEnd; ++k)
-      if (!cq[k].empty()) out.push_back(TileQueue{ fs_queue_line(k), fs_queue_pass(k), std::move(cq[k]) });
+    for (int k = 1; k < kFsQueueEnd; ++k) {
+      if (!cq[k].tiles) continue;
+      cq[k].line = fs_queue_line(k);
+      cq[k].pass = fs_queue_pass(k);
+      out.push_back(std::move(cq[k]));
+    }
     chunk.clear();
     used = 0;
   };
@@ -207,34 +212,6 @@ std::vector<TileQueue> chunked_fs_queues(const std::vector<BatchJob> &jobs, cons
   return out;
 }
 
-void make_batch_fft_tiles(const BatchJob &j, int ji, std::vector<BatchTile> q[kBatchQueues])
-{
-  push_col_tiles(q[fs_queue(0, j.n1)], j, ji, BT_FS_FFT_A, 0, j.rows);
-  const int lines = j.n1 / batch_fs_lines_per_group(j.n2);
-  std::vector<BatchTile> &b = q[fs_queue(1, j.n2)];
-  for (long r = 0; r < j.rows; ++r)
-    for (int g = 0; g < lines; ++g) b.push_back(BatchTile{ ji, BT_FS_FFT_B, (int)r, g });
-}
-
-hipError_t capture_batch_launches(const BatchJob *jobs, BatchTile *const tiles[kBatchQueues], int *meta,
-                                  const int *counts, bool all, hipStream_t cap)
-{
-  hipError_t e = hipSuccess;
-  if (all || counts[0] > 0) e = launch_batch(jobs, tiles[0], meta, device_cu_count(), cap);
-  if (e == hipSuccess && (all || counts[kMidQueue] > 0))
-    e = launch_batch_mid(jobs, tiles[kMidQueue], meta + kMidQueue, kBatchMidBlocksPerCu * device_cu_count(), cap);
-  for (int k = 1; k < kFsQueueEnd && e == hipSuccess; ++k) {
-    if (!all && counts[k] == 0) continue;
-    const int line = fs_queue_line(k);
-    // a batch with known counts launches one workgroup per tile (as the
-    // standalone passes do); the server's graph, whose counts change per
-    // batch, strides a resident grid over the queue
-    const int grid = all ? batch_fs_blocks_per_cu(line) * device_cu_count() : counts[k];
-    e = launch_batch_fs(line, fs_queue_pass(k), jobs, tiles[k], meta + k, grid, cap);
-  }
-  return e;
-}
-
 GraphBatch::~GraphBatch() { release_graph(); }
 
 void GraphBatch::release_graph()
@@ -245,36 +222,28 @@ void GraphBatch::release_graph()
   graph = nullptr;
 }
 
-// Upload jobs and the tile queues; capture the launches once, in queue order.
+// Upload jobs and the queues' spans; capture the launches once, in queue order.
 int GraphBatch::build(const std::vector<BatchJob> &jobs, const std::vector<TileQueue> &queues, hipStream_t s)
 {
   release_graph();
-  const int nq = (int)queues.size();
-  size_t nt = 0;
-  for (const auto &q : queues) nt += q.tiles.size();
+  std::vector<BatchSpan> all;
+  nlaunch = 0;
+  ntiles = 0;
+  for (const auto &q : queues) {
+    all.insert(all.end(), q.spans.begin(), q.spans.end());
+    ntiles += (size_t)q.tiles;
+    if (q.tiles) ++nlaunch;
+  }
   int st;
   if ((st = d_jobs.alloc(std::max<size_t>(jobs.size(), 1) * sizeof(BatchJob))) ||
-      (st = d_tiles.alloc(std::max<size_t>(nt, 1) * sizeof(BatchTile))) || (st = d_meta.alloc(std::max(nq, 1) * sizeof(int))))
+      (st = d_spans.alloc(std::max<size_t>(all.size(), 1) * sizeof(BatchSpan))))
     return st;
-  std::vector<BatchTile> all;
-  all.reserve(nt);
-  std::vector<int> counts((size_t)std::max(nq, 1), 0); // tile counts
-  std::vector<size_t> offset(nq);
-  nlaunch = 0;
-  for (int k = 0; k < nq; ++k) {
-    offset[k] = all.size();
-    counts[k] = (int)queues[k].tiles.size();
-    all.insert(all.end(), queues[k].tiles.begin(), queues[k].tiles.end());
-    if (counts[k]) ++nlaunch;
-  }
   hipError_t e = hipSuccess;
   if (!jobs.empty()) e = hipMemcpyAsync(d_jobs.p, jobs.data(), jobs.size() * sizeof(BatchJob), hipMemcpyHostToDevice, s);
   if (e == hipSuccess && !all.empty())
-    e = hipMemcpyAsync(d_tiles.p, all.data(), all.size() * sizeof(BatchTile), hipMemcpyHostToDevice, s);
-  if (e == hipSuccess) e = hipMemcpyAsync(d_meta.p, counts.data(), counts.size() * sizeof(int), hipMemcpyHostToDevice, s);
+    e = hipMemcpyAsync(d_spans.p, all.data(), all.size() * sizeof(BatchSpan), hipMemcpyHostToDevice, s);
   if (e == hipSuccess) e = hipStreamSynchronize(s);
   if (e != hipSuccess) return hip_fail(e, "batch table upload");
-  ntiles = nt;
   if (nlaunch == 0) return OVX_OK;
 
   hipStream_t cap;
@@ -282,15 +251,10 @@ int GraphBatch::build(const std::vector<BatchJob> &jobs, const std::vector<TileQ
   if (e != hipSuccess) return hip_fail(e, "capture stream");
   e = hipStreamBeginCapture(cap, hipStreamCaptureModeThreadLocal);
   if (e == hipSuccess) {
-    const BatchJob *dj = (const BatchJob *)d_jobs.p;
-    int *meta = (int *)d_meta.p;
-    for (int k = 0; k < nq && e == hipSuccess; ++k) {
-      if (!counts[k]) continue;
-      const BatchTile *t = (const BatchTile *)d_tiles.p + offset[k];
-      if (queues[k].line == 0) e = launch_batch(dj, t, meta + k, device_cu_count(), cap);
-      else if (queues[k].line == kMidLine)
-        e = launch_batch_mid(dj, t, meta + k, kBatchMidBlocksPerCu * device_cu_count(), cap);
-      else e = launch_batch_fs(queues[k].line, queues[k].pass, dj, t, meta + k, counts[k], cap); // one workgroup per tile
+    const BatchSpan *spans = (const BatchSpan *)d_spans.p;
+    for (const auto &q : queues) {
+      if (e == hipSuccess) e = launch_queue(q, (const BatchJob *)d_jobs.p, spans, cap);
+      spans += q.spans.size();
     }
     hipError_t e2 = hipStreamEndCapture(cap, &graph);
     if (e == hipSuccess) e = e2;
@@ -402,12 +366,10 @@ extern "C" int ovx_batch_commit(ovx_batch b, void *stream)
   // (1024-thread rows, then the shorter ones), then the four-step jobs' rows
   // in Infinity-Cache-sized chunks, one launch per non-empty (pass, line
   // length) queue of a chunk, in pass order.
-  std::vector<BatchTile> q[kBatchQueues];
+  std::vector<TileQueue> queues(2);
+  queues[1].line = kMidLine;
   for (int i : order)
-    if (b->djobs[i].path != BP_FS) make_batch_tiles(b->djobs[i], i, q, 1);
-  std::vector<TileQueue> queues;
-  if (!q[0].empty()) queues.push_back(TileQueue{ 0, 0, std::move(q[0]) });
-  if (!q[kMidQueue].empty()) queues.push_back(TileQueue{ kMidLine, 0, std::move(q[kMidQueue]) });
+    if (b->djobs[i].path != BP_FS) push_row_tiles(b->djobs[i], i, false, queues[0], queues[1]);
   for (auto &fq : chunked_fs_queues(b->djobs, order, kFsChunkBytes)) queues.push_back(std::move(fq));
   int st = b->gb.build(b->djobs, queues, s);
   if (st) return st;

@@ -26,26 +26,12 @@ int batch_path_of(const LineFFT &f);
 int device_cu_count();
 int make_batch_job(const LineFFT &f, long rows, const float2 *x, long ldx, float2 *y, long ldy, const float2 *wprep,
                    BatchJob *job);
-// Tiles of job `ji` appended to the batch's queues (kBatchQueues of them);
-// conv_rows: rows per tile of a four-step job's middle pass.
-void make_batch_tiles(const BatchJob &j, int ji, std::vector<BatchTile> q[kBatchQueues], int conv_rows);
 // Middle-pass workgroups of one row each that `rows` rows of a four-step job
 // of n = n1 * n2 points make (fs_conv_rows turns their sum over a launch into
 // rows per tile).
 long batch_conv_workgroups(int n1, int n2, long rows);
-// Four-step forward Fftm tiles (x -> workspace -> y) of job `ji`.
-void make_batch_fft_tiles(const BatchJob &j, int ji, std::vector<BatchTile> q[kBatchQueues]);
-// Capture the launches of a batch into `graph` on stream `cap`: the
-// persistent launches over queue 0 and kMidQueue, then one launch per
-// four-step queue in pass order; `all` launches every queue (tile counts read from device memory at
-// run time), otherwise only the non-empty ones in `counts`.
-hipError_t capture_batch_launches(const BatchJob *jobs, BatchTile *const tiles[kBatchQueues], int *meta,
-                                  const int *counts, bool all, hipStream_t cap);
 // Prepared spectrum of a resident replica in the layout of path `f`.
 int replica_prepared(int id, const float2 **prep, long *n, const LineFFT *f);
-
-// Server slot tables: tile counts [0 .. kBatchQueues).
-constexpr int kMetaInts = 16;
 
 // One launch of a batch: a persistent kernel over LDS-resident tiles
 // (line == 0: the 1024-thread one, line == kMidLine: the 512-thread one) or
@@ -54,8 +40,16 @@ constexpr int kMidLine = -1;
 struct TileQueue {
   int line = 0;
   int pass = 0;
-  std::vector<BatchTile> tiles;
+  std::vector<BatchSpan> spans;
+  int tiles = 0;
+  // `count` tiles of operation `op` over rows [row0, row1) of job `job`
+  void push(int job, int op, long row0, long row1, long count, int conv_rows = 0);
 };
+// Launch queue `q` whose spans are at `spans` in device memory.
+hipError_t launch_queue(const TileQueue &q, const BatchJob *jobs, const BatchSpan *spans, hipStream_t s);
+// Append job `ji`, whose rows are LDS-resident, to the queue of its persistent
+// launch: fastconv rows, or a forward Fftm's.
+void push_row_tiles(const BatchJob &j, int ji, bool fft, TileQueue &big, TileQueue &mid);
 
 // Four-step passes of a batch in chunks of about kFsChunkBytes of rows
 // (rows of one job may fall into different chunks), each chunk's three passes
@@ -65,14 +59,14 @@ struct TileQueue {
 // up, which is what one pass over all of a batch's four-step rows gives.
 constexpr size_t kFsChunkBytes = (size_t)128 << 20;
 // Four-step queues (in launch order) of jobs order[0], order[1], ... that
-// take the four-step path.
+// take the four-step path; a job with a workspace is a forward Fftm.
 std::vector<TileQueue> chunked_fs_queues(const std::vector<BatchJob> &jobs, const std::vector<int> &order,
                                          size_t chunk_bytes);
 
-// Device job/tile tables plus the batch's launches (queues in launch order)
+// Device job/span tables plus the batch's launches (queues in launch order)
 // captured in one hipGraph.
 struct GraphBatch {
-  DevBuf d_jobs, d_tiles, d_meta;
+  DevBuf d_jobs, d_spans;
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
   int nlaunch = 0;

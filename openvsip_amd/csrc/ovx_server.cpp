@@ -2,12 +2,14 @@
 //
 // Requests (fast convolution against a resident replica, forward Fftm,
 // FFT-based correlation against a prepared reference) arrive on a queue.  A
-// scheduler thread takes a free slot -- a stream with its own device tile
-// tables, four-step workspace and a hipGraph of tile-queue launches (the
-// persistent launches, one per four-step pass and line length) captured once
-// at start-up -- admits queued requests into it in
-// arrival order while their device working sets fit the HBM budget, uploads
-// the slot's tables and replays the graph.  A completion thread retires slots
+// scheduler thread takes a free slot -- a stream with its own device tables and
+// four-step workspace -- admits queued requests into it in arrival order while
+// their device working sets fit the HBM budget, uploads the slot's job and span
+// tables in one copy and launches its tile queues (the persistent launches,
+// one per four-step pass and line length; empty ones are left out).  Launched
+// one by one, the first runs while the host issues the next; a graph captured
+// once at start-up had to launch every queue, 4.6 us each when empty, and took
+// up to nine copies.  A completion thread retires slots
 // in launch order, stamps completion times and returns their budget.  With
 // several slots, requests that arrive while others run are admitted as slots
 // free up and their batches overlap on the device.  In plain mode every
@@ -103,12 +105,8 @@ struct Req {
 struct Slot {
   hipStream_t stream = nullptr;
   hipEvent_t done = nullptr;
-  DevBuf d_jobs, d_tiles[kBatchQueues], d_meta, ws;
-  BatchJob *h_jobs = nullptr;
-  BatchTile *h_tiles[kBatchQueues] = {};
-  int *h_meta = nullptr;
-  hipGraph_t graph = nullptr;
-  hipGraphExec_t exec = nullptr;
+  DevBuf d_tab, ws;
+  char *h_tab = nullptr; // jobs, then the queues' spans
   std::vector<Req *> reqs;
   size_t bytes = 0;
 };
@@ -129,6 +127,7 @@ struct Server {
   int error = OVX_OK;
   std::thread sched, compl_;
   long max_tiles = 0;
+  size_t table_bytes = 0;
   int device = 0;
 
   ~Server();
@@ -161,13 +160,9 @@ Server::~Server()
   cv_done.notify_all();
   if (compl_.joinable()) compl_.join();
   for (auto &s : slots) {
-    if (s->exec) (void)hipGraphExecDestroy(s->exec);
-    if (s->graph) (void)hipGraphDestroy(s->graph);
     if (s->done) (void)hipEventDestroy(s->done);
     if (s->stream) (void)hipStreamDestroy(s->stream);
-    free_pinned(s->h_jobs);
-    for (int k = 0; k < kBatchQueues; ++k) free_pinned(s->h_tiles[k]);
-    free_pinned(s->h_meta);
+    free_pinned(s->h_tab);
   }
 }
 
@@ -177,34 +172,10 @@ int Server::build_slot(Slot &s)
   if (e == hipSuccess) e = hipEventCreateWithFlags(&s.done, hipEventDisableTiming);
   if (e != hipSuccess) return hip_fail(e, "slot stream");
   int st;
-  size_t jb = (size_t)cfg.max_jobs * sizeof(BatchJob), tb = (size_t)max_tiles * sizeof(BatchTile);
-  if ((st = s.d_jobs.alloc(jb)) || (st = s.d_meta.alloc(kMetaInts * sizeof(int)))) return st;
-  for (int k = 0; k < kBatchQueues; ++k)
-    if ((st = s.d_tiles[k].alloc(tb))) return st;
+  if ((st = s.d_tab.alloc(table_bytes))) return st;
   if (cfg.workspace_mb > 0 && (st = s.ws.alloc((size_t)cfg.workspace_mb << 20))) return st;
-  e = hipHostMalloc((void **)&s.h_jobs, jb, hipHostMallocDefault);
-  for (int k = 0; k < kBatchQueues && e == hipSuccess; ++k)
-    e = hipHostMalloc((void **)&s.h_tiles[k], tb, hipHostMallocDefault);
-  if (e == hipSuccess) e = hipHostMalloc((void **)&s.h_meta, kMetaInts * sizeof(int), hipHostMallocDefault);
+  e = hipHostMalloc((void **)&s.h_tab, table_bytes, hipHostMallocDefault);
   if (e != hipSuccess) return hip_fail(e, "pinned staging");
-  if (cfg.plain) return OVX_OK;
-  // capture the launches (the persistent one and one per four-step queue)
-  // once; every batch reuses them with new table contents (tile counts are
-  // read from device memory, an empty queue's launch exits at once)
-  hipStream_t cap;
-  e = hipStreamCreateWithFlags(&cap, hipStreamNonBlocking);
-  if (e != hipSuccess) return hip_fail(e, "capture stream");
-  e = hipStreamBeginCapture(cap, hipStreamCaptureModeThreadLocal);
-  if (e == hipSuccess) {
-    BatchTile *tiles[kBatchQueues];
-    for (int k = 0; k < kBatchQueues; ++k) tiles[k] = (BatchTile *)s.d_tiles[k].p;
-    e = capture_batch_launches((const BatchJob *)s.d_jobs.p, tiles, (int *)s.d_meta.p, nullptr, true, cap);
-    hipError_t e2 = hipStreamEndCapture(cap, &s.graph);
-    if (e == hipSuccess) e = e2;
-  }
-  if (e == hipSuccess) e = hipGraphInstantiate(&s.exec, s.graph, nullptr, nullptr, 0);
-  (void)hipStreamDestroy(cap);
-  if (e != hipSuccess) return hip_fail(e, "slot graph capture");
   return OVX_OK;
 }
 
@@ -216,6 +187,11 @@ int Server::init(const ovx_server_config &c)
   if (cfg.plain) cfg.max_jobs = 1; // one request per launch, `slots` requests in flight
   budget = (size_t)std::max(cfg.hbm_budget_mb, 1l) << 20;
   max_tiles = cfg.max_tiles > 0 ? cfg.max_tiles : 65536;
+  // one span per LDS-resident job, three per part of a four-step one; the parts
+  // are at most the jobs and the ends of chunks together (a chunk is full when
+  // the next row, 2 MB at most, does not fit)
+  const size_t chunks = budget / (kFsChunkBytes - ((size_t)4 << 20)) + 1;
+  table_bytes = (size_t)cfg.max_jobs * sizeof(BatchJob) + 3 * ((size_t)cfg.max_jobs + chunks) * sizeof(BatchSpan);
   (void)hipGetDevice(&device);
   for (int i = 0; i < cfg.slots; ++i) {
     slots.emplace_back(new (std::nothrow) Slot());
@@ -248,16 +224,10 @@ static long tiles_of(const Req &q, const LineFFT *f, const CorrRef *cr)
 int Server::admit_and_launch(Slot &s, std::vector<Req *> &batch)
 {
   std::vector<BatchJob> jobs;
-  std::vector<BatchTile> q[kBatchQueues];
+  std::vector<int> order;
+  std::vector<TileQueue> queues(2);
+  queues[1].line = kMidLine;
   size_t ws_off = 0;
-  long conv_wgs = 0; // middle-pass workgroups of the batch's four-step fastconvs
-  for (const Req *q0 : batch) {
-    int st;
-    const LineFFT *f = q0->r.kind == OVX_REQ_FASTCONV ? shared_path(q0->r.n, q0->r.rows, &st) : nullptr;
-    if (f && f->kind == LineFFT::FOURSTEP && batch_supported(BP_FS, (int)f->n))
-      conv_wgs += batch_conv_workgroups((int)f->n1, (int)f->n2, q0->r.rows);
-  }
-  const int conv_rows = fs_conv_rows(conv_wgs, false);
   for (size_t i = 0; i < batch.size(); ++i) {
     const ovx_request &r = batch[i]->r;
     int st;
@@ -270,9 +240,8 @@ int Server::admit_and_launch(Slot &s, std::vector<Req *> &batch)
       j.ols = corr_ols_args(*cr, (const float2 *)r.x, (float2 *)r.y, r.bias);
       j.ols_len = cr->L;
       jobs.push_back(j);
-      int spt = batch_ols_segments_per_tile(cr->L);
-      std::vector<BatchTile> &dst = q[batch_ols_queue(cr->L)];
-      for (long sgm = 0; sgm < corr_segments(*cr); sgm += spt) dst.push_back(BatchTile{ (int)i, BT_OLS, (int)sgm, 0 });
+      const long seg = corr_segments(*cr), spt = batch_ols_segments_per_tile(cr->L);
+      queues[batch_ols_queue(cr->L) == kMidQueue].push((int)i, BT_OLS, 0, seg, (seg + spt - 1) / spt);
       continue;
     }
     const LineFFT *f = shared_path(r.n, r.rows, &st);
@@ -282,41 +251,37 @@ int Server::admit_and_launch(Slot &s, std::vector<Req *> &batch)
       long rn;
       if ((st = replica_prepared(r.ref, &prep, &rn, f))) return st;
       if ((st = make_batch_job(*f, r.rows, (const float2 *)r.x, r.ldx, (float2 *)r.y, r.ldy, prep, &j))) return st;
-      jobs.push_back(j);
-      make_batch_tiles(j, (int)i, q, conv_rows);
     } else { // forward Fftm
       if ((st = make_batch_job(*f, r.rows, (const float2 *)r.x, r.ldx, (float2 *)r.y, r.ldy, nullptr, &j))) return st;
-      j.scale = 1.0f;
       if (j.path == BP_FS) {
         j.ws = (float2 *)((char *)s.ws.p + ws_off);
         ws_off += batch[i]->ws_need;
-        make_batch_fft_tiles(j, (int)i, q);
-      } else {
-        int rpt = batch_rows_per_tile(j.path, j.n);
-        int op = j.path == BP_HIER ? BT_HIER_FFT_FWD : BT_ROW_FFT_FWD;
-        std::vector<BatchTile> &dst = q[batch_queue(j.path, j.n)];
-        for (long rr = 0; rr < j.rows; rr += rpt) dst.push_back(BatchTile{ (int)i, op, (int)rr, 0 });
       }
-      jobs.push_back(j);
     }
+    jobs.push_back(j);
+    if (j.path == BP_FS) order.push_back((int)i);
+    else push_row_tiles(j, (int)i, r.kind == OVX_REQ_FFTM, queues[0], queues[1]);
   }
-  for (int k = 0; k < kBatchQueues; ++k)
-    if ((long)q[k].size() > max_tiles) return fail(OVX_ERR_STATE, "slot tile table overflow");
-  std::copy(jobs.begin(), jobs.end(), s.h_jobs);
-  int meta[kMetaInts] = { 0 };
-  for (int k = 0; k < kBatchQueues; ++k) {
-    std::copy(q[k].begin(), q[k].end(), s.h_tiles[k]);
-    meta[k] = (int)q[k].size();
+  for (auto &fq : chunked_fs_queues(jobs, order, kFsChunkBytes)) queues.push_back(std::move(fq));
+  const size_t job_bytes = jobs.size() * sizeof(BatchJob);
+  static_assert(sizeof(BatchJob) % alignof(BatchSpan) == 0, "the spans follow the jobs");
+  size_t used = job_bytes;
+  long tiles[kBatchQueues] = { 0 }; // of all chunks together
+  for (const auto &q : queues) {
+    const int k = q.line == 0 ? 0 : q.line == kMidLine ? kMidQueue : fs_queue(q.pass, q.line);
+    if ((tiles[k] += q.tiles) > max_tiles) return fail(OVX_ERR_STATE, "slot tile table overflow");
+    used += q.spans.size() * sizeof(BatchSpan);
   }
-  std::copy(meta, meta + kMetaInts, s.h_meta);
-  hipError_t e = hipMemcpyAsync(s.d_jobs.p, s.h_jobs, jobs.size() * sizeof(BatchJob), hipMemcpyHostToDevice, s.stream);
-  for (int k = 0; k < kBatchQueues && e == hipSuccess; ++k)
-    if (!q[k].empty())
-      e = hipMemcpyAsync(s.d_tiles[k].p, s.h_tiles[k], q[k].size() * sizeof(BatchTile), hipMemcpyHostToDevice,
-                         s.stream);
-  if (e == hipSuccess)
-    e = hipMemcpyAsync(s.d_meta.p, s.h_meta, kMetaInts * sizeof(int), hipMemcpyHostToDevice, s.stream);
-  if (e == hipSuccess) e = hipGraphLaunch(s.exec, s.stream);
+  if (used > table_bytes) return fail(OVX_ERR_STATE, "slot span table overflow");
+  std::copy(jobs.begin(), jobs.end(), (BatchJob *)s.h_tab);
+  BatchSpan *h = (BatchSpan *)(s.h_tab + job_bytes);
+  for (const auto &q : queues) h = std::copy(q.spans.begin(), q.spans.end(), h);
+  hipError_t e = hipMemcpyAsync(s.d_tab.p, s.h_tab, used, hipMemcpyHostToDevice, s.stream);
+  const BatchSpan *spans = (const BatchSpan *)((char *)s.d_tab.p + job_bytes);
+  for (const auto &q : queues) {
+    if (e == hipSuccess) e = launch_queue(q, (const BatchJob *)s.d_tab.p, spans, s.stream);
+    spans += q.spans.size();
+  }
   if (e != hipSuccess) return hip_fail(e, "batch launch");
   return OVX_OK;
 }

@@ -282,11 +282,9 @@ int autotune_batch(long n, long rows, int *best_variant, double *best_us)
     BatchJob j;
     if ((st = make_batch_job(f, rows, (const float2 *)x.p, n, (float2 *)y.p, n, (const float2 *)wp.p, &j))) break;
     std::vector<BatchJob> jobs(1, j);
-    std::vector<BatchTile> q[kBatchQueues];
-    make_batch_tiles(j, 0, q, 1);
-    std::vector<TileQueue> queues;
-    if (!q[0].empty()) queues.push_back(TileQueue{ 0, 0, std::move(q[0]) });
-    if (!q[kMidQueue].empty()) queues.push_back(TileQueue{ kMidLine, 0, std::move(q[kMidQueue]) });
+    std::vector<TileQueue> queues(2);
+    queues[1].line = kMidLine;
+    push_row_tiles(j, 0, false, queues[0], queues[1]);
     GraphBatch gb;
     if ((st = gb.build(jobs, queues, s))) break;
     auto t0 = std::chrono::steady_clock::now();
