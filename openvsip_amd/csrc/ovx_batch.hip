@@ -327,7 +327,7 @@ __device__ __forceinline__ void fs_col_tile(const Tile &t, int groups, int &row,
 // workgroups run independently and overlap their loads with other groups'
 // arithmetic.  The job descriptor is read from global memory (uniform per tile,
 // scalar loads).
-template <int L, int PASS>
+template <int L, int PASS, bool STREAM>
 __global__ __launch_bounds__(FsCfg<L>::NT, 4) void k_batch_fs(
     const BatchJob *__restrict__ jobs, const BatchSpan *__restrict__ spans, int nspans)
 {
@@ -347,7 +347,7 @@ __global__ __launch_bounds__(FsCfg<L>::NT, 4) void k_batch_fs(
     a.out = fft ? j.ws : j.y;
     a.ld_out = fft ? (long)j.n : j.ldy;
     fs_col_tile(tile, j.n2 / F::C, row, group);
-    fs_col_body<L, F::P, F::C, -1>(a, row, group, tid, lds);
+    fs_col_body<L, F::P, F::C, -1, false, false, STREAM>(a, row, group, tid, lds);
   } else if constexpr (PASS == 1) {
     if (tile.op == BT_FS_B) { // fastconv: middle pass in place on y
       a.in = j.y;
@@ -372,25 +372,31 @@ __global__ __launch_bounds__(FsCfg<L>::NT, 4) void k_batch_fs(
     a.out = j.y;
     a.ld_out = j.ldy;
     fs_col_tile(tile, j.n2 / F::C, row, group);
-    fs_col_body<L, F::P, F::C, +1>(a, row, group, tid, lds);
+    fs_col_body<L, F::P, F::C, +1, false, false, STREAM, STREAM>(a, row, group, tid, lds);
   }
 }
 
-template <int L>
-static hipError_t launch_fs_pass(int pass, const BatchQueue &q, hipStream_t s)
+template <int L, int PASS, bool STREAM>
+static hipError_t launch_fs(const BatchQueue &q, hipStream_t s)
 {
-  constexpr int NT = FsCfg<L>::NT;
-  if (pass == 0) hipLaunchKernelGGL((k_batch_fs<L, 0>), dim3(q.tiles), dim3(NT), 0, s, q.jobs, q.spans, q.nspans);
-  else if (pass == 1) hipLaunchKernelGGL((k_batch_fs<L, 1>), dim3(q.tiles), dim3(NT), 0, s, q.jobs, q.spans, q.nspans);
-  else hipLaunchKernelGGL((k_batch_fs<L, 2>), dim3(q.tiles), dim3(NT), 0, s, q.jobs, q.spans, q.nspans);
+  hipLaunchKernelGGL((k_batch_fs<L, PASS, STREAM>), dim3(q.tiles), dim3(FsCfg<L>::NT), 0, s, q.jobs, q.spans,
+                     q.nspans);
   return hipGetLastError();
 }
 
-hipError_t launch_batch_fs(int n_line, int pass, const BatchQueue &q, hipStream_t s)
+template <int L>
+static hipError_t launch_fs_pass(int pass, bool stream, const BatchQueue &q, hipStream_t s)
+{
+  if (pass == 0) return stream ? launch_fs<L, 0, true>(q, s) : launch_fs<L, 0, false>(q, s);
+  if (pass == 1) return launch_fs<L, 1, false>(q, s);
+  return stream ? launch_fs<L, 2, true>(q, s) : launch_fs<L, 2, false>(q, s);
+}
+
+hipError_t launch_batch_fs(int n_line, int pass, bool stream, const BatchQueue &q, hipStream_t s)
 {
   if (q.tiles <= 0) return hipSuccess;
-  if (n_line == 256) return launch_fs_pass<256>(pass, q, s);
-  if (n_line == 512) return launch_fs_pass<512>(pass, q, s);
+  if (n_line == 256) return launch_fs_pass<256>(pass, stream, q, s);
+  if (n_line == 512) return launch_fs_pass<512>(pass, stream, q, s);
   return hipErrorInvalidValue;
 }
 

@@ -108,8 +108,9 @@ hipError_t launch_batch(const BatchQueue &q, int grid, hipStream_t s);
 hipError_t launch_batch_mid(const BatchQueue &q, int grid, hipStream_t s);
 constexpr int kBatchMidBlocksPerCu = 2;
 // Four-step pass `pass` (0, 1, 2) over a queue of line length n_line (256 or
-// 512), one tile per workgroup.
-hipError_t launch_batch_fs(int n_line, int pass, const BatchQueue &q, hipStream_t s);
+// 512), one tile per workgroup; `stream`: a column pass with non-temporal access
+// (fs_streams_in, fs_streams_out).
+hipError_t launch_batch_fs(int n_line, int pass, bool stream, const BatchQueue &q, hipStream_t s);
 inline int fs_queue_pass(int q) { return (q - 1) / 2; }
 
 } // namespace ovx

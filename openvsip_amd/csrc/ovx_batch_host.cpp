@@ -139,7 +139,9 @@ hipError_t launch_queue(const TileQueue &q, const BatchJob *jobs, const BatchSpa
   const BatchQueue bq{ jobs, spans, (int)q.spans.size(), q.tiles };
   if (q.line == 0) return launch_batch(bq, std::min(q.tiles, device_cu_count()), s);
   if (q.line == kMidLine) return launch_batch_mid(bq, std::min(q.tiles, kBatchMidBlocksPerCu * device_cu_count()), s);
-  return launch_batch_fs(q.line, q.pass, bq, s);
+  // a chunk's first and last pass access memory as a standalone call's
+  const bool stream = q.pass == 0 ? fs_streams_in(q.bytes) : fs_streams_out(q.bytes);
+  return launch_batch_fs(q.line, q.pass, stream, bq, s);
 }
 
 void push_row_tiles(const BatchJob &j, int ji, bool fft, TileQueue &big, TileQueue &mid)
@@ -186,6 +188,7 @@ std::vector<TileQueue> chunked_fs_queues(const std::vector<BatchJob> &jobs, cons
       if (!cq[k].tiles) continue;
       cq[k].line = fs_queue_line(k);
       cq[k].pass = fs_queue_pass(k);
+      cq[k].bytes = used;
       out.push_back(std::move(cq[k]));
     }
     chunk.clear();

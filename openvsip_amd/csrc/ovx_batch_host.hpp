@@ -42,6 +42,7 @@ struct TileQueue {
   int pass = 0;
   std::vector<BatchSpan> spans;
   int tiles = 0;
+  size_t bytes = 0; // four-step: rows of the chunk
   // `count` tiles of operation `op` over rows [row0, row1) of job `job`
   void push(int job, int op, long row0, long row1, long count, int conv_rows = 0);
 };
@@ -54,10 +55,12 @@ void push_row_tiles(const BatchJob &j, int ji, bool fft, TileQueue &big, TileQue
 // Four-step passes of a batch in chunks of about kFsChunkBytes of rows
 // (rows of one job may fall into different chunks), each chunk's three passes
 // launched back to back: a chunk's matrix then stays in the 256 MB Infinity
-// Cache from one pass to the next.  Standalone 65536-point fastconvs run at
-// 0.56 us per row with 96-128 MB matrices and at 0.70 us per row from 512 MB
-// up, which is what one pass over all of a batch's four-step rows gives.
-constexpr size_t kFsChunkBytes = (size_t)128 << 20;
+// Cache from one pass to the next, X and the result passing it by
+// (fs_streams_in, fs_streams_out).  Chunks of 96 / 128 / 160 / 192 / 224 / 256 /
+// 512 MB, us: 400 rows of 65536 247 / 228 / 230 / 222 / 207 / 212 / 209, 800 rows
+// 467 / 437 / 425 / 422 / 402 / 413 / 431, 2000 rows 1118 / 1050 / 1032 / 1011 /
+// 995 / 1002 / 1072, 240 rows of 262144 567 / 543 / 524 / 532 / 538 / 527 / 563.
+constexpr size_t kFsChunkBytes = (size_t)192 << 20;
 // Four-step queues (in launch order) of jobs order[0], order[1], ... that
 // take the four-step path; a job with a workspace is a forward Fftm.
 std::vector<TileQueue> chunked_fs_queues(const std::vector<BatchJob> &jobs, const std::vector<int> &order,
