@@ -471,6 +471,15 @@ int LineFFT::fastconv_split(const float *xr, const float *xi, long ldx, const fl
   return hier_fastconv(a, HIER_FASTCONV_SPLIT, ldx, w, ldy, lines, scale, s);
 }
 
+// Whether the spectra (one of n values, or one per line) and the result share
+// memory: a spectrum read beside or after the first writes has to be laid out
+// beforehand.
+static bool spectrum_meets_result(const float2 *w, long ldw, const float2 *y, long ldy, long lines, long n)
+{
+  const float2 *w1 = w + (ldw ? (lines - 1) * ldw : 0) + n, *y1 = y + (lines - 1) * ldy + n;
+  return w < y1 && y < w1;
+}
+
 int LineFFT::fastconv(const float2 *x, long ldx, const float2 *w, long ldw, float2 *y, long ldy, long lines,
                       float scale, hipStream_t s, const ExtScratch *ext) const
 {
@@ -494,8 +503,11 @@ int LineFFT::fastconv(const float2 *x, long ldx, const float2 *w, long ldw, floa
     if (lines > 65535) return fail(OVX_ERR_UNSUPPORTED, "more than 65535 lines of a four-step fastconv");
     long wrows = ldw ? lines : 1;
     float2 *wpp;
+    if (ext && ext->wp_elems < (size_t)wrows * n)
+      return fail(OVX_ERR_UNSUPPORTED, "lent scratch too small for the spectrum");
+    if (fs_takes_natural(n2, n, lines) && !spectrum_meets_result(w, ldw, y, ldy, lines, n))
+      return fs_fastconv(x, ldx, w, ldw, y, ldy, lines, s, &scale);
     if (ext) {
-      if (ext->wp_elems < (size_t)wrows * n) return fail(OVX_ERR_UNSUPPORTED, "lent scratch too small for the spectrum");
       wpp = ext->wp;
     } else {
       int st = wp.alloc((size_t)wrows * n * 8);
@@ -516,12 +528,15 @@ int LineFFT::fastconv(const float2 *x, long ldx, const float2 *w, long ldw, floa
 // slower at every chunk size from 16 to 128 MiB of X (the passes lose
 // parallelism faster than they gain cache hits), so one launch per pass
 // covers every row.
+// `natural`: the spectra are in natural order, to be scaled by it.
 int LineFFT::fs_fastconv(const float2 *x, long ldx, const float2 *wprep, long ldwp, float2 *y, long ldy, long lines,
-                         hipStream_t s) const
+                         hipStream_t s, const float *natural) const
 {
   FsArgs a = fs_args(*this);
   a.wp = wprep;
   a.ldwp = ldwp;
+  a.natural = natural != nullptr;
+  a.wscale = natural ? *natural : 1.0f;
   a.in = x;
   a.ld_in = ldx;
   a.out = y;

@@ -18,6 +18,10 @@ struct FsArgs {
   const float2 *tfull;     // W_N^{k1 n2} at [k1 * n2count + n2], or null (two-level)
   const float2 *wp;        // fastconv: permuted, scaled spectrum [k1][k2]
   long ldwp;               // 0: one spectrum for every row
+  // wp is instead the spectrum in natural order, W[k1 + N1 k2], to be scaled by
+  // wscale (fs_takes_natural)
+  bool natural = false;
+  float wscale = 1.0f;
   float scale;
   // split storage for a call's first read / last write (separate real and
   // imaginary arrays at the strides ld_in / ld_out); null: in / out are used
@@ -52,6 +56,19 @@ inline bool fs_stays_in_l2(long n, long rows)
 // 256 x 65536 127 / 124 / 120 / 120; at 32 MB 41 / 43 / 48 / 49.
 inline bool fs_streams_in(size_t bytes) { return bytes >= ((size_t)64 << 20); }
 inline bool fs_streams_out(size_t bytes) { return bytes >= ((size_t)96 << 20); }
+
+// Whether the middle pass reads spectra in natural order itself, or
+// launch_fs_permute lays them out first.  The C neighbouring lines of a
+// workgroup (16 to 4 up to 512 points) make runs of 128 to 32 bytes, which
+// neighbouring groups complete in L2; 32-byte runs only pay while the call fits
+// there.  Laid out / natural, us: 256-point lines, one spectrum, 1 row of 65536
+// 12.8 / 10.9, a spectrum per row, 64 rows 54.4 / 42.4, 256 rows 190 / 169;
+// 512-point lines, one spectrum, 1 row of 262144 18.9 / 16.6, a spectrum per row,
+// 24 rows of 131072 42.9 / 37.5, 100 rows 151 / 162, 16 rows of 262144 57.5 / 62.2.
+inline bool fs_takes_natural(long n2, long n, long rows)
+{
+  return n2 <= 256 || (n2 == 512 && rows * n * 8 < 8 * (4l << 20));
+}
 
 // Column pass of `rows` rows in direction dir; row pass of a transform; middle
 // pass of a fastconv.

@@ -161,7 +161,9 @@ struct FsConv {
   static constexpr int T = L / P;
   static constexpr int LROW = LdsLayout<L, P>::elems | 1;
 };
-template <int L, int C, typename LP>
+// NATURAL: the spectrum is W[k1 + N1 k2], read in runs of the C lines and
+// turned over in LDS (fs_takes_natural()).
+template <int L, int C, bool NATURAL = false, typename LP>
 __device__ __forceinline__ void fs_conv_body(const FsArgs &a, long row0, int nrows, int step, long group, int tid, LP lds_all)
 {
   constexpr int P = FsConv<L>::P, T = FsConv<L>::T;
@@ -172,12 +174,34 @@ __device__ __forceinline__ void fs_conv_body(const FsArgs &a, long row0, int nro
   const rsrc_t rtw = make_rsrc(a.tw2c, (uint32_t)(E::plan.twtotal + 1) * 8u);
   LP lds = lds_all + c * FsConv<L>::LROW;
   const uint32_t lane = (uint32_t)k1 * L + t;
-  const float2 *wp = a.wp + row0 * a.ldwp + k1 * L + t;
+  // this thread's entry of the spectrum: its own in [k1][k2] order, or entry tid,
+  // tid + C T, ... of the lines' C values of each k2
+  const float2 *wp = a.wp + row0 * a.ldwp;
+  if constexpr (NATURAL) wp += group * C + tid % C + (long)(tid / C) * a.n1;
+  else wp += k1 * L + t;
 
   float2 w[P], ws[P], st[E::HELD];
-  fs_line_twiddles<L, P>(a, k1, t, w);
+  auto spectrum = [&] {
 #pragma unroll
-  for (int q = 0; q < P; ++q) ws[q] = wp[T * q];
+    for (int q = 0; q < P; ++q) {
+      if constexpr (NATURAL) ws[q] = cscale(wp[(long)(T * q) * a.n1], a.wscale);
+      else ws[q] = wp[T * q];
+    }
+  };
+  // natural order: from entries by number to the thread's own
+  auto turn = [&] {
+    if constexpr (NATURAL) {
+      __syncthreads(); // the exchanges before are done with the lines
+#pragma unroll
+      for (int q = 0; q < P; ++q) lds_st(lds_all, tid % C * FsConv<L>::LROW + tid / C + T * q, ws[q]);
+      __syncthreads();
+#pragma unroll
+      for (int q = 0; q < P; ++q) ws[q] = lds_ld(lds, t + T * q);
+      asm volatile("" ::: "memory"); // read before the line is written again
+    }
+  };
+  fs_line_twiddles<L, P>(a, k1, t, w);
+  spectrum();
   E::load_held(t, rtw, st);
 #pragma unroll 1
   for (int r = 0; r < nrows; ++r) {
@@ -186,6 +210,7 @@ __device__ __forceinline__ void fs_conv_body(const FsArgs &a, long row0, int nro
     float2 v[P];
 #pragma unroll
     for (int q = 0; q < P; ++q) v[q] = in.ld((uint32_t)(T * q));
+    if (a.ldwp || r == 0) turn();
 #pragma unroll
     for (int q = 0; q < P; ++q) v[q] = cmul(v[q], w[q]);
     E::template fft_held<-1>(v, lds, t, st);
@@ -193,8 +218,7 @@ __device__ __forceinline__ void fs_conv_body(const FsArgs &a, long row0, int nro
     for (int q = 0; q < P; ++q) v[q] = cmul(v[q], ws[q]);
     if (a.ldwp && r + 1 < nrows) { // one spectrum per row: the next one
       wp += a.ldwp * step;
-#pragma unroll
-      for (int q = 0; q < P; ++q) ws[q] = wp[T * q];
+      spectrum();
     }
     E::template fft_held<+1>(v, lds, t, st);
 #pragma unroll
