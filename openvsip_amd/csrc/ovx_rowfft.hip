@@ -246,19 +246,23 @@ int row_config_with(int n, int p)
   }
 }
 
-// The first configuration of a length, or for few lines (up to two per CU) the
-// one with fewer values per thread, as long as its lines keep to 256 threads:
-// fastconv of 256 lines, first / few-line form, 384 5.8 / 4.9, 576 6.9 / 5.2,
-// 640 7.6 / 6.3, 1024 5.3 / 4.7, 1536 7.1 / 7.1 (7.3 / 6.7 at 64), 2048
-// 6.9 / 5.7 us; of 1000 lines 5.9 / 5.6, 7.0 / 6.2, 7.6 / 7.4, 6.4 / 7.0,
-// 8.9 / 10.5 and 10.5 / 11.2 us.  Above 256 threads (6144, 12288) the form
-// with fewer values is the slower one from one line on.
+// The first configuration of a length, or the one with fewer values per thread
+// for up to 8 lines a CU if its lines keep to a wave, to one a CU with 128
+// threads and 4 with 256; above 256 threads (6144, 12288) it is the slower one
+// from one line on.  Fastconv, first / fewer values, us: 384 points, 256 lines 5.7 /
+// 4.4, 2000 6.5 / 6.0; 576, 256 6.5 / 4.3, 2000 7.9 / 7.5; 640, 256 7.2 / 5.5, 2000
+// 8.9 / 8.8; 1024, 256 4.8 / 4.4, 400 5.2 / 5.3, 1000 6.2 / 6.4; 1536, 256 6.8 / 6.8
+// (64 7.3 / 6.7), 400 7.4 / 8.2; 2048, 256 6.8 / 5.3, 600 9.6 / 8.4, 1000 11.2 / 11.0
+// (a spectrum per line 13.7 / 11.1), 2000 17.3 / 18.3; 6144, 400 15.9 / 18.3.
 int row_pick(int n, long rows)
 {
   const Entry *first = find_entry(n, 0);
-  if (first && rows <= 2 * kRowSpread)
-    for (int v = 1; const Entry *e = find_entry(n, v); ++v)
-      if (e->p < first->p && n / e->p <= 256) return v;
+  if (!first) return 0;
+  for (int v = 1; const Entry *e = find_entry(n, v); ++v) {
+    const int threads = n / e->p;
+    const long per_cu = threads <= 64 ? 8 : threads <= 128 ? 1 : threads <= 256 ? 4 : 0;
+    if (e->p < first->p && rows <= per_cu * kRowSpread) return v;
+  }
   return 0;
 }
 
