@@ -375,69 +375,66 @@ int LineFFT::transform_split(int dir, const float *in_re, const float *in_im, lo
   return e == hipSuccess ? OVX_OK : hip_fail(e, "row fft launch");
 }
 
-// Split X, Y and a single split spectrum vector: one kernel permutes and
-// scales the spectrum straight from its two arrays, then the split fastconv.
-int LineFFT::fastconv_split_vec(const float *xr, const float *xi, long ldx, const float *wr, const float *wi,
-                                float *yr, float *yi, long ldy, long lines, float scale, hipStream_t s) const
+// Whether `lines` lines of n values at a stride of ld and `lines2` at ld2 share
+// memory.
+template <typename T>
+static bool lines_meet(const T *a, long lines, long ld, const T *b, long lines2, long ld2, long n)
 {
-  if (lines <= 0) return OVX_OK;
-  if (!native_split()) return fail(OVX_ERR_UNSUPPORTED, "no split-storage fastconv kernel on this path");
-  if (!tables_ready()) return fail(OVX_ERR_STATE, "fastconv plan has no twiddle tables");
-  if (kind == FOURSTEP) {
-    // interleave the spectrum into the workspace's tail; fastconv_split
-    // permutes it before its first pass writes the head
-    int st = work.alloc((size_t)(lines + 1) * n * 8);
-    if (st) return st;
-    float2 *wi2 = (float2 *)work.p + (size_t)lines * n;
-    hipError_t e = launch_interleave(wr, wi, 0, wi2, n, 1, n, s);
-    if (e != hipSuccess) return hip_fail(e, "interleave");
-    return fastconv_split(xr, xi, ldx, wi2, 0, yr, yi, ldy, lines, scale, s);
-  }
-  int st = wp.alloc((size_t)n * 8);
-  if (st) return st;
-  if (kind == LDS) {
-    // the register-Stockham kernel reads the spectrum in natural order
-    hipError_t e = launch_interleave(wr, wi, 0, (float2 *)wp.p, n, 1, n, s);
-    if (e != hipSuccess) return hip_fail(e, "interleave");
-    return fastconv_split(xr, xi, ldx, (const float2 *)wp.p, 0, yr, yi, ldy, lines, scale, s);
-  }
-  if (!offsets_fit(hier_rows_per_block(n), std::max(ldx, ldy)))
-    return fail(OVX_ERR_UNSUPPORTED, "row stride too large for 32-bit buffer offsets");
-  hipError_t e = launch_hier_permute_split(wr, wi, (float2 *)wp.p, n, scale, s);
-  if (e != hipSuccess) return hip_fail(e, "spectrum permutation");
-  HierArgs a = hier_args(*this);
-  a.xr = xr;
-  a.xi = xi;
-  a.ldx = ldx;
-  a.yr = yr;
-  a.yi = yi;
-  a.ldy = ldy;
-  a.rows = lines;
-  a.w = (const float2 *)wp.p;
-  e = launch_hier(HIER_FASTCONV_SPLIT, n, a, s);
-  return e == hipSuccess ? OVX_OK : hip_fail(e, "fastconv launch");
+  return a < b + (lines2 - 1) * ld2 + n && b < a + (lines - 1) * ld + n;
 }
 
-int LineFFT::fastconv_split(const float *xr, const float *xi, long ldx, const float2 *w, long ldw, float *yr,
-                            float *yi, long ldy, long lines, float scale, hipStream_t s) const
+// Up to this many lines the register-Stockham kernel, which reads a spectrum
+// vector as it is, takes less than the hierarchical one and its permutation
+// launch.  Hierarchical / register-Stockham, us: 8192 points, 1 row 11.4 / 10.6,
+// 64 rows 11.9 / 11.0, 256 15.3 / 14.9, 300 21.0 / 20.2, 600 28.4 / 29.1; 16384
+// points, 1 row 20.2 / 19.1, 64 rows 21.3 / 19.8, 256 25.6 / 25.3, 300 41.2 / 43.1,
+// 1000 88.3 / 98.3.
+constexpr long kHierVectorLines = 256;
+
+// Whether a fastconv goes to the register-Stockham kernel, which reads spectra in
+// natural order (those of a hierarchical path: see hier_fastconv).
+bool LineFFT::rows_fastconv(long ldw, long lines) const
+{
+  return kind == LDS || (kind == HIER && (ldw != 0 || (n >= 8192 && lines <= kHierVectorLines)));
+}
+
+bool LineFFT::row_strides_fit(long ldx, long ldw, long ldy) const
+{
+  return (unsigned long)rc.rows_per_block * (unsigned long)std::max(std::max(ldx, ldy), ldw) * 8ul < (1ul << 32);
+}
+
+// Fastconv of split X, W and Y.  The register-Stockham kernels read the
+// spectra's two arrays themselves; interleaved by a kernel of its own first, 256 x
+// 1024 took 6.4 us and now 4.4, 256 x 4096 9.7 and 7.7.  For the
+// hierarchical kernel one kernel permutes and scales a vector straight from them.
+int LineFFT::fastconv_split(const float *xr, const float *xi, long ldx, const float *wr, const float *wi, long ldw,
+                            float *yr, float *yi, long ldy, long lines, float scale, hipStream_t s) const
 {
   if (lines <= 0) return OVX_OK;
   if (!native_split()) return fail(OVX_ERR_UNSUPPORTED, "no split-storage fastconv kernel on this path");
   if (!tables_ready()) return fail(OVX_ERR_STATE, "fastconv plan has no twiddle tables");
+  const long wrows = ldw ? lines : 1;
+  int st;
+  hipError_t e;
   if (kind == FOURSTEP) {
     // the three passes of fs_fastconv with X read split by the first and Y
-    // written split by the last; the middle pass works in the workspace
+    // written split by the last; the middle pass works in the workspace, whose
+    // tail takes the spectra interleaved
     if (lines > 65535) return fail(OVX_ERR_UNSUPPORTED, "more than 65535 lines of a four-step fastconv");
-    const long wrows = ldw ? lines : 1;
-    int st = wp.alloc((size_t)wrows * n * 8);
-    if (st) return st;
-    hipError_t e = launch_fs_permute(w, ldw, (float2 *)wp.p, n1, n2, wrows, scale, s);
-    if (e != hipSuccess) return hip_fail(e, "spectrum permutation");
-    if ((st = work.alloc((size_t)lines * n * 8))) return st;
-    float2 *ws = (float2 *)work.p;
+    if ((st = work.alloc((size_t)(lines + wrows) * n * 8))) return st;
+    float2 *ws = (float2 *)work.p, *wi2 = ws + (size_t)lines * n;
+    if ((e = launch_interleave(wr, wi, ldw, wi2, n, wrows, n, s)) != hipSuccess) return hip_fail(e, "interleave");
     FsArgs a = fs_args(*this);
-    a.wp = (const float2 *)wp.p;
+    a.wp = wi2;
     a.ldwp = ldw ? n : 0;
+    a.natural = fs_takes_natural(n2, n, lines);
+    a.wscale = scale;
+    if (!a.natural) {
+      if ((st = wp.alloc((size_t)wrows * n * 8))) return st;
+      if ((e = launch_fs_permute(wi2, a.ldwp, (float2 *)wp.p, n1, n2, wrows, scale, s)) != hipSuccess)
+        return hip_fail(e, "spectrum permutation");
+      a.wp = (const float2 *)wp.p;
+    }
     a.in_re = xr;
     a.in_im = xi;
     a.ld_in = ldx;
@@ -455,29 +452,42 @@ int LineFFT::fastconv_split(const float *xr, const float *xi, long ldx, const fl
     if ((e = launch_fs_col(+1, a, lines, s)) != hipSuccess) return hip_fail(e, "four-step column pass");
     return OVX_OK;
   }
-  if (kind == LDS || (kind == HIER && ldw != 0)) {
-    long ld = std::max(std::max(ldx, ldy), ldw);
-    if ((unsigned long)rc.rows_per_block * (unsigned long)ld * 8ul >= (1ul << 32))
+  if (rows_fastconv(ldw, lines) && (kind == LDS || ldw != 0 || row_strides_fit(ldx, ldw, ldy))) {
+    if (!row_strides_fit(ldx, ldw, ldy))
       return fail(OVX_ERR_UNSUPPORTED, "row stride too large for 32-bit buffer offsets");
-    hipError_t e = launch_row_fastconv_split(rc, xr, xi, ldx, w, ldw, yr, yi, ldy, lines, (const float2 *)tw.p,
-                                             scale, s);
+    const bool meet = lines_meet(wr, wrows, ldw, yr, lines, ldy, n) || lines_meet(wr, wrows, ldw, yi, lines, ldy, n) ||
+                      lines_meet(wi, wrows, ldw, yr, lines, ldy, n) || lines_meet(wi, wrows, ldw, yi, lines, ldy, n);
+    if (meet) { // copy the spectra out of the result's way
+      const size_t values = (size_t)wrows * n;
+      if ((st = wp.alloc(2 * values * 8))) return st;
+      float2 *both = (float2 *)wp.p;
+      float *re = (float *)(both + values), *im = re + values;
+      e = launch_interleave(wr, wi, ldw, both, n, wrows, n, s);
+      if (e == hipSuccess) e = launch_deinterleave(both, n, re, im, n, wrows, n, s);
+      if (e != hipSuccess) return hip_fail(e, "spectrum copy");
+      wr = re;
+      wi = im;
+      if (ldw) ldw = n;
+    }
+    e = launch_row_fastconv_split(rc, xr, xi, ldx, wr, wi, ldw, yr, yi, ldy, lines, (const float2 *)tw.p, scale, s);
     return e == hipSuccess ? OVX_OK : hip_fail(e, "fastconv launch");
   }
+  if (!offsets_fit(hier_rows_per_block(n), std::max(ldx, ldy)))
+    return fail(OVX_ERR_UNSUPPORTED, "row stride too large for 32-bit buffer offsets");
+  if ((st = wp.alloc((size_t)n * 8))) return st;
+  if ((e = launch_hier_permute_split(wr, wi, (float2 *)wp.p, n, scale, s)) != hipSuccess)
+    return hip_fail(e, "spectrum permutation");
   HierArgs a = hier_args(*this);
   a.xr = xr;
   a.xi = xi;
+  a.ldx = ldx;
   a.yr = yr;
   a.yi = yi;
-  return hier_fastconv(a, HIER_FASTCONV_SPLIT, ldx, w, ldy, lines, scale, s);
-}
-
-// Whether the spectra (one of n values, or one per line) and the result share
-// memory: a spectrum read beside or after the first writes has to be laid out
-// beforehand.
-static bool spectrum_meets_result(const float2 *w, long ldw, const float2 *y, long ldy, long lines, long n)
-{
-  const float2 *w1 = w + (ldw ? (lines - 1) * ldw : 0) + n, *y1 = y + (lines - 1) * ldy + n;
-  return w < y1 && y < w1;
+  a.ldy = ldy;
+  a.rows = lines;
+  a.w = (const float2 *)wp.p;
+  e = launch_hier(HIER_FASTCONV_SPLIT, n, a, s);
+  return e == hipSuccess ? OVX_OK : hip_fail(e, "fastconv launch");
 }
 
 int LineFFT::fastconv(const float2 *x, long ldx, const float2 *w, long ldw, float2 *y, long ldy, long lines,
@@ -485,16 +495,34 @@ int LineFFT::fastconv(const float2 *x, long ldx, const float2 *w, long ldw, floa
 {
   if (lines <= 0) return OVX_OK;
   if (!tables_ready()) return fail(OVX_ERR_STATE, "fastconv plan has no twiddle tables");
-  if (kind == HIER && ldw == 0) {
+  const bool meet = lines_meet(w, ldw ? lines : 1, ldw, (const float2 *)y, lines, ldy, n);
+  if (kind == HIER && ldw == 0 && (meet || !rows_fastconv(ldw, lines) || !row_strides_fit(ldx, ldw, ldy))) {
     HierArgs a = hier_args(*this);
     a.x = x;
     a.y = y;
     return hier_fastconv(a, HIER_FASTCONV, ldx, w, ldy, lines, scale, s, ext);
   }
-  if (kind == LDS || (kind == HIER && ldw != 0)) {
-    long ld = std::max(std::max(ldx, ldy), ldw);
-    if ((unsigned long)rc.rows_per_block * (unsigned long)ld * 8ul >= (1ul << 32))
+  if (kind == LDS || kind == HIER) {
+    if (!row_strides_fit(ldx, ldw, ldy))
       return fail(OVX_ERR_UNSUPPORTED, "row stride too large for 32-bit buffer offsets");
+    if (ext && ext->wp_elems < fastconv_scratch_wp(lines, ldw))
+      return fail(OVX_ERR_UNSUPPORTED, "lent scratch too small for the spectrum");
+    // a line's spectrum is read before its result is written; other overlaps
+    // have the spectra copied out of the result's way
+    const size_t values = (size_t)(ldw ? lines : 1) * n;
+    if (meet && !(ldw != 0 && w == y && ldw == ldy) && (!ext || ext->wp_elems >= values)) {
+      float2 *copy = ext ? ext->wp : nullptr;
+      if (!ext) {
+        int st = wp.alloc(values * 8);
+        if (st) return st;
+        copy = (float2 *)wp.p;
+      }
+      hipError_t e = hipMemcpy2DAsync(copy, (size_t)n * 8, w, (size_t)(ldw ? ldw : n) * 8, (size_t)n * 8,
+                                      values / (size_t)n, hipMemcpyDeviceToDevice, s);
+      if (e != hipSuccess) return hip_fail(e, "spectrum copy");
+      w = copy;
+      if (ldw) ldw = n;
+    }
     hipError_t e = launch_row_fastconv(rc, x, ldx, w, ldw, y, ldy, lines, (const float2 *)tw.p, scale, s);
     if (e != hipSuccess) return hip_fail(e, "fastconv launch");
     return OVX_OK;
@@ -505,7 +533,7 @@ int LineFFT::fastconv(const float2 *x, long ldx, const float2 *w, long ldw, floa
     float2 *wpp;
     if (ext && ext->wp_elems < (size_t)wrows * n)
       return fail(OVX_ERR_UNSUPPORTED, "lent scratch too small for the spectrum");
-    if (fs_takes_natural(n2, n, lines) && !spectrum_meets_result(w, ldw, y, ldy, lines, n))
+    if (fs_takes_natural(n2, n, lines) && !meet)
       return fs_fastconv(x, ldx, w, ldw, y, ldy, lines, s, &scale);
     if (ext) {
       wpp = ext->wp;
@@ -1243,18 +1271,8 @@ extern "C" int ovx_fastconv_split_exec(ovx_plan p, const void *x_re, const void 
   hipStream_t s = (hipStream_t)stream;
   const long wlines = ldw ? rows : 1;
   auto run = [&](SplitIn x, SplitIn w, SplitOut y) -> int {
-    if (p->line.native_split() && ldw == 0)
-      return p->line.fastconv_split_vec(x.re, x.im, ldx, w.re, w.im, y.re, y.im, ldy, rows, p->scale, s);
-    if (p->line.native_split()) {
-      // the kernel reads and writes the split arrays itself; only the
-      // coefficient matrix is interleaved first
-      int r = p->split_ws.alloc((size_t)wlines * n * 8);
-      if (r) return r;
-      float2 *ww = (float2 *)p->split_ws.p;
-      hipError_t e = launch_interleave(w.re, w.im, ldw, ww, n, wlines, n, s);
-      if (e != hipSuccess) return hip_fail(e, "interleave");
-      return p->line.fastconv_split(x.re, x.im, ldx, ww, ldw ? n : 0, y.re, y.im, ldy, rows, p->scale, s);
-    }
+    if (p->line.native_split())
+      return p->line.fastconv_split(x.re, x.im, ldx, w.re, w.im, ldw, y.re, y.im, ldy, rows, p->scale, s);
     int r = p->split_ws.alloc((size_t)(rows + wlines) * n * 8);
     if (r) return r;
     float2 *wx = (float2 *)p->split_ws.p, *ww = wx + (size_t)rows * n;

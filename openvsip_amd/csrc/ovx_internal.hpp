@@ -50,7 +50,7 @@ hipError_t launch_row_fft_split(const RowConfig &cfg, int dir, const float *in_r
                                 float *out_re, float *out_im, long ld_out, long rows, const float2 *tw, float scale,
                                 hipStream_t s);
 hipError_t launch_row_fastconv_split(const RowConfig &cfg, const float *xr, const float *xi, long ldx,
-                                     const float2 *w, long ldw, float *yr, float *yi, long ldy, long rows,
+                                     const float *wr, const float *wi, long ldw, float *yr, float *yi, long ldy, long rows,
                                      const float2 *tw, float scale, hipStream_t s);
 
 // Real <-> complex rows in one pass: `lines` real lines of 2 * cfg.n values,

@@ -67,19 +67,18 @@ struct LineFFT {
                    float2 *ws, hipStream_t s) const;
   int fastconv(const float2 *x, long ldx, const float2 *w, long ldw, float2 *y, long ldy, long lines, float scale,
                hipStream_t s, const ExtScratch *ext = nullptr) const;
+  bool rows_fastconv(long ldw, long lines) const;
+  bool row_strides_fit(long ldx, long ldw, long ldy) const;
   // permuted-spectrum elements fastconv() needs for `lines` lines and
   // spectrum row stride ldw (0 when it permutes nothing)
   size_t fastconv_scratch_wp(long lines, long ldw) const;
-  // fastconv with X and Y in split storage (line strides in floats) and an
-  // interleaved spectrum, and the plain transform on split lines, read and
-  // written by the kernels themselves (native_split(): every transform path)
+  // fastconv and plain transform in split storage (line strides in floats),
+  // read and written by the kernels themselves (native_split(): every path)
   bool native_split() const { return kind == HIER || kind == LDS || kind == FOURSTEP; }
-  int fastconv_split(const float *xr, const float *xi, long ldx, const float2 *w, long ldw, float *yr, float *yi,
-                     long ldy, long lines, float scale, hipStream_t s) const;
+  int fastconv_split(const float *xr, const float *xi, long ldx, const float *wr, const float *wi, long ldw, float *yr,
+                     float *yi, long ldy, long lines, float scale, hipStream_t s) const;
   int transform_split(int dir, const float *in_re, const float *in_im, long ld_in, float *out_re, float *out_im,
                       long ld_out, long lines, float scale, hipStream_t s) const;
-  int fastconv_split_vec(const float *xr, const float *xi, long ldx, const float *wr, const float *wi, float *yr,
-                         float *yi, long ldy, long lines, float scale, hipStream_t s) const;
   int hier_fastconv(HierArgs a, int launch_kind, long ldx, const float2 *w, long ldy, long lines, float scale,
                     hipStream_t s, const ExtScratch *ext = nullptr) const;
   int fs_fastconv(const float2 *x, long ldx, const float2 *wprep, long ldwp, float2 *y, long ldy, long lines,

@@ -16,20 +16,19 @@ constexpr bool row_holds_twiddles(int N, int P) { return P == 16 && N >= 1024 &&
 // Rows row0 + lrow of the job, thread t of the row's T = N/P threads, LDS row
 // region `lds` (Engine LROW elements).  Every thread of the workgroup calls
 // it; rows at or beyond `rows` compute on zeros and store nothing.  ix / iy
-// access the thread's input and output line (interleaved IoC or split IoS),
-// element e of the thread at ld(e) / st(v, e).
-template <int N, int P, typename IX, typename IY, typename LP>
-__device__ __forceinline__ void row_fastconv_io(const IX &ix, const IY &iy, const float2 *__restrict__ w, long ldw,
-                                                long rows, const float2 *__restrict__ tw, float scale, long row0,
-                                                int lrow, int t, LP lds)
+// access the thread's input and output line and iw its spectrum (interleaved IoC
+// or split IoS), element e of the thread at ld(e) / st(v, e).  The spectrum of a
+// row at or beyond `rows` is some row's below.
+template <int N, int P, typename IX, typename IW, typename IY, typename LP>
+__device__ __forceinline__ void row_fastconv_io(const IX &ix, const IW &iw, const IY &iy, long rows,
+                                                const float2 *__restrict__ tw, float scale, long row0, int lrow, int t,
+                                                LP lds)
 {
   using E = Engine<N, P, line_in_wave(N / P)>;
   constexpr int T = E::T;
   const long row = row0 + lrow;
   const bool valid = row < rows;
-  const rsrc_t rw = make_rsrc(w + row0 * ldw, 0xffffffffu);
   const rsrc_t rtw = make_rsrc(tw, (uint32_t)(E::plan.twtotal + 1) * 8u);
-  const uint32_t vw = (uint32_t)(lrow * ldw + t) * 8u;
 
   float2 v[P];
   if (valid) {
@@ -49,10 +48,7 @@ __device__ __forceinline__ void row_fastconv_io(const IX &ix, const IY &iy, cons
   }
   // multiply by the replica spectrum; slot q holds frequency t + T q
 #pragma unroll
-  for (int q = 0; q < P; ++q) {
-    float2 ww = bload(rw, vw, (uint32_t)(T * q) * 8u);
-    v[q] = cmul(v[q], ww);
-  }
+  for (int q = 0; q < P; ++q) v[q] = cmul(v[q], iw.ld((uint32_t)(T * q)));
   if (scale != 1.0f) {
 #pragma unroll
     for (int q = 0; q < P; ++q) v[q] = cscale(v[q], scale);
@@ -72,9 +68,11 @@ __device__ __forceinline__ void row_fastconv_body(const float2 *__restrict__ x, 
                                                   const float2 *__restrict__ tw, float scale, long row0, int lrow,
                                                   int t, LP lds)
 {
+  const int wrow = row0 + lrow < rows ? lrow : 0;
   row_fastconv_io<N, P>(IoC{make_rsrc(x + row0 * ldx, 0xffffffffu), (uint32_t)(lrow * ldx + t) * 8u},
-                        IoC{make_rsrc(y + row0 * ldy, 0xffffffffu), (uint32_t)(lrow * ldy + t) * 8u}, w, ldw,
-                        rows, tw, scale, row0, lrow, t, lds);
+                        IoC{make_rsrc(w + row0 * ldw, 0xffffffffu), (uint32_t)(wrow * ldw + t) * 8u},
+                        IoC{make_rsrc(y + row0 * ldy, 0xffffffffu), (uint32_t)(lrow * ldy + t) * 8u}, rows, tw, scale,
+                        row0, lrow, t, lds);
 }
 
 // Forward (DIR = -1) or inverse (+1) transform of rows row0 + lrow, times

@@ -32,8 +32,8 @@ __global__ __launch_bounds__((RowCfg<N, P>::NT)) void k_row_fastconv(const float
   row_fastconv_body<N, P>(x, ldx, w, ldw, y, ldy, rows, tw, scale, r.row0, r.lrow, r.t, r.lds);
 }
 
-// Split-storage forms: real and imaginary parts of the lines in two float
-// arrays with the same strides (the spectrum stays interleaved).
+// Split-storage forms: real and imaginary parts of the lines, and of a
+// fastconv's spectra, in two float arrays with the same strides.
 template <int N, int P, int DIR>
 __global__ __launch_bounds__((RowCfg<N, P>::NT)) void k_row_fft_split(const float *__restrict__ in_re,
                                                                      const float *__restrict__ in_im, long ld_in,
@@ -53,16 +53,20 @@ __global__ __launch_bounds__((RowCfg<N, P>::NT)) void k_row_fft_split(const floa
 
 template <int N, int P>
 __global__ __launch_bounds__((RowCfg<N, P>::NT)) void k_row_fastconv_split(
-    const float *__restrict__ xr, const float *__restrict__ xi, long ldx, const float2 *__restrict__ w, long ldw,
-    float *__restrict__ yr, float *__restrict__ yi, long ldy, long rows, const float2 *__restrict__ tw, float scale)
+    const float *__restrict__ xr, const float *__restrict__ xi, long ldx, const float *__restrict__ wr,
+    const float *__restrict__ wi, long ldw, float *__restrict__ yr, float *__restrict__ yi, long ldy, long rows,
+    const float2 *__restrict__ tw, float scale)
 {
   const RowPlace<N, P> r;
+  const int wrow = r.row0 + r.lrow < rows ? r.lrow : 0;
   row_fastconv_io<N, P>(
       IoS{make_rsrc(xr + r.row0 * ldx, 0xffffffffu), make_rsrc(xi + r.row0 * ldx, 0xffffffffu),
           (uint32_t)(r.lrow * ldx + r.t) * 4u},
+      IoS{make_rsrc(wr + r.row0 * ldw, 0xffffffffu), make_rsrc(wi + r.row0 * ldw, 0xffffffffu),
+          (uint32_t)(wrow * ldw + r.t) * 4u},
       IoS{make_rsrc(yr + r.row0 * ldy, 0xffffffffu), make_rsrc(yi + r.row0 * ldy, 0xffffffffu),
           (uint32_t)(r.lrow * ldy + r.t) * 4u},
-      w, ldw, rows, tw, scale, r.row0, r.lrow, r.t, r.lds);
+      rows, tw, scale, r.row0, r.lrow, r.t, r.lds);
 }
 
 // ---------------------------------------------------------------- twiddles
@@ -184,12 +188,13 @@ static hipError_t do_fft_split(int dir, const float *ir, const float *ii, long l
 }
 
 template <int N, int P>
-static hipError_t do_fastconv_split(const float *xr, const float *xi, long ldx, const float2 *w, long ldw, float *yr,
-                                    float *yi, long ldy, long rows, const float2 *tw, float scale, hipStream_t s)
+static hipError_t do_fastconv_split(const float *xr, const float *xi, long ldx, const float *wr, const float *wi,
+                                    long ldw, float *yr, float *yi, long ldy, long rows, const float2 *tw, float scale,
+                                    hipStream_t s)
 {
   const RowLaunch<N, P> l(rows);
-  hipLaunchKernelGGL((k_row_fastconv_split<N, P>), l.grid, l.block, l.lds, s, xr, xi, ldx, w, ldw, yr, yi, ldy, rows,
-                     tw, scale);
+  hipLaunchKernelGGL((k_row_fastconv_split<N, P>), l.grid, l.block, l.lds, s, xr, xi, ldx, wr, wi, ldw, yr, yi, ldy,
+                     rows, tw, scale);
   return hipGetLastError();
 }
 
@@ -201,7 +206,7 @@ struct Entry {
                       hipStream_t);
   hipError_t (*fft_split)(int, const float *, const float *, long, float *, float *, long, long, const float2 *,
                           float, hipStream_t);
-  hipError_t (*fconv_split)(const float *, const float *, long, const float2 *, long, float *, float *, long, long,
+  hipError_t (*fconv_split)(const float *, const float *, long, const float *, const float *, long, float *, float *, long, long,
                             const float2 *, float, hipStream_t);
 };
 
@@ -295,13 +300,13 @@ hipError_t launch_row_fft_split(const RowConfig &cfg, int dir, const float *in_r
 }
 
 hipError_t launch_row_fastconv_split(const RowConfig &cfg, const float *xr, const float *xi, long ldx,
-                                     const float2 *w, long ldw, float *yr, float *yi, long ldy, long rows,
+                                     const float *wr, const float *wi, long ldw, float *yr, float *yi, long ldy, long rows,
                                      const float2 *tw, float scale, hipStream_t s)
 {
   const Entry *e = find_entry(cfg.n, cfg.variant);
   if (!e) return hipErrorInvalidValue;
   if (rows <= 0) return hipSuccess;
-  return e->fconv_split(xr, xi, ldx, w, ldw, yr, yi, ldy, rows, tw, scale, s);
+  return e->fconv_split(xr, xi, ldx, wr, wi, ldw, yr, yi, ldy, rows, tw, scale, s);
 }
 
 } // namespace ovx

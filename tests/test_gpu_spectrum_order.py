@@ -64,3 +64,34 @@ def test_result_over_the_spectrum(ovx, n, rows):
     fc(x, over[0], out=over)
     for r in range(rows):
         assert rel(over[r].cpu().numpy(), vec[r]) < REL_L2
+
+
+@pytest.mark.parametrize("n,rows", [(64, 5), (1024, 3), (2048, 9), (4096, 70), (8192, 9), (8192, 257), (16384, 5), (32768, 3),
+                                    (131072, 40)])
+@pytest.mark.parametrize("matrix", [False, True])
+def test_split_spectra(ovx, n, rows, matrix):
+    """Split storage, spectra included, equals interleaved storage bit for bit, and
+    the result may take the spectra's place."""
+    import ctypes
+    import torch
+    from openvsip_amd import _lib
+    gen = torch.Generator(device="cuda").manual_seed(n + rows + matrix)
+    x = torch.randn(rows, n, dtype=torch.complex64, device="cuda", generator=gen)
+    w = torch.randn(rows, n, dtype=torch.complex64, device="cuda", generator=gen)
+    fc = ovx.Fastconv(rows, n)
+    want = fc(x, w if matrix else w[0].clone())
+
+    def ptr(t):
+        return ctypes.c_void_p(t.data_ptr())
+
+    xr, xi, wr, wi = (t.contiguous() for t in (x.real, x.imag, w.real, w.imag))
+    yr, yi = torch.empty_like(xr), torch.empty_like(xi)
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    for outr, outi in ((yr, yi), (wr, wi)):
+        assert _lib.lib().ovx_fastconv_split_exec(fc._h, ptr(xr), ptr(xi), n, ptr(wr), ptr(wi), n if matrix else 0,
+                                                  ptr(outr), ptr(outi), n, rows, stream) == 0
+        if outr is yr or n not in (8192, 16384):  # those take another kernel beside an overlapping vector
+            assert torch.equal(torch.complex(outr, outi), want)
+        else:
+            got = torch.complex(outr, outi).cpu().numpy()
+            assert rel(got, want.cpu().numpy()) < REL_L2
