@@ -226,7 +226,7 @@ bool offsets_fit(long rows_per_block, long ld)
 }
 
 int LineFFT::transform(int dir, const float2 *in, long ld_in, float2 *out, long ld_out, long lines, float scale,
-                       hipStream_t s) const
+                       hipStream_t s, bool reread) const
 {
   if (lines <= 0) return OVX_OK;
   if (!tables_ready()) return fail(OVX_ERR_STATE, "transform plan has no twiddle tables");
@@ -254,13 +254,13 @@ int LineFFT::transform(int dir, const float2 *in, long ld_in, float2 *out, long 
   if (kind == FOURSTEP) {
     int st = work.alloc((size_t)lines * n * 8);
     if (st) return st;
-    return transform_ws(dir, in, ld_in, out, ld_out, lines, scale, (float2 *)work.p, s);
+    return transform_ws(dir, in, ld_in, out, ld_out, lines, scale, (float2 *)work.p, s, reread);
   }
   return fail(OVX_ERR_UNSUPPORTED, "no transform path");
 }
 
 int LineFFT::transform_ws(int dir, const float2 *in, long ld_in, float2 *out, long ld_out, long lines, float scale,
-                          float2 *ws, hipStream_t s) const
+                          float2 *ws, hipStream_t s, bool reread) const
 {
   if (kind != FOURSTEP) return transform(dir, in, ld_in, out, ld_out, lines, scale, s);
   if (lines <= 0) return OVX_OK;
@@ -279,6 +279,7 @@ int LineFFT::transform_ws(int dir, const float2 *in, long ld_in, float2 *out, lo
     a.out = out;
     a.ld_out = ld_out;
     a.scale = scale;
+    a.reread = reread;
     e = launch_fs_row(dir, a, lines, s);
     if (e != hipSuccess) return hip_fail(e, "four-step row pass");
     return OVX_OK;
@@ -976,7 +977,7 @@ static int real_run(ovx_plan p, const RealLines &g, const void *din, void *dout,
   if (p->line.kind == LineFFT::LDS)
     return g.fwd ? real_fused(p, g, din, dout, nullptr, nullptr, s) : real_fused(p, g, dout, din, nullptr, nullptr, s);
   if (g.fwd) {
-    int r = p->line.transform(-1, (const float2 *)din, g.ldz, (float2 *)dout, ldc, g.lines, 1.0f, s);
+    int r = p->line.transform(-1, (const float2 *)din, g.ldz, (float2 *)dout, ldc, g.lines, 1.0f, s, true);
     if (r) return r;
     hipError_t e = launch_r2c_post((float2 *)dout, ldc, g.lines, g.h, (const float2 *)p->wtab.p, p->scale, s);
     return e == hipSuccess ? OVX_OK : hip_fail(e, "r2c pass");
@@ -1331,7 +1332,7 @@ extern "C" int ovx_fftm_r2c_split(ovx_plan p, const void *in, long in_s0, long i
     int r = p->split_ws.alloc((size_t)g.lines * hc * 8);
     if (r) return r;
     float2 *ws = (float2 *)p->split_ws.p;
-    if ((r = p->line.transform(-1, (const float2 *)din, g.ldz, ws, hc, g.lines, 1.0f, s))) return r;
+    if ((r = p->line.transform(-1, (const float2 *)din, g.ldz, ws, hc, g.lines, 1.0f, s, true))) return r;
     hipError_t e = launch_r2c_post_split(ws, hc, o.re, o.im, g.ldc, g.lines, g.h, (const float2 *)p->wtab.p,
                                          p->scale, s);
     return e == hipSuccess ? OVX_OK : hip_fail(e, "r2c pass");

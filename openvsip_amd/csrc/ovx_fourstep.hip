@@ -23,40 +23,24 @@
 
 namespace ovx {
 
-// Row and column group of workgroup w: the groups of a row on one XCD
-// (workgroups go to the eight XCDs in turn), so that its accesses cover whole
-// matrix rows, not every eighth 128-byte run of each, which at a row of
-// 256 columns left an XCD two of its L2's sixteen channels.  256 x 256 lines,
-// 256 rows: 58 to 52 us; 512 x 512: 62 to 58.
-__device__ __forceinline__ void fs_place(unsigned w, unsigned groups, unsigned rows, long &row, long &group)
-{
-  const unsigned whole = rows & ~7u;
-  if (w < whole * groups) {
-    row = (w / 8 / groups) * 8 + w % 8;
-    group = (w / 8) % groups;
-  } else {
-    const unsigned r = w - whole * groups;
-    row = whole + r / groups;
-    group = r % groups;
-  }
-}
-
 template <int L, int P, int C, int DIR, bool SIN, bool SOUT, bool STREAM>
 __global__ __launch_bounds__(C *(L / P)) void k_fs_col(FsArgs a, unsigned groups, unsigned rows)
 {
   __shared__ float2 lds_all[C * FsLds<L>::LROW];
   long row, group;
   fs_place(blockIdx.x, groups, rows, row, group);
+  if (C == 8 && row >= (rows & ~7u)) group = fs_neighbours(group);
   fs_col_body<L, P, C, DIR, SIN, SOUT, STREAM, STREAM && (DIR > 0)>(a, row, group, threadIdx.x, lds_all);
 }
 
-template <int L, int P, int C, int DIR, bool SOUT>
+template <int L, int P, int C, int DIR, bool SOUT, bool REREAD>
 __global__ __launch_bounds__(C *(L / P)) void k_fs_row(FsArgs a, unsigned groups, unsigned rows)
 {
   __shared__ float2 lds_all[C * FsLds<L>::LROW];
   long row = blockIdx.x / groups, group = blockIdx.x % groups;
   if (a.placed) fs_place(blockIdx.x, groups, rows, row, group);
-  fs_row_body<L, P, C, DIR, SOUT>(a, row, group, threadIdx.x, lds_all);
+  if (C == 8 && !(a.placed && row < (rows & ~7u))) group = fs_neighbours(group);
+  fs_row_body<L, P, C, DIR, SOUT, REREAD>(a, row, group, threadIdx.x, lds_all);
 }
 
 // 256 threads: fewer lines per workgroup leave it sooner (C = 16 / 4 at 512:
@@ -153,13 +137,13 @@ static hipError_t col_launch(const FsArgs &a, long rows, hipStream_t s)
   return col_launch_c<L, DIR, C, false, false, false>(a, rows, s);
 }
 
-template <int L, int DIR, int C, bool SPLIT>
+template <int L, int DIR, int C, bool SPLIT, bool REREAD = false>
 static hipError_t row_launch_c(FsArgs a, long rows, hipStream_t s)
 {
   constexpr int P = FsCfg<L>::P, CL = C < FsSplitCfg<L>::C ? C : FsSplitCfg<L>::C;
   const unsigned groups = (unsigned)(a.n1 / CL);
   a.placed = fs_stays_in_l2(a.nbig, rows);
-  hipLaunchKernelGGL((k_fs_row<L, P, CL, DIR, SPLIT>), dim3(groups * (unsigned)rows), dim3(CL * (L / P)), 0, s, a,
+  hipLaunchKernelGGL((k_fs_row<L, P, CL, DIR, SPLIT, REREAD>), dim3(groups * (unsigned)rows), dim3(CL * (L / P)), 0, s, a,
                      groups, (unsigned)rows);
   return hipGetLastError();
 }
@@ -178,7 +162,13 @@ static hipError_t row_launch(const FsArgs &a, long rows, hipStream_t s)
   if (a.out_re)
     return rows * a.n1 < 128 * 32 ? row_launch_c<L, DIR, 8, true>(a, rows, s)
                                   : row_launch_c<L, DIR, 32, true>(a, rows, s);
-  return rows * a.nbig * 8 <= (64l << 20) ? row_launch_c<L, DIR, 8, false>(a, rows, s)
+  const long bytes = rows * a.nbig * 8;
+  if constexpr (DIR < 0) {
+    if (a.reread)
+      return bytes <= (64l << 20) ? row_launch_c<L, DIR, 8, false, true>(a, rows, s)
+                                  : row_launch_c<L, DIR, FsCfg<L>::C, false, true>(a, rows, s);
+  }
+  return bytes <= (64l << 20) ? row_launch_c<L, DIR, 8, false>(a, rows, s)
                                          : row_launch_c<L, DIR, FsCfg<L>::C, false>(a, rows, s);
 }
 

@@ -22,6 +22,30 @@ __device__ __forceinline__ float2 big_twiddle(const float2 *__restrict__ tlo, co
   return cmul(hi, lo);
 }
 
+// Row and column group of workgroup w: the groups of a row on one XCD
+// (workgroups go to the eight XCDs in turn), so that its accesses cover whole
+// matrix rows, not every eighth 128-byte run of each, which at a row of
+// 256 columns left an XCD two of its L2's sixteen channels.  256 x 256 lines,
+// 256 rows: 58 to 52 us; 512 x 512: 62 to 58.
+__device__ __forceinline__ void fs_place(unsigned w, unsigned groups, unsigned rows, long &row, long &group)
+{
+  const unsigned whole = rows & ~7u;
+  if (w < whole * groups) {
+    row = (w / 8 / groups) * 8 + w % 8;
+    group = (w / 8) % groups;
+  } else {
+    const unsigned r = w - whole * groups;
+    row = whole + r / groups;
+    group = r % groups;
+  }
+}
+
+// Order of a row's groups of 8 (a multiple of 16 of them) dealt to the XCDs in
+// turn: the two that share 128-byte lines get the same one, or each line is put
+// together from two L2s.  Inverse transform in place, in turn / paired, us: 6 x
+// 65536 9.6 / 8.3, 6 x 131072 14.5 / 12.1, 4 x 262144 18.9 / 15.8.
+__device__ __forceinline__ long fs_neighbours(long g) { return (g & ~15l) | (g & 7) << 1 | (g >> 3 & 1); }
+
 // The passes' global reads and writes: one row's buffer, element offsets of at
 // most N values.  Interleaved lines (a.in, a.out) or, when SPLIT, separate real
 // and imaginary arrays (a.in_re / a.in_im, a.out_re / a.out_im).  NT:
@@ -103,8 +127,11 @@ __device__ __forceinline__ void fs_line_twiddles(const FsArgs &a, long k1, int t
 // [group*C, group*C + C) of one row.
 // The result is written once, non-temporally where a run is 64 bytes or more:
 // 512 x 512 lines, 24 rows, both passes 42 to 36 us, 64 rows 95 to 88; 256 x
-// 256, 256 rows, 84 to 80; runs of 32 bytes (split, 2048 lines) 57 to 75.
-template <int L, int P, int C, int DIR, bool SOUT = false, typename LP>
+// 256, 256 rows, 84 to 80; runs of 32 bytes (split, 2048 lines) 57 to 75.  REREAD:
+// a kernel of the same call reads it again (a real transform's recombination), so
+// it is stored the ordinary way: 63 x 65536 real values forward 30.4 us
+// non-temporally, 25.3 so, 256 113 and 87.
+template <int L, int P, int C, int DIR, bool SOUT = false, bool REREAD = false, typename LP>
 __device__ __forceinline__ void fs_row_body(const FsArgs &a, long row, long group, int tid, LP lds_all)
 {
   // a line's L/P threads are consecutive; when they fit one wavefront its
@@ -138,7 +165,7 @@ __device__ __forceinline__ void fs_row_body(const FsArgs &a, long row, long grou
   const int c2 = tid % C;
   const int t2 = tid / C;
   LP lsrc = lds_all + c2 * LROW;
-  const auto out = fs_out<SOUT, (C * (SOUT ? 4 : 8) >= 64)>(a, row, (uint32_t)t2 * N1 + (uint32_t)(group * C + c2));
+  const auto out = fs_out<SOUT, !REREAD && (C * (SOUT ? 4 : 8) >= 64)>(a, row, (uint32_t)t2 * N1 + (uint32_t)(group * C + c2));
 #pragma unroll
   for (int q = 0; q < P; ++q) out.st(lds_ld(lsrc, t2 + T * q), (uint32_t)(T * q) * N1);
 }
