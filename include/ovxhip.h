@@ -106,8 +106,8 @@ int ovx_length_variants(long n);
    with FFTW_MEASURE, src/ovxx/fftw/fft.cpp:44-52): time every variant of
    length n on a rows x n fastconv, record the fastest under (n, rows rounded
    up to a power of two) in the cache file $OVX_TUNE_CACHE (default
-   ~/.cache/ovxhip/tune.txt).  Plans created without an explicit variant use
-   the cached choice. */
+   ~/.cache/ovxhip/tune.txt).  Fastconv plans created without an explicit
+   variant use the cached choice (transform plans do not). */
 int ovx_autotune_fastconv(long n, long rows, int *best_variant, double *best_us);
 /* Cached variant for (n, rows), or -1. */
 int ovx_tuned_variant(long n, long rows);
@@ -328,7 +328,7 @@ int ovx_storage_info(ovx_storage storage, unsigned *valid, uint64_t *h2d_bytes,
    persistent-kernel launches over (instance, rows) tile queues (one of
    1024-thread workgroups for rows of 12288 and 16384 points, one of
    512-thread workgroups for shorter rows); the rows of jobs on the
-   four-step path run in chunks of about 128 MiB, each chunk one launch per
+   four-step path run in chunks of about 192 MB, each chunk one launch per
    pass and line length (one line group per workgroup), so that a chunk
    stays in the Infinity Cache between its passes.  The launches are
    captured once into a hipGraph at commit and replayed by every exec.  Each job's result is bitwise the same as

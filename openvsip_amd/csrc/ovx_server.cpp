@@ -369,8 +369,7 @@ void Server::scheduler()
       st = launch_plain(*s, *batch[0]);
     } else if ((int)batch.size() <= kDirectMax) {
       // a small batch (light load): the requests' standalone launches on the
-      // slot's stream cost less than replaying the slot graph (a persistent
-      // launch over every CU plus one launch per four-step queue); same
+      // slot's stream cost less than the tables and the batch's launches; same
       // device bodies, same results
       for (Req *r : batch)
         if ((st = launch_plain(*s, *r))) break;
