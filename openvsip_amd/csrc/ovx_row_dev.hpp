@@ -61,7 +61,7 @@ __device__ __forceinline__ void row_fastconv_io(const IX &ix, const IW &iw, cons
   }
 }
 
-template <int N, int P, typename LP>
+template <int N, int P, bool NTL = false, typename LP>
 __device__ __forceinline__ void row_fastconv_body(const float2 *__restrict__ x, long ldx,
                                                   const float2 *__restrict__ w, long ldw,
                                                   float2 *__restrict__ y, long ldy, long rows,
@@ -69,7 +69,7 @@ __device__ __forceinline__ void row_fastconv_body(const float2 *__restrict__ x, 
                                                   int t, LP lds)
 {
   const int wrow = row0 + lrow < rows ? lrow : 0;
-  row_fastconv_io<N, P>(IoC{make_rsrc(x + row0 * ldx, 0xffffffffu), (uint32_t)(lrow * ldx + t) * 8u},
+  row_fastconv_io<N, P>(IoCx<NTL>{make_rsrc(x + row0 * ldx, 0xffffffffu), (uint32_t)(lrow * ldx + t) * 8u},
                         IoC{make_rsrc(w + row0 * ldw, 0xffffffffu), (uint32_t)(wrow * ldw + t) * 8u},
                         IoC{make_rsrc(y + row0 * ldy, 0xffffffffu), (uint32_t)(lrow * ldy + t) * 8u}, rows, tw, scale,
                         row0, lrow, t, lds);
