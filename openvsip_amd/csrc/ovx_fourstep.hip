@@ -156,6 +156,9 @@ static hipError_t row_launch_c(FsArgs a, long rows, hipStream_t s)
 // 1024 x 1024, 8 rows 66.3 / 60.7.  Split storage, whose runs are half as long:
 // 32 lines, 8 where those would leave half the CUs without one (32 / 8, 256 x
 // 256, 1 row 10.9 / 8.5, 9 rows 11.8 / 10.3, 24 rows 14.5 / 15.2).
+// A result that is read again (REREAD) is better in whole lines: 16 from 320
+// workgroups on; real forward, 8 / 16, 63 x 65536 25.4 / 25.0, 256 81.4 / 78.3, 18 x
+// 131072 (288 workgroups) 19.2 / 20.2.
 template <int L, int DIR>
 static hipError_t row_launch(const FsArgs &a, long rows, hipStream_t s)
 {
@@ -165,8 +168,8 @@ static hipError_t row_launch(const FsArgs &a, long rows, hipStream_t s)
   const long bytes = rows * a.nbig * 8;
   if constexpr (DIR < 0) {
     if (a.reread)
-      return bytes <= (64l << 20) ? row_launch_c<L, DIR, 8, false, true>(a, rows, s)
-                                  : row_launch_c<L, DIR, FsCfg<L>::C, false, true>(a, rows, s);
+      return rows * a.n1 < 320 * 16 ? row_launch_c<L, DIR, 8, false, true>(a, rows, s)
+                                    : row_launch_c<L, DIR, FsCfg<L>::C, false, true>(a, rows, s);
   }
   return bytes <= (64l << 20) ? row_launch_c<L, DIR, 8, false>(a, rows, s)
                                          : row_launch_c<L, DIR, FsCfg<L>::C, false>(a, rows, s);
