@@ -16,6 +16,7 @@
 #include <algorithm>
 
 #include "../../include/ovxhip.h"
+#include "ovx_fs_dev.hpp"
 #include "ovx_plan.hpp"
 
 namespace ovx {
@@ -58,7 +59,17 @@ struct VmmulArgs {
   long outer, inner;
   int v_inner;
   float alpha;
+  unsigned groups; // placed: workgroups of a line, else 0
 };
+
+// Bytes of output up to which lines are placed: line o on XCD o mod 8, where the
+// row kernels (one line a workgroup, dealt to the XCDs in turn) and the four-step
+// passes leave and take lines.  Workgroups of a line in turn over the XCDs / placed,
+// us: 256 x 4097 complex values 5.2 / 4.7, in place 5.1 / 4.5, 256 x 16384 13.6 /
+// 11.7, 300 x 16384 15.0 / 13.3, 500 x 16384 in place 22.9 / 20.5; beyond, 64 x
+// 262144 59.9 / 64.2.  A filter's transform, product and inverse, 256 x 8192 real
+// values 19.8 / 18.9, 56 x 65536 55.0 / 51.5.
+constexpr long kPlacedBytes = 64l << 20;
 
 template <bool VC, bool MC>
 __global__ __launch_bounds__(256) void k_vmmul(VmmulArgs a)
@@ -69,13 +80,22 @@ __global__ __launch_bounds__(256) void k_vmmul(VmmulArgs a)
   const vt *v = static_cast<const vt *>(a.v);
   const mt *m = static_cast<const mt *>(a.m);
   ot *out = static_cast<ot *>(a.out);
+  auto one = [&](long o, long i) {
+    const vt vv = v[(a.v_inner ? i : o) * a.vs];
+    const mt mm = m[o * a.m_outer + i * a.m_inner];
+    if constexpr (VC || MC) out[o * a.o_outer + i * a.o_inner] = cmul(as_c(vv), as_c(mm), a.alpha);
+    else out[o * a.o_outer + i * a.o_inner] = cmul(vv, mm, a.alpha);
+  };
+  if (a.groups) {
+    long o, group;
+    fs_place(blockIdx.x, a.groups, (unsigned)a.outer, o, group);
+    const long i = group * blockDim.x + threadIdx.x;
+    if (i < a.inner) one(o, i);
+    return;
+  }
   for (long o = blockIdx.y; o < a.outer; o += gridDim.y) {
-    for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < a.inner; i += (long)gridDim.x * blockDim.x) {
-      vt vv = v[(a.v_inner ? i : o) * a.vs];
-      mt mm = m[o * a.m_outer + i * a.m_inner];
-      if constexpr (VC || MC) out[o * a.o_outer + i * a.o_inner] = cmul(as_c(vv), as_c(mm), a.alpha);
-      else out[o * a.o_outer + i * a.o_inner] = cmul(vv, mm, a.alpha);
-    }
+    for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < a.inner; i += (long)gridDim.x * blockDim.x)
+      one(o, i);
   }
 }
 
@@ -124,8 +144,12 @@ extern "C" int ovx_vmmul(int dim, int v_complex, const void *v, long v_stride, i
   long by = std::min<long>(a.outer, 65535);
   // enough workgroups to fill the chip when the lines are short
   dim3 grid((unsigned)bx, (unsigned)by);
+  const bool vc = v_complex != 0, mc = m_complex != 0;
+  if (a.outer >= 8 && a.outer <= 65535 && a.inner <= kPlacedBytes && a.outer * a.inner * (vc || mc ? 8 : 4) <= kPlacedBytes) {
+    a.groups = (unsigned)((a.inner + threads - 1) / threads);
+    grid = dim3(a.groups * (unsigned)a.outer);
+  }
   hipStream_t s = static_cast<hipStream_t>(stream);
-  bool vc = v_complex != 0, mc = m_complex != 0;
   if (vc && mc) k_vmmul<true, true><<<grid, threads, 0, s>>>(a);
   else if (vc) k_vmmul<true, false><<<grid, threads, 0, s>>>(a);
   else if (mc) k_vmmul<false, true><<<grid, threads, 0, s>>>(a);
