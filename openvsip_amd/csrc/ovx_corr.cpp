@@ -65,6 +65,24 @@ static int choose_L(const CorrState &c)
 // The reference's spectrum in every segment or once in a launch of its own.
 static bool ols_fuse_ref(const CorrState &c) { return !c.is_conv && segment_count(c, c.L) <= kOlsFew; }
 
+// Whether two runs of values share memory.
+static bool runs_meet(const float2 *a, long na, const float2 *b, long nb) { return a < b + nb && b < a + na; }
+
+// A single segment reads all of its samples before its first store, so a result
+// over the signal is right; several segments run at once and store over each
+// other's samples.  A signal that one segment of the greatest length could hold
+// is copied out of the result's way then.
+static bool ols_copies_meeting(const CorrState &c) { return c.N <= kMaxRowN && segment_count(c, c.L) > 1; }
+
+// The samples to read for a result at `out`: `in` itself, or its copy.
+static int ols_input(CorrState &c, const float2 *&in, const float2 *out, hipStream_t s)
+{
+  if (!ols_copies_meeting(c) || !runs_meet(in, c.N, out, c.P)) return OVX_OK;
+  hipError_t e = hipMemcpyAsync(c.in_stage.p, in, (size_t)c.N * 8, hipMemcpyDeviceToDevice, s);
+  in = (const float2 *)c.in_stage.p;
+  return e == hipSuccess ? OVX_OK : hip_fail(e, "signal copy");
+}
+
 static int ols_init(CorrState &c)
 {
   if (c.M - 1 >= kMaxRowN) return fail(OVX_ERR_UNSUPPORTED, "kernel length %ld too long for overlap-save", c.M);
@@ -76,7 +94,8 @@ static int ols_init(CorrState &c)
   if (st) return st;
   if (c.fftL.kind != LineFFT::LDS || c.fftL.rc.p != c.Lp || !c.fftL.tw.p)
     return fail(OVX_ERR_UNSUPPORTED, "no register-Stockham configuration for segment length %d", c.L);
-  return ols_fuse_ref(c) ? OVX_OK : c.H.alloc((size_t)c.L * 8);
+  if ((st = c.H.alloc((size_t)c.L * 8))) return st;
+  return ols_copies_meeting(c) ? c.in_stage.alloc((size_t)c.N * 8) : OVX_OK;
 }
 
 // H = FFT_L(h padded); h is a device pointer of M values
@@ -214,7 +233,10 @@ extern "C" int ovx_corr_exec(ovx_plan p, int bias, const void *ref, const void *
     din = (const float2 *)c.in_stage.p;
     dout = (float2 *)c.out_stage.p;
   }
-  const bool fuse = ols_fuse_ref(c);
+  if (!host && (st = ols_input(c, din, dout, s))) return st;
+  // a reference that the result is written over is read whole by a launch of
+  // its own first
+  const bool fuse = ols_fuse_ref(c) && !runs_meet(dref, c.M, dout, c.P);
   if (!fuse && (st = ols_spectrum(c, dref, 1, s))) return st;
   if ((st = ols_run(c, fuse ? dref : nullptr, din, dout, 1, bias == OVX_UNBIASED, s))) return st;
   if (host) {
@@ -302,6 +324,7 @@ extern "C" int ovx_conv_exec(ovx_plan p, const void *in, void *out, void *stream
     din = (const float2 *)c.in_stage.p;
     dout = (float2 *)c.out_stage.p;
   }
+  if (!host && (st = ols_input(c, din, dout, s))) return st;
   if ((st = ols_run(c, nullptr, din, dout, 0, 0, s))) return st;
   if (host) {
     hipError_t e = hipMemcpyAsync(out, c.out_stage.p, (size_t)c.P * 8, hipMemcpyDeviceToHost, s);

@@ -78,3 +78,34 @@ def test_convolution_segments_and_decimation(ovx, m, n, d):
         scale = np.linalg.norm(want) if want.size > 8 else np.sqrt(want.size) * np.sqrt(np.mean(np.abs(c) ** 2)) * 4
         assert np.linalg.norm(got[: want.size] - want) / scale < REL_L2, (support, m, n, d)
         assert np.all(got[want.size:] == 7.0)
+
+
+@pytest.mark.parametrize("support,m,n", [("same", 200, 800), ("min", 150, 1000), ("full", 300, 900), ("min", 1024, 9000),
+                                         ("same", 17, 300), ("same", 2000, 16384)])
+def test_result_over_the_operands(ovx, support, m, n):
+    """A result that is stored over the signal, and one over the reference: in
+    one segment and in several, whose stores meet each other's samples."""
+    import torch
+    rng = np.random.default_rng(m * 3 + n)
+    ref, x = cg(rng, m), cg(rng, n)
+    rd, xd = torch.from_numpy(ref).cuda(), torch.from_numpy(x).cuda()
+    shift = {"full": m - 1, "same": m // 2, "min": 0}[support]
+    corr = ovx.Correlation(support, m, n)
+    conv = ovx.Convolution(ref, "nonsym", support, n, 1)
+    p = corr.output_size
+    c = fftconvolve(ref[::-1].astype(np.complex128), x.conj().astype(np.complex128))[m - 1 - shift:][:p]
+    for operand, at in ((xd, 0), (rd, 0), (rd, p - m // 2)):
+        buf = torch.zeros(2 * (n + m), dtype=torch.complex64, device="cuda")
+        # the operand begins `at` values into the result
+        over = buf[at: at + operand.numel()]
+        over.copy_(operand)
+        out = buf[:p]
+        corr("biased", over if operand is rd else rd, over if operand is xd else xd, out=out)
+        assert rel(out.cpu().numpy(), c) < REL_L2, (support, m, n, at)
+    q = conv.output_size
+    c = fftconvolve(ref.astype(np.complex128), x.astype(np.complex128))
+    off = {"full": 0, "same": m // 2, "min": m - 1}[support]
+    buf = torch.zeros(2 * (n + m), dtype=torch.complex64, device="cuda")
+    buf[:n].copy_(xd)
+    conv(buf[:n], out=buf[:q])
+    assert rel(buf[:q].cpu().numpy(), c[off: off + q]) < REL_L2, (support, m, n)
