@@ -572,12 +572,12 @@ int LineFFT::fs_fastconv(const float2 *x, long ldx, const float2 *wprep, long ld
   a.ld_out = ldy;
   const size_t bytes = (size_t)lines * (size_t)n * sizeof(float2);
   hipError_t e;
-  a.stream = fs_streams_in(bytes);
+  a.stream = fs_streams_in(bytes) && fs_whole_lines(x, ldx, lines);
   if ((e = launch_fs_col(-1, a, lines, s)) != hipSuccess) return hip_fail(e, "four-step column pass");
   a.in = y;
   a.ld_in = ldy;
   if ((e = launch_fs_conv(a, lines, s)) != hipSuccess) return hip_fail(e, "four-step row pass");
-  a.stream = fs_streams_out(bytes);
+  a.stream = fs_streams_out(bytes) && fs_whole_lines(y, ldy, lines);
   if ((e = launch_fs_col(+1, a, lines, s)) != hipSuccess) return hip_fail(e, "four-step column pass");
   return OVX_OK;
 }

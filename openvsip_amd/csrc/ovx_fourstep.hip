@@ -158,7 +158,10 @@ static hipError_t row_launch_c(FsArgs a, long rows, hipStream_t s)
 // 256, 1 row 10.9 / 8.5, 9 rows 11.8 / 10.3, 24 rows 14.5 / 15.2).
 // A result that is read again (REREAD) is better in whole lines: 16 from 320
 // workgroups on; real forward, 8 / 16, 63 x 65536 25.4 / 25.0, 256 81.4 / 78.3, 18 x
-// 131072 (288 workgroups) 19.2 / 20.2.
+// 131072 (288 workgroups) 19.2 / 20.2.  Rows off the 128-byte lines
+// (fs_whole_lines) are stored the same way, 16 from 144 workgroups on; rows of n +
+// 33 values, 8 / 16, 5 x 262144 21.3 / 19.8, 6 20.9 / 22.0, 13 x 131072 19.3 / 18.0, 2 x
+// 262144 13.1 / 14.6.
 template <int L, int DIR>
 static hipError_t row_launch(const FsArgs &a, long rows, hipStream_t s)
 {
@@ -166,11 +169,10 @@ static hipError_t row_launch(const FsArgs &a, long rows, hipStream_t s)
     return rows * a.n1 < 128 * 32 ? row_launch_c<L, DIR, 8, true>(a, rows, s)
                                   : row_launch_c<L, DIR, 32, true>(a, rows, s);
   const long bytes = rows * a.nbig * 8;
-  if constexpr (DIR < 0) {
-    if (a.reread)
-      return rows * a.n1 < 320 * 16 ? row_launch_c<L, DIR, 8, false, true>(a, rows, s)
-                                    : row_launch_c<L, DIR, FsCfg<L>::C, false, true>(a, rows, s);
-  }
+  const bool whole = fs_whole_lines(a.out, a.ld_out, rows);
+  if (a.reread || !whole)
+    return rows * a.n1 < (whole ? 320 : 144) * 16 ? row_launch_c<L, DIR, 8, false, true>(a, rows, s)
+                                  : row_launch_c<L, DIR, FsCfg<L>::C, false, true>(a, rows, s);
   return bytes <= (64l << 20) ? row_launch_c<L, DIR, 8, false>(a, rows, s)
                                          : row_launch_c<L, DIR, FsCfg<L>::C, false>(a, rows, s);
 }

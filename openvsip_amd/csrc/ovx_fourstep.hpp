@@ -50,6 +50,17 @@ inline bool fs_stays_in_l2(long n, long rows)
   return n * 8 <= (1l << 20) && rows * n * 8 <= 8 * (4l << 20);
 }
 
+// Whether every row begins on a 128-byte line.  Runs of other rows straddle
+// lines: each part loaded or stored past the caches is a memory access of its
+// own, where ordinary ones meet in L2.  Rows of n + 33 values, past the caches /
+// ordinary, us: fastconv 64 x 262144 225 / 160, 50 x 262144 179 / 135, 200 x
+// 65536 167 / 115 (n + 8 values 132 / 115); transforms (last pass) 20 x 262144 55 /
+// 45, 8 x 262144 28.2 / 22.0, 24 x 131072 32.2 / 24.9, 30 x 65536 21.2 / 17.6.
+inline bool fs_whole_lines(const float2 *p, long ld, long rows)
+{
+  return (size_t)p % 128 == 0 && (rows == 1 || ld % 16 == 0);
+}
+
 // Whether the first / last pass of a fastconv over `bytes` of rows goes past
 // the caches: X, which is read once, should not push Y out of the 256 MB
 // Infinity Cache, nor the result the rows of Y still to be read.  All ordinary

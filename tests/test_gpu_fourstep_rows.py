@@ -56,3 +56,26 @@ def test_four_step_rows(ovx, n, rows):
     rep = ovx.Replica(n, w.cpu().numpy(), is_spectrum=True)
     fc.with_replica(x, rep, out=x)  # in place
     assert torch.equal(x, y)
+
+
+@pytest.mark.parametrize("rows,n,pad", [(1, 65536, 1), (3, 65536, 33), (9, 16 * 2048, 8), (9, 131072, 5),
+                                        (24, 131072, 33), (13, 1 << 20, 24), (50, 262144, 33)])
+def test_rows_off_the_cache_lines(ovx, rows, n, pad):
+    """Rows of other strides and bases than whole 128-byte lines are stored by
+    other launches: the arithmetic of a line is the same, so the same bits."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(rows * n + pad)
+    x = torch.randn(rows, n, dtype=torch.complex64, device="cuda", generator=g)
+    w = torch.randn(n, dtype=torch.complex64, device="cuda", generator=g)
+    xo, yo = (torch.full((rows * (n + pad) + 1,), 7.0, dtype=torch.complex64, device="cuda") for _ in range(2))
+    xp, yp = (t[1:].view(rows, n + pad) for t in (xo, yo))
+    xp[:, :n].copy_(x)
+    plans = [ovx.Fftm(rows, n, ovx.ROW, d, 0.5) for d in (ovx.FFT_FWD, ovx.FFT_INV)]
+    calls = [lambda a, b, p=p: p(a, out=b) for p in plans]
+    fc = ovx.Fastconv(rows, n)
+    calls.append(lambda a, b: fc(a, w, out=b))
+    for call in calls:
+        want = call(x, torch.empty_like(x))
+        call(xp[:, :n], yp[:, :n])
+        assert torch.equal(yp[:, :n], want)
+        assert bool((yp[:, n:] == 7.0).all()) and bool(yo[0] == 7.0)
