@@ -30,7 +30,7 @@ struct FsArgs {
   // interleaved column pass: non-temporal loads (forward) or loads and stores
   // (inverse), see fs_streams_in / fs_streams_out
   bool stream = false;
-  // row pass of a forward transform: the result is read again in this call
+  // row pass: the result is read again in this call
   bool reread = false;
   // row and middle passes: each row on the XCD of its column pass
   // (fs_stays_in_l2)

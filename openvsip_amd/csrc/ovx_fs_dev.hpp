@@ -131,6 +131,7 @@ __device__ __forceinline__ void fs_line_twiddles(const FsArgs &a, long k1, int t
 // a kernel of the same call reads it again (a real transform's recombination), so
 // it is stored the ordinary way: 63 x 65536 real values forward 30.4 us
 // non-temporally, 25.3 so, 256 113 and 87.
+// Rows off the 128-byte lines are stored so too (fs_whole_lines).
 template <int L, int P, int C, int DIR, bool SOUT = false, bool REREAD = false, typename LP>
 __device__ __forceinline__ void fs_row_body(const FsArgs &a, long row, long group, int tid, LP lds_all)
 {
