@@ -331,8 +331,12 @@ int ovx_storage_info(ovx_storage storage, unsigned *valid, uint64_t *h2d_bytes,
    four-step path run in chunks of about 192 MB, each chunk one launch per
    pass and line length (one line group per workgroup), so that a chunk
    stays in the Infinity Cache between its passes.  The launches are
-   captured once into a hipGraph at commit and replayed by every exec.  Each job's result is bitwise the same as
-   ovx_fastconv_exec_replica on the same job.  ovx_batch_launches returns
+   captured once into a hipGraph at commit and replayed by every exec.  Each
+   job's result is bitwise the same as ovx_fastconv_exec_replica on the same job
+   with a plan of the job's rows and n made without a variant -- at 6144 and
+   12288 points, and where the autotuner has chosen another variant for the plan
+   or the job, with a plan of the variant that ovx_batch_job_variant reports.
+   ovx_batch_launches returns
    the number of kernel launches per replay.  A committed batch holds the
    device addresses of its jobs' buffers and replica spectra: they must stay
    valid (and the replicas not destroyed) until the batch is destroyed. */

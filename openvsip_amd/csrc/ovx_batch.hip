@@ -7,8 +7,8 @@
 // workgroups (one per CU; rows of 12288 and 16384 points) and one of
 // 512-thread workgroups (two per CU; every shorter row), whose fixed grids
 // stride over their queues, workgroup w taking tiles w, w + grid, ...  Every
-// tile runs the same device body as the standalone kernels, so a job's
-// result is bitwise the same alone and in a batch.  Four-step jobs need their
+// tile runs the same device body as the standalone kernel of its variant, so a
+// job's result is bitwise the same alone and in a batch.  Four-step jobs need their
 // three passes in order; each pass is a launch of its own over its queue.  A
 // batch's launches are captured in one hipGraph; the server issues its own.
 #include "ovx_batch.hpp"
@@ -188,13 +188,13 @@ __device__ __forceinline__ FsArgs fs_args_of(const J &j)
 // runs in the launch of NT threads: the host routes each to exactly one of
 // the two (batch_queue, batch_ols_queue), and the other launch's switch has
 // no code for it.
-template <int NT, int PATH, int N>
-constexpr bool runs_in() { return batch_mid_routed(PATH, N) == (NT == kBatchMidThreads); }
+template <int NT, int PATH, int N, int P = 0>
+constexpr bool runs_in() { return batch_mid_routed(PATH, N, P) == (NT == kBatchMidThreads); }
 template <int NT, int L>
 constexpr bool ols_runs_in() { return batch_ols_mid_routed(L) == (NT == kBatchMidThreads); }
-static_assert(batch_mid_routed(BP_HIER, 8192) && !batch_mid_routed(BP_HIER, 16384) &&
-                  batch_mid_routed(BP_ROW, 6144) && !batch_mid_routed(BP_ROW, 12288) &&
-                  batch_mid_routed(BP_ROW, 256) && batch_ols_mid_routed(8192) && !batch_ols_mid_routed(16384),
+static_assert(batch_mid_routed(BP_HIER, 8192, 0) && !batch_mid_routed(BP_HIER, 16384, 0) &&
+                  batch_mid_routed(BP_ROW, 6144, 12) && !batch_mid_routed(BP_ROW, 12288, 12) &&
+                  batch_ols_mid_routed(8192) && !batch_ols_mid_routed(16384),
               "rows of 12288 and 16384 points (and segments of 16384) need the 1024-thread launch, all others "
               "run in the 512-thread one");
 
@@ -209,7 +209,7 @@ __device__ __forceinline__ void run_hier(bool fwd_only, const BatchJob &j, const
 template <int NT, int N, int P>
 __device__ __forceinline__ void run_row(bool fwd_only, const BatchJob &j, const Tile &tile, lds_ptr lds)
 {
-  if constexpr (runs_in<NT, BP_ROW, N>()) {
+  if constexpr (runs_in<NT, BP_ROW, N, P>()) {
     if (fwd_only) tile_row_fwd<NT, N, P>(j, tile, lds);
     else tile_row_fastconv<NT, N, P>(j, tile, lds);
   }
@@ -250,14 +250,11 @@ __device__ __forceinline__ void batch_loop(const BatchJob *__restrict__ jobs, co
     case BT_ROW_FASTCONV:
     case BT_ROW_FFT_FWD: {
       const bool fwd = tile.op == BT_ROW_FFT_FWD;
-      switch (j.n) {
-      case 256: run_row<NT, 256, 16>(fwd, j, tile, lds); break;
-      case 512: run_row<NT, 512, 16>(fwd, j, tile, lds); break;
-      case 2048: run_row<NT, 2048, 16>(fwd, j, tile, lds); break;
-      case 4096: run_row<NT, 4096, 16>(fwd, j, tile, lds); break;
-      case 3072: run_row<NT, 3072, 12>(fwd, j, tile, lds); break;
-      case 6144: run_row<NT, 6144, 12>(fwd, j, tile, lds); break;
-      case 12288: run_row<NT, 12288, 12>(fwd, j, tile, lds); break;
+      switch (j.n + j.p) { // lengths are multiples of 256, values per thread fewer
+#define X(N, P) \
+      case N + P: run_row<NT, N, P>(fwd, j, tile, lds); break;
+      OVX_ROW_TILES(X)
+#undef X
       default: break;
       }
       break;
@@ -403,18 +400,18 @@ hipError_t launch_batch_fs(int n_line, int pass, bool stream, const BatchQueue &
   return hipErrorInvalidValue;
 }
 
-bool batch_supported(int path, int n)
+bool batch_supported(int path, int n, int p)
 {
   if (path == BP_HIER) return hier_supported(n);
-  if (path == BP_ROW) return n == 256 || n == 512 || n == 2048 || n == 4096 || n == 3072 || n == 6144 || n == 12288;
+  if (path == BP_ROW) return batch_row_tile(n, p);
   if (path == BP_FS) return n == 65536 || n == 131072 || n == 262144;
   return false;
 }
 
-int batch_rows_per_tile(int path, int n)
+int batch_rows_per_tile(int path, int n, int p)
 {
   if (path != BP_HIER && path != BP_ROW) return 1;
-  return (batch_mid_routed(path, n) ? kBatchMidThreads : kBatchThreads) / batch_line_threads(path, n);
+  return (batch_mid_routed(path, n, p) ? kBatchMidThreads : kBatchThreads) / batch_line_threads(path, n, p);
 }
 
 int batch_fs_lines_per_group(int n_line)

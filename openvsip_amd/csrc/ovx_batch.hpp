@@ -25,6 +25,7 @@ enum BatchOp {
 struct alignas(16) BatchJob { // spans may follow a table of jobs
   int path;
   int n;
+  int p;             // ROW: values per thread
   long rows;
   const float2 *x;
   long ldx;
@@ -69,10 +70,25 @@ constexpr int kFsLines[2] = { 256, 512 };
 inline int fs_queue(int pass, int n_line) { return 1 + 2 * pass + (n_line == 512 ? 1 : 0); }
 inline int fs_queue_line(int q) { return kFsLines[(q - 1) % 2]; }
 
-// Values per thread of a register-Stockham batch tile: 12 for the 3 * 2^k
-// lengths (so that 1024 threads fit the 128-VGPR budget of a 1024-thread
-// workgroup), 16 for the powers of two.
-constexpr int batch_row_p(int n) { return (n == 256 || n == 512 || n == 2048 || n == 4096) ? 16 : 12; }
+// X(N, P): the register-Stockham tile bodies, N points with P values per
+// thread.  A length has the configurations that a fastconv plan of it runs by
+// default (row_pick), so that a job gives the same floats in a batch as alone:
+// at 1024 points that is the hierarchical body (16 values a thread, the same
+// operations).  6144 and 12288 points, whose plans run 24 values a thread, have
+// 12, which fit the 128-VGPR budget of both kernels.  16 values a thread for
+// every power of two / the plans' own: 47 jobs of 512 points 20.2 / 20.1 us, 50
+// of 2048 60.5 / 72.3, 47 of 256 13.2 / 14.6, the 512-job benchmark 5.93 / 5.95
+// ms.
+#define OVX_ROW_TILES(X)                                                                        \
+  X(256, 4) X(512, 8) X(2048, 16) X(2048, 8) X(4096, 16) X(3072, 12) X(6144, 12) X(12288, 12)
+constexpr bool batch_row_tile(int n, int p)
+{
+#define X(N, P) \
+  if (n == N && p == P) return true;
+  OVX_ROW_TILES(X)
+#undef X
+  return false;
+}
 
 // Threads per persistent workgroup.  Rows whose line takes at most 512
 // threads (every LDS-resident length up to 8192; overlap-save segments up to
@@ -81,19 +97,19 @@ constexpr int batch_row_p(int n) { return (n == 256 || n == 512 || n == 2048 || 
 // 16384 need the 1024-thread workgroup, one per CU.
 constexpr int kBatchThreads = 1024;
 constexpr int kBatchMidThreads = 512;
-constexpr int batch_line_threads(int path, int n) // threads of one row's transform
+constexpr int batch_line_threads(int path, int n, int p) // threads of one row's transform
 {
-  return path == BP_HIER ? 64 * (n / 1024) : n / batch_row_p(n);
+  return path == BP_HIER ? 64 * (n / 1024) : n / p;
 }
-constexpr bool batch_mid_routed(int path, int n) { return batch_line_threads(path, n) <= kBatchMidThreads; }
+constexpr bool batch_mid_routed(int path, int n, int p) { return batch_line_threads(path, n, p) <= kBatchMidThreads; }
 constexpr bool batch_ols_mid_routed(int L) { return L / 16 <= kBatchMidThreads; }
-inline int batch_queue(int path, int n) { return batch_mid_routed(path, n) ? kMidQueue : 0; }
+inline int batch_queue(int path, int n, int p) { return batch_mid_routed(path, n, p) ? kMidQueue : 0; }
 inline int batch_ols_queue(int L) { return batch_ols_mid_routed(L) ? kMidQueue : 0; }
-int batch_rows_per_tile(int path, int n);
+int batch_rows_per_tile(int path, int n, int p);
 int batch_ols_segments_per_tile(int L);
 int batch_fs_lines_per_group(int n_line); // C of a four-step group of lines of length n_line
 int batch_fs_conv_lines_per_group(int n_line); // of a fastconv's middle pass
-bool batch_supported(int path, int n);
+bool batch_supported(int path, int n, int p);
 
 // A queue in device memory: spans by first tile, `tiles` tiles in all.
 struct BatchQueue {

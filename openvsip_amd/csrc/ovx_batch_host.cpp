@@ -28,15 +28,14 @@ static std::map<std::pair<long, int>, std::unique_ptr<LineFFT>> g_paths;
 
 // Variant the batch tiles of an (n, rows) job run: the autotuner's batch
 // entry for (n, rows) when it names a tile body (an older cache file may hold
-// other variant numbers), else at 2048 and 4096 points the register-Stockham
-// body, else the first.  Lengths without a tile run the standalone default.
+// other variant numbers), else the last candidate, a plan's own default where
+// it has a tile.  Lengths without a tile run the standalone default.
 int batch_variant(long n, long rows)
 {
-  const std::vector<int> cands = batch_candidates(n);
+  const std::vector<int> cands = batch_candidates(n, rows);
   if (cands.empty()) return LineFFT::default_variant(n, rows);
   const int v = tuned_batch_variant(n, rows);
-  if (std::find(cands.begin(), cands.end(), v) != cands.end()) return v;
-  return n == 2048 || n == 4096 ? cands.back() : cands.front();
+  return std::find(cands.begin(), cands.end(), v) != cands.end() ? v : cands.back();
 }
 
 const LineFFT *shared_path(long n, int variant, int *status)
@@ -88,7 +87,8 @@ int make_batch_job(const LineFFT &f, long rows, const float2 *x, long ldx, float
   BatchJob j{};
   j.path = batch_path_of(f);
   j.n = (int)f.n;
-  if (!batch_supported(j.path, j.n))
+  j.p = j.path == BP_ROW ? f.rc.p : 0;
+  if (!batch_supported(j.path, j.n, j.p))
     return fail(OVX_ERR_UNSUPPORTED, "length %ld has no batch tile (path %d)", f.n, j.path);
   if (!f.tables_ready()) return fail(OVX_ERR_STATE, "length %ld: twiddle tables missing", f.n);
   if (rows > 0x7fffffff) return fail(OVX_ERR_UNSUPPORTED, "too many rows in one job");
@@ -103,11 +103,6 @@ int make_batch_job(const LineFFT &f, long rows, const float2 *x, long ldx, float
     j.tw0 = (const float2 *)f.tw_outer.p;
     j.tw1 = (const float2 *)f.tw_wave.p;
   } else if (j.path == BP_ROW) {
-    // the tile body is Engine<n, batch_row_p(n)>: the path must be exactly
-    // that configuration, or its twiddle table would not match
-    if (f.rc.p != batch_row_p(j.n))
-      return fail(OVX_ERR_STATE, "length %ld: path has %d values per thread, batch tile needs %d", f.n, f.rc.p,
-                  batch_row_p(j.n));
     j.tw0 = (const float2 *)f.tw.p;
   } else {
     j.tw0 = (const float2 *)f.tw1.p;
@@ -146,9 +141,9 @@ hipError_t launch_queue(const TileQueue &q, const BatchJob *jobs, const BatchSpa
 
 void push_row_tiles(const BatchJob &j, int ji, bool fft, TileQueue &big, TileQueue &mid)
 {
-  const int rpt = batch_rows_per_tile(j.path, j.n);
+  const int rpt = batch_rows_per_tile(j.path, j.n, j.p);
   const int op = j.path == BP_HIER ? (fft ? BT_HIER_FFT_FWD : BT_HIER_FASTCONV) : (fft ? BT_ROW_FFT_FWD : BT_ROW_FASTCONV);
-  TileQueue &q = batch_queue(j.path, j.n) == kMidQueue ? mid : big;
+  TileQueue &q = batch_queue(j.path, j.n, j.p) == kMidQueue ? mid : big;
   q.push(ji, op, 0, j.rows, (j.rows + rpt - 1) / rpt);
 }
 
@@ -340,7 +335,7 @@ extern "C" int ovx_batch_commit(ovx_batch b, void *stream)
   if (!getenv("OVX_NO_BATCH_TUNE")) {
     for (size_t i = 0; i < b->jobs.size(); ++i) {
       const auto &h = b->jobs[i];
-      if (batch_candidates(h.n).size() > 1 && tuned_batch_variant(h.n, h.rows) < 0) {
+      if (batch_candidates(h.n, h.rows).size() > 1 && tuned_batch_variant(h.n, h.rows) < 0) {
         int st = autotune_batch(h.n, h.rows, nullptr, nullptr);
         if (st) return st;
       }

@@ -19,7 +19,7 @@ int batch_variant(long n, long rows);
 // Batch tile autotuner (ovx_tune.cpp): the variants whose device body a
 // batch tile can run for length n, the cached choice for (n, rows) or -1,
 // and the tuning itself (records the choice).
-std::vector<int> batch_candidates(long n);
+std::vector<int> batch_candidates(long n, long rows);
 int tuned_batch_variant(long n, long rows);
 int autotune_batch(long n, long rows, int *best_variant, double *best_us);
 int batch_path_of(const LineFFT &f);

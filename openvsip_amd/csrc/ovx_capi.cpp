@@ -93,10 +93,13 @@ static int make_row_twiddles(const RowConfig &rc, DevBuf &tw, size_t room = 0, b
 // hierarchical fastconv at 8192 and 16384 points (256 rows: 12.9 against 14.6
 // and 24.1 against 24.5 us), the register-Stockham kernel at the lengths below,
 // where it is faster at every row count (1024: 6.2 against 5.3, 2048: 8.7
-// against 6.9, 4096: 8.7 against 8.1 us).
+// against 6.9, 4096: 8.7 against 8.1 us).  At 1024 points always with 16 values
+// per thread, the operations of the batch's tile body (8 and 16 values: 64 rows
+// 4.1 and 4.7 us, 256 rows 4.3 and 4.8, 600 rows 6.2 and 5.5).
 int LineFFT::default_variant(long n, long rows)
 {
   if (n < 1 || n > kMaxRowN || n == 8192 || n == 16384) return 0;
+  if (n == 1024) return row_variant(n, row_config_with(1024, 16));
   return row_variant(n, row_pick((int)n, rows));
 }
 

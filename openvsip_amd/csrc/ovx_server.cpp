@@ -217,7 +217,7 @@ static long tiles_of(const Req &q, const LineFFT *f, const CorrRef *cr)
     long gr = f->n1 / batch_fs_lines_per_group((int)f->n2);
     return r.rows * std::max(gc, gr);
   }
-  long rpt = batch_rows_per_tile(path, (int)r.n);
+  long rpt = batch_rows_per_tile(path, (int)r.n, f->rc.p);
   return (r.rows + rpt - 1) / rpt;
 }
 

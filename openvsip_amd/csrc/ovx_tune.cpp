@@ -226,23 +226,25 @@ extern "C" int ovx_autotune_fastconv(long n, long rows, int *best_variant, doubl
 extern "C" int ovx_tuned_variant(long n, long rows) { return tuned_variant(n, rows); }
 
 // ---------------------------------------------------------------- batch tiles
-// The tile bodies a batch (and the server) can run for length n: the
-// hierarchical body and the register-Stockham body with batch_row_p(n)
-// values per thread, each the device body of one standalone variant.
+// The tile bodies a batch (and the server) can run for a job of n x rows, each
+// the device body of one standalone variant: the hierarchical one, then a
+// plan's default or, where that has no tile, the configuration that has.
 namespace ovx {
 
-std::vector<int> batch_candidates(long n)
+std::vector<int> batch_candidates(long n, long rows)
 {
   std::vector<int> out;
   if (n < 1 || n > kMaxRowN) return out;
-  const bool hier = hier_supported(n);
-  if (hier && batch_supported(BP_HIER, (int)n)) out.push_back(0);
-  if (batch_supported(BP_ROW, (int)n)) {
-    for (int v = 0; v < row_variants((int)n); ++v) {
-      RowConfig rc;
-      if (row_config((int)n, v, &rc) && rc.p == batch_row_p((int)n)) out.push_back(hier ? v + 1 : v);
-    }
-  }
+  if (hier_supported(n) && batch_supported(BP_HIER, (int)n, 0)) out.push_back(0);
+  auto has_tile = [&](int config) {
+    RowConfig rc;
+    return row_config((int)n, config, &rc) && batch_supported(BP_ROW, (int)n, rc.p);
+  };
+  const int configs = row_variants((int)n);
+  int config = row_pick((int)n, rows);
+  if (!has_tile(config))
+    for (config = 0; config < configs && !has_tile(config);) ++config;
+  if (config < configs) out.push_back(LineFFT::row_variant(n, config));
   return out;
 }
 
@@ -260,7 +262,7 @@ int tuned_batch_variant(long n, long rows)
 // rounds of 20 replays counts.
 int autotune_batch(long n, long rows, int *best_variant, double *best_us)
 {
-  std::vector<int> cands = batch_candidates(n);
+  std::vector<int> cands = batch_candidates(n, rows);
   if (cands.empty()) return fail(OVX_ERR_UNSUPPORTED, "length %ld has no batch tile to tune", n);
   DevBuf x, y, w, wp;
   const size_t bytes = (size_t)rows * n * 8;
