@@ -22,6 +22,7 @@
 #include "ovx_hier.hpp"
 #include "ovx_internal.hpp"
 #include "ovx_batch_host.hpp"
+#include "ovx_overlap.hpp"
 #include "ovx_plan.hpp"
 
 using namespace ovx;
@@ -377,14 +378,6 @@ int LineFFT::transform_split(int dir, const float *in_re, const float *in_im, lo
   a.scale = scale;
   hipError_t e = launch_hier(dir < 0 ? HIER_FWD_SPLIT : HIER_INV_SPLIT, n, a, s);
   return e == hipSuccess ? OVX_OK : hip_fail(e, "row fft launch");
-}
-
-// Whether `lines` lines of n values at a stride of ld and `lines2` at ld2 share
-// memory.
-template <typename T>
-static bool lines_meet(const T *a, long lines, long ld, const T *b, long lines2, long ld2, long n)
-{
-  return a < b + (lines2 - 1) * ld2 + n && b < a + (lines - 1) * ld + n;
 }
 
 // Up to this many lines the register-Stockham kernel, which reads a spectrum
