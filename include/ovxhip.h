@@ -200,8 +200,10 @@ int ovx_fastconv_exec(ovx_plan plan, const void *x, long ldx, const void *w,
    each GPU until the process ends, instead of a plan buffer made on first
    use.  The call allocates nothing (no hipMalloc, no hipFree; the plan's
    tables were made by ovx_fastconv_plan_create).  A call that would need
-   more scratch (a four-step plan with a coefficient matrix of many rows, or
-   a spectrum longer than 2^19 points) fails with OVX_ERR_UNSUPPORTED;
+   more scratch (a four-step plan with a coefficient matrix of many rows, a
+   spectrum longer than 2^19 points, or more than 2^19 values of spectra that
+   share memory with the result, other than each row's with its own result)
+   fails with OVX_ERR_UNSUPPORTED;
    host-pointer plans are refused.  Every call on one GPU shares that GPU's
    array and leaves its last contents there (each call writes all of the
    scratch it reads before reading it): calls that overlap on one GPU --

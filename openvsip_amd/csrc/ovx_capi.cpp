@@ -507,7 +507,9 @@ int LineFFT::fastconv(const float2 *x, long ldx, const float2 *w, long ldw, floa
     // a line's spectrum is read before its result is written; other overlaps
     // have the spectra copied out of the result's way
     const size_t values = (size_t)(ldw ? lines : 1) * n;
-    if (meet && !(ldw != 0 && w == y && ldw == ldy) && (!ext || ext->wp_elems >= values)) {
+    if (meet && !(ldw != 0 && w == y && ldw == ldy)) {
+      if (ext && ext->wp_elems < values)
+        return fail(OVX_ERR_UNSUPPORTED, "lent scratch too small for spectra that share memory with the result");
       float2 *copy = ext ? ext->wp : nullptr;
       if (!ext) {
         int st = wp.alloc(values * 8);
