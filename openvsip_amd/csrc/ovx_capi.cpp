@@ -487,12 +487,25 @@ int LineFFT::fastconv_split(const float *xr, const float *xi, long ldx, const fl
   return e == hipSuccess ? OVX_OK : hip_fail(e, "fastconv launch");
 }
 
+bool LineFFT::spectra_meet(const float2 *w, long ldw, const float2 *y, long ldy, long lines) const
+{
+  return lines_meet(w, ldw ? lines : 1, ldw, y, lines, ldy, n);
+}
+
+// A line's spectrum is read before its result is written: spectra in the places
+// of their own results need no copy.
+bool LineFFT::copies_spectra(const float2 *w, long ldw, const float2 *y, long ldy, long lines) const
+{
+  return (kind == LDS || kind == HIER) && spectra_meet(w, ldw, y, ldy, lines) &&
+         !(ldw != 0 && w == y && (lines == 1 || ldw == ldy));
+}
+
 int LineFFT::fastconv(const float2 *x, long ldx, const float2 *w, long ldw, float2 *y, long ldy, long lines,
                       float scale, hipStream_t s, const ExtScratch *ext) const
 {
   if (lines <= 0) return OVX_OK;
   if (!tables_ready()) return fail(OVX_ERR_STATE, "fastconv plan has no twiddle tables");
-  const bool meet = lines_meet(w, ldw ? lines : 1, ldw, (const float2 *)y, lines, ldy, n);
+  const bool meet = spectra_meet(w, ldw, y, ldy, lines);
   if (kind == HIER && ldw == 0 && (meet || !rows_fastconv(ldw, lines) || !row_strides_fit(ldx, ldw, ldy))) {
     HierArgs a = hier_args(*this);
     a.x = x;
@@ -504,10 +517,8 @@ int LineFFT::fastconv(const float2 *x, long ldx, const float2 *w, long ldw, floa
       return fail(OVX_ERR_UNSUPPORTED, "row stride too large for 32-bit buffer offsets");
     if (ext && ext->wp_elems < fastconv_scratch_wp(lines, ldw))
       return fail(OVX_ERR_UNSUPPORTED, "lent scratch too small for the spectrum");
-    // a line's spectrum is read before its result is written; other overlaps
-    // have the spectra copied out of the result's way
     const size_t values = (size_t)(ldw ? lines : 1) * n;
-    if (meet && !(ldw != 0 && w == y && ldw == ldy)) {
+    if (copies_spectra(w, ldw, y, ldy, lines)) { // out of the result's way
       if (ext && ext->wp_elems < values)
         return fail(OVX_ERR_UNSUPPORTED, "lent scratch too small for spectra that share memory with the result");
       float2 *copy = ext ? ext->wp : nullptr;
@@ -1050,8 +1061,8 @@ extern "C" int ovx_fastconv_plan_create(ovx_plan *plan, long rows, long n, float
 // 3 us between back-to-back launches).  The check is conservative: it also
 // refuses when the other stream's pending work is not this plan's.  Calls
 // that use no plan scratch (a prepared replica spectrum, the
-// register-Stockham and BF16x3 kernels reading the spectrum as given) skip
-// it.
+// register-Stockham and BF16x3 kernels reading the spectrum as given, unless the
+// result shares its memory) skip it.
 static int claim_plan(ovx_plan p, hipStream_t s)
 {
   if (!p->scratch_used || p->scratch_stream == s) return OVX_OK;
@@ -1062,7 +1073,29 @@ static int claim_plan(ovx_plan p, hipStream_t s)
   return OVX_OK;
 }
 
-static int mark_plan(ovx_plan p, hipStream_t s, int status)
+// The same for calls that once used no scratch and ran on several streams at
+// once: the other stream's work is waited for instead of refusing the call
+// (under capture, where it cannot be waited for, the call is refused).
+int ovx::order_plan(ovx_plan_s *p, hipStream_t s)
+{
+  if (!p->scratch_used || p->scratch_stream == s) return OVX_OK;
+  hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+  hipError_t e = hipStreamIsCapturing(s, &capturing);
+  if (e != hipSuccess) return hip_fail(e, "capture status");
+  if (capturing != hipStreamCaptureStatusNone) return claim_plan(p, s);
+  if (hipStreamQuery(p->scratch_stream) != hipErrorNotReady) {
+    (void)hipGetLastError();
+    return OVX_OK;
+  }
+  hipEvent_t last;
+  if ((e = hipEventCreateWithFlags(&last, hipEventDisableTiming)) != hipSuccess) return hip_fail(e, "scratch event");
+  e = hipEventRecord(last, p->scratch_stream);
+  if (e == hipSuccess) e = hipStreamWaitEvent(s, last, 0);
+  (void)hipEventDestroy(last);
+  return e == hipSuccess ? OVX_OK : hip_fail(e, "wait for the plan's scratch");
+}
+
+int ovx::mark_plan(ovx_plan_s *p, hipStream_t s, int status)
 {
   if (status) return status;
   p->scratch_used = true;
@@ -1081,8 +1114,11 @@ extern "C" int ovx_fastconv_exec(ovx_plan p, const void *x, long ldx, const void
   hipStream_t s = (hipStream_t)stream;
   if (p->flags & OVX_FLAG_HOST_POINTERS) return fastconv_exec_body(p, x, ldx, w, ldw, y, ldy, rows, s);
   // the hierarchical and four-step kernels read the spectrum permuted into
-  // the plan's buffer
-  const bool scratch = !p->bf16x3 && (p->line.kind == LineFFT::HIER || p->line.kind == LineFFT::FOURSTEP);
+  // the plan's buffer, the register-Stockham ones a copy there of spectra that
+  // share memory with the result
+  const bool fits = rows > 0 && rows <= p->rows && (rows == 1 || ldy >= p->cols); // else the body refuses it
+  const bool scratch = !p->bf16x3 && (p->line.kind == LineFFT::HIER || p->line.kind == LineFFT::FOURSTEP ||
+                                      (fits && p->line.copies_spectra((const float2 *)w, ldw, (const float2 *)y, ldy, rows)));
   if (!scratch) return fastconv_exec_body(p, x, ldx, w, ldw, y, ldy, rows, s);
   if ((st = claim_plan(p, s))) return st;
   return mark_plan(p, s, fastconv_exec_body(p, x, ldx, w, ldw, y, ldy, rows, s));

@@ -74,10 +74,9 @@ static bool runs_meet(const float2 *a, long na, const float2 *b, long nb) { retu
 // is copied out of the result's way then.
 static bool ols_copies_meeting(const CorrState &c) { return c.N <= kMaxRowN && segment_count(c, c.L) > 1; }
 
-// The samples to read for a result at `out`: `in` itself, or its copy.
-static int ols_input(CorrState &c, const float2 *&in, const float2 *out, hipStream_t s)
+// Puts the samples in `in` out of the way of a result over them.
+static int ols_copy_input(CorrState &c, const float2 *&in, hipStream_t s)
 {
-  if (!ols_copies_meeting(c) || !runs_meet(in, c.N, out, c.P)) return OVX_OK;
   hipError_t e = hipMemcpyAsync(c.in_stage.p, in, (size_t)c.N * 8, hipMemcpyDeviceToDevice, s);
   in = (const float2 *)c.in_stage.p;
   return e == hipSuccess ? OVX_OK : hip_fail(e, "signal copy");
@@ -233,12 +232,16 @@ extern "C" int ovx_corr_exec(ovx_plan p, int bias, const void *ref, const void *
     din = (const float2 *)c.in_stage.p;
     dout = (float2 *)c.out_stage.p;
   }
-  if (!host && (st = ols_input(c, din, dout, s))) return st;
   // a reference that the result is written over is read whole by a launch of
   // its own first
   const bool fuse = ols_fuse_ref(c) && !runs_meet(dref, c.M, dout, c.P);
+  const bool copy = !host && ols_copies_meeting(c) && runs_meet(din, c.N, dout, c.P);
+  const bool scratch = !host && (copy || !fuse);
+  if (scratch && (st = order_plan(p, s))) return st;
+  if (copy && (st = ols_copy_input(c, din, s))) return st;
   if (!fuse && (st = ols_spectrum(c, dref, 1, s))) return st;
   if ((st = ols_run(c, fuse ? dref : nullptr, din, dout, 1, bias == OVX_UNBIASED, s))) return st;
+  if (scratch) return mark_plan(p, s, OVX_OK);
   if (host) {
     hipError_t e = hipMemcpyAsync(out, c.out_stage.p, (size_t)c.P * 8, hipMemcpyDeviceToHost, s);
     if (e == hipSuccess) e = hipStreamSynchronize(s);
@@ -324,8 +327,10 @@ extern "C" int ovx_conv_exec(ovx_plan p, const void *in, void *out, void *stream
     din = (const float2 *)c.in_stage.p;
     dout = (float2 *)c.out_stage.p;
   }
-  if (!host && (st = ols_input(c, din, dout, s))) return st;
+  const bool copy = !host && ols_copies_meeting(c) && runs_meet(din, c.N, dout, c.P);
+  if (copy && ((st = order_plan(p, s)) || (st = ols_copy_input(c, din, s)))) return st;
   if ((st = ols_run(c, nullptr, din, dout, 0, 0, s))) return st;
+  if (copy) return mark_plan(p, s, OVX_OK);
   if (host) {
     hipError_t e = hipMemcpyAsync(out, c.out_stage.p, (size_t)c.P * 8, hipMemcpyDeviceToHost, s);
     if (e == hipSuccess) e = hipStreamSynchronize(s);

@@ -70,6 +70,10 @@ struct LineFFT {
                hipStream_t s, const ExtScratch *ext = nullptr) const;
   bool rows_fastconv(long ldw, long lines) const;
   bool row_strides_fit(long ldx, long ldw, long ldy) const;
+  // spectra that share memory with the result, and whether fastconv() copies
+  // them to `wp` (or a lent buffer) for it
+  bool spectra_meet(const float2 *w, long ldw, const float2 *y, long ldy, long lines) const;
+  bool copies_spectra(const float2 *w, long ldw, const float2 *y, long ldy, long lines) const;
   // permuted-spectrum elements fastconv() needs for `lines` lines and
   // spectrum row stride ldw (0 when it permutes nothing)
   size_t fastconv_scratch_wp(long lines, long ldw) const;
@@ -128,3 +132,11 @@ struct ovx_plan_s {
   const char *name() const;
   size_t device_bytes() const;
 };
+
+namespace ovx {
+// Before and after a call that uses the plan's scratch: order_plan makes the
+// stream wait for the scratch's last user if that is another stream with work
+// queued, mark_plan remembers the stream.
+int order_plan(ovx_plan_s *p, hipStream_t s);
+int mark_plan(ovx_plan_s *p, hipStream_t s, int status);
+} // namespace ovx
