@@ -70,9 +70,13 @@ static bool runs_meet(const float2 *a, long na, const float2 *b, long nb) { retu
 
 // A single segment reads all of its samples before its first store, so a result
 // over the signal is right; several segments run at once and store over each
-// other's samples.  A signal that one segment of the greatest length could hold
-// is copied out of the result's way then.
-static bool ols_copies_meeting(const CorrState &c) { return c.N <= kMaxRowN && segment_count(c, c.L) > 1; }
+// other's samples.  A signal of which one segment of the greatest length could
+// hold all that the outputs need is copied out of the result's way then (with a
+// decimation the signal itself may be longer).
+static bool ols_copies_meeting(const CorrState &c)
+{
+  return segment_count(c, c.L) > 1 && (c.N <= kMaxRowN || (c.P - 1) * c.D + 1 + c.M - 1 <= kMaxRowN);
+}
 
 // Puts the samples in `in` out of the way of a result over them.
 static int ols_copy_input(CorrState &c, const float2 *&in, hipStream_t s)
