@@ -282,7 +282,12 @@ int Server::admit_and_launch(Slot &s, std::vector<Req *> &batch)
     if (e == hipSuccess) e = launch_queue(q, (const BatchJob *)s.d_tab.p, spans, s.stream);
     spans += q.spans.size();
   }
-  if (e != hipSuccess) return hip_fail(e, "batch launch");
+  if (e != hipSuccess) {
+    // the slot goes back to the free ones: what was issued must be done with its
+    // tables before the next batch is written into them
+    (void)hipStreamSynchronize(s.stream);
+    return hip_fail(e, "batch launch");
+  }
   return OVX_OK;
 }
 
