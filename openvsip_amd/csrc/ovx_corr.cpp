@@ -39,8 +39,10 @@ static long segment_count(const CorrState &c, int L)
   return (span + step - 1) / step;
 }
 
-// Segments up to which a segment is a matter of latency: four per CU.
+// Segments up to which a segment is a matter of latency: four per CU (those of
+// less than 512 points are so many times fewer).
 constexpr long kOlsFew = 1024;
+static bool few_segments(const CorrState &c, int L) { return segment_count(c, L) * std::min(L, 512) <= kOlsFew * 512; }
 
 // Segment length: the shortest power of two from 512 of which the kernel
 // overlap takes no more than half (the chain of stages is what a call waits
@@ -51,19 +53,26 @@ constexpr long kOlsFew = 1024;
 // the overlap takes no more than a quarter: the rounding error of an output goes
 // with the root of the samples in a segment over its length, and next to a long
 // segment's padding a short one's would be up to 1.4 times larger (1630 x 574,
-// unbiased, 1.9e-6 in segments of 2048, 1.5e-6 in 4096).
+// unbiased, 1.9e-6 in segments of 2048, 1.5e-6 in 4096).  Kernels of up to 33
+// values keep segments of which the overlap takes a quarter for the same
+// reason, fewer levels of rounding: error against 64 bits and time of 126694 x
+// 17, segments of 64 / 512, 1.45e-7 / 1.70e-7 and 3.6 / 4.6 us, of 126694 x 33,
+// 128 / 512, 1.58e-7 / 1.73e-7 and 4.6 / 4.7 us (2 * 10^6 x 17 13.4 / 12.6, x 33
+// 13.6 / 13.3).
 static int choose_L(const CorrState &c)
 {
+  if (c.M <= 17) return 64;
+  if (c.M <= 33) return 128;
   long L = 512, longer = 512;
   while (L < 2 * (c.M - 1) && L < kMaxRowN) L *= 2;
   while (longer < 4 * (c.M - 1) && longer < kMaxRowN) longer *= 2;
   while (L < longer && c.N * L < longer * (L - (c.M - 1))) L *= 2;
-  while (L < kMaxRowN && segment_count(c, (int)L) > kOlsFew && 10 * (c.M - 1) > 3 * L) L *= 2;
+  while (L < kMaxRowN && !few_segments(c, (int)L) && 10 * (c.M - 1) > 3 * L) L *= 2;
   return (int)L;
 }
 
 // The reference's spectrum in every segment or once in a launch of its own.
-static bool ols_fuse_ref(const CorrState &c) { return !c.is_conv && segment_count(c, c.L) <= kOlsFew; }
+static bool ols_fuse_ref(const CorrState &c) { return !c.is_conv && few_segments(c, c.L); }
 
 // Whether two runs of values share memory.
 static bool runs_meet(const float2 *a, long na, const float2 *b, long nb) { return a < b + nb && b < a + na; }
@@ -90,7 +99,7 @@ static int ols_init(CorrState &c)
 {
   if (c.M - 1 >= kMaxRowN) return fail(OVX_ERR_UNSUPPORTED, "kernel length %ld too long for overlap-save", c.M);
   c.L = choose_L(c);
-  c.Lp = c.L <= 2048 ? 8 : 16;
+  c.Lp = c.L == 64 ? 4 : c.L <= 2048 ? 8 : 16;
   // the overlap-save kernels are built on the register-Stockham engine: take
   // the configuration of that length and values per thread and its twiddles
   int st = c.fftL.init(c.L, LineFFT::row_variant(c.L, row_config_with(c.L, c.Lp)));

@@ -13,7 +13,7 @@
 // gathers g[i0 - (M-1) + u] (zero outside [0, N)), runs forward FFT,
 // multiplies by H = FFT_L(h) / L, inverse FFT, and scatters the valid outputs
 // u >= M-1, applying the unbiased divisors (correlation) or the decimation
-// (convolution).  One workgroup per segment.
+// (convolution).  One workgroup per segment, or per wave of short segments.
 //
 // A call is bound by the latency of one segment's chain of stages (a 65536 x
 // 1024 correlation has 65 segments for 256 CUs), so short segments run with 8
@@ -30,11 +30,23 @@
 
 namespace ovx {
 
+// Segments of less than 64 threads share a wave: 256 threads a workgroup took
+// 3.7 instead of 3.2 us for 20000 x 17, 3.8 instead of 3.6 for 126694 x 17.
+template <int L, int P>
+struct OlsCfg {
+  static constexpr int T = L / P;
+  static constexpr int B = T < 64 ? 64 / T : 1;
+  static constexpr int NT = T * B;
+};
+
 template <int L, int P, bool REF>
-__global__ __launch_bounds__(L / P) void k_ols(OlsArgs a)
+__global__ __launch_bounds__((OlsCfg<L, P>::NT)) void k_ols(OlsArgs a)
 {
-  __shared__ float2 lds[Engine<L, P>::LROW];
-  ols_body<L, P, REF>(a, blockIdx.x, 0, threadIdx.x, lds);
+  using C = OlsCfg<L, P>;
+  __shared__ float2 lds[C::B * Engine<L, P>::LROW];
+  const int copy = C::B == 1 ? 0 : (int)threadIdx.x / C::T;
+  const int t = C::B == 1 ? (int)threadIdx.x : (int)threadIdx.x % C::T;
+  ols_body<L, P, REF>(a, (long)blockIdx.x * C::B, copy, t, lds + copy * Engine<L, P>::LROW);
 }
 
 // H = FFT_L of the reversed (correlation) or plain (convolution) kernel,
@@ -57,16 +69,17 @@ __global__ __launch_bounds__(L / P) void k_ols_spectrum(const float2 *__restrict
 // segments; 16 for the longer ones and for every length of the server's
 // references, whose batch tiles run the same body.
 #define OVX_OLS_CONFIGS(X) \
-  X(512, 8) X(1024, 8) X(2048, 8) X(1024, 16) X(2048, 16) X(4096, 16) X(8192, 16) X(16384, 16)
+  X(64, 4) X(128, 8) X(512, 8) X(1024, 8) X(2048, 8) X(1024, 16) X(2048, 16) X(4096, 16) X(8192, 16) X(16384, 16)
 
 hipError_t launch_ols(int L, int P, const OlsArgs &a, long segments, hipStream_t s)
 {
   if (segments <= 0) return hipSuccess;
-  const dim3 grid((unsigned)segments);
 #define X(L_, P_)                                                                                  \
   if (L == L_ && P == P_) {                                                                        \
-    if (a.H) hipLaunchKernelGGL((k_ols<L_, P_, false>), grid, dim3(L_ / P_), 0, s, a);             \
-    else hipLaunchKernelGGL((k_ols<L_, P_, true>), grid, dim3(L_ / P_), 0, s, a);                  \
+    using C = OlsCfg<L_, P_>;                                                                      \
+    const dim3 grid((unsigned)((segments + C::B - 1) / C::B)), block(C::NT);                       \
+    if (a.H) hipLaunchKernelGGL((k_ols<L_, P_, false>), grid, block, 0, s, a);                     \
+    else hipLaunchKernelGGL((k_ols<L_, P_, true>), grid, block, 0, s, a);                          \
     return hipGetLastError();                                                                      \
   }
   OVX_OLS_CONFIGS(X)

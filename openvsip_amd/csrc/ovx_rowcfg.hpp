@@ -75,10 +75,11 @@ struct RowPlace {
 // Where one P is best or within a few per cent everywhere it is the only one;
 // else row_pick() chooses by the number of lines.  16 values per thread at
 // powers of two from 64 and 12 at 3072, 6144 and 12288 are also what the
-// four-step, overlap-save and batch kernels run.
+// four-step, overlap-save and batch kernels run; 8 at 128 points is there for
+// the overlap-save segments alone.
 #define OVX_ROW_CONFIGS(X)                                                      \
   X(2, 2) X(4, 4) X(8, 8) X(16, 4) X(32, 4) X(64, 4) X(64, 16) X(128, 4)        \
-  X(128, 16) X(256, 4) X(256, 16) X(512, 8) X(512, 16) X(1024, 16) X(1024, 8)   \
+  X(128, 16) X(128, 8) X(256, 4) X(256, 16) X(512, 8) X(512, 16) X(1024, 16) X(1024, 8)   \
   X(2048, 16) X(2048, 8) X(4096, 16) X(8192, 16) X(16384, 16)                   \
   X(3, 3) X(6, 6) X(12, 12) X(24, 24) X(48, 6) X(96, 6) X(192, 6) X(384, 12)    \
   X(384, 6) X(768, 12) X(1536, 24) X(1536, 12) X(3072, 12) X(6144, 24)          \
