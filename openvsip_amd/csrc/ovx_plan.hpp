@@ -44,9 +44,11 @@ struct LineFFT {
   int variant = 0;
   RowConfig rc;
   DevBuf tw;
-  // hierarchical (outer stage + per-wave 1024-point transforms); `rc` and
-  // `tw` are then the register-Stockham path that takes coefficient matrices
-  DevBuf tw_outer, tw_wave;
+  // hierarchical (outer stage + per-wave 1024-point transforms): its tables and,
+  // for a fastconv plan, that of the register-Stockham path `rc` which takes
+  // coefficient matrices, one after the other in `tw`
+  const float2 *tw_outer = nullptr, *tw_wave = nullptr;
+  const float2 *tw_rows = nullptr; // of `rc`, on the register-Stockham path `tw` itself
   // two-pass four-step (n = n1 * n2)
   long n1 = 0, n2 = 0;
   int sbits = 0;
@@ -55,7 +57,8 @@ struct LineFFT {
   const float2 *tw2c = nullptr; // lines of a fastconv's middle pass, in tw2 after its own
   mutable DevBuf work, wp; // Fftm workspace, permuted spectrum
 
-  int init(long n, int variant);
+  // fastconv: with what a plan's fastconv calls need beyond prepared spectra
+  int init(long n, int variant, bool fastconv = false);
   const char *name() const;
   size_t device_bytes() const;
   // lines x n at line strides ld_in / ld_out; dir = -1 forward, +1 inverse
