@@ -21,8 +21,12 @@
 namespace ovx {
 
 // ---------------------------------------------------------------- kernels
+// 8192 points: two workgroups a CU, four waves per SIMD, 128 VGPRs.  Left to
+// itself the compiler takes 134 in split storage, one workgroup a CU (1000 rows
+// 48.2 / 38.5 us, 600 35.7 / 30.3, 300 21.8 / 21.0, though three values spill);
+// at 4096 points, 129, the bound is the slower way (256 rows 8.1 / 8.4).
 template <int N, bool SPLIT, bool NTL>
-__global__ __launch_bounds__(Hier<N>::NT) void k_hier_fastconv(HierArgs a)
+__global__ __launch_bounds__(Hier<N>::NT, N == 8192 ? 4 : 1) void k_hier_fastconv(HierArgs a)
 {
   using H = Hier<N>;
   __shared__ float2 lds_all[H::B * H::LROW];
