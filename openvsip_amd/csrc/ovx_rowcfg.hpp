@@ -6,7 +6,7 @@
 
 namespace ovx {
 
-constexpr long kRowSpread = 256; // workgroups that fill the chip, one per CU
+constexpr long kRowCus = 256; // CUs, for rules that go by lines per CU
 
 // Compiled configurations: (N, P).  Rows per block B makes blocks of at
 // least 256 threads for short lines.
@@ -17,9 +17,15 @@ struct RowCfg {
   static constexpr int NT = T * B;
 };
 
-// The launch of `rows` lines: as few lines per workgroup (RowCfg::B at most)
-// as leave no more than one workgroup per CU, so that a few short lines spread
-// over the chip instead of sharing a CU.
+// The launch of `rows` lines.  Lines share a workgroup (RowCfg::B at most) once
+// there are more than four workgroups per CU, so that few lines spread over the
+// chip; below that as many as fill a wave, whose threads a workgroup has anyway.
+// One line a workgroup up to one per CU and packed from there / so, fastconv, us:
+// 600 x 2560 16.5 / 13.8, 1300 x 1280 12.4 / 11.2, 3000 x 576 11.9 / 10.5, 1000 x
+// 576 5.9 / 5.3; 256 lines of 2 points 2.8 / 2.2, 16 2.5 / 2.4, 72 3.4 / 3.1, 160
+// 5.5 / 5.0.  One-thread lines of more than 16 points wait for each other's LDS
+// banks in a wave: theirs is spread as far as it goes (256 x 24 3.0 us, a full
+// wave 3.4; 256 x 40 4.0 and 5.4).
 template <int N, int P>
 struct RowLaunch {
   dim3 grid, block;
@@ -27,7 +33,10 @@ struct RowLaunch {
   explicit RowLaunch(long rows)
   {
     using C = RowCfg<N, P>;
-    const long b = std::min<long>(C::B, std::max<long>((rows + kRowSpread - 1) / kRowSpread, 1));
+    constexpr bool ALONE = C::T == 1 && N > 16;
+    constexpr long spread = ALONE ? kRowCus : 4 * kRowCus, least = ALONE || C::T > 64 ? 1 : 64 / C::T;
+    const long packed = std::max<long>((rows + spread - 1) / spread, least);
+    const long b = std::max<long>(std::min({ (long)C::B, packed, rows }), 1);
     grid = dim3((unsigned)((rows + b - 1) / b));
     block = dim3((unsigned)(b * C::T));
     lds = C::B == 1 ? 0 : (unsigned)(b * Engine<N, P>::LROW * sizeof(float2));

@@ -266,7 +266,7 @@ int row_pick(int n, long rows)
   for (int v = 1; const Entry *e = find_entry(n, v); ++v) {
     const int threads = n / e->p;
     const long per_cu = threads <= 64 ? 8 : threads <= 128 ? 1 : threads <= 256 ? 4 : 0;
-    if (e->p < first->p && rows <= per_cu * kRowSpread) return v;
+    if (e->p < first->p && rows <= per_cu * kRowCus) return v;
   }
   return 0;
 }
