@@ -767,11 +767,11 @@ static int variant_of(unsigned flags, long n = 0, long rows = 0)
 // 10.3 / 10.0 and 12.0 / 10.0, 16384 18.2 / 17.0 and 20.6 / 16.9 us; 1000 rows
 // of 16384 68.9 / 64.0 and 78.4 / 63.9 us).  The autotuner times fastconv, so
 // its choice is not asked here.
-static int fft_variant_of(unsigned flags, long n, long rows)
+static int fft_variant_of(unsigned flags, long n, long rows, bool plain)
 {
   if ((flags >> 8) & 0xffu) return variant_of(flags);
   if (n < 1 || n > kMaxRowN) return 0;
-  return LineFFT::row_variant(n, row_pick((int)n, rows));
+  return LineFFT::row_variant(n, row_pick((int)n, rows, plain));
 }
 
 extern "C" int ovx_supported_length(long n)
@@ -801,7 +801,7 @@ extern "C" int ovx_fftm_plan_create(ovx_plan *plan, long rows, long cols, int ax
   p->flags = flags;
   long n = axis == OVX_ROW ? cols : rows;
   if (n > 0) {
-    int st = p->line.init(n, fft_variant_of(flags, n, axis == OVX_ROW ? rows : cols));
+    int st = p->line.init(n, fft_variant_of(flags, n, axis == OVX_ROW ? rows : cols, true));
     if (st) return st;
   }
   *plan = p.release();
@@ -907,7 +907,7 @@ extern "C" int ovx_fftm_real_plan_create(ovx_plan *plan, long rows, long cols, i
     const long h = n / 2;
     // the one-pass real kernels are built on the register-Stockham
     // configurations
-    int st = p->line.init(h, fft_variant_of(flags, h, axis == OVX_ROW ? rows : cols));
+    int st = p->line.init(h, fft_variant_of(flags, h, axis == OVX_ROW ? rows : cols, false));
     if (st) return st;
     if ((st = p->wtab.alloc((size_t)(h / 2 + 1) * 8))) return st;
     hipError_t e = launch_unit_roots(n, h / 2 + 1, (float2 *)p->wtab.p, nullptr);

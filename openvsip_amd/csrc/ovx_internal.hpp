@@ -27,7 +27,8 @@ bool row_config(int n, int variant, RowConfig *out);
 // The configuration with p values per thread: its index, or -1.
 int row_config_with(int n, int p);
 // The configuration a transform or fastconv of `rows` lines runs by default.
-int row_pick(int n, long rows);
+// plain: a transform of complex lines.
+int row_pick(int n, long rows, bool plain = false);
 // Largest length with an LDS-resident configuration.
 constexpr int kMaxRowN = 16384;
 

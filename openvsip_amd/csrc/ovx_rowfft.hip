@@ -259,13 +259,15 @@ int row_config_with(int n, int p)
 // 8.9 / 8.8; 1024, 256 4.8 / 4.4, 400 5.2 / 5.3, 1000 6.2 / 6.4; 1536, 256 6.8 / 6.8
 // (64 7.3 / 6.7), 400 7.4 / 8.2; 2048, 256 6.8 / 5.3, 600 9.6 / 8.4, 1000 11.2 / 11.0
 // (a spectrum per line 13.7 / 11.1), 2000 17.3 / 18.3; 6144, 400 15.9 / 18.3.
-int row_pick(int n, long rows)
+// Plain transforms of 256 threads a line cross over sooner: 2048, 700 6.5 / 6.3,
+// 800 7.1 / 7.75 (in place 8.2 / 8.9), 900 7.7 / 7.9, 1000 8.0 / 8.0.
+int row_pick(int n, long rows, bool plain)
 {
   const Entry *first = find_entry(n, 0);
   if (!first) return 0;
   for (int v = 1; const Entry *e = find_entry(n, v); ++v) {
     const int threads = n / e->p;
-    const long per_cu = threads <= 64 ? 8 : threads <= 128 ? 1 : threads <= 256 ? 4 : 0;
+    const long per_cu = threads <= 64 ? 8 : threads <= 128 ? 1 : threads <= 256 ? (plain ? 3 : 4) : 0;
     if (e->p < first->p && rows <= per_cu * kRowCus) return v;
   }
   return 0;
