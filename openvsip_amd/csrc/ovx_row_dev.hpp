@@ -105,12 +105,12 @@ __device__ __forceinline__ void row_fft_io(const IX &ix, const IY &iy, long rows
   }
 }
 
-template <int N, int P, int DIR, typename LP>
+template <int N, int P, int DIR, bool NTL = false, typename LP>
 __device__ __forceinline__ void row_fft_body(const float2 *__restrict__ in, long ld_in, float2 *__restrict__ out,
                                              long ld_out, long rows, const float2 *__restrict__ tw, float scale,
                                              long row0, int lrow, int t, LP lds)
 {
-  row_fft_io<N, P, DIR>(IoC{make_rsrc(in + row0 * ld_in, 0xffffffffu), (uint32_t)(lrow * ld_in + t) * 8u},
+  row_fft_io<N, P, DIR>(IoCx<NTL>{make_rsrc(in + row0 * ld_in, 0xffffffffu), (uint32_t)(lrow * ld_in + t) * 8u},
                         IoC{make_rsrc(out + row0 * ld_out, 0xffffffffu), (uint32_t)(lrow * ld_out + t) * 8u}, rows,
                         tw, scale, row0, lrow, t, lds);
 }

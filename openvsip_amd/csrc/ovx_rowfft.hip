@@ -13,13 +13,13 @@
 
 namespace ovx {
 
-template <int N, int P, int DIR>
+template <int N, int P, int DIR, bool NTL>
 __global__ __launch_bounds__((RowCfg<N, P>::NT)) void k_row_fft(const float2 *__restrict__ in, long ld_in,
                                                                float2 *__restrict__ out, long ld_out, long rows,
                                                                const float2 *__restrict__ tw, float scale)
 {
   const RowPlace<N, P> r;
-  row_fft_body<N, P, DIR>(in, ld_in, out, ld_out, rows, tw, scale, r.row0, r.lrow, r.t, r.lds);
+  row_fft_body<N, P, DIR, NTL>(in, ld_in, out, ld_out, rows, tw, scale, r.row0, r.lrow, r.t, r.lds);
 }
 
 template <int N, int P>
@@ -152,16 +152,39 @@ static void fill_cfg(RowConfig *c, int variant)
   c->variant = variant;
 }
 
+// Whether a transform loads its lines past the caches.  In place the result
+// follows the line into its cache lines, and while all of them are in the 32 MB
+// of L2, or too many for the Infinity Cache, the load is better not kept.
+// Ordinary / non-temporal loads, in place, us: 4000 x 512 8.6 / 7.9, 2000 x 1024
+// 8.9 / 7.5, 1000 x 2048 9.8 / 8.3, 1000 x 3072 12.6 / 10.8, 600 x 6144 15.5 /
+// 14.2; between, 4000 x 1024 13.2 / 14.5, 1000 x 4096 14.2 / 15.6, 1000 x 6144 22.6 /
+// 23.2; 4000 x 4096 57.1 / 53.8, 1000 x 16384 68.9 / 66.0; from 8192 points on, a
+// line a CU, ordinary ones stay ahead, 300 x 8192 13.8 / 14.4.  Out of place:
+// 2000 x 2048 12.3 / 15.6, 1000 x 4096 12.1 / 16.1.
+static bool row_streams_in(const float2 *in, const float2 *out, long rows, int n)
+{
+  const long bytes = rows * n * (long)sizeof(float2);
+  return in == out && ((n < 8192 && bytes <= (30l << 20)) || bytes >= (120l << 20));
+}
+
+template <int N, int P, int DIR>
+static hipError_t do_fft_dir(const float2 *in, long ld_in, float2 *out, long ld_out, long rows, const float2 *tw,
+                             float scale, hipStream_t s)
+{
+  const RowLaunch<N, P> l(rows);
+  if (row_streams_in(in, out, rows, N))
+    hipLaunchKernelGGL((k_row_fft<N, P, DIR, true>), l.grid, l.block, l.lds, s, in, ld_in, out, ld_out, rows, tw, scale);
+  else
+    hipLaunchKernelGGL((k_row_fft<N, P, DIR, false>), l.grid, l.block, l.lds, s, in, ld_in, out, ld_out, rows, tw, scale);
+  return hipGetLastError();
+}
+
 template <int N, int P>
 static hipError_t do_fft(int dir, const float2 *in, long ld_in, float2 *out, long ld_out, long rows,
                          const float2 *tw, float scale, hipStream_t s)
 {
-  const RowLaunch<N, P> l(rows);
-  if (dir < 0)
-    hipLaunchKernelGGL((k_row_fft<N, P, -1>), l.grid, l.block, l.lds, s, in, ld_in, out, ld_out, rows, tw, scale);
-  else
-    hipLaunchKernelGGL((k_row_fft<N, P, +1>), l.grid, l.block, l.lds, s, in, ld_in, out, ld_out, rows, tw, scale);
-  return hipGetLastError();
+  return dir < 0 ? do_fft_dir<N, P, -1>(in, ld_in, out, ld_out, rows, tw, scale, s)
+                 : do_fft_dir<N, P, +1>(in, ld_in, out, ld_out, rows, tw, scale, s);
 }
 
 template <int N, int P>
