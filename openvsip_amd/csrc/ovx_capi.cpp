@@ -294,6 +294,7 @@ int LineFFT::transform_ws(int dir, const float2 *in, long ld_in, float2 *out, lo
     a.ld_out = ld_out;
     a.scale = scale;
     a.reread = reread;
+    a.in_place = fs_keeps_in_place(in, out, (size_t)lines * (size_t)n * sizeof(float2));
     e = launch_fs_row(dir, a, lines, s);
     if (e != hipSuccess) return hip_fail(e, "four-step row pass");
     return OVX_OK;

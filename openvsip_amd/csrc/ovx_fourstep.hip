@@ -170,6 +170,7 @@ static hipError_t row_launch(const FsArgs &a, long rows, hipStream_t s)
                                   : row_launch_c<L, DIR, 32, true>(a, rows, s);
   const long bytes = rows * a.nbig * 8;
   const bool whole = fs_whole_lines(a.out, a.ld_out, rows);
+  if (a.in_place && whole) return row_launch_c<L, DIR, 8, false, true>(a, rows, s);
   if (a.reread || !whole)
     return rows * a.n1 < (whole ? 320 : 144) * 16 ? row_launch_c<L, DIR, 8, false, true>(a, rows, s)
                                   : row_launch_c<L, DIR, FsCfg<L>::C, false, true>(a, rows, s);

@@ -30,8 +30,10 @@ struct FsArgs {
   // interleaved column pass: non-temporal loads (forward) or loads and stores
   // (inverse), see fs_streams_in / fs_streams_out
   bool stream = false;
-  // row pass: the result is read again in this call
+  // row pass: the result is read again in this call; it takes the input's place
+  // and is stored the ordinary way (fs_keeps_in_place)
   bool reread = false;
+  bool in_place = false;
   // row and middle passes: each row on the XCD of its column pass
   // (fs_stays_in_l2)
   bool placed = false;
@@ -69,6 +71,17 @@ inline bool fs_whole_lines(const float2 *p, long ld, long rows)
 // 256 x 65536 127 / 124 / 120 / 120; at 32 MB 41 / 43 / 48 / 49.
 inline bool fs_streams_in(size_t bytes) { return bytes >= ((size_t)64 << 20); }
 inline bool fs_streams_out(size_t bytes) { return bytes >= ((size_t)96 << 20); }
+
+// Whether the result of a transform in place is stored the ordinary way: the
+// column pass has left the lines it replaces in the caches.  Non-temporal /
+// ordinary stores, in place, us: 128 x 32768 29.7 / 26.7, 64 x 65536 30.5 / 27.5, 32
+// x 131072 31.8 / 30.1, 20 x 262144 39.0 / 37.3, 12 x 524288 47.9 / 47.2, 6 x
+// 1048576 56.2 / 52.4, 4 x 2097152 75.8 / 71.4; fewer or more rows, 64 x 32768
+// 16.8 / 17.8, 32 x 65536 17.4 / 18.1, 256 x 65536 88 / 93.
+inline bool fs_keeps_in_place(const void *in, const void *out, size_t bytes)
+{
+  return in == out && bytes >= ((size_t)20 << 20) && bytes <= ((size_t)64 << 20);
+}
 
 // Whether the middle pass reads spectra in natural order itself, or
 // launch_fs_permute lays them out first.  The C neighbouring lines of a
