@@ -159,12 +159,13 @@ static void fill_cfg(RowConfig *c, int variant)
 // 8.9 / 7.5, 1000 x 2048 9.8 / 8.3, 1000 x 3072 12.6 / 10.8, 600 x 6144 15.5 /
 // 14.2; between, 4000 x 1024 13.2 / 14.5, 1000 x 4096 14.2 / 15.6, 1000 x 6144 22.6 /
 // 23.2; 4000 x 4096 57.1 / 53.8, 1000 x 16384 68.9 / 66.0; from 8192 points on, a
-// line a CU, ordinary ones stay ahead, 300 x 8192 13.8 / 14.4.  Out of place:
-// 2000 x 2048 12.3 / 15.6, 1000 x 4096 12.1 / 16.1.
+// line a CU, ordinary ones stay ahead, 300 x 8192 13.8 / 14.4, and for lines of a
+// thread or a few, whose loads of a wave lie apart, 256 x 18 3.2 / 3.5, 4000 x 12
+// 2.5 / 2.8.  Out of place: 2000 x 2048 12.3 / 15.6, 1000 x 4096 12.1 / 16.1.
 static bool row_streams_in(const float2 *in, const float2 *out, long rows, int n)
 {
   const long bytes = rows * n * (long)sizeof(float2);
-  return in == out && ((n < 8192 && bytes <= (30l << 20)) || bytes >= (120l << 20));
+  return in == out && n >= 256 && ((n < 8192 && bytes <= (30l << 20)) || bytes >= (120l << 20));
 }
 
 template <int N, int P, int DIR>

@@ -6,7 +6,7 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("n,rows", [(64, 100), (1024, 3840), (1024, 3841), (6144, 640), (6144, 641), (8192, 20),
+@pytest.mark.parametrize("n,rows", [(64, 100), (192, 300), (256, 300), (1024, 3840), (1024, 3841), (6144, 640), (6144, 641), (8192, 20),
                                     (2048, 7679), (2048, 7680), (16384, 959), (16384, 960), (65536, 39),
                                     (65536, 40), (131072, 64), (131072, 65), (262144, 10), (1 << 20, 3), (1 << 21, 4)])
 @pytest.mark.parametrize("inverse", [False, True])
