@@ -240,7 +240,7 @@ bool offsets_fit(long rows_per_block, long ld)
 }
 
 int LineFFT::transform(int dir, const float2 *in, long ld_in, float2 *out, long ld_out, long lines, float scale,
-                       hipStream_t s, bool reread) const
+                       hipStream_t s, Around around) const
 {
   if (lines <= 0) return OVX_OK;
   if (!tables_ready()) return fail(OVX_ERR_STATE, "transform plan has no twiddle tables");
@@ -268,13 +268,13 @@ int LineFFT::transform(int dir, const float2 *in, long ld_in, float2 *out, long 
   if (kind == FOURSTEP) {
     int st = work.alloc((size_t)lines * n * 8);
     if (st) return st;
-    return transform_ws(dir, in, ld_in, out, ld_out, lines, scale, (float2 *)work.p, s, reread);
+    return transform_ws(dir, in, ld_in, out, ld_out, lines, scale, (float2 *)work.p, s, around);
   }
   return fail(OVX_ERR_UNSUPPORTED, "no transform path");
 }
 
 int LineFFT::transform_ws(int dir, const float2 *in, long ld_in, float2 *out, long ld_out, long lines, float scale,
-                          float2 *ws, hipStream_t s, bool reread) const
+                          float2 *ws, hipStream_t s, Around around) const
 {
   if (kind != FOURSTEP) return transform(dir, in, ld_in, out, ld_out, lines, scale, s);
   if (lines <= 0) return OVX_OK;
@@ -293,8 +293,8 @@ int LineFFT::transform_ws(int dir, const float2 *in, long ld_in, float2 *out, lo
     a.out = out;
     a.ld_out = ld_out;
     a.scale = scale;
-    a.reread = reread;
-    a.in_place = fs_keeps_in_place(in, out, (size_t)lines * (size_t)n * sizeof(float2));
+    a.reread = around == READ_AFTER;
+    a.in_place = around == ALONE && fs_keeps_in_place(in, out, (size_t)lines * (size_t)n * sizeof(float2));
     e = launch_fs_row(dir, a, lines, s);
     if (e != hipSuccess) return hip_fail(e, "four-step row pass");
     return OVX_OK;
@@ -999,7 +999,8 @@ static int real_run(ovx_plan p, const RealLines &g, const void *din, void *dout,
   if (p->line.kind == LineFFT::LDS)
     return g.fwd ? real_fused(p, g, din, dout, nullptr, nullptr, s) : real_fused(p, g, dout, din, nullptr, nullptr, s);
   if (g.fwd) {
-    int r = p->line.transform(-1, (const float2 *)din, g.ldz, (float2 *)dout, ldc, g.lines, 1.0f, s, true);
+    int r = p->line.transform(-1, (const float2 *)din, g.ldz, (float2 *)dout, ldc, g.lines, 1.0f, s,
+                              LineFFT::READ_AFTER);
     if (r) return r;
     hipError_t e = launch_r2c_post((float2 *)dout, ldc, g.lines, g.h, (const float2 *)p->wtab.p, p->scale, s);
     return e == hipSuccess ? OVX_OK : hip_fail(e, "r2c pass");
@@ -1007,7 +1008,8 @@ static int real_run(ovx_plan p, const RealLines &g, const void *din, void *dout,
   hipError_t e = launch_c2r_pre((const float2 *)din, ldc, (float2 *)dout, g.ldz, g.lines, g.h,
                                 (const float2 *)p->wtab.p, s);
   if (e != hipSuccess) return hip_fail(e, "c2r pass");
-  return p->line.transform(+1, (const float2 *)dout, g.ldz, (float2 *)dout, g.ldz, g.lines, p->scale, s);
+  return p->line.transform(+1, (const float2 *)dout, g.ldz, (float2 *)dout, g.ldz, g.lines, p->scale, s,
+                           LineFFT::WRITTEN_BEFORE);
 }
 
 extern "C" int ovx_fftm_real_out_of_place(ovx_plan p, const void *in, long in_s0, long in_s1, void *out, long out_s0,
@@ -1255,7 +1257,7 @@ static int fftm_split_exec(ovx_plan p, const void *in_re, const void *in_im, lon
     float2 *ws = (float2 *)p->split_ws.p;
     hipError_t e = launch_interleave(a.re, a.im, ldi, ws, n, lines, n, s);
     if (e != hipSuccess) return hip_fail(e, "interleave");
-    if ((r = p->line.transform(dir, ws, n, ws, n, lines, p->scale, s))) return r;
+    if ((r = p->line.transform(dir, ws, n, ws, n, lines, p->scale, s, LineFFT::WRITTEN_BEFORE))) return r;
     e = launch_deinterleave(ws, n, b.re, b.im, ldo, lines, n, s);
     return e == hipSuccess ? OVX_OK : hip_fail(e, "deinterleave");
   };
@@ -1379,7 +1381,8 @@ extern "C" int ovx_fftm_r2c_split(ovx_plan p, const void *in, long in_s0, long i
     int r = p->split_ws.alloc((size_t)g.lines * hc * 8);
     if (r) return r;
     float2 *ws = (float2 *)p->split_ws.p;
-    if ((r = p->line.transform(-1, (const float2 *)din, g.ldz, ws, hc, g.lines, 1.0f, s, true))) return r;
+    if ((r = p->line.transform(-1, (const float2 *)din, g.ldz, ws, hc, g.lines, 1.0f, s,
+                              LineFFT::READ_AFTER))) return r;
     hipError_t e = launch_r2c_post_split(ws, hc, o.re, o.im, g.ldc, g.lines, g.h, (const float2 *)p->wtab.p,
                                          p->scale, s);
     return e == hipSuccess ? OVX_OK : hip_fail(e, "r2c pass");
@@ -1418,7 +1421,8 @@ extern "C" int ovx_fftm_c2r_split(ovx_plan p, const void *in_re, const void *in_
     hipError_t e = launch_c2r_pre_split(i.re, i.im, g.ldc, (float2 *)dout, g.ldz, g.lines, g.h,
                                         (const float2 *)p->wtab.p, s);
     if (e != hipSuccess) return hip_fail(e, "c2r pass");
-    return p->line.transform(+1, (const float2 *)dout, g.ldz, (float2 *)dout, g.ldz, g.lines, p->scale, s);
+    return p->line.transform(+1, (const float2 *)dout, g.ldz, (float2 *)dout, g.ldz, g.lines, p->scale, s,
+                           LineFFT::WRITTEN_BEFORE);
   };
   if (!host) return run({(const float *)in_re, (const float *)in_im}, out);
   const HostLines gr = host_lines(g.lines, g.ldr, g.n, 4), gc = host_lines(g.lines, g.ldc, hc, 4);

@@ -72,8 +72,11 @@ inline bool fs_whole_lines(const float2 *p, long ld, long rows)
 inline bool fs_streams_in(size_t bytes) { return bytes >= ((size_t)64 << 20); }
 inline bool fs_streams_out(size_t bytes) { return bytes >= ((size_t)96 << 20); }
 
-// Whether the result of a transform in place is stored the ordinary way: the
-// column pass has left the lines it replaces in the caches.  Non-temporal /
+// Whether the result of a transform in place of a caller's data is stored the
+// ordinary way: the column pass has left the lines it replaces in the caches
+// (where the call itself has just written them, before a real inverse transform,
+// it is the slower way: 24 x 524288 real values 59.4 / 64.5, 48 x 262144 54.4 /
+// 58.8).  Non-temporal /
 // ordinary stores, in place, us: 128 x 32768 29.7 / 26.7, 64 x 65536 30.5 / 27.5, 32
 // x 131072 31.8 / 30.1, 20 x 262144 39.0 / 37.3, 12 x 524288 47.9 / 47.2, 6 x
 // 1048576 56.2 / 52.4, 4 x 2097152 75.8 / 71.4; fewer or more rows, 64 x 32768

@@ -62,13 +62,15 @@ struct LineFFT {
   const char *name() const;
   size_t device_bytes() const;
   // lines x n at line strides ld_in / ld_out; dir = -1 forward, +1 inverse
-  // (reread: this call's next kernel reads the result)
+  // (around: whether another kernel of the call wrote the input or reads the
+  // result)
+  enum Around { ALONE, WRITTEN_BEFORE, READ_AFTER };
   int transform(int dir, const float2 *in, long ld_in, float2 *out, long ld_out, long lines, float scale,
-                hipStream_t s, bool reread = false) const;
+                hipStream_t s, Around around = ALONE) const;
   // same, with a caller-provided four-step workspace of lines * n elements
   // (so that concurrent callers of one path do not share `work`)
   int transform_ws(int dir, const float2 *in, long ld_in, float2 *out, long ld_out, long lines, float scale,
-                   float2 *ws, hipStream_t s, bool reread = false) const;
+                   float2 *ws, hipStream_t s, Around around = ALONE) const;
   int fastconv(const float2 *x, long ldx, const float2 *w, long ldw, float2 *y, long ldy, long lines, float scale,
                hipStream_t s, const ExtScratch *ext = nullptr) const;
   bool rows_fastconv(long ldw, long lines) const;
