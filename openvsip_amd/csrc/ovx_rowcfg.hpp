@@ -23,9 +23,9 @@ struct RowCfg {
 // One line a workgroup up to one per CU and packed from there / so, fastconv, us:
 // 600 x 2560 16.5 / 13.8, 1300 x 1280 12.4 / 11.2, 3000 x 576 11.9 / 10.5, 1000 x
 // 576 5.9 / 5.3; 256 lines of 2 points 2.8 / 2.2, 16 2.5 / 2.4, 72 3.4 / 3.1, 160
-// 5.5 / 5.0.  One-thread lines of more than 16 points wait for each other's LDS
-// banks in a wave: theirs is spread as far as it goes (256 x 24 3.0 us, a full
-// wave 3.4; 256 x 40 4.0 and 5.4).
+// 5.5 / 5.0.  One-thread lines wait for each other's LDS banks in a wave: up to 16
+// points they fill half of one (4000 x 12 2.57 us, a whole one 2.72), beyond they
+// spread as far as they go (256 x 24 3.0, a whole wave 3.4; 256 x 40 4.0 and 5.4).
 template <int N, int P>
 struct RowLaunch {
   dim3 grid, block;
@@ -34,7 +34,7 @@ struct RowLaunch {
   {
     using C = RowCfg<N, P>;
     constexpr bool ALONE = C::T == 1 && N > 16;
-    constexpr long spread = ALONE ? kRowCus : 4 * kRowCus, least = ALONE || C::T > 64 ? 1 : 64 / C::T;
+    constexpr long spread = ALONE ? kRowCus : 4 * kRowCus, least = ALONE || C::T > 64 ? 1 : C::T == 1 ? 32 : 64 / C::T;
     const long packed = std::max<long>((rows + spread - 1) / spread, least);
     const long b = std::max<long>(std::min({ (long)C::B, packed, rows }), 1);
     grid = dim3((unsigned)((rows + b - 1) / b));

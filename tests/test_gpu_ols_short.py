@@ -52,7 +52,7 @@ def test_segments_that_share_a_wave(ovx, m, length, segments, more):
 
 
 @pytest.mark.parametrize("m,n", [(8, 700000), (33, 1100000)])
-def test_reference_in_a_launch_of_its_own(ovx, m, n):
+def test_reference_in_many_segments(ovx, m, n):
     import torch
     rng = np.random.default_rng(m)
     ref, x = cg(rng, m), cg(rng, n)
