@@ -11,6 +11,7 @@
 // A = X[k] + conj X[h-k], C = W^-k (X[k] - conj X[h-k]), then
 // z = IFFT_h(Z) holds x[2m] + i x[2m+1].
 #include "ovx_fs_dev.hpp"
+#include "ovx_pair_dev.hpp"
 #include "ovx_real.hpp"
 
 namespace ovx {
@@ -38,24 +39,6 @@ struct SLine {
     im[k] = v.y;
   }
 };
-
-// The pair (k, h - k) of Z in the row becomes that of X; k = 0 takes Z[0] twice.
-__device__ __forceinline__ void r2c_pair(float2 zk, float2 zm, float2 w, float scale, float2 &xk, float2 &xm)
-{
-  const float2 e = make_float2(0.5f * (zk.x + zm.x), 0.5f * (zk.y - zm.y));
-  const float2 o = make_float2(0.5f * (zk.y + zm.y), -0.5f * (zk.x - zm.x));
-  const float2 wo = cmul(w, o);
-  xk = cscale(cadd(e, wo), scale);
-  const float2 d = csub(e, wo);
-  xm = cscale(make_float2(d.x, -d.y), scale);
-}
-__device__ __forceinline__ void c2r_pair(float2 xk, float2 xm, float2 w, float2 &zk, float2 &zm)
-{
-  const float2 a = make_float2(xk.x + xm.x, xk.y - xm.y);            // X[k] + conj X[h-k]
-  const float2 c = cmulc(make_float2(xk.x - xm.x, xk.y + xm.y), w);  // W^-k (X[k] - conj X[h-k])
-  zk = make_float2(a.x - c.y, a.y + c.x);                            // A + i C
-  zm = make_float2(a.x + c.y, c.x - a.y);                            // conj(A - i C)
-}
 
 template <int kPairs, typename Out>
 __device__ __forceinline__ void r2c_row(const float2 *z, const Out out, long group, long h,

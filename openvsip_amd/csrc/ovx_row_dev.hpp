@@ -3,6 +3,7 @@
 // persistent batch kernel.
 #pragma once
 #include "ovx_internal.hpp"
+#include "ovx_pair_dev.hpp"
 
 namespace ovx {
 
@@ -120,25 +121,9 @@ __device__ __forceinline__ void row_fft_body(const float2 *__restrict__ in, long
 // and W = e^{-2 pi i/n} its spectrum is, for k = 0 .. N/2,
 //   X[k] = E + W^k O,  X[N-k] = conj(E - W^k O),
 //   E = (Z[k] + conj Z[N-k]) / 2,  O = -i (Z[k] - conj Z[N-k]) / 2
-// (Z[N] standing for Z[0]).  r2c_pair gives both from Z[k] and Z[N-k], c2r_pair
+// (Z[N] standing for Z[0]).  r2c_pair (ovx_pair_dev.hpp) gives both from Z[k] and Z[N-k], c2r_pair
 // the way back: Z[k] = A + i C, Z[N-k] = conj(A - i C) with
 // A = X[k] + conj X[N-k], C = W^-k (X[k] - conj X[N-k]).
-__device__ __forceinline__ void r2c_pair(float2 zk, float2 zm, float2 w, float scale, float2 &xk, float2 &xm)
-{
-  const float2 e = make_float2(0.5f * (zk.x + zm.x), 0.5f * (zk.y - zm.y));
-  const float2 o = make_float2(0.5f * (zk.y + zm.y), -0.5f * (zk.x - zm.x));
-  const float2 wo = cmul(w, o);
-  const float2 d = csub(e, wo);
-  xk = cscale(cadd(e, wo), scale);
-  xm = cscale(make_float2(d.x, -d.y), scale);
-}
-__device__ __forceinline__ void c2r_pair(float2 xk, float2 xm, float2 w, float2 &zk, float2 &zm)
-{
-  const float2 a = make_float2(xk.x + xm.x, xk.y - xm.y);
-  const float2 c = cmulc(make_float2(xk.x - xm.x, xk.y + xm.y), w);
-  zk = make_float2(a.x - c.y, a.y + c.x);
-  zm = make_float2(a.x + c.y, c.x - a.y);
-}
 
 // The pairs (k, N-k) of one thread: k = t + T q for q < NQ, so that the thread
 // holds Z[k] itself (slot form) and finds Z[N-k] in another thread's upper
