@@ -362,8 +362,9 @@ int ovx_batch_destroy(ovx_batch batch);
 /* No reference counterpart: serving pulse-compression jobs, standalone
    forward Fftms and correlations as they arrive.  A scheduler thread admits
    queued requests (in arrival order, while their device working sets fit the
-   HBM budget) into a free slot -- a stream with a hipGraph of persistent
-   tile-queue launches captured at creation -- and replays it; requests that
+   HBM budget) into a free slot -- a stream with its own tables and workspace --
+   and launches their tile queues there (the persistent launches and the
+   four-step passes, empty queues left out); requests that
    arrive meanwhile go into the next free slot, so batches overlap on the
    device.  Data pointers are device pointers owned by the caller and must
    stay valid until the request completes, and the replicas and correlation
@@ -378,7 +379,8 @@ typedef struct ovx_server_s *ovx_server;
 typedef struct {
   int slots;          /* batches in flight at once (>= 1)                    */
   int max_jobs;       /* requests per batch                                  */
-  long max_tiles;     /* tile-table capacity per queue (0 = 65536)           */
+  long max_tiles;     /* a batch of several requests takes requests of at
+                         most half as many tiles together (0 = 65536)        */
   long hbm_budget_mb; /* admission budget for request working sets           */
   long workspace_mb;  /* four-step Fftm workspace per slot                   */
   int plain;          /* 1: one standalone launch per request                */

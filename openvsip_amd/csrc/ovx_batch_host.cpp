@@ -134,7 +134,9 @@ hipError_t launch_queue(const TileQueue &q, const BatchJob *jobs, const BatchSpa
   const BatchQueue bq{ jobs, spans, (int)q.spans.size(), q.tiles };
   if (q.line == 0) return launch_batch(bq, std::min(q.tiles, device_cu_count()), s);
   if (q.line == kMidLine) return launch_batch_mid(bq, std::min(q.tiles, kBatchMidBlocksPerCu * device_cu_count()), s);
-  // a chunk's first and last pass access memory as a standalone call's
+  // A chunk's first and last pass go past the caches by its bytes, as a standalone
+  // call's do; rows off the 128-byte lines, which standalone calls then keep in the
+  // caches (fs_whole_lines), are not told apart here.
   const bool stream = q.pass == 0 ? fs_streams_in(q.bytes) : fs_streams_out(q.bytes);
   return launch_batch_fs(q.line, q.pass, stream, bq, s);
 }

@@ -60,6 +60,8 @@ void push_row_tiles(const BatchJob &j, int ji, bool fft, TileQueue &big, TileQue
 // 512 MB, us: 400 rows of 65536 247 / 228 / 230 / 222 / 207 / 212 / 209, 800 rows
 // 467 / 437 / 425 / 422 / 402 / 413 / 431, 2000 rows 1118 / 1050 / 1032 / 1011 /
 // 995 / 1002 / 1072, 240 rows of 262144 567 / 543 / 524 / 532 / 538 / 527 / 563.
+// (224 MB is the fastest on three of the four lists; with 192, 400 rows of 65536
+// stay two chunks, as the tests of a batch's launches count them.)
 constexpr size_t kFsChunkBytes = (size_t)192 << 20;
 // Four-step queues (in launch order) of jobs order[0], order[1], ... that
 // take the four-step path; a job with a workspace is a forward Fftm.

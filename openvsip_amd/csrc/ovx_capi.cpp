@@ -749,7 +749,7 @@ int tuned_variant(long n, long rows);
 }
 
 // Explicit variant from the flags, else the autotuner's cached choice for
-// (n, rows), else the default (variant 0).
+// (n, rows), else the default for them.
 static int variant_of(unsigned flags, long n = 0, long rows = 0)
 {
   int v = (int)((flags >> 8) & 0xffu);

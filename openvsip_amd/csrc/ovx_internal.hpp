@@ -16,7 +16,6 @@ struct RowConfig {
   int p = 0;            // values per thread
   int rows_per_block = 0;
   int threads = 0;      // block size
-  size_t lds_bytes = 0; // static LDS per block
   RadixPlan plan{};
   int variant = 0;      // index among the configurations compiled for n
 };
@@ -46,7 +45,7 @@ hipError_t launch_row_fastconv(const RowConfig &cfg, const float2 *x, long ldx,
                                const float2 *tw, float scale, hipStream_t s);
 
 // The same two on split storage: real and imaginary parts of the lines in
-// two float arrays with the same strides (ld in floats); w stays interleaved.
+// two float arrays with the same strides (ld in floats), the spectra likewise.
 hipError_t launch_row_fft_split(const RowConfig &cfg, int dir, const float *in_re, const float *in_im, long ld_in,
                                 float *out_re, float *out_im, long ld_out, long rows, const float2 *tw, float scale,
                                 hipStream_t s);

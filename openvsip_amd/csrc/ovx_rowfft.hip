@@ -147,7 +147,6 @@ static void fill_cfg(RowConfig *c, int variant)
   c->p = P;
   c->rows_per_block = C::B;
   c->threads = C::NT;
-  c->lds_bytes = (size_t)C::B * Engine<N, P>::LROW * sizeof(float2);
   c->plan = Engine<N, P>::plan;
   c->variant = variant;
 }

@@ -205,7 +205,8 @@ int Server::init(const ovx_server_config &c)
   return OVX_OK;
 }
 
-// Tiles a request needs (to respect the slot's table capacity).
+// Tiles of a request, a four-step one's in its widest transform pass.  They bound a
+// batch (max_tiles / 2), not a table: a slot holds spans.
 static long tiles_of(const Req &q, const LineFFT *f, const CorrRef *cr)
 {
   const ovx_request &r = q.r;
@@ -266,12 +267,7 @@ int Server::admit_and_launch(Slot &s, std::vector<Req *> &batch)
   const size_t job_bytes = jobs.size() * sizeof(BatchJob);
   static_assert(sizeof(BatchJob) % alignof(BatchSpan) == 0, "the spans follow the jobs");
   size_t used = job_bytes;
-  long tiles[kBatchQueues] = { 0 }; // of all chunks together
-  for (const auto &q : queues) {
-    const int k = q.line == 0 ? 0 : q.line == kMidLine ? kMidQueue : fs_queue(q.pass, q.line);
-    if ((tiles[k] += q.tiles) > max_tiles) return fail(OVX_ERR_STATE, "slot tile table overflow");
-    used += q.spans.size() * sizeof(BatchSpan);
-  }
+  for (const auto &q : queues) used += q.spans.size() * sizeof(BatchSpan);
   if (used > table_bytes) return fail(OVX_ERR_STATE, "slot span table overflow");
   std::copy(jobs.begin(), jobs.end(), (BatchJob *)s.h_tab);
   BatchSpan *h = (BatchSpan *)(s.h_tab + job_bytes);
