@@ -193,7 +193,7 @@ template <int L>
 static hipError_t conv_launch(FsArgs a, long rows, hipStream_t s)
 {
   const int groups = (int)(a.n1 / FsConvCfg<L>::C), whole = (int)rows & ~7;
-  a.placed = fs_stays_in_l2(a.nbig, rows);
+  a.placed = fs_stays_in_l2(a.nbig, rows, true);
   const int per = fs_conv_rows(groups * rows, a.placed);
   const long sets = a.placed ? 8l * fs_conv_sets(whole, per) + (rows - whole) : (rows + per - 1) / per;
   const dim3 grid((unsigned)(groups * sets));

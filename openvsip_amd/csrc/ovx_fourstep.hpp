@@ -44,12 +44,17 @@ struct FsArgs {
 // same.  Otherwise its groups go to the XCDs in turn, which suits rows that are
 // not in L2 better.  In turn / on the row's XCD, us: fastconv 256 x 256 lines,
 // 9 rows 16.8 / 14.7, 24 25.9 / 21.7, 40 33.0 / 27.8, 64 38.6 / 36.7, 96 54.0 /
-// 54.2; 256 x 512, 24 rows 35.9 / 31.2; rows of 2 MB and more, of which an L2
-// holds two: 512 x 512, 12 rows 41.3 / 42.5, 24 59 / 64.  Fftm 256 x 256, 24
-// rows 16.5 / 13.3, 256 x 512, 24 rows 22.3 / 21.7.
-inline bool fs_stays_in_l2(long n, long rows)
+// 54.2; 256 x 512, 24 rows 35.9 / 31.2.  Fftm 256 x 256, 24 rows 16.5 / 13.3, 256 x
+// 512, 24 rows 22.3 / 21.7.  Of rows of 2 MB an L2 holds one beside what is being
+// loaded, so eight of them, the middle pass, which works in place, two more: Fftm
+// 512 x 512, 8 rows 20.9 / 20.1, in place 22.7 / 20.9, 9 rows 24.0 / 25.0; fastconv 8
+// rows 37.4 / 31.5, in place 42.5 / 30.1, 9 rows 41.2 / 38.5, 10 40.4 / 39.7, 12 40.8 /
+// 44.2.
+inline bool fs_stays_in_l2(long n, long rows, bool middle = false)
 {
-  return n * 8 <= (1l << 20) && rows * n * 8 <= 8 * (4l << 20);
+  const long row = n * 8, all = rows * row;
+  if (row <= (1l << 20)) return all <= 8 * (4l << 20);
+  return row <= (2l << 20) && rows >= 8 && all <= (middle ? 10 : 8) * (2l << 20);
 }
 
 // Whether every row begins on a 128-byte line.  Runs of other rows straddle
