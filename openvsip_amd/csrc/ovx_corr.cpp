@@ -251,7 +251,7 @@ extern "C" int ovx_corr_exec(ovx_plan p, int bias, const void *ref, const void *
   // a reference that the result is written over is read whole by a launch of
   // its own first
   const bool fuse = ols_fuse_ref(c) && !runs_meet(dref, c.M, dout, c.P);
-  const bool copy = !host && ols_copies_meeting(c) && runs_meet(din, c.N, dout, c.P);
+  const bool copy = !host && runs_meet(din, c.N, dout, c.P) && ols_copies_meeting(c);
   const bool scratch = !host && (copy || !fuse);
   if (scratch && (st = order_plan(p, s))) return st;
   if (copy && (st = ols_copy_input(c, din, s))) return st;
@@ -343,7 +343,7 @@ extern "C" int ovx_conv_exec(ovx_plan p, const void *in, void *out, void *stream
     din = (const float2 *)c.in_stage.p;
     dout = (float2 *)c.out_stage.p;
   }
-  const bool copy = !host && ols_copies_meeting(c) && runs_meet(din, c.N, dout, c.P);
+  const bool copy = !host && runs_meet(din, c.N, dout, c.P) && ols_copies_meeting(c);
   if (copy && ((st = order_plan(p, s)) || (st = ols_copy_input(c, din, s)))) return st;
   if ((st = ols_run(c, nullptr, din, dout, 0, 0, s))) return st;
   if (copy) return mark_plan(p, s, OVX_OK);

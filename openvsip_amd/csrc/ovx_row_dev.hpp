@@ -121,8 +121,8 @@ __device__ __forceinline__ void row_fft_body(const float2 *__restrict__ in, long
 // and W = e^{-2 pi i/n} its spectrum is, for k = 0 .. N/2,
 //   X[k] = E + W^k O,  X[N-k] = conj(E - W^k O),
 //   E = (Z[k] + conj Z[N-k]) / 2,  O = -i (Z[k] - conj Z[N-k]) / 2
-// (Z[N] standing for Z[0]).  r2c_pair (ovx_pair_dev.hpp) gives both from Z[k] and Z[N-k], c2r_pair
-// the way back: Z[k] = A + i C, Z[N-k] = conj(A - i C) with
+// (Z[N] standing for Z[0]).  r2c_pair (ovx_pair_dev.hpp) gives both from Z[k] and
+// Z[N-k], c2r_pair the way back: Z[k] = A + i C, Z[N-k] = conj(A - i C) with
 // A = X[k] + conj X[N-k], C = W^-k (X[k] - conj X[N-k]).
 
 // The pairs (k, N-k) of one thread: k = t + T q for q < NQ, so that the thread
